@@ -238,6 +238,29 @@ def lib():
     return _lib
 
 
+_torch_calls = None
+
+
+def torch_calls():
+    """The native module behind the compute calls on torch tensors (``csrc/torch_calls.cpp``), loaded once.  Raises if it
+    has not been built; torch must have been imported."""
+    global _torch_calls
+    if _torch_calls is None:
+        import importlib.machinery
+        import importlib.util
+
+        lib()
+        path = os.path.join(_HERE, "lib", "rpu_torch.so")
+        if not os.path.exists(path):
+            raise RuntimeError(f"{path} is missing: build it with `make -C aihwkit_amd/csrc`.")
+        loader = importlib.machinery.ExtensionFileLoader("rpu_torch", path)
+        spec = importlib.util.spec_from_file_location("rpu_torch", path, loader=loader)
+        module = importlib.util.module_from_spec(spec)
+        loader.exec_module(module)
+        _torch_calls = module
+    return _torch_calls
+
+
 def check(code):
     """Turn a non-zero return code into the RuntimeError the reference's bindings raise."""
     if code != 0:

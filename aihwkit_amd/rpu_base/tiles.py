@@ -11,11 +11,12 @@ argument order is the reference's; it is what its Python callers rely on
 (src/aihwkit/simulator/tiles/periphery.py:1061,1165,1225).
 """
 import ctypes as C
+import struct
 from typing import List
 
 import torch
 
-from .._cabi import MAX_MODIFIER_COEFFS, ModifierParams, RemapParams, check, lib
+from .._cabi import MAX_MODIFIER_COEFFS, ModifierParams, RemapParams, check, lib, torch_calls
 # the reference binds these parameter structs in its tiles module (rpu_base_utils.cpp:17-58)
 from .devices import (WeightClipParameter, WeightClipType, WeightModifierParameter,  # noqa: F401
                       WeightModifierType, WeightRemapParameter, WeightRemapType)
@@ -42,6 +43,8 @@ class _TileBase:
 
     def __init__(self, handle):
         self._h = C.c_void_p(handle)
+        self._x_size = lib().rpu_tile_get_x_size(self._h)
+        self._d_size = lib().rpu_tile_get_d_size(self._h)
 
     def __del__(self):
         handle, self._h = getattr(self, "_h", None), None
@@ -133,10 +136,10 @@ class _TileBase:
 
     # -- sizes / learning rate (rpu_base_tiles.cpp get_x_size, get_d_size, get/set_learning_rate)
     def get_x_size(self) -> int:
-        return lib().rpu_tile_get_x_size(self._h)
+        return self._x_size
 
     def get_d_size(self) -> int:
-        return lib().rpu_tile_get_d_size(self._h)
+        return self._d_size
 
     def get_learning_rate(self) -> float:
         return float(lib().rpu_tile_get_learning_rate(self._h))
@@ -260,7 +263,7 @@ class _CudaTileMixin:
 
     @staticmethod
     def _stream_for(tensor: torch.Tensor):
-        return C.c_void_p(torch.cuda.current_stream(tensor.device).cuda_stream)
+        return torch._C._cuda_getCurrentRawStream(tensor.device.index)
 
     def _finish(self, tensor: torch.Tensor, non_blocking: bool):
         if not non_blocking:
@@ -280,6 +283,11 @@ class _CudaTileMixin:
     # rpu_base_tiles_cuda.cpp:159-236
     def forward(self, x_input: torch.Tensor, bias: bool = False, x_trans: bool = False, d_trans: bool = False,
                 is_test: bool = False, non_blocking: bool = False) -> torch.Tensor:
+        done = torch_calls().forward(self._h.value, x_input, self._x_size - 1 if bias else self._x_size, self._d_size,
+                                     bias, x_trans, d_trans, is_test, non_blocking)
+        if done is not None:
+            return done
+        # not plain tensors of the right sizes: convert what can be converted, word the errors
         x_input = _check_input(x_input, True, "x_input")
         if x_input.dim() < 1:
             raise RuntimeError("Invalid x_input dimensions: expected at least 1 dimensional tensor")
@@ -299,6 +307,10 @@ class _CudaTileMixin:
     # rpu_base_tiles_cuda.cpp:237-309
     def backward(self, d_input: torch.Tensor, bias: bool = False, d_trans: bool = False, x_trans: bool = False,
                  non_blocking: bool = False) -> torch.Tensor:
+        done = torch_calls().backward(self._h.value, d_input, self._d_size, self._x_size - 1 if bias else self._x_size,
+                                      bias, d_trans, x_trans, False, non_blocking)
+        if done is not None:
+            return done
         d_input = _check_input(d_input, True, "d_input")
         if d_input.dim() < 1:
             raise RuntimeError("Invalid d_input dimensions: expected at least 1 dimensional tensor")
@@ -320,7 +332,8 @@ class _CudaTileMixin:
     # reference (py::arg("d_trans") precedes py::arg("x_trans")); positions are what callers use.
     def update(self, x_input: torch.Tensor, d_input: torch.Tensor, bias: bool, x_trans: bool = False,
                d_trans: bool = False, non_blocking: bool = False) -> None:
-        if self.get_learning_rate() == 0.0:
+        if torch_calls().update(self._h.value, x_input, d_input, self._x_size - 1 if bias else self._x_size, self._d_size,
+                                bias, x_trans, d_trans, self._update_without_allocation, non_blocking):
             return
         d_input = _check_input(d_input, True, "d_input")
         x_input = _check_input(x_input, True, "x_input")
@@ -618,6 +631,8 @@ class TileGroup:
         self._tiles = list(tile_list)
         if not self._tiles:
             raise RuntimeError("empty tile list")
+        # (x_size, d_size) of every tile, for the native calls
+        self._sizes = b"".join(struct.pack("=ii", t.get_x_size(), t.get_d_size()) for t in self._tiles)
         handles = (C.c_void_p * len(self._tiles))(*[t._h for t in self._tiles])
         self._g = C.c_void_p()
         check(lib().rpu_group_create(C.byref(self._g), handles, len(self._tiles)))
@@ -647,6 +662,8 @@ class TileGroup:
         """Stochastic pulsed update of every tile with its own ``x_inputs[i]`` [m_batch, x_size_i] and ``d_inputs[i]``
         [m_batch, d_size_i] (column slices of larger matrices are read in place): what each tile's own ``update`` does,
         in three launches for the whole group."""
+        if torch_calls().group_update(self._g.value, self._sizes, x_inputs, d_inputs, non_blocking):
+            return
         if len(x_inputs) != len(self._tiles) or len(d_inputs) != len(self._tiles):
             raise RuntimeError("one input and one output gradient per tile expected")
         xs = [self._rows(x, "x_input") for x in x_inputs]
@@ -677,6 +694,9 @@ class TileGroup:
     def backward(self, d_inputs, non_blocking: bool = False, outs=None):
         """d_inputs[i]: CUDA tensor [m_batch, d_size_i]; returns the input gradients [m_batch, x_size_i] of every tile
         (``outs``: tensors to fill, e.g. column slices), each what the tile's own ``backward`` gives."""
+        done = torch_calls().group_backward(self._g.value, self._sizes, d_inputs, outs, False, non_blocking)
+        if done is not None:
+            return done
         if len(d_inputs) != len(self._tiles):
             raise RuntimeError("one input per tile expected")
         ds = [self._rows(d, "d_input") for d in d_inputs]
@@ -708,6 +728,9 @@ class TileGroup:
         """x_inputs[i]: CUDA tensor [m_batch, x_size_i] (column slices of one matrix are read in place); returns the
         list of outputs [m_batch, d_size_i].  ``outs`` may give the output tensors, e.g. column slices of one
         [m_batch, out_total] matrix, which the tiles then fill in place."""
+        done = torch_calls().group_forward(self._g.value, self._sizes, x_inputs, outs, is_test, non_blocking)
+        if done is not None:
+            return done
         if len(x_inputs) != len(self._tiles):
             raise RuntimeError("one input per tile expected")
         xs = [self._rows(x, "x_input") for x in x_inputs]
