@@ -292,18 +292,20 @@ struct UpdateArgs {
   int *bl;       // [B] bit-line length per sample
   float *prob_a; // [B] probability scale of d
   float *prob_b; // [B] probability scale of x
-  uint32_t *x_words; // [B][X] packed pulse words
-  uint32_t *d_words; // [B][D]
+  uint32_t *x_words; // [B][X] packed pulse words: written where bit lines are longer than seven pulses, else only their
+  uint32_t *d_words; // [B][D] bit planes (launch_words_from_planes makes them for the inspection hook)
   // bit lines beyond 31 pulses: a sample takes words_per_sample consecutive rows of words (and bit positions in the
   // planes); m_batch then counts those rows, bl / prob_a / prob_b / x / d stay per sample (row r belongs to sample
   // r / words_per_sample and holds its pulse slots 31 (r % words_per_sample) + 1 ..).  0 or 1: one row per sample.
   int words_per_sample;
   // sample-transposed pulse bits: plane (chunk c, slot k) of line element e is the 32-bit word whose bit q
-  // is pulse slot k of sample 32 c + q; element (c, k, e) at planes[(c * plane_slots + k) * size + e];
-  // slot plane_slots - 1 holds the sign bits (bit 0 of the packed words)
+  // is pulse slot k of sample 32 c + q; element (c, k, e) at planes[(c * slots + k) * size + e] with slots = the batch's
+  // longest bit line (kmax[kmax_slot]) + 1; the last slot holds the sign bits (bit 0 of the packed words)
   uint32_t *x_planes;
   uint32_t *d_planes;
-  int plane_slots; // slots per chunk the plane buffers are laid out for
+  // 1: the x lines are kept as 64-bit lane masks instead (bit lines of up to seven pulses): bit l of word
+  // ((row of words * ceil(x_size / 64) + block) * slots + k) is slot k of element 64 block + l, k = slots - 1 its sign
+  int x_lane_masks;
   int n_chunks;    // ceil(m_batch / 32)
   int *row_cost;   // [d_size] work of the pulse loop on each d row of this call (zeroed by the prepare kernel, summed by
                    // the kernel that makes the d pulse trains); null: not kept
@@ -332,6 +334,7 @@ int update_lines_blocks(const UpdateArgs &a, bool wide);
 int update_pulsed_variant(const UpdateArgs &a);
 bool update_reads_row_cost(const UpdateArgs &a); // by its shape: whether the pulse loop of this call looks at row_cost
 int update_pulsed_workgroups(const UpdateArgs &a);
+bool update_takes_stream(const UpdateArgs &a); // by its shape: the call may set x_lane_masks (launch_update_lines, launch_update_pulsed)
 void launch_update_pulsed_group(const UpdateGroup &g, int variant, int total_workgroups, hipStream_t s);
 
 // tables of the update kernels on the current device (once per GPU; blocking copy, no allocation)
@@ -339,6 +342,7 @@ void ensure_update_tables();
 void launch_update_prepare(const UpdateArgs &a, hipStream_t s);       // BL, A, B per sample
 void launch_update_lines(const UpdateArgs &a, hipStream_t s);         // stochastic pulse words and their bit planes
 void launch_update_implicit_lines(const UpdateArgs &a, hipStream_t s); // deterministic line values
+void launch_words_from_planes(const UpdateArgs &a, hipStream_t s);    // x_words / d_words of an update that kept bit planes only
 void launch_update_planes(const UpdateArgs &a, hipStream_t s);        // bit planes of pulse words made elsewhere
 void launch_words_kmax(const UpdateArgs &a, hipStream_t s);           // a.kmax[a.kmax_slot] = longest bit line among such words
 void launch_update_pulsed(const UpdateArgs &a, hipStream_t s);        // coincidences + device steps

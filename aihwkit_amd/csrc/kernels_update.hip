@@ -231,6 +231,10 @@ __device__ __forceinline__ float discretize_prob(float pp, float res, int sto_ro
   return rintf(q) * res;
 }
 
+// slots per chunk of the bit planes: those of the batch's longest bit line and the sign bits (known on the device only;
+// fixed at 32 the planes of one-pulse bit lines were spread over sixteen times the memory they fill)
+__device__ __forceinline__ unsigned plane_slots(const UpdateArgs &a) { return (unsigned)a.kmax[a.kmax_slot] + 1u; }
+
 // packed pulse word of line element j (an x line or a d line) for sample b: bit 0 = sign, bits 1..K = pulses;
 // `row` numbers the sample's rows of words (pulse slots 31 row + 1 ..), each with its own uniforms
 __device__ __forceinline__ uint32_t pulse_word(const UpdateArgs &a, bool is_x, int j, int b, float v, float P, int K,
@@ -254,6 +258,9 @@ __device__ __forceinline__ uint32_t pulse_word(const UpdateArgs &a, bool is_x, i
   }
   return word;
 }
+
+// longest bit line of a batch whose packed words are not written: only the loop for longer ones reads them
+constexpr int UPDATE_PLANES_ONLY_KMAX = 7;
 
 // Pulse words and their sample-transposed bit planes in one pass.  A workgroup owns 64 samples x LINES_E line elements
 // (x lines first, then d lines): the values are read 4 LINES_E bytes per sample row into LDS, then each wave takes every
@@ -324,14 +331,15 @@ __device__ __forceinline__ void update_lines_block(const UpdateArgs &a, const in
   const int sample = wps > 1 ? b / wps : b, wrow = wps > 1 ? b - sample * wps : 0;
   const float P = b_ok ? (is_x ? a.prob_b[sample] : a.prob_a[sample]) : 0.0f;
   const int K = b_ok ? min(max(a.bl[sample] - 31 * wrow, 0), 31) : 0;
-  const int kmax = a.kmax[a.kmax_slot];
+  const int kmax = a.kmax[a.kmax_slot], slots = kmax + 1;
+  const bool keep_words = kmax > UPDATE_PLANES_ONLY_KMAX;
   uint32_t *planes = is_x ? a.x_planes : a.d_planes;
   const int c0 = 2 * by;
   for (int el = wave; el < LINES_E; el += 4) {
     const int e = e0 + el;
     if (e >= size) break; // wave-uniform
     const uint32_t word = b_ok ? pulse_word(a, is_x, e, sample, vals[lane][el], P, K, wrow) : 0u;
-    wt[lane][el] = word;
+    if (keep_words) wt[lane][el] = word;
     unsigned long long any = 0ull;
     int passes = 0;
     for (int k = 0; k < kmax; ++k) {
@@ -339,19 +347,19 @@ __device__ __forceinline__ void update_lines_block(const UpdateArgs &a, const in
       any |= m;
       passes += __popcll(m);
       if (lane == 0) {
-        planes[((long)c0 * a.plane_slots + k) * size + e] = (uint32_t)m;
-        if (c0 + 1 < a.n_chunks) planes[((long)(c0 + 1) * a.plane_slots + k) * size + e] = (uint32_t)(m >> 32);
+        planes[((long)c0 * slots + k) * size + e] = (uint32_t)m;
+        if (c0 + 1 < a.n_chunks) planes[((long)(c0 + 1) * slots + k) * size + e] = (uint32_t)(m >> 32);
       }
     }
     // what the pulse loop will spend on this d row for these samples: a pass per pulse, a set-up per sample with pulses
     if (!is_x && a.row_cost && lane == 0 && passes) atomicAdd(&a.row_cost[e], 9 * passes + 4 * __popcll(any));
     const unsigned long long sg = __ballot(word & 1u); // the last slot of a chunk holds the sign bits
     if (lane == 0) {
-      const int ks = a.plane_slots - 1;
-      planes[((long)c0 * a.plane_slots + ks) * size + e] = (uint32_t)sg;
-      if (c0 + 1 < a.n_chunks) planes[((long)(c0 + 1) * a.plane_slots + ks) * size + e] = (uint32_t)(sg >> 32);
+      planes[((long)c0 * slots + kmax) * size + e] = (uint32_t)sg;
+      if (c0 + 1 < a.n_chunks) planes[((long)(c0 + 1) * slots + kmax) * size + e] = (uint32_t)(sg >> 32);
     }
   }
+  if (!keep_words) return; // nothing reads the words of short bit lines: the planes hold them (k_words_from_planes)
   __syncthreads();
   uint32_t *words = is_x ? a.x_words : a.d_words;
 #pragma unroll
@@ -398,6 +406,76 @@ __global__ __launch_bounds__(256) void k_update_lines(UpdateArgs a) {
     return;
   }
   update_lines_block<LINES_E, IN_PLACE>(a, (int)blockIdx.x, (int)blockIdx.y, vals, wt);
+}
+
+// The pulse trains as k_update_pulsed_stream reads them: those of the d lines as bit planes, those of the x lines with a
+// word's bits along 64 elements of one sample instead of along the samples (UpdateArgs::x_lane_masks).  Workgroups of
+// 64 samples x 64 x elements, then 64 samples x 16 d elements; the random numbers are keyed by element and sample, so the
+// pulses are those of k_update_lines.  Bit lines of more than seven pulses leave planes and words as that kernel does.
+template <bool IN_PLACE>
+__global__ __launch_bounds__(256) void k_update_lines_stream(UpdateArgs a) {
+  __shared__ float vals[64][65];
+  __shared__ uint32_t wt[64][17];
+  const int blocks_x = (a.x_size + 63) / 64, blocks_d = (a.d_size + 15) / 16;
+  const int bx = (int)blockIdx.x, by = (int)blockIdx.y;
+  if (bx >= blocks_x + blocks_d) { // only launched with a.wt_src set
+    update_copy_weights(a, blocks_x + blocks_d, reinterpret_cast<float (*)[33]>(&vals[0][0]));
+    return;
+  }
+  const int kmax = a.kmax[a.kmax_slot];
+  float (*narrow)[17] = reinterpret_cast<float (*)[17]>(&vals[0][0]);
+  const int tiles_x = (a.x_size + 15) / 16; // x blocks in update_lines_block's numbering
+  if (bx >= blocks_x) {
+    update_lines_block<16, IN_PLACE>(a, tiles_x + bx - blocks_x, by, narrow, wt);
+    return;
+  }
+  if (kmax > UPDATE_PLANES_ONLY_KMAX) {
+    for (int q = 4 * bx; q < min(4 * bx + 4, tiles_x); ++q) {
+      update_lines_block<16, IN_PLACE>(a, q, by, narrow, wt);
+      __syncthreads();
+    }
+    return;
+  }
+  const int lane = (int)threadIdx.x & 63, wave = (int)threadIdx.x >> 6;
+  const int e0 = bx * 64, b0 = by * 64;
+  const int wps = max(a.words_per_sample, 1);
+  if (IN_PLACE && a.x_index) { // lanes along the patches, as in update_lines_block
+    const int b = b0 + lane;
+    const int sample = wps > 1 ? b / wps : b;
+    const int n = sample / a.x_group;
+    const int *idx = a.x_index_lines + (sample - n * a.x_group);
+    const float *image = a.x + (long)n * a.x_gs - 2;
+    int at[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int e = e0 + wave * 16 + i;
+      at[i] = (b < a.m_batch && e < a.x_size) ? idx[(long)e * a.x_group] : 0;
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) vals[lane][wave * 16 + i] = at[i] <= 1 ? (float)at[i] : image[at[i]];
+  } else {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int b = b0 + wave * 16 + i, e = e0 + lane;
+      const int sample = wps > 1 ? b / wps : b;
+      vals[wave * 16 + i][lane] = (b < a.m_batch && e < a.x_size) ? a.x[(long)sample * a.x_sb + (long)e * a.x_sj] : 0.0f;
+    }
+  }
+  __syncthreads();
+  const int e = e0 + lane;
+  for (int i = 0; i < 16; ++i) {
+    const int b = b0 + wave * 16 + i;
+    if (b >= a.m_batch) break; // wave-uniform
+    const int sample = wps > 1 ? b / wps : b, wrow = wps > 1 ? b - sample * wps : 0;
+    const int K = min(max(a.bl[sample] - 31 * wrow, 0), 31);
+    const uint32_t word = e < a.x_size ? pulse_word(a, true, e, sample, vals[wave * 16 + i][lane], a.prob_b[sample], K, wrow) : 0u;
+    unsigned long long mine = __ballot(word & 1u); // lane kmax keeps the signs
+    for (int k = 0; k < kmax; ++k) {
+      const unsigned long long m = __ballot((word >> (k + 1)) & 1u);
+      mine = lane == k ? m : mine;
+    }
+    if (lane <= kmax) reinterpret_cast<unsigned long long *>(a.x_planes)[((long)b * blocks_x + bx) * (kmax + 1) + lane] = mine;
+  }
 }
 
 // Several tiles in one launch: start[t] .. start[t + 1] are the element blocks of tile t.
@@ -577,21 +655,45 @@ __global__ __launch_bounds__(256) void k_update_planes(UpdateArgs a) {
   uint32_t *planes = is_x ? a.x_planes : a.d_planes;
   const int b = sb * 64 + lane;
   const uint32_t word = (b < a.m_batch) ? words[(long)b * size + el] : 0u;
-  const int kmax = a.kmax[a.kmax_slot];
+  const int kmax = a.kmax[a.kmax_slot], slots = kmax + 1;
   const int c0 = 2 * sb;
   for (int k = 0; k < kmax; ++k) {
     const unsigned long long m = __ballot((word >> (k + 1)) & 1u);
     if (lane == 0) {
-      planes[((long)c0 * a.plane_slots + k) * size + el] = (uint32_t)m;
-      if (c0 + 1 < a.n_chunks) planes[((long)(c0 + 1) * a.plane_slots + k) * size + el] = (uint32_t)(m >> 32);
+      planes[((long)c0 * slots + k) * size + el] = (uint32_t)m;
+      if (c0 + 1 < a.n_chunks) planes[((long)(c0 + 1) * slots + k) * size + el] = (uint32_t)(m >> 32);
     }
   }
   // the last slot of a chunk holds the sign bits of its samples
   const unsigned long long sg = __ballot(word & 1u);
   if (lane == 0) {
-    const int ks = a.plane_slots - 1;
-    planes[((long)c0 * a.plane_slots + ks) * size + el] = (uint32_t)sg;
-    if (c0 + 1 < a.n_chunks) planes[((long)(c0 + 1) * a.plane_slots + ks) * size + el] = (uint32_t)(sg >> 32);
+    planes[((long)c0 * slots + kmax) * size + el] = (uint32_t)sg;
+    if (c0 + 1 < a.n_chunks) planes[((long)(c0 + 1) * slots + kmax) * size + el] = (uint32_t)(sg >> 32);
+  }
+}
+
+// The packed words of the last update from its bit planes, for the inspection hook (bit lines that are longer left the
+// words themselves).
+__global__ __launch_bounds__(256) void k_words_from_planes(UpdateArgs a) {
+  const int kmax = a.kmax[a.kmax_slot];
+  if (kmax > UPDATE_PLANES_ONLY_KMAX) return;
+  const long slots = kmax + 1, per = (long)a.x_size + a.d_size, total = per * a.m_batch;
+  for (long idx = blockIdx.x * 256L + threadIdx.x; idx < total; idx += gridDim.x * 256L) {
+    const int b = (int)(idx / per), el = (int)(idx % per);
+    const bool is_x = el < a.x_size;
+    const int e = is_x ? el : el - a.x_size, size = is_x ? a.x_size : a.d_size;
+    if (is_x && a.x_lane_masks) {
+      const unsigned long long *m = reinterpret_cast<const unsigned long long *>(a.x_planes) +
+                                    ((long)b * ((a.x_size + 63) / 64) + (e >> 6)) * slots;
+      uint32_t word = (uint32_t)(m[kmax] >> (e & 63)) & 1u;
+      for (int k = 0; k < kmax; ++k) word |= ((uint32_t)(m[k] >> (e & 63)) & 1u) << (k + 1);
+      a.x_words[(long)b * size + e] = word;
+      continue;
+    }
+    const uint32_t *planes = (is_x ? a.x_planes : a.d_planes) + (long)(b >> 5) * slots * size + e;
+    uint32_t word = (planes[(long)kmax * size] >> (b & 31)) & 1u;
+    for (int k = 0; k < kmax; ++k) word |= ((planes[(long)k * size] >> (b & 31)) & 1u) << (k + 1);
+    (is_x ? a.x_words : a.d_words)[(long)b * size + e] = word;
   }
 }
 
@@ -679,8 +781,8 @@ __device__ __forceinline__ float select_bits(uint32_t m, float a, float b) {
 // x bit planes of one 32-sample chunk for the C columns of a lane: NK pulse slots and the sign plane
 template <int NK, int C> struct ChunkPlanes {
   uint32_t k[C][NK], sg[C];
-  __device__ __forceinline__ void load(const UpdateArgs &a, const int (&j)[C], unsigned chunk) {
-    const unsigned xs = (unsigned)a.x_size, slots = (unsigned)a.plane_slots;
+  __device__ __forceinline__ void load(const UpdateArgs &a, const int (&j)[C], unsigned chunk, unsigned slots) {
+    const unsigned xs = (unsigned)a.x_size;
     const unsigned base = chunk * slots;
 #pragma unroll
     for (int c = 0; c < C; ++c) {
@@ -709,11 +811,12 @@ template <int KIND, bool MULT, int NK, bool NOISE, int C> struct PulsedRows {
   float (&w)[C];
   const PulseCell<KIND> (&cp)[C];
   const float *tbl;
+  const unsigned slots;
   uint32_t s0 = 1u, s1 = 0u;
   float fnext[C];
 
   __device__ __forceinline__ PulsedRows(const UpdateArgs &a_, float (&w_)[C], const PulseCell<KIND> (&cp_)[C], const float *tbl_)
-      : a(a_), w(w_), cp(cp_), tbl(tbl_) {}
+      : a(a_), w(w_), cp(cp_), tbl(tbl_), slots(plane_slots(a_)) {}
 
   __device__ __forceinline__ void draw() {
     if (!NOISE) return;
@@ -732,7 +835,7 @@ template <int KIND, bool MULT, int NK, bool NOISE, int C> struct PulsedRows {
   }
 
   __device__ __forceinline__ void chunk(const ChunkPlanes<NK, C> &x, unsigned ch, int i, int kmax, uint32_t lr_mask) {
-    const unsigned ds = (unsigned)a.d_size, slots = (unsigned)a.plane_slots;
+    const unsigned ds = (unsigned)a.d_size;
     const uint32_t *dpl = a.d_planes + i;
     const unsigned base = ch * slots;
     uint32_t dk[NK], any = 0u; // wave-uniform
@@ -789,9 +892,9 @@ template <int KIND, bool MULT, int NK, bool NOISE, int C> struct PulsedRows {
     uint32_t dk[NK], dsg; // of chunk (first chunk of the block + lane)
   };
   __device__ __forceinline__ void load_block(Block &b, const int (&j)[C], unsigned ch0, int i, int kmax) {
-    const unsigned n_chunks = (unsigned)a.n_chunks, ds = (unsigned)a.d_size, slots = (unsigned)a.plane_slots;
+    const unsigned n_chunks = (unsigned)a.n_chunks, ds = (unsigned)a.d_size;
 #pragma unroll
-    for (int p = 0; p < PB; ++p) b.x[p].load(a, j, min(ch0 + (unsigned)p, n_chunks - 1u));
+    for (int p = 0; p < PB; ++p) b.x[p].load(a, j, min(ch0 + (unsigned)p, n_chunks - 1u), slots);
     const unsigned chl = min(ch0 + (threadIdx.x & 63u), n_chunks - 1u);
     const uint32_t *dpl = a.d_planes + i;
 #pragma unroll
@@ -844,19 +947,19 @@ template <int KIND, bool MULT, int NK, bool NOISE, int C> struct PulsedRows {
     if (NK > 3) { // one register set: the longer lines are the rarer case, and two sets would not fit
       ChunkPlanes<NK, C> p;
       for (unsigned ch = 0; ch < n_chunks; ++ch) {
-        p.load(a, j, ch);
+        p.load(a, j, ch, slots);
         chunk(p, ch, i, kmax, lr_mask);
       }
       return;
     }
     ChunkPlanes<NK, C> pa, pb;
-    pa.load(a, j, 0u);
+    pa.load(a, j, 0u, slots);
     for (unsigned ch = 0; ch < n_chunks; ch += 2u) {
       const bool second = ch + 1u < n_chunks;
-      if (second) pb.load(a, j, ch + 1u);
+      if (second) pb.load(a, j, ch + 1u, slots);
       chunk(pa, ch, i, kmax, lr_mask);
       if (second) {
-        if (ch + 2u < n_chunks) pa.load(a, j, ch + 2u);
+        if (ch + 2u < n_chunks) pa.load(a, j, ch + 2u, slots);
         chunk(pb, ch + 1u, i, kmax, lr_mask);
       }
     }
@@ -879,7 +982,7 @@ __device__ __forceinline__ float pulsed_gather(const UpdateArgs &a, float w, con
   const uint32_t *xwp = a.x_words + j;
   const uint32_t *dwp = a.d_words + i;
   const unsigned xs = (unsigned)a.x_size, ds = (unsigned)a.d_size;
-  const int slots = a.plane_slots;
+  const int slots = kmax + 1;
 
   uint32_t refill = 0;
   for (int c0 = 0; c0 < n_chunks; c0 += 4) {
@@ -1011,6 +1114,304 @@ __global__ __launch_bounds__(256, ((C > 1 || DEEP) ? 4 : 8)) void k_update_pulse
   update_pulsed_row<KIND, MULT, NOISE, C, DEEP>(a, (int)blockIdx.x, row, tbl);
 }
 
+// ---- the pulse loop as a pipeline of waves -------------------------------------------------------------------------
+// Long batches on tiles of few rows (the patches of a convolution are samples to its tile).  A cross-point takes its
+// pulses one after the other, and with less than a wave of cross-points per SIMD nothing overlaps the chain of a pass:
+// PulsedRows takes 257 cycles for one (dependent instructions of a wave issue 8 cycles apart, a taken branch costs 30,
+// a table read 120), of which the step itself is 25.  Here the chain keeps only what depends on the weight.  A workgroup
+// shares one row among PARTS teams of three waves, each team on 64 columns, and one more wave:
+//   wave 0               lists the row's passes -- (sample, slot) pairs with a d pulse, in batch order -- in a ring in
+//                        LDS, eight chunks at a time, all of its lanes at once
+//   first of a team      draws the lane's noise factor for every pass
+//   second               zeroes it where the lane's x line did not fire
+//   third                owns the weights: w <- med3(w + (slope w + scale) f), three dependent operations and two selects
+// in blocks of STREAM_PASSES passes, each stage one block behind the one before it, one barrier per block.  Which lanes
+// fire in a pass and which go down are 64-bit lane masks (k_update_lines_stream), 64 passes of them to a load (lane p
+// fetches those of pass p), spread to the wave by v_readlane.
+// A factor of zero leaves w where it is -- bit for bit, unless w is outside its bounds or a parameter is not finite: such
+// a wave selects by the factor's bits instead.  Passes, noise bytes and the arithmetic of a step are those of
+// PulsedRows: same weights, bit for bit.
+// 433 x 48 tile, 131 072 samples, 21 000 passes a row: 1973 -> 493 us (55 cycles a pass; draw and steps take 45 each on
+// their own, the seven waves of a workgroup share four SIMDs).
+template <int PARTS> struct PulseStream {
+  float tbl[CTOC_LEVELS]; // first: its offset goes into the reads
+  float4 fac[PARTS][3][16][64]; // [team][block modulo 3][four passes][column]
+  uint32_t ring[4096];          // pass: row of words << 8 | direction flip << 3 | slot
+  int listed[2], done[2]; // by the parity of the step: passes listed so far, whether these are all
+};
+constexpr int STREAM_PASSES = 64, STREAM_RING = 4096, STREAM_APPEND = 8; // STREAM_APPEND chunks: at most 1792 passes
+
+// Step s of the pipeline has been done by this wave; whether that was the last one (the weights have taken the blocks up
+// to s - 2).  The words of a parity are rewritten two steps later, behind the barrier of the step between.
+template <typename SH> __device__ __forceinline__ bool pulse_stream_over(const SH &sh, int s) {
+  __syncthreads();
+  return sh.done[s & 1] && (s - 1) * STREAM_PASSES >= sh.listed[s & 1];
+}
+
+// wave 0: the passes of row i, as many as the other waves are about to need.  NK: pulse slots in use at most
+template <int NK, typename SH>
+__device__ __forceinline__ void pulse_stream_list(const UpdateArgs &a, SH &sh, const int i, const int kmax, const int lane) {
+  const unsigned ds = (unsigned)a.d_size, slots = (unsigned)kmax + 1u, n_chunks = (unsigned)a.n_chunks;
+  const uint32_t lr_mask = a.lr < 0.0f ? 0xffffffffu : 0u;
+  const uint32_t *dpl = a.d_planes + i;
+  const int q0 = (lane & 7) * 4; // lane: four samples of chunk (lane >> 3) of the next STREAM_APPEND chunks
+  uint32_t dk[NK], dsg = 0u;
+  auto load_d = [&](unsigned first) {
+    const unsigned ch = first + ((unsigned)lane >> 3);
+    const unsigned chc = min(ch, n_chunks - 1u);
+#pragma unroll
+    for (int k = 0; k < NK; ++k) dk[k] = (k < kmax && ch < n_chunks) ? dpl[(chc * slots + (unsigned)k) * ds] : 0u;
+    dsg = dpl[(chc * slots + slots - 1u) * ds];
+  };
+  int listed = 0;
+  unsigned next_chunk = 0u;
+  load_d(0u);
+  __syncthreads();
+  for (int s = 0;; ++s) {
+    const int wanted = (s + 2) * STREAM_PASSES;
+    while (listed < wanted && next_chunk < n_chunks) {
+      const unsigned ch = next_chunk + ((unsigned)lane >> 3);
+      uint32_t nib[NK], n = 0u;
+#pragma unroll
+      for (int k = 0; k < NK; ++k) {
+        nib[k] = (dk[k] >> q0) & 15u;
+        n += (uint32_t)__popc(nib[k]);
+      }
+      const uint32_t flip = (~dsg ^ lr_mask) >> q0;
+      next_chunk += STREAM_APPEND;
+      if (next_chunk < n_chunks) load_d(next_chunk);
+      // passes of the lanes before this one: the bits of the counts, counted over the lower lanes
+      unsigned before = 0u, all = 0u;
+#pragma unroll
+      for (int bit = 0; (4 * NK) >> bit; ++bit) {
+        const unsigned long long m = __ballot((n >> bit) & 1u);
+        before += (unsigned)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u)) << bit;
+        all += (unsigned)__popcll(m) << bit;
+      }
+      unsigned pos = (unsigned)listed + before;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const uint32_t entry = ((32u * ch + (unsigned)(q0 + t)) << 8) | (((flip >> t) & 1u) << 3);
+#pragma unroll
+        for (int k = 0; k < NK; ++k) { // slots beyond kmax hold no pulses
+          if ((nib[k] >> t) & 1u) {
+            sh.ring[pos & (STREAM_RING - 1)] = entry | (uint32_t)k;
+            ++pos;
+          }
+        }
+      }
+      listed += (int)all;
+    }
+    if (lane == 0) {
+      sh.listed[s & 1] = listed;
+      sh.done[s & 1] = next_chunk >= n_chunks ? 1 : 0;
+    }
+    if (pulse_stream_over(sh, s)) return;
+  }
+}
+
+// One 64-bit lane mask for each of the 64 passes from `first` on, lane p holding that of pass first + p: its fire mask (all
+// zero behind the end of the list) or, SIGN, the lanes that step down
+template <bool SIGN, typename SH>
+__device__ __forceinline__ void pulse_stream_masks(const UpdateArgs &a, const SH &sh, int first, int known, int block, int blocks,
+                                                   unsigned slots, int lane, uint32_t &lo, uint32_t &hi) {
+  const int p = first + lane;
+  const bool ok = p < known;
+  const uint32_t e = ok ? sh.ring[p & (STREAM_RING - 1)] : 0u;
+  const unsigned long long *masks = reinterpret_cast<const unsigned long long *>(a.x_planes);
+  const unsigned long long m = masks[((long)(e >> 8) * blocks + block) * slots + (SIGN ? slots - 1u : (e & 7u))];
+  const unsigned long long turn = SIGN ? (((e >> 3) & 1u) ? ~0ull : 0ull) : 0ull;
+  const unsigned long long keep = (SIGN || ok) ? ~0ull : 0ull;
+  lo = (uint32_t)((m ^ turn) & keep);
+  hi = (uint32_t)(((m ^ turn) & keep) >> 32);
+}
+__device__ __forceinline__ bool pulse_stream_lane_bit(uint32_t lo, uint32_t hi, int pass) {
+  const unsigned long long m = ((unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)hi, pass) << 32) |
+                               (uint32_t)__builtin_amdgcn_readlane((int)lo, pass);
+  return __builtin_amdgcn_inverse_ballot_w64(m);
+}
+
+// noise factors of every pass for 64 columns (cell: the lane's cross-point)
+template <bool NOISE, typename SH>
+__device__ __forceinline__ void pulse_stream_draw(const UpdateArgs &a, SH &sh, float4 (*fac)[16][64], const unsigned cell,
+                                                  const int lane) {
+  uint32_t s0 = 1u, s1 = 0u;
+  if (NOISE) {
+    const Philox4 r = philox4x32_10(cell, 0u, a.call, RNG_CTOC, a.key.k0, a.key.k1);
+    s0 = r.v[0] | 1u; // as PulsedRows::run
+    s1 = r.v[1];
+  }
+  auto draw4 = [&](float (&f)[4]) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      if (NOISE) {
+        const uint32_t r = s0 + s1;
+        s1 ^= s0;
+        s0 = __builtin_amdgcn_bitop3_b32(__builtin_rotateleft32(s0, 26), s1, s1 << 9, 0x96);
+        s1 = __builtin_rotateleft32(s1, 13);
+        f[u] = *(const float *)((const char *)sh.tbl + ((r & 0xffu) << 2));
+      } else {
+        f[u] = 1.0f;
+      }
+    }
+  };
+  __syncthreads();
+  float f[2][4]; // the factors of the next four passes are on their way while these are stored
+  draw4(f[0]);
+  for (int s = 0, buf = 0;; ++s, buf = buf == 2 ? 0 : buf + 1) {
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+      draw4(f[(q + 1) & 1]);
+      fac[buf][q][lane] = make_float4(f[q & 1][0], f[q & 1][1], f[q & 1][2], f[q & 1][3]);
+    }
+    if (pulse_stream_over(sh, s)) return;
+  }
+}
+
+// the factors of block s - 1, in place
+template <typename SH>
+__device__ __forceinline__ void pulse_stream_fire(const UpdateArgs &a, const SH &sh, float4 (*fac)[16][64], const int block,
+                                                  const int blocks, const int lane) {
+  const unsigned slots = plane_slots(a);
+  __builtin_amdgcn_s_setprio(2); // the longest stage where it shares its SIMD with another wave of the workgroup
+  __syncthreads();
+  if (pulse_stream_over(sh, 0)) return;
+  uint32_t lo, hi, lo_next, hi_next;
+  pulse_stream_masks<false>(a, sh, 0, sh.listed[0], block, blocks, slots, lane, lo, hi);
+  for (int s = 1, buf = 0;; ++s, buf = buf == 2 ? 0 : buf + 1) {
+    // the list covers this block and the next one, or is all there is
+    pulse_stream_masks<false>(a, sh, s * STREAM_PASSES, sh.listed[(s - 1) & 1], block, blocks, slots, lane, lo_next, hi_next);
+    float4 v[2] = {fac[buf][0][lane], fac[buf][1][lane]};
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+      float4 f = v[q & 1];
+      if (q + 2 < 16) v[q & 1] = fac[buf][q + 2][lane];
+      f.x = pulse_stream_lane_bit(lo, hi, 4 * q) ? f.x : 0.0f;
+      f.y = pulse_stream_lane_bit(lo, hi, 4 * q + 1) ? f.y : 0.0f;
+      f.z = pulse_stream_lane_bit(lo, hi, 4 * q + 2) ? f.z : 0.0f;
+      f.w = pulse_stream_lane_bit(lo, hi, 4 * q + 3) ? f.w : 0.0f;
+      fac[buf][q][lane] = f;
+    }
+    lo = lo_next;
+    hi = hi_next;
+    if (pulse_stream_over(sh, s)) return;
+  }
+}
+
+// The steps of a block.  The selects of the next pass (and the lane mask of the one after it) stand between the dependent
+// operations of this one.
+// BY_BITS: a factor of all bits zero leaves w untouched whatever it is
+template <int KIND, bool MULT, bool BY_BITS>
+__device__ __forceinline__ void pulse_stream_block(const float4 (*fac)[64], const PulseCell<KIND> &cp, const uint32_t lo,
+                                                   const uint32_t hi, float &w, const int lane) {
+#define RPU_IN_ORDER() __builtin_amdgcn_sched_barrier(0)
+  float4 f0 = fac[0][lane], f1 = fac[1][lane];
+  const bool down = pulse_stream_lane_bit(lo, hi, 0);
+  float slope = down ? cp.slope_dn : cp.slope_up, scale = down ? cp.scale_dn : cp.scale_up;
+  unsigned m_lo = (unsigned)__builtin_amdgcn_readlane((int)lo, 1), m_hi = (unsigned)__builtin_amdgcn_readlane((int)hi, 1);
+#pragma unroll
+  for (int q = 0; q < 16; ++q) {
+    const float fv[4] = {f0.x, f0.y, f0.z, f0.w};
+    f0 = f1;
+    if (q + 2 < 16) f1 = fac[q + 2][lane];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int p = 4 * q + u;
+      const bool down_next = __builtin_amdgcn_inverse_ballot_w64(((unsigned long long)m_hi << 32) | m_lo);
+      if (BY_BITS) {
+        const float wn = pulse<KIND, MULT>(w, slope, scale, fv[u], cp.lo, cp.hi);
+        w = __float_as_uint(fv[u]) == 0u ? w : wn;
+        m_lo = (unsigned)__builtin_amdgcn_readlane((int)lo, (p + 2) & 63);
+        m_hi = (unsigned)__builtin_amdgcn_readlane((int)hi, (p + 2) & 63);
+        slope = down_next ? cp.slope_dn : cp.slope_up;
+        scale = down_next ? cp.scale_dn : cp.scale_up;
+        continue;
+      }
+      // pulse(), spread out
+      RPU_IN_ORDER();
+      float t = 0.0f;
+      if (KIND != RPU_DEVICE_CONSTANT_STEP) t = MULT ? __builtin_fmaf(slope, w, scale) : __builtin_fmaf(slope, w, w);
+      RPU_IN_ORDER();
+      m_lo = (unsigned)__builtin_amdgcn_readlane((int)lo, (p + 2) & 63);
+      RPU_IN_ORDER();
+      const float wn = KIND == RPU_DEVICE_CONSTANT_STEP ? __builtin_fmaf(scale, fv[u], w)
+                                                        : (MULT ? __builtin_fmaf(t, fv[u], w) : __builtin_fmaf(scale, fv[u], t));
+      RPU_IN_ORDER();
+      m_hi = (unsigned)__builtin_amdgcn_readlane((int)hi, (p + 2) & 63);
+      slope = down_next ? cp.slope_dn : cp.slope_up;
+      RPU_IN_ORDER();
+      w = __builtin_amdgcn_fmed3f(wn, cp.lo, cp.hi);
+      RPU_IN_ORDER();
+      scale = down_next ? cp.scale_dn : cp.scale_up;
+    }
+  }
+#undef RPU_IN_ORDER
+}
+
+template <int KIND, bool MULT, typename SH>
+__device__ __forceinline__ void pulse_stream_steps(const UpdateArgs &a, const SH &sh, const float4 (*fac)[16][64],
+                                                   const PulseCell<KIND> &cp, float &w, const int block, const int blocks,
+                                                   const int lane) {
+  const unsigned slots = plane_slots(a);
+  const float big = fmaxf(fmaxf(fabsf(cp.slope_up), fabsf(cp.slope_dn)), fmaxf(fabsf(cp.scale_up), fabsf(cp.scale_dn)));
+  const bool by_bits = __any(!(w >= cp.lo && w <= cp.hi && big < 1e15f && fabsf(w) < 1e15f));
+  __syncthreads();
+  if (pulse_stream_over(sh, 0)) return;
+  uint32_t lo = 0u, hi = 0u, lo_next, hi_next;
+  for (int s = 1, buf = 2;; ++s, buf = buf == 2 ? 0 : buf + 1) {
+    // of block s - 1, which this wave takes in the next step
+    pulse_stream_masks<true>(a, sh, (s - 1) * STREAM_PASSES, sh.listed[(s - 1) & 1], block, blocks, slots, lane, lo_next, hi_next);
+    if (s >= 2) {
+      if (by_bits) pulse_stream_block<KIND, MULT, true>(fac[buf], cp, lo, hi, w, lane);
+      else pulse_stream_block<KIND, MULT, false>(fac[buf], cp, lo, hi, w, lane);
+    }
+    lo = lo_next;
+    hi = hi_next;
+    if (pulse_stream_over(sh, s)) return;
+  }
+}
+
+template <int KIND, bool MULT, bool NOISE, int PARTS>
+__global__ __launch_bounds__(64 * (1 + 3 * PARTS)) void k_update_pulsed_stream(UpdateArgs a) {
+  __shared__ __attribute__((aligned(16))) PulseStream<PARTS> sh;
+  const int lane = (int)threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int part = max(wave - 1, 0) / 3, role = max(wave - 1, 0) % 3;
+  const int i = (int)blockIdx.y, blocks = (a.x_size + 63) / 64;
+  const int block = min((int)blockIdx.x * PARTS + part, blocks - 1); // a team beyond the row repeats the last one
+  const int jt = ((int)blockIdx.x * PARTS + part) * 64 + lane;
+  const bool valid = jt < a.x_size;
+  const int j = min(block * 64 + lane, a.x_size - 1);
+  const unsigned cell = (unsigned)i * (unsigned)a.x_size + (unsigned)j;
+  const int kmax = a.kmax[a.kmax_slot];
+  if (kmax > UPDATE_PLANES_ONLY_KMAX && (wave == 0 || role != 2)) return; // see below
+  if (NOISE) {
+    for (int t = (int)threadIdx.x; t < CTOC_LEVELS; t += 64 * (1 + 3 * PARTS)) {
+      const float f = __builtin_fmaf(a.dev.dw_min_std, g_ctoc_xi[t], 1.0f);
+      sh.tbl[t] = f == 0.0f ? -0.0f : f; // all bits zero stands for "no pulse"
+    }
+  }
+  if (wave == 0) {
+    if (kmax <= 1) pulse_stream_list<1>(a, sh, i, kmax, lane);
+    else if (kmax <= 3) pulse_stream_list<3>(a, sh, i, kmax, lane);
+    else pulse_stream_list<7>(a, sh, i, kmax, lane);
+  } else if (role == 0) {
+    pulse_stream_draw<NOISE>(a, sh, sh.fac[part], cell, lane);
+  } else if (role == 1) {
+    pulse_stream_fire(a, sh, sh.fac[part], block, blocks, lane);
+  } else {
+    PulseCell<KIND> cp;
+    cp.load(a.dev, cell);
+    float w = a.w[cell];
+    // the noise of longer bit lines is drawn per pulse: these waves walk them as k_update_pulsed does
+    if (kmax > UPDATE_PLANES_ONLY_KMAX) w = pulsed_gather<KIND, MULT>(a, w, cp, cell, i, j, valid, kmax);
+    else pulse_stream_steps<KIND, MULT>(a, sh, sh.fac[part], cp, w, block, blocks, lane);
+    if (valid) {
+      if (a.w_out) a.w_out[(long)i * a.wo_si + (long)j * a.wo_sj] = w; // see UpdateArgs::w_out
+      else a.w[cell] = w;
+    }
+  }
+}
+
 // The same pulse loop with the rows dealt out by their work.  The time a row takes follows its number of d pulses, which
 // varies by several percent between rows, and a CU holds four rows at a time: whichever CU draws four long ones sets
 // the kernel's time.  Here a workgroup of 1024 threads fills a CU and takes four rows, one per 256 threads, chosen so
@@ -1139,10 +1540,10 @@ template <bool NOISE, int R> struct AggregatedRows {
   // kk < 3, or the sign plane for kk = 3.  One gather per four chunks instead of a scalar load (and its latency) per
   // row, chunk and slot; the counting loop reads the words back with v_readlane.
   __device__ __forceinline__ uint32_t gather_d(unsigned block, int kmax) const {
+    const unsigned slots = (unsigned)kmax + 1u;
     static_assert(R == 4, "lane layout of the d-plane gather");
     const unsigned lane = threadIdx.x & 63u;
     const unsigned ch = 4u * block + (lane >> 4), r = (lane >> 2) & 3u, kk = lane & 3u;
-    const unsigned slots = (unsigned)a.plane_slots;
     const unsigned slot = kk < 3u ? kk : slots - 1u;
     const unsigned row = min((unsigned)i0 + r, (unsigned)a.d_size - 1u);
     const bool wanted = ch < (unsigned)a.n_chunks && (kk == 3u || (int)kk < kmax);
@@ -1177,7 +1578,7 @@ template <bool NOISE, int R> struct AggregatedRows {
 
   // any bit-line length: planes read where they are used
   __device__ __forceinline__ void count_generic(int j, unsigned ch, int kmax) {
-    const unsigned xs = (unsigned)a.x_size, ds = (unsigned)a.d_size, slots = (unsigned)a.plane_slots, base = ch * slots;
+    const unsigned xs = (unsigned)a.x_size, ds = (unsigned)a.d_size, slots = (unsigned)kmax + 1u, base = ch * slots;
     const uint32_t *xpl = a.x_planes + j;
     const uint32_t xsg = xpl[(base + slots - 1u) * xs];
 #pragma unroll
@@ -1238,12 +1639,12 @@ template <bool NOISE, int R> struct AggregatedRows {
       ChunkPlanes<3, 1> cur[4], nxt[4];
       uint32_t dcur = gather_d(0u, kmax), dnxt = 0u;
 #pragma unroll
-      for (int q = 0; q < 4; ++q) cur[q].load(a, jj, (unsigned)min(q, n_chunks - 1));
+      for (int q = 0; q < 4; ++q) cur[q].load(a, jj, (unsigned)min(q, n_chunks - 1), (unsigned)kmax + 1u);
       for (int b = 0; b < n_blocks; ++b) {
         if (b + 1 < n_blocks) {
           dnxt = gather_d((unsigned)b + 1u, kmax);
 #pragma unroll
-          for (int q = 0; q < 4; ++q) nxt[q].load(a, jj, (unsigned)min(4 * b + 4 + q, n_chunks - 1));
+          for (int q = 0; q < 4; ++q) nxt[q].load(a, jj, (unsigned)min(4 * b + 4 + q, n_chunks - 1), (unsigned)kmax + 1u);
         }
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
@@ -1345,7 +1746,7 @@ __global__ __launch_bounds__(256) void k_count_pulses(UpdateArgs a, unsigned lon
   const int j = blockIdx.x * blockDim.x + threadIdx.x;
   if (j >= a.x_size) return;
   const int kmax = a.kmax[a.kmax_slot];
-  const unsigned xs = (unsigned)a.x_size, ds = (unsigned)a.d_size, slots = (unsigned)a.plane_slots;
+  const unsigned xs = (unsigned)a.x_size, ds = (unsigned)a.d_size, slots = (unsigned)kmax + 1u;
   const uint32_t *xpl = a.x_planes + j;
   const uint32_t *dpl = a.d_planes + i;
   unsigned n_same = 0, n_diff = 0;
@@ -1395,7 +1796,7 @@ __global__ __launch_bounds__(256) void k_write_noise_touched(UpdateArgs a, float
     for (int b = 0; b < a.m_batch && !touched; ++b) touched = implicit_count(a, b, i, j) != 0;
   } else {
     const int kmax = a.kmax[a.kmax_slot];
-    const unsigned xs = (unsigned)a.x_size, ds = (unsigned)a.d_size, slots = (unsigned)a.plane_slots;
+    const unsigned xs = (unsigned)a.x_size, ds = (unsigned)a.d_size, slots = (unsigned)kmax + 1u;
     const uint32_t *xpl = a.x_planes + j;
     const uint32_t *dpl = a.d_planes + i;
     uint32_t any = 0u;
@@ -1497,6 +1898,12 @@ void launch_update_lines(const UpdateArgs &a, hipStream_t s) {
     extra = (extra + sample_tiles - 1) / sample_tiles;
   }
   const bool in_place = a.x_index || a.d_group;
+  if (a.x_lane_masks) {
+    const dim3 grid((a.x_size + 63) / 64 + (a.d_size + 15) / 16 + extra, sample_tiles);
+    if (in_place) hipLaunchKernelGGL(k_update_lines_stream<true>, grid, dim3(256), 0, s, a);
+    else hipLaunchKernelGGL(k_update_lines_stream<false>, grid, dim3(256), 0, s, a);
+    return;
+  }
   const dim3 narrow((a.x_size + 3) / 4 + (a.d_size + 3) / 4 + extra, sample_tiles);
   if (wide * sample_tiles >= 256) {
     if (in_place) hipLaunchKernelGGL((k_update_lines<16, true>), dim3(wide + extra, sample_tiles), dim3(256), 0, s, a);
@@ -1529,6 +1936,10 @@ void launch_words_kmax(const UpdateArgs &a, hipStream_t s) {
   hipLaunchKernelGGL(k_zero_word, dim3(1), dim3(64), 0, s, a.kmax + a.kmax_slot);
   hipLaunchKernelGGL(k_words_kmax, dim3((unsigned)std::max<size_t>(blocks, 1)), dim3(256), 0, s, a.x_words, nx, a.d_words, nd,
                      a.kmax + a.kmax_slot);
+}
+
+void launch_words_from_planes(const UpdateArgs &a, hipStream_t s) {
+  hipLaunchKernelGGL(k_words_from_planes, dim3(grid_for(((long)a.x_size + a.d_size) * a.m_batch)), dim3(256), 0, s, a);
 }
 
 void launch_update_planes(const UpdateArgs &a, hipStream_t s) {
@@ -1585,8 +1996,39 @@ static int update_pulsed_columns(const UpdateArgs &a) {
   return 1;
 }
 
+// Whether the pulse loop of this call runs as a pipeline of waves (k_update_pulsed_stream): a batch that fills the
+// pipeline, on a tile with at most one wave of cross-points per SIMD (with more, the plain loop's waves overlap each
+// other and its fewer instructions per pass count: 25 against 40).
+bool update_takes_stream(const UpdateArgs &a) {
+  return update_pulsed_columns(a) == 1 && a.n_chunks >= 32 && a.m_batch < (1 << 23) &&
+         (long)((a.x_size + 63) / 64) * a.d_size <= 1024;
+}
+template <bool NOISE, int PARTS> static void launch_update_pulsed_stream(const UpdateArgs &a, hipStream_t s) {
+  const dim3 grid(((a.x_size + 63) / 64 + PARTS - 1) / PARTS, a.d_size), block(64 * (1 + 3 * PARTS));
+  if (a.dev.kind == RPU_DEVICE_CONSTANT_STEP) {
+    hipLaunchKernelGGL((k_update_pulsed_stream<RPU_DEVICE_CONSTANT_STEP, true, NOISE, PARTS>), grid, block, 0, s, a);
+  } else if (a.dev.ls_mult_noise) {
+    hipLaunchKernelGGL((k_update_pulsed_stream<RPU_DEVICE_LINEAR_STEP, true, NOISE, PARTS>), grid, block, 0, s, a);
+  } else {
+    hipLaunchKernelGGL((k_update_pulsed_stream<RPU_DEVICE_LINEAR_STEP, false, NOISE, PARTS>), grid, block, 0, s, a);
+  }
+}
+
 void launch_update_pulsed(const UpdateArgs &a, hipStream_t s) {
   const int cols = update_pulsed_columns(a);
+  if (a.x_lane_masks) {
+    // two teams to a workgroup where single ones would be more than the CUs: seven waves on a CU's four SIMDs, evenly
+    // over the chip, instead of two workgroups on some CUs and one on the others
+    const bool noise = a.dev.dw_min_std > 0.0f;
+    if ((long)((a.x_size + 63) / 64) * a.d_size <= 256) {
+      if (noise) launch_update_pulsed_stream<true, 1>(a, s);
+      else launch_update_pulsed_stream<false, 1>(a, s);
+    } else {
+      if (noise) launch_update_pulsed_stream<true, 2>(a, s);
+      else launch_update_pulsed_stream<false, 2>(a, s);
+    }
+    return;
+  }
   if (a.dev.dw_min_std > 0.0f) {
     if (cols == 4) launch_update_pulsed_t<true, 4>(a, s);
     else if (cols == 2) launch_update_pulsed_t<true, 2>(a, s);

@@ -236,7 +236,8 @@ struct Tile {
   // where the last pulsed update left its per-sample values and packed words (own buffers or the static scratch)
   int *last_bl = nullptr;
   float *last_a = nullptr, *last_b = nullptr;
-  uint32_t *last_xw = nullptr, *last_dw = nullptr;
+  UpdateArgs last_update{};   // its arguments: where its words (or the planes that hold them) are
+  bool last_in_planes = false; // the words have not been made from the planes yet
   int last_words_per_sample = 1;
   // transfer compound (rpu_transfer_device.{h,cpp}): device 0 takes the gradient update, device j is read
   // column by column and written onto device j + 1; the tile's weights d_w are the weighted sum, or the
@@ -422,7 +423,7 @@ struct Tile {
     u_bl.release(); u_a.release(); u_b.release(); u_xval.release(); u_dval.release(); u_xw.release(); u_dw.release();
     u_xpl.release(); u_dpl.release(); u_kmax.release();
     r_wmax.release(); r_wmin.release(); r_sup.release(); r_sdown.release(); r_slup.release(); r_sldown.release(); u_wrm.release();
-    last_bl = nullptr; last_a = last_b = nullptr; last_xw = last_dw = nullptr;
+    last_bl = nullptr; last_a = last_b = nullptr; last_update = UpdateArgs{}; last_in_planes = false;
     t_unit.release(); t_read.release();
     i_ref.release(); i_prog.release(); i_nu_plus.release(); i_nu_minus.release(); i_scalar.release(); i_absmax.release();
     has_reference = programmed = false;
@@ -985,7 +986,7 @@ struct Tile {
     float *rows = bias ? (float *)take((size_t)B * X * 4) : nullptr;
     if (a) {
       a->kmax = kmax; a->row_cost = row_cost; a->bl = bl; a->prob_a = pa; a->prob_b = pb; a->x_words = xw; a->d_words = dw;
-      a->x_planes = xpl; a->d_planes = dpl; a->plane_slots = (int)slots; a->n_chunks = (int)chunks;
+      a->x_planes = xpl; a->d_planes = dpl; a->n_chunks = (int)chunks;
     }
     if (bias_rows) *bias_rows = rows;
     return off;
@@ -994,14 +995,14 @@ struct Tile {
   void set_plane_args(UpdateArgs &a, int B) {
     const int slots = 32; // 31 pulse slots and the sign plane
     const int chunks = (B + 31) / 32;
-    u_xpl.ensure((size_t)chunks * slots * X);
+    u_xpl.ensure((size_t)chunks * slots * std::max(X, 16)); // 16: lane masks of a row of up to 64 elements
     u_dpl.ensure((size_t)chunks * slots * D);
     if (!u_kmax.p) {
       u_kmax.ensure(4);
       const int init[4] = {0, 0, 31, 0};
       RPU_HIP_CHECK(hipMemcpy(u_kmax.p, init, sizeof(init), hipMemcpyHostToDevice));
     }
-    a.x_planes = u_xpl.p; a.d_planes = u_dpl.p; a.plane_slots = slots; a.n_chunks = chunks;
+    a.x_planes = u_xpl.p; a.d_planes = u_dpl.p; a.n_chunks = chunks;
     a.kmax = u_kmax.p;
   }
 
@@ -1018,6 +1019,7 @@ struct Tile {
     a.dev.slope_up = d_slup.p; a.dev.slope_down = d_sldown.p;
     a.x_words = const_cast<uint32_t *>(x_words); a.d_words = const_cast<uint32_t *>(d_words);
     a.key = key(); a.call = call++;
+    make_last_words(s); // the planes are used again
     set_plane_args(a, B);
     if (xd) { // see r_wmax
       row_major_pulse_loop(a);
@@ -1503,13 +1505,22 @@ struct Tile {
   // row-major tile, with x and d exchanged on one that stores [x_size][d_size] (UpdateArgs::swapped)
   UpdateArgs cross_point_view(const UpdateArgs &a) const { return xd ? update_swapped_view(a) : a; }
 
+  // the packed words of the last stochastic update, which may have left their bit planes only
+  void make_last_words(hipStream_t s) {
+    if (!last_in_planes) return;
+    launch_words_from_planes(last_update, s);
+    last_in_planes = false;
+  }
+
   // what the debug hooks read after a pulsed update
   void note_pulsed_update(const UpdateArgs &a, int B, int wps, int pulse_type, hipStream_t s) {
     last_stream = s;
     last_update_batch = B;
     last_words_per_sample = wps;
     last_update_pulse = pulse_type;
-    last_bl = a.bl; last_a = a.prob_a; last_b = a.prob_b; last_xw = a.x_words; last_dw = a.d_words;
+    last_bl = a.bl; last_a = a.prob_a; last_b = a.prob_b;
+    last_update = a;
+    last_in_planes = pulse_type == RPU_PULSE_STOCHASTIC_COMPRESSED;
   }
 
   void pulsed_update_on(const DeviceView &dv, const UpdatePar &up, float lr, const float *xin, long x_sb, long x_sj,
@@ -1532,6 +1543,8 @@ struct Tile {
         row_major_pulse_loop(a);
         a.wt_src = d_w.p; // the launch of the pulse trains makes the row-major copy
       }
+      // (pulse counters and write noise read the bit planes; the static block is laid out for planes)
+      a.x_lane_masks = (!ws && !aggregated && !counting && !(dv.w == d_wp.p && persistent()) && update_takes_stream(a)) ? 1 : 0;
       launch_update_lines(a, s);
       prof_mark(s, "update_lines");
       if (counting) count_pulses(a, false, s);
@@ -3400,8 +3413,10 @@ int rpu_tile_get_update_words(rpu_tile_t *tile, uint32_t *x_words_host, uint32_t
     DeviceGuard g(t.device_id);
     t.sync_last();
     const size_t rows = (size_t)m_batch * t.last_words_per_sample;
-    RPU_HIP_CHECK(hipMemcpy(x_words_host, t.last_xw, rows * t.X * 4, hipMemcpyDeviceToHost));
-    RPU_HIP_CHECK(hipMemcpy(d_words_host, t.last_dw, rows * t.D * 4, hipMemcpyDeviceToHost));
+    t.make_last_words(t.last_stream);
+    t.sync_last();
+    RPU_HIP_CHECK(hipMemcpy(x_words_host, t.last_update.x_words, rows * t.X * 4, hipMemcpyDeviceToHost));
+    RPU_HIP_CHECK(hipMemcpy(d_words_host, t.last_update.d_words, rows * t.D * 4, hipMemcpyDeviceToHost));
     RPU_HIP_CHECK(hipMemcpy(bl_host, t.last_bl, (size_t)m_batch * 4, hipMemcpyDeviceToHost));
   });
 }
