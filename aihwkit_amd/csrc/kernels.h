@@ -73,6 +73,7 @@ struct MvmArgs {
   int m_batch;
   int K, O;       // contraction length and number of outputs
   int k_pad;      // K rounded up to the step of the contraction kernel (mvm_k_pad)
+  float x_step;   // > 0: the quantized inputs are multiples of this step, at most 256 of them (mvm_input_step); 0: any values
   float *xq[2];   // ping-pong scratch [rows][k_pad]: DAC-quantized inputs, zero padded (rows: see MvmState::row)
   int transposed; // 0: forward pass (out = W in), 1: backward pass (out = W^T in); decides the scales of a round, not
                   // how the weights are addressed (w_oc)
@@ -174,8 +175,9 @@ int mvm_round_workgroups(const MvmArgs &a);            // workgroups of a round 
 int mvm_big_workgroups(const MvmArgs &a, int bb);
 // bb: samples of a workgroup tile, 128 or 64 (mvm_big_sample_tile: by the workgroups the launch would have with 128)
 int mvm_big_sample_tile(int workgroups_128, int n_cus);
+float mvm_input_step(const IoDev &io);
 // w_oc: how the tiles of the launch address their weights (MvmArgs::w_oc; the same for all of them)
-void launch_mvm_big_group(const MvmGroup &g, int total_workgroups, int bb, bool w_oc, hipStream_t s);
+void launch_mvm_big_group(const MvmGroup &g, int total_workgroups, int bb, bool w_oc, bool stepped, hipStream_t s);
 void mvm_round_variant(const MvmArgs &a, int &prefetch_depth, int &weight_mode);
 
 // Fused convolution forward (unfold + noisy MVM with its bound-management rounds) for tiles of at most 32 outputs:

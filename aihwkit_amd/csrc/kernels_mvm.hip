@@ -23,14 +23,15 @@
 //                  between two rounds.
 //   k_mvm_round_tail   later rounds of a launch whose full grid would be large: a fixed number of workgroups walk
 //                  the tiles of the samples that are listed (usually few).
-//   k_mvm_big      large batches on wide tiles: 128 x 128 workgroup tiles, both operands staged through LDS and
-//                  shared by the four waves (64 x 64 per wave), same state / epilogue / random streams; a round is
+//   k_mvm_big      large batches on wide tiles: 128 x 128 workgroup tiles, both operands staged through LDS, the product
+//                  on the bf16 matrix pipe with operands split into bf16 parts without loss; same state / epilogue / random streams; a round is
 //                  run by this or by the 32 x 32 kernel, by the number of samples it lists.
 //   k_conv_forward convolution forward of a narrow tile (at most 32 outputs): unfold by the index matrix, noise
 //                  management, DAC, contraction, ADC and the bound-management rounds in one kernel.
 //   *_group        the same kernels over the tiles of a group in one launch.
 #include "kernels.h"
 
+#include <cmath>
 #include <mutex>
 
 namespace rpu_amd {
@@ -1549,16 +1550,18 @@ __global__ __launch_bounds__(256) void k_mvm_round(MvmArgs a) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// Large-batch round: one workgroup (4 waves as 2 x 2) owns 128 outputs x 128 samples, each wave a 64 x 64 block as
-// 2 x 2 MFMA tiles.  Both operands go through LDS stages of 32 k-values shared by the four waves (a stage is
-// fetched into registers while the previous one is multiplied, then written to the other LDS buffer: one barrier
-// per stage), so a byte fetched from L2 feeds 64 multiply-adds instead of 16 and the matrix pipe, not the memory
-// path, sets the pace.  Same per-sample state, lists, epilogue and random streams as the 32 x 32 kernel: a round
+// Large-batch round: one workgroup (4 waves) owns 128 outputs x 128 samples, each wave 32 outputs of all samples, so
+// that a weight is split into its bf16 parts by one wave only (five operations, next to 3 x 4 MFMAs per 16 of them in a
+// lane).  Both operands go through LDS stages of 32 k-values shared by the four waves (a stage is fetched into registers
+// while the previous one is multiplied, then written to the other LDS buffer: one barrier per stage), so a byte fetched
+// from L2 feeds 64 multiply-adds instead of 16.
+// On the fp32 matrix pipe, which set the pace before, a round of 16384 samples on a 1024 x 1024 tile took 316 us
+// (backward), the four linear layers of a 768-wide transformer block 69 + 34 + 80 + 69 us at 1024 tokens; with the split
+// operands 164 us and 49 + 30 + 54 + 50 us.  Error against 64-bit sums (relative, 1024 terms): 5.7e-7 before, 3.1e-7 with
+// quantized inputs, 4.9e-7 with any other.  Same per-sample state, lists, epilogue and random streams as the 32 x 32 kernel: a round
 // may be run by either (the launcher picks by the number of samples in the round).
 // WT = 0: weights contiguous along k (forward), 1: contiguous along the outputs (backward, W read in place).
 
-constexpr int BT = 128;        // outputs of a workgroup tile; its samples: BB = 128, or 64 (each wave 64 x 32: twice the
-                               // workgroups, for launches that would put fewer than about three of the square tiles on a CU)
 constexpr int BKS = 32;        // k-values per stage
 constexpr int BROW = 32;       // floats per staged row of a k-contiguous operand, no padding.  LDS has 64 banks: two rows
                                // fill the 16 chunk slots (of 16 bytes) of a 256-byte line, and chunk c of row `row` sits in
@@ -1567,11 +1570,10 @@ constexpr int BROW = 32;       // floats per staged row of a k-contiguous operan
 __device__ __forceinline__ int big_lds_offset(int row, int chunk) {
   return (row >> 1) * (2 * BROW) + ((((row & 1) << 3) + chunk + (row >> 1)) & 15) * 4;
 }
-constexpr int BPITCH_T = 132;  // floats per staged k-row of an output-contiguous weight tile
 
 template <int BB>
-__device__ __forceinline__ void big_prepare_next_rows(const MvmArgs &a, int round, int tile_o, int tile_b, int n_act,
-                                                      int *sh_b, float *sh_scale) {
+__device__ __forceinline__ void big_prepare_next_rows(const MvmArgs &a, int round, int tile_o, int tiles_o, int tile_b,
+                                                      int n_act, int *sh_b, float *sh_scale) {
   if (threadIdx.x < BB) {
     const int slot = tile_b * BB + threadIdx.x;
     int b = 0;
@@ -1584,7 +1586,6 @@ __device__ __forceinline__ void big_prepare_next_rows(const MvmArgs &a, int roun
     sh_scale[threadIdx.x] = scale;
   }
   __syncthreads();
-  const int tiles_o = (a.O + BT - 1) / BT;
   const int chunk = (((a.k_pad + tiles_o - 1) / tiles_o) + 31) & ~31;
   const int k_lo = tile_o * chunk;
   const int k_hi = min(k_lo + chunk, a.k_pad);
@@ -1612,73 +1613,83 @@ __device__ __forceinline__ void big_prepare_next_rows(const MvmArgs &a, int roun
   }
 }
 
-// Instruction order of 16 MFMAs and the LDS reads of the operands that follow them (a hint to the scheduler): the
-// reads are spread behind the first MFMAs so that they complete underneath the rest.
-template <int WT, int NB>
-__device__ __forceinline__ void mvm_big_schedule() {
-  // NB sample blocks per wave: 8 NB MFMAs.  WT = 0: 2 + NB wide LDS reads; WT = 1: NB wide reads and the 8 single
-  // reads of the transposed weight tile
-  constexpr int mfmas = 8 * NB;
-  constexpr int paired = WT == 0 ? 2 + NB : (NB == 2 ? 6 : 5);
-  constexpr int doubled = (WT == 1 && NB == 1) ? 4 : 0; // pairs that carry two LDS reads
-#pragma unroll
-  for (int i = 0; i < doubled; ++i) {
-    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0); // one MFMA
-    __builtin_amdgcn_sched_group_barrier(0x100, 2, 0); // two LDS reads
-  }
-#pragma unroll
-  for (int i = doubled; i < paired; ++i) {
-    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0); // one MFMA
-    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0); // one LDS read
-  }
-  __builtin_amdgcn_sched_group_barrier(0x008, mfmas - paired, 0);
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
+// Offset (in bf16) of 16-byte chunk `chunk` (8 values, 0 .. 3) of staged input row `row`: four rows of 64 bytes fill a
+// 256-byte line, and the rotation by row / 4 lets 16 rows that read the same chunk touch all 64 banks once.
+__device__ __forceinline__ int big_x_offset(int row, int chunk) {
+  return (row >> 2) * 128 + (((row & 3) << 2) + ((chunk + (row >> 2)) & 3)) * 8;
+}
+
+// v = hi + mid + lo with every part rounded to bf16: 3 x 8 bits hold the 24 of a float, so the sum is exact (above
+// 2^-110; the low part of a smaller value may drop out)
+__device__ __forceinline__ void split_bf16(const f32x4 v, bf16x4 &hi, bf16x4 &mid, bf16x4 &lo) {
+  hi = __builtin_convertvector(v, bf16x4);
+  const f32x4 r1 = v - __builtin_convertvector(hi, f32x4);
+  mid = __builtin_convertvector(r1, bf16x4);
+  const f32x4 r2 = r1 - __builtin_convertvector(mid, f32x4);
+  lo = __builtin_convertvector(r2, bf16x4);
+}
+__device__ __forceinline__ float max_abs4(float m, const f32x4 v) {
+  return fmaxf(fmaxf(m, fmaxf(fabsf(v.x), fabsf(v.y))), fmaxf(fabsf(v.z), fabsf(v.w)));
 }
 
 // work of workgroup number n of a large-tile round launch of one tile; BB: samples of a workgroup tile (128 or 64)
-// NARROW (tiles of at most 64 outputs, BB = 128): every wave takes outputs 0 .. 63 and one of the four 32-sample
-// blocks, instead of two waves on outputs that do not exist: half of the MFMAs, spread over all four SIMDs; the
-// k order of every sum is the same.
-// NBUF = 1 (contractions of one or two stages): a single staging buffer, half of the LDS, so that a third workgroup
-// fits a CU and covers the ADC stage of the other two, which is all such a call consists of.
+// WO: waves along the outputs, 32 outputs each: 4, or 2 for tiles of at most 64 outputs (the other two waves then take
+// the second half of the samples instead of outputs that do not exist).
+// XP: bf16 planes of a staged input.  The product of two floats is made on the bf16 matrix pipe, 16 times as fast as the
+// fp32 one, from operands split into bf16 parts without loss: three parts for a weight, and
+//   XP = 1  one for an input that the DAC has rounded to a multiple k of its step, |k| <= 256 (MvmArgs::x_step): the
+//           rows hold k * step, k is what is staged, and the step multiplies the finished sum.  3 exact products of 8 x 8
+//           bits per element against the one rounded input k * step of the fp32 pipe;
+//   XP = 3  three for any other input, of whose nine products the three below 2^-24 of the whole are left out.
+// Sums are kept in fp32 as before, in chains an eighth as long.  A stage with a value outside the range in which the
+// parts and their products are safe (infinities among them, whose parts would be NaN) is multiplied on the fp32 pipe.
 // LAZY (calls with speculate = 0): nothing is quantized ahead; the last workgroup of a sample tile writes the rows of
 // the samples that go on.  The other instantiations always quantize ahead, as their callers ask for.
-template <int WT, int BB, bool NARROW = false, int NBUF = 2, bool LAZY = false>
+template <int WT, int BB, int WO, int XP, bool LAZY>
 __device__ __forceinline__ void mvm_big_workgroup(const MvmArgs &a, const int round, const int n, const int min_active) {
   static_assert(BB == 128 || BB == 64, "sample tile of 128 or 64");
-  static_assert(!NARROW || BB == 128, "the narrow wave layout covers four sample blocks");
-  constexpr int NB = NARROW ? 1 : BB / 64; // 32-sample blocks per wave
-  constexpr int XJ = BB / 32; // staged sample rows per thread
-  __shared__ __attribute__((aligned(16))) float lds_x[NBUF][BB * BROW];
-  __shared__ __attribute__((aligned(16))) float lds_w[NBUF][WT ? BKS * BPITCH_T : BT * BROW];
+  static_assert(WO == 4 || WO == 2, "two or four waves along the outputs");
+  constexpr int OT = 32 * WO;            // outputs of a workgroup tile
+  constexpr int WB = 4 / WO;             // waves along the samples
+  constexpr int NB = BB / 32 / WB;       // 32-sample blocks per wave
+  constexpr int XJ = BB / 32;            // staged sample rows per thread
+  constexpr int WJ = OT / 32;            // staged chunks of weights per thread
+  constexpr int WPITCH = OT + 4;         // floats per staged k-row of an output-contiguous weight tile
+  __shared__ __attribute__((aligned(16))) __bf16 lds_x[2][XP][BB * BKS];
+  __shared__ __attribute__((aligned(16))) float lds_w[2][WT ? BKS * WPITCH : OT * BROW];
   __shared__ int sh_hits[2 * BB];
   __shared__ int sh_b[BB];
   __shared__ float sh_scale[BB];
   __shared__ int sh_last;
+  __shared__ int sh_slow[2]; // the last stage in this buffer that the fp32 pipe has to multiply
 
   const int n_act = (round > 0) ? a.st.count[round] : a.m_batch;
   if (n_act < min_active) return; // this round is run by the 32 x 32 kernel
   // workgroup n runs on XCD n % 8: an XCD walks the output tiles of one sample tile after the other, so a tile of
   // quantized inputs (the large operand) enters one L2 only and the small weight matrix is what every XCD streams
-  const int tile_o = (n >> 3) % ((a.O + BT - 1) / BT);
-  const int tile_b = ((n >> 3) / ((a.O + BT - 1) / BT)) * 8 + (n & 7);
+  const int tiles_o = (a.O + OT - 1) / OT;
+  const int tile_o = (n >> 3) % tiles_o;
+  const int tile_b = ((n >> 3) / tiles_o) * 8 + (n & 7);
   if (tile_b * BB >= n_act) return;
   const bool more_rounds = round + 1 < a.max_rounds;
   if (more_rounds && !LAZY && !(round == 0 && a.rows_ahead_in_init)) {
-    big_prepare_next_rows<BB>(a, round, tile_o, tile_b, n_act, sh_b, sh_scale);
+    big_prepare_next_rows<BB>(a, round, tile_o, tiles_o, tile_b, n_act, sh_b, sh_scale);
   }
 
   const int t = threadIdx.x;
   const int lane = t & 63, wave = t >> 6;
   const int r = lane & 31, h = lane >> 5;
-  const int wy = NARROW ? 0 : wave >> 1, wx = wave & 1;
-  const int blk = NARROW ? wave >> 1 : 0; // NARROW: this wave's sample block within its half
+  const int wo = WO == 4 ? wave : (wave & 1), wb = WO == 4 ? 0 : (wave >> 1);
   const int K = a.K;
 
   // global -> LDS assignment.  k-contiguous operand: chunk c = t + 256 j covers row c / 8, floats 4 (c % 8) ..;
-  // output-contiguous weights: chunk c covers k-row c / 32, outputs 4 (c % 32) ..
+  // output-contiguous weights: chunk c covers k-row c / (OT / 4), outputs 4 (c % (OT / 4)) ..
   const float *xq = round_rows(a, round);
   const float *x_src[XJ];
-  const float *w_src[4];
+  const float *w_src[WJ];
   const int st_col = (t & 7) * 4;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
@@ -1686,13 +1697,16 @@ __device__ __forceinline__ void mvm_big_workgroup(const MvmArgs &a, const int ro
     if (j < XJ) {
       const int slot = min(tile_b * BB + row, n_act - 1);
       const int xrow = (round > 0) ? pick2(a.st.row, round & 1)[slot] : slot;
-      x_src[j] = xq + (long)xrow * a.k_pad + st_col;
+      x_src[j < XJ ? j : 0] = xq + (long)xrow * a.k_pad + st_col;
     }
-    if (WT == 0) w_src[j] = a.w + (long)min(tile_o * BT + row, a.O - 1) * a.w_ld;
+    if (WT == 0 && j < WJ) w_src[j < WJ ? j : 0] = a.w + (long)min(tile_o * OT + row, a.O - 1) * a.w_ld;
   }
-  const int wt_o = tile_o * BT + (t & 31) * 4; // WT = 1: first of this thread's four outputs
+  constexpr int WROWS = 1024 / OT; // k-rows of an output-contiguous tile that the threads cover at a time
+  const int wt_k = t / (OT / 4);
+  const int wt_col = (t % (OT / 4)) * 4;
+  const int wt_o = tile_o * OT + wt_col; // WT = 1: first of this thread's four outputs
 
-  auto gload = [&](int s, f32x4 (&gx)[XJ], f32x4 (&gw)[4]) {
+  auto gload = [&](int s, f32x4 (&gx)[XJ], f32x4 (&gw)[WJ]) __attribute__((always_inline)) {
     const int k0 = s * BKS;
 #pragma unroll
     for (int j = 0; j < XJ; ++j) gx[j] = *reinterpret_cast<const f32x4 *>(x_src[j] + k0);
@@ -1700,10 +1714,10 @@ __device__ __forceinline__ void mvm_big_workgroup(const MvmArgs &a, const int ro
       const int kc = k0 + st_col;
       if (kc + 4 <= K) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) gw[j] = *reinterpret_cast<const f32x4_unaligned *>(w_src[j] + kc);
+        for (int j = 0; j < WJ; ++j) gw[j] = *reinterpret_cast<const f32x4_unaligned *>(w_src[j] + kc);
       } else {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
+        for (int j = 0; j < WJ; ++j) {
           f32x4 z;
           z.x = (kc < K) ? w_src[j][kc] : 0.0f;
           z.y = (kc + 1 < K) ? w_src[j][kc + 1] : 0.0f;
@@ -1714,8 +1728,8 @@ __device__ __forceinline__ void mvm_big_workgroup(const MvmArgs &a, const int ro
       }
     } else {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int k = min(k0 + (t >> 5) + 8 * j, K - 1); // rows past K meet the zero padding of the inputs
+      for (int j = 0; j < WJ; ++j) {
+        const int k = min(k0 + wt_k + WROWS * j, K - 1); // rows past K meet the zero padding of the inputs
         const float *row = a.w + (long)k * a.w_ld;
         if (wt_o + 4 <= a.O) {
           gw[j] = *reinterpret_cast<const f32x4_unaligned *>(row + wt_o);
@@ -1730,140 +1744,181 @@ __device__ __forceinline__ void mvm_big_workgroup(const MvmArgs &a, const int ro
       }
     }
   };
-  auto lds_store = [&](int buf, const f32x4 (&gx)[XJ], const f32x4 (&gw)[4]) {
+  // k * step times 1 / step is k up to a few units in the 24th bit: rounding to bf16 returns k itself
+  const float inv_step = XP == 1 ? 1.0f / a.x_step : 1.0f;
+  constexpr float SAFE = XP == 1 ? 0x1p100f : 0x1p60f; // parts and products stay finite below it
+  auto lds_store = [&](int s, const f32x4 (&gx)[XJ], const f32x4 (&gw)[WJ]) __attribute__((always_inline)) {
+    const int buf = s & 1;
+    float m = 0.0f;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int row = (t >> 3) + 32 * j;
-      if (j < XJ) *reinterpret_cast<f32x4 *>(&lds_x[buf][big_lds_offset(row, t & 7)]) = gx[j < XJ ? j : 0];
-      if (WT == 0) {
-        *reinterpret_cast<f32x4 *>(&lds_w[buf][big_lds_offset(row, t & 7)]) = gw[j];
+    for (int j = 0; j < XJ; ++j) {
+      __bf16 *dst = &lds_x[buf][0][big_x_offset((t >> 3) + 32 * j, (t & 7) >> 1) + (t & 1) * 4];
+      if (XP == 1) {
+        *reinterpret_cast<bf16x4 *>(dst) = __builtin_convertvector(gx[j] * inv_step, bf16x4);
       } else {
-        const int krow = (t >> 5) + 8 * j;
-        *reinterpret_cast<f32x4 *>(&lds_w[buf][krow * BPITCH_T + (t & 31) * 4]) = gw[j];
+        bf16x4 hi, mid, lo;
+        split_bf16(gx[j], hi, mid, lo);
+        *reinterpret_cast<bf16x4 *>(dst) = hi;
+        *reinterpret_cast<bf16x4 *>(dst + BB * BKS) = mid;
+        *reinterpret_cast<bf16x4 *>(dst + 2 * BB * BKS) = lo;
+        m = max_abs4(m, gx[j]);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < WJ; ++j) {
+      m = max_abs4(m, gw[j]);
+      if (WT == 0) {
+        *reinterpret_cast<f32x4 *>(&lds_w[buf][big_lds_offset((t >> 3) + 32 * j, t & 7)]) = gw[j];
+      } else {
+        *reinterpret_cast<f32x4 *>(&lds_w[buf][(wt_k + WROWS * j) * WPITCH + wt_col]) = gw[j];
+      }
+    }
+    if (!(m < SAFE)) {
+      sh_slow[buf] = s;
+      if (XP == 3) { // rounded up, the upper part of a value at the end of the range would be infinite: cut it off instead
+#pragma unroll
+        for (int j = 0; j < XJ; ++j) {
+          __bf16 *dst = &lds_x[buf][0][big_x_offset((t >> 3) + 32 * j, (t & 7) >> 1) + (t & 1) * 4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float v = gx[j][e];
+            const float hi = fabsf(v) < __builtin_inff() ? __uint_as_float(__float_as_uint(v) & 0xffff0000u) : v;
+            const __bf16 mid = (__bf16)(v - hi);
+            dst[e] = (__bf16)hi;
+            dst[BB * BKS + e] = mid;
+            dst[2 * BB * BKS + e] = (__bf16)(v - hi - (float)mid);
+          }
+        }
       }
     }
   };
 
-  // accumulators of the 2 x 2 MFMA tiles (output block, sample block), named one by one so that they stay in
-  // registers whatever the inlining order
-  floatx16 acc00, acc01, acc10, acc11;
+  floatx16 acc[NB];
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    acc00[i] = 0.0f;
-    acc01[i] = 0.0f;
-    acc10[i] = 0.0f;
-    acc11[i] = 0.0f;
+  for (int i = 0; i < NB; ++i) {
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[i][e] = 0.0f;
   }
 
-  // lane (r, h) multiplies k = 16 h .. 16 h + 15 of a stage, four values at a time; the operands of the next four
-  // are read from LDS before the 16 MFMAs of the current four are issued, so that the reads complete underneath them
-  struct Operands {
-    f32x4 xb0, xb1, wa0, wa1;
-  };
-  // staged offsets of this lane's four operand chunks (rows 32 further on: 32 * BROW floats further on)
-  int x_off[4], w_off[4];
+  // lane (r, h) multiplies k = 16 h .. 16 h + 15 of a stage, eight values per MFMA: the order of k within a stage does
+  // not matter as long as both operands agree
+  int x_off[2], w_off[4];
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    x_off[q] = big_lds_offset(wx * (BB / 2) + blk * 32 + r, h * 4 + q);
-    w_off[q] = big_lds_offset(wy * 64 + r, h * 4 + q);
-  }
-  auto read_operands = [&](int buf, int q, Operands &o) __attribute__((always_inline)) {
-    const int kk = h * 16 + q * 4;
-    o.xb0 = *reinterpret_cast<const f32x4 *>(&lds_x[buf][x_off[q]]);
-    if (NB == 2) o.xb1 = *reinterpret_cast<const f32x4 *>(&lds_x[buf][x_off[q] + 32 * BROW]);
-    if (WT == 0) {
-      o.wa0 = *reinterpret_cast<const f32x4 *>(&lds_w[buf][w_off[q]]);
-      o.wa1 = *reinterpret_cast<const f32x4 *>(&lds_w[buf][w_off[q] + 32 * BROW]);
-    } else {
-      const float *col = &lds_w[buf][kk * BPITCH_T + wy * 64 + r];
-      o.wa0.x = col[0];
-      o.wa0.y = col[BPITCH_T];
-      o.wa0.z = col[2 * BPITCH_T];
-      o.wa0.w = col[3 * BPITCH_T];
-      o.wa1.x = col[32];
-      o.wa1.y = col[BPITCH_T + 32];
-      o.wa1.z = col[2 * BPITCH_T + 32];
-      o.wa1.w = col[3 * BPITCH_T + 32];
-    }
-  };
-  auto multiply = [&](const Operands &o) __attribute__((always_inline)) {
+  for (int q = 0; q < 2; ++q) x_off[q] = big_x_offset(wb * (BB / WB) + r, h * 2 + q);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      acc00 = __builtin_amdgcn_mfma_f32_32x32x2f32(o.wa0[e], o.xb0[e], acc00, 0, 0, 0);
-      if (NB == 2) acc01 = __builtin_amdgcn_mfma_f32_32x32x2f32(o.wa0[e], o.xb1[e], acc01, 0, 0, 0);
-      acc10 = __builtin_amdgcn_mfma_f32_32x32x2f32(o.wa1[e], o.xb0[e], acc10, 0, 0, 0);
-      if (NB == 2) acc11 = __builtin_amdgcn_mfma_f32_32x32x2f32(o.wa1[e], o.xb1[e], acc11, 0, 0, 0);
-    }
+  for (int q = 0; q < 4; ++q) w_off[q] = big_lds_offset(wo * 32 + r, h * 4 + q);
+  auto read_w = [&](int buf, int q) __attribute__((always_inline)) { // k = 16 h + 4 q .. + 3 of this lane's output
+    if (WT == 0) return *reinterpret_cast<const f32x4 *>(&lds_w[buf][w_off[q]]);
+    const float *col = &lds_w[buf][(h * 16 + q * 4) * WPITCH + wo * 32 + r];
+    f32x4 v;
+    v.x = col[0];
+    v.y = col[WPITCH];
+    v.z = col[2 * WPITCH];
+    v.w = col[3 * WPITCH];
+    return v;
+  };
+  auto read_x = [&](int buf, int plane, int j, int nb) __attribute__((always_inline)) { // 32 rows further on: 8 lines
+    return *reinterpret_cast<const bf16x8 *>(&lds_x[buf][plane][x_off[j] + nb * 32 * BKS]);
   };
   auto compute = [&](int buf) __attribute__((always_inline)) {
-    Operands even, odd;
-    read_operands(buf, 0, even);
-    read_operands(buf, 1, odd);
-    multiply(even);
-    mvm_big_schedule<WT, NB>();
-    read_operands(buf, 2, even);
-    multiply(odd);
-    mvm_big_schedule<WT, NB>();
-    read_operands(buf, 3, odd);
-    multiply(even);
-    mvm_big_schedule<WT, NB>();
-    multiply(odd);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      bf16x8 x[NB][XP];
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) {
+#pragma unroll
+        for (int p = 0; p < XP; ++p) x[nb][p] = read_x(buf, p, j, nb);
+      }
+      bf16x4 h0, m0, l0, h1, m1, l1;
+      split_bf16(read_w(buf, 2 * j), h0, m0, l0);
+      split_bf16(read_w(buf, 2 * j + 1), h1, m1, l1);
+      const bf16x8 w[3] = {__builtin_shufflevector(h0, h1, 0, 1, 2, 3, 4, 5, 6, 7),
+                           __builtin_shufflevector(m0, m1, 0, 1, 2, 3, 4, 5, 6, 7),
+                           __builtin_shufflevector(l0, l1, 0, 1, 2, 3, 4, 5, 6, 7)};
+#pragma unroll
+      for (int p = 0; p < XP; ++p) {
+#pragma unroll
+        for (int q = 0; q + p < 3; ++q) {
+#pragma unroll
+          for (int nb = 0; nb < NB; ++nb) {
+            acc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[q], x[nb][p], acc[nb], 0, 0, 0);
+          }
+        }
+      }
+    }
+  };
+  auto compute_fp32 = [&](int buf) __attribute__((always_inline)) { // the parts of an input add up to it again
+#pragma unroll 1
+    for (int e = 0; e < 16; ++e) {
+      const int k = h * 16 + e;
+      const float w = WT ? lds_w[buf][k * WPITCH + wo * 32 + r] : lds_w[buf][big_lds_offset(wo * 32 + r, k >> 2) + (k & 3)];
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) {
+        float x = 0.0f;
+#pragma unroll
+        for (int p = XP - 1; p >= 0; --p) {
+          const float part = (float)lds_x[buf][p][big_x_offset(wb * (BB / WB) + nb * 32 + r, k >> 3) + (k & 7)];
+          x = (p == 0 && !(fabsf(part) < __builtin_inff())) ? part : x + part; // an infinity's lower parts are NaN
+        }
+        acc[nb] = __builtin_amdgcn_mfma_f32_32x32x2f32(w, x, acc[nb], 0, 0, 0);
+      }
+    }
   };
 
   const int stages = a.k_pad / BKS;
+  if (t < 2) sh_slow[t] = -1;
+  __syncthreads();
   {
-    f32x4 gx[XJ], gw[4];
+    f32x4 gx[XJ], gw[WJ];
     gload(0, gx, gw);
     lds_store(0, gx, gw);
     __syncthreads();
     for (int s = 0; s < stages; ++s) {
       const bool next = s + 1 < stages;
       if (next) gload(s + 1, gx, gw);
-      compute(NBUF == 1 ? 0 : s & 1);
-      if (NBUF == 1 && next) __syncthreads(); // every wave is done with the one buffer
-      if (next) lds_store(NBUF == 1 ? 0 : (s + 1) & 1, gx, gw);
+      if (__builtin_expect(__builtin_amdgcn_readfirstlane(sh_slow[s & 1]) == s, 0)) compute_fp32(s & 1);
+      else compute(s & 1);
+      if (next) lds_store(s + 1, gx, gw);
       __syncthreads();
     }
   }
 
-  // ADC stage: lane (r, h) of wave (wy, wx) holds, for its 2 x 2 tiles, sample column r and output rows
-  // g * 8 + h * 4 + q of each tile
+  // ADC stage: lane (r, h) of a wave holds, for each of its NB blocks, sample column r and output rows g * 8 + h * 4 + q
   if (t < 2 * BB) sh_hits[t] = 0;
   __syncthreads();
   const bool flags = !a.io.perfect && a.io.bound_management != RPU_BM_NONE;
-  // sample block bi of this wave: its two output blocks
-  auto finish_block = [&](const int bi, const floatx16 &acc_o0, const floatx16 &acc_o1) __attribute__((always_inline)) {
-    const int local_b = wx * (BB / 2) + bi * 32 + r;
+  auto finish_block = [&](const int nb, const floatx16 &sums) __attribute__((always_inline)) {
+    const int local_b = wb * (BB / WB) + nb * 32 + r;
     const int slot = tile_b * BB + local_b;
-    if (slot >= n_act) return;
-    int b_out = slot;
-    float fin_out = 1.0f;
-    if (!a.io.perfect) {
-      if (round > 0) b_out = pick2(a.st.list, round & 1)[slot];
-      fin_out = a.st.fin[b_out];
-    }
-    int up_max = 0, lo_max = 0;
-#pragma unroll
-    for (int oi = 0; oi < 2; ++oi) {
+    if (slot < n_act) {
+      int b_out = slot;
+      float fin_out = 1.0f;
+      if (!a.io.perfect) {
+        if (round > 0) b_out = pick2(a.st.list, round & 1)[slot];
+        fin_out = a.st.fin[b_out];
+      }
+      int up_max = 0, lo_max = 0;
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
-        const int o0 = tile_o * BT + wy * 64 + oi * 32 + g * 8 + h * 4;
+        const int o0 = tile_o * OT + wo * 32 + g * 8 + h * 4;
         float v[4];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) v[q] = oi ? acc_o1[4 * g + q] : acc_o0[4 * g + q];
+        for (int q = 0; q < 4; ++q) v[q] = XP == 1 ? sums[4 * g + q] * a.x_step : sums[4 * g + q];
         int up = 0, lo = 0;
         if (o0 < a.O) mvm_finish_outputs(a, round, b_out, fin_out, o0, v, up, lo);
         up_max = max(up_max, up);
         lo_max = max(lo_max, lo);
       }
-    }
-    if (flags) {
-      if (up_max) atomicMax(&sh_hits[local_b], up_max);
-      if (lo_max) atomicMax(&sh_hits[BB + local_b], lo_max);
+      if (flags) {
+        if (up_max) atomicMax(&sh_hits[local_b], up_max);
+        if (lo_max) atomicMax(&sh_hits[BB + local_b], lo_max);
+      }
     }
   };
-  finish_block(blk, acc00, acc10);
-  if (NB == 2) finish_block(1, acc01, acc11);
+  finish_block(0, acc[0]); // call by call: a loop over the blocks is too long to be unrolled, and would index registers
+  if (NB > 1) finish_block(1, acc[NB > 1 ? 1 : 0]);
+  if (NB > 2) finish_block(2, acc[NB > 2 ? 2 : 0]);
+  if (NB > 3) finish_block(3, acc[NB > 3 ? 3 : 0]);
   if (!flags) return;
   __syncthreads();
   if (t < 2 * BB) {
@@ -1880,7 +1935,6 @@ __device__ __forceinline__ void mvm_big_workgroup(const MvmArgs &a, const int ro
   // the last workgroup of this sample tile decides which of its samples go on (see mvm_tile_finished)
   __syncthreads();
   if (t == 0) {
-    const int tiles_o = (a.O + BT - 1) / BT;
     const int tiles_b = (a.m_batch + BB - 1) / BB;
     const int prev = atomicAdd(&a.st.tile_done[round * tiles_b + tile_b], 1);
     sh_last = (prev == tiles_o - 1) ? 1 : 0;
@@ -1916,30 +1970,19 @@ __device__ __forceinline__ void mvm_big_workgroup(const MvmArgs &a, const int ro
   }
 }
 
-template <int WT, int BB>
+template <int WT, int BB, int WO, int XP, bool LAZY>
 __global__ __launch_bounds__(256, 2) void k_mvm_big(MvmArgs a, int min_active) {
-  mvm_big_workgroup<WT, BB>(a, a.round, (int)blockIdx.x, min_active);
-}
-template <int BB>
-__global__ __launch_bounds__(256, 3) void k_mvm_big_short(MvmArgs a, int min_active) {
-  mvm_big_workgroup<1, BB, false, 1>(a, a.round, (int)blockIdx.x, min_active);
-}
-__global__ __launch_bounds__(256, 2) void k_mvm_big_narrow(MvmArgs a, int min_active) {
-  mvm_big_workgroup<0, 128, true, 2, true>(a, a.round, (int)blockIdx.x, min_active);
-}
-template <int WT, int BB>
-__global__ __launch_bounds__(256, 2) void k_mvm_big_lazy(MvmArgs a, int min_active) {
-  mvm_big_workgroup<WT, BB, false, 2, true>(a, a.round, (int)blockIdx.x, min_active);
+  mvm_big_workgroup<WT, BB, WO, XP, LAZY>(a, a.round, (int)blockIdx.x, min_active);
 }
 
 // several tiles in one launch (round 0): a tile that is not run by this kernel has no workgroups in the table
-template <int WT, int BB>
+template <int WT, int BB, int XP>
 __global__ __launch_bounds__(256, 2) void k_mvm_big_group(MvmGroup g, int round) {
   int t = 0;
   while (t + 1 < g.n && (int)blockIdx.x >= g.start[t + 1]) ++t;
   const MvmArgs &a = g.args[t];
   if (round > 0 && round >= a.max_rounds) return;
-  mvm_big_workgroup<WT, BB>(a, round, (int)blockIdx.x - g.start[t], 0);
+  mvm_big_workgroup<WT, BB, 4, XP, false>(a, round, (int)blockIdx.x - g.start[t], 0);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -2376,6 +2419,17 @@ int mvm_max_rounds(const IoDev &io) {
   return rounds > 32 ? 32 : rounds;
 }
 
+// The DAC step if every quantized input is a multiple k of it with |k| <= 256 up to rounding (a bf16 holds those k), 0
+// otherwise: no input noise or asymmetry on top, and an input range that is itself a multiple of the step, because
+// values beyond it are clipped to the range.
+float mvm_input_step(const IoDev &io) {
+  if (io.perfect || !(io.inp_res > 0.0f) || io.inp_noise > 0.0f || io.inp_asym != 0.0f) return 0.0f;
+  const double steps = (double)io.inp_bound / (double)io.inp_res;
+  if (!(steps >= 1.0 && steps < 256.5) || std::fabs(steps - std::rint(steps)) > 1e-6 * steps) return 0.0f;
+  if (!(io.inp_res > 0x1p-60f && io.inp_res < 0x1p60f)) return 0.0f;
+  return io.inp_res;
+}
+
 // prefetch depth used for a contraction length: deep for long contractions, where each of the few
 // resident waves must cover the memory latency alone
 static int mvm_prefetch_depth(int K, int k_pad) {
@@ -2476,15 +2530,21 @@ int mvm_big_sample_tile(int workgroups_128, int n_cus) {
   return 10 * idle <= rounds * slots ? 128 : 64;
 }
 
-void launch_mvm_big_group(const MvmGroup &g, int total_workgroups, int bb, bool w_oc, hipStream_t s) {
+void launch_mvm_big_group(const MvmGroup &g, int total_workgroups, int bb, bool w_oc, bool stepped, hipStream_t s) {
   const dim3 grid(total_workgroups);
+#define RPU_LAUNCH_BIG(WT, BB) \
+  do { \
+    if (stepped) hipLaunchKernelGGL((k_mvm_big_group<WT, BB, 1>), grid, dim3(256), 0, s, g, 0); \
+    else hipLaunchKernelGGL((k_mvm_big_group<WT, BB, 3>), grid, dim3(256), 0, s, g, 0); \
+  } while (0)
   if (bb == 128) {
-    if (w_oc) hipLaunchKernelGGL((k_mvm_big_group<1, 128>), grid, dim3(256), 0, s, g, 0);
-    else hipLaunchKernelGGL((k_mvm_big_group<0, 128>), grid, dim3(256), 0, s, g, 0);
+    if (w_oc) RPU_LAUNCH_BIG(1, 128);
+    else RPU_LAUNCH_BIG(0, 128);
   } else {
-    if (w_oc) hipLaunchKernelGGL((k_mvm_big_group<1, 64>), grid, dim3(256), 0, s, g, 0);
-    else hipLaunchKernelGGL((k_mvm_big_group<0, 64>), grid, dim3(256), 0, s, g, 0);
+    if (w_oc) RPU_LAUNCH_BIG(1, 64);
+    else RPU_LAUNCH_BIG(0, 64);
   }
+#undef RPU_LAUNCH_BIG
 }
 
 // samples of a round from which the large-tile kernel takes over, 0 when a call of this shape never uses it: it
@@ -2659,31 +2719,31 @@ void launch_mvm_round(const MvmArgs &a_in, hipStream_t s) {
   // the round is one launch
   if (a.round > 0 && !a.speculate) a.big_from = 0;
   if (a.big_from > 0) {
-    // the variants below exist for the way a tile that stores [d_size][x_size] addresses its weights (forward: rows
-    // along k, backward: rows along the outputs); the other storage takes the general kernels where its case has none
     const bool lazy = !a.transposed && !a.speculate && a.max_rounds > 1;
-    const bool narrow = !a.transposed && !a.w_oc && a.O <= 64; // see mvm_big_workgroup
+    const bool narrow = a.O <= 64; // see mvm_big_workgroup, WO
     const int bb = narrow ? 128 : mvm_big_sample_tile(big_workgroups(a, 128), current_device_cus());
     const dim3 big_grid(big_workgroups(a, bb));
     const int min_active = a.round > 0 ? a.big_from : 0;
-    if (narrow) {
-      hipLaunchKernelGGL(k_mvm_big_narrow, big_grid, dim3(256), 0, s, a, min_active);
-    } else if (lazy && !a.w_oc) {
-      if (bb == 128) hipLaunchKernelGGL((k_mvm_big_lazy<0, 128>), big_grid, dim3(256), 0, s, a, min_active);
-      else hipLaunchKernelGGL((k_mvm_big_lazy<0, 64>), big_grid, dim3(256), 0, s, a, min_active);
-    } else if (lazy) {
-      if (bb == 128) hipLaunchKernelGGL((k_mvm_big_lazy<1, 128>), big_grid, dim3(256), 0, s, a, min_active);
-      else hipLaunchKernelGGL((k_mvm_big_lazy<1, 64>), big_grid, dim3(256), 0, s, a, min_active);
-    } else if (a.transposed && a.w_oc && a.k_pad <= 2 * BKS) { // see mvm_big_workgroup, NBUF
-      if (bb == 128) hipLaunchKernelGGL((k_mvm_big_short<128>), big_grid, dim3(256), 0, s, a, min_active);
-      else hipLaunchKernelGGL((k_mvm_big_short<64>), big_grid, dim3(256), 0, s, a, min_active);
-    } else if (bb == 128) {
-      if (a.w_oc) hipLaunchKernelGGL((k_mvm_big<1, 128>), big_grid, dim3(256), 0, s, a, min_active);
-      else hipLaunchKernelGGL((k_mvm_big<0, 128>), big_grid, dim3(256), 0, s, a, min_active);
+#define RPU_LAUNCH_BIG(WT, BB, WO, XP, LAZY) \
+  hipLaunchKernelGGL((k_mvm_big<WT, BB, WO, XP, LAZY>), big_grid, dim3(256), 0, s, a, min_active)
+#define RPU_PICK_BIG(WT, XP) \
+  do { \
+    if (narrow && lazy) RPU_LAUNCH_BIG(WT, 128, 2, XP, true); \
+    else if (narrow) RPU_LAUNCH_BIG(WT, 128, 2, XP, false); \
+    else if (bb == 128 && lazy) RPU_LAUNCH_BIG(WT, 128, 4, XP, true); \
+    else if (bb == 128) RPU_LAUNCH_BIG(WT, 128, 4, XP, false); \
+    else if (lazy) RPU_LAUNCH_BIG(WT, 64, 4, XP, true); \
+    else RPU_LAUNCH_BIG(WT, 64, 4, XP, false); \
+  } while (0)
+    if (a.x_step > 0.0f) {
+      if (a.w_oc) RPU_PICK_BIG(1, 1);
+      else RPU_PICK_BIG(0, 1);
     } else {
-      if (a.w_oc) hipLaunchKernelGGL((k_mvm_big<1, 64>), big_grid, dim3(256), 0, s, a, min_active);
-      else hipLaunchKernelGGL((k_mvm_big<0, 64>), big_grid, dim3(256), 0, s, a, min_active);
+      if (a.w_oc) RPU_PICK_BIG(1, 3);
+      else RPU_PICK_BIG(0, 3);
     }
+#undef RPU_PICK_BIG
+#undef RPU_LAUNCH_BIG
     if (a.round == 0) return; // later rounds: whichever kernel the number of listed samples calls for
   }
   const int all = mvm_round_workgroups(a);

@@ -598,6 +598,7 @@ struct Tile {
     a.transposed = transposed ? 1 : 0;
     mvm_set_weights(a, w_other ? w_other : wdev(), w_ld(), xd);
     a.io = io_dev(io);
+    a.x_step = mvm_input_step(a.io);
     a.alpha = io.p.out_scale; a.beta = 0.0f;
     a.key = key(); a.call = call++;
     a.st.next_scale[0] = s_nsc0.p; a.st.next_scale[1] = s_nsc1.p;
@@ -2716,6 +2717,7 @@ static int group_mvm(rpu_group_t *group, const float *const *x_dev, const long *
     // with the half tiles, one workgroup on every second CU already beats the 32 x 32 kernel
     const bool use_big = big_total >= (big_bb == 128 ? 256 : 128);
     bool all_big = use_big;
+    bool all_stepped = true; // of the tiles on the large-tile kernel (MvmArgs::x_step)
     // per tile: arguments of a plain forward call (row-major x [m_batch][x_size], y [m_batch][d_size])
     std::vector<MvmArgs> args(n);
     std::vector<int> depth(n), mode(n);
@@ -2736,6 +2738,7 @@ static int group_mvm(rpu_group_t *group, const float *const *x_dev, const long *
       if (a.in_sb < in_size || a.out_sb < out_size) throw RpuError("A row stride is shorter than the row.");
       a.big_from = big ? -1 : 0;
       if (!big) all_big = false;
+      else if (a.x_step <= 0.0f) all_stepped = false;
       mvm_round_variant(a, depth[i], mode[i]);
       rounds = std::max(rounds, a.max_rounds);
       args[i] = a;
@@ -2852,7 +2855,7 @@ static int group_mvm(rpu_group_t *group, const float *const *x_dev, const long *
     for (int r = 0; r < rounds; ++r) {
       if (use_big && r == 0) {
         MvmGroup g{group->d_args.p, group->d_start.p + big_offset, n, m_batch};
-        launch_mvm_big_group(g, big_total, big_bb, transposed != storage_xd, s);
+        launch_mvm_big_group(g, big_total, big_bb, transposed != storage_xd, all_stepped, s);
         if (all_big) continue;
       }
       for (size_t k = 0; k < segments.size(); ++k) {

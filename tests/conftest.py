@@ -27,7 +27,8 @@ def gpu_device():
 # shared tensor, as the reference's Python binds every CUDA tile (the library then works on that layout in place)
 BOTH_STORAGES = ("test_gpu_parity", "test_gpu_statistics", "test_gpu_benchmark_configs", "test_gpu_fused_rounds",
                  "test_gpu_group_update", "test_gpu_inference", "test_gpu_indexed", "test_gpu_long_batches",
-                 "test_gpu_state", "test_gpu_hwa", "test_zz_no_alloc", "test_gpu_pulse_stream")
+                 "test_gpu_state", "test_gpu_hwa", "test_zz_no_alloc", "test_gpu_pulse_stream",
+                 "test_gpu_large_tiles")
 
 
 def pytest_generate_tests(metafunc):

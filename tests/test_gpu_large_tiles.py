@@ -1,0 +1,89 @@
+"""Contraction of the large-tile kernel on the bf16 matrix pipe (operands split into bf16 parts without loss) against
+64-bit sums: inputs on the DAC grid (one part), any other inputs (three parts), and values that only the fp32 pipe takes."""
+import numpy as np
+import pytest
+import torch
+
+from helpers import make_meta, noise_free_io
+from aihwkit_amd.rpu_base import devices as dv
+from aihwkit_amd.rpu_base import tiles
+
+pytestmark = pytest.mark.gpu
+
+# tile edges of 64 and 128 outputs and 64 and 128 samples, contraction stages of 32, each with a remainder
+SHAPES = [(33, 64, 16384), (65, 65, 16400), (433, 48, 16500), (31, 129, 1536), (160, 130, 1601), (513, 257, 2049),
+          (1024, 128, 8193), (96, 1000, 8192)]
+
+
+def _tile(x_size, d_size, io, w):
+    meta = make_meta(io, io, pulse_type=dv.PulseType.NONE)
+    host = meta.create_array(x_size, d_size, dv.IdealResistiveDeviceParameter())
+    host.set_weights(torch.from_numpy(w))
+    return tiles.CudaAnalogTile(host)
+
+
+def _close(got, want, terms, lengths):
+    """A sum of n products in fp32 is off by at most (n + 2) half units of the sum of the absolute products; random signs
+    leave far less than a quarter of that bound."""
+    bound = 0.25 * (lengths + 2) * 2.0 ** -24 * terms + 1e-37
+    assert np.all(np.abs(got.double().cpu().numpy() - want) <= bound)
+
+
+@pytest.mark.parametrize("scale", [0.3, 1e-12, 1e10])
+@pytest.mark.parametrize("x_size,d_size,batch", SHAPES)
+def test_unquantized_products_against_64_bit_sums(gpu_device, x_size, d_size, batch, scale):
+    rng = np.random.default_rng(x_size)
+    io = noise_free_io()
+    io.is_perfect = True
+    w = (scale * rng.standard_normal((d_size, x_size))).astype(np.float32)
+    tile = _tile(x_size, d_size, io, w)
+    x = rng.standard_normal((batch, x_size)).astype(np.float32)
+    d = rng.standard_normal((batch, d_size)).astype(np.float32)
+    w64 = w.astype(np.float64)
+    _close(tile.forward(torch.from_numpy(x).cuda()), x @ w64.T, np.abs(x) @ np.abs(w64).T, x_size)
+    _close(tile.backward(torch.from_numpy(d).cuda()), d @ w64, np.abs(d) @ np.abs(w64), d_size)
+
+
+@pytest.mark.parametrize("x_size,d_size,batch", SHAPES)
+@pytest.mark.parametrize("steps", [63, 256, 300])  # of the DAC on either side of zero: the last is not held by one bf16
+def test_quantized_products_against_64_bit_sums(gpu_device, x_size, d_size, batch, steps):
+    rng = np.random.default_rng(d_size)
+    io = noise_free_io(inp_res=1.0 / (2 * steps))
+    io.out_res, io.out_bound = -1.0, float("inf")
+    w = rng.uniform(-0.6, 0.6, (d_size, x_size)).astype(np.float32)
+    tile = _tile(x_size, d_size, io, w)
+    w64 = w.astype(np.float64)
+    step = np.float32(2.0 * np.float32(1.0 / (2 * steps)))  # the range is [-1, 1]
+    for call, width, axis in ((tile.forward, x_size, w64.T), (tile.backward, d_size, w64)):
+        v = rng.uniform(-1.0, 1.0, (batch, width)).astype(np.float32)
+        # away from the middle between two steps, where the fp32 quotient may round to either; the range itself is met
+        k = np.rint(v / step)
+        v = ((k + np.clip(v / step - k, -0.4, 0.4)) * step).astype(np.float32)
+        v[:, 0] = 1.0
+        q = np.clip(np.rint(v / step), -steps, steps).astype(np.float64) * float(step)
+        got = call(torch.from_numpy(v).cuda())
+        # the reference's own rounding of k * step and of the clipped range: one half unit per product
+        _close(got, q @ axis, np.abs(q) @ np.abs(axis), 4 * width + 16)
+
+
+@pytest.mark.parametrize("x_size,d_size,batch", [(100, 50, 16500), (256, 256, 2048), (300, 300, 8192)])
+def test_values_out_of_the_range_of_the_parts(gpu_device, x_size, d_size, batch):
+    """Infinities, NaN and values near the end of the fp32 range give what fp32 products give."""
+    rng = np.random.default_rng(1)
+    io = noise_free_io()
+    io.is_perfect = True
+    w = rng.uniform(-0.5, 0.5, (d_size, x_size)).astype(np.float32)
+    w[3, 7], w[40, 9], w[5, 5], w[6, 6], w[7, -1] = np.inf, -np.inf, 3.4e38, np.nan, 2e38
+    tile = _tile(x_size, d_size, io, w)
+    x = (rng.random((batch, x_size)) + 0.5).astype(np.float32)
+    x[10, 3], x[11, 3], x[12, 1], x[13, 0] = np.inf, 3e38, np.nan, -np.inf
+    with np.errstate(all="ignore"):
+        want = (x.astype(np.float64) @ w.astype(np.float64).T).astype(np.float32)
+    got = tile.forward(torch.from_numpy(x).cuda()).cpu().numpy()
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
+    fine = np.isfinite(want)
+    # the bound of _close: where products of 1e38 cancel, the error is relative to them and not to what is left
+    with np.errstate(all="ignore"):
+        bound = (x_size + 2) * 2.0 ** -24 * (np.abs(x.astype(np.float64)) @ np.abs(w.astype(np.float64)).T)
+        assert np.all((np.abs(got.astype(np.float64) - want) <= bound + 1e-37)[fine])
