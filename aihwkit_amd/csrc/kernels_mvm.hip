@@ -24,8 +24,8 @@
 //   k_mvm_round_tail   later rounds of a launch whose full grid would be large: a fixed number of workgroups walk
 //                  the tiles of the samples that are listed (usually few).
 //   k_mvm_big      large batches on wide tiles: 128 x 128 workgroup tiles, both operands staged through LDS, the product
-//                  on the bf16 matrix pipe with operands split into bf16 parts without loss; same state / epilogue / random streams; a round is
-//                  run by this or by the 32 x 32 kernel, by the number of samples it lists.
+//                  on the bf16 matrix pipe with operands split into bf16 parts without loss; same state / epilogue /
+//                  random streams; a round is run by this or by the 32 x 32 kernel, by the number of samples it lists.
 //   k_conv_forward convolution forward of a narrow tile (at most 32 outputs): unfold by the index matrix, noise
 //                  management, DAC, contraction, ADC and the bound-management rounds in one kernel.
 //   *_group        the same kernels over the tiles of a group in one launch.
@@ -1613,7 +1613,6 @@ __device__ __forceinline__ void big_prepare_next_rows(const MvmArgs &a, int roun
   }
 }
 
-typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 // Offset (in bf16) of 16-byte chunk `chunk` (8 values, 0 .. 3) of staged input row `row`: four rows of 64 bytes fill a
@@ -1622,17 +1621,32 @@ __device__ __forceinline__ int big_x_offset(int row, int chunk) {
   return (row >> 2) * 128 + (((row & 3) << 2) + ((chunk + (row >> 2)) & 3)) * 8;
 }
 
-// v = hi + mid + lo with every part rounded to bf16: 3 x 8 bits hold the 24 of a float, so the sum is exact (above
-// 2^-110; the low part of a smaller value may drop out)
-__device__ __forceinline__ void split_bf16(const f32x4 v, bf16x4 &hi, bf16x4 &mid, bf16x4 &lo) {
-  hi = __builtin_convertvector(v, bf16x4);
-  const f32x4 r1 = v - __builtin_convertvector(hi, f32x4);
-  mid = __builtin_convertvector(r1, bf16x4);
-  const f32x4 r2 = r1 - __builtin_convertvector(mid, f32x4);
-  lo = __builtin_convertvector(r2, bf16x4);
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ uint32_t pack_bf16(float lower, float upper) { // both rounded to nearest even
+  uint32_t p;
+  asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(p) : "v"(lower), "v"(upper));
+  return p;
 }
-__device__ __forceinline__ float max_abs4(float m, const f32x4 v) {
-  return fmaxf(fmaxf(m, fmaxf(fabsf(v.x), fabsf(v.y))), fmaxf(fabsf(v.z), fabsf(v.w)));
+// v = hi + mid + lo with every part rounded to bf16: 3 x 8 bits hold the 24 of a float, so the sum is exact (above
+// 2^-110; the low part of a smaller value may drop out).  On the packed pairs: written with conversions of the single
+// parts, the compiler rounds every value a second time before it widens it again.
+__device__ __forceinline__ void split_bf16(const f32x4 v, u32x2 &hi, u32x2 &mid, u32x2 &lo) {
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const float a = v[2 * i], b = v[2 * i + 1];
+    hi[i] = pack_bf16(a, b);
+    const float a1 = a - __uint_as_float(hi[i] << 16), b1 = b - __uint_as_float(hi[i] & 0xffff0000u);
+    mid[i] = pack_bf16(a1, b1);
+    lo[i] = pack_bf16(a1 - __uint_as_float(mid[i] << 16), b1 - __uint_as_float(mid[i] & 0xffff0000u));
+  }
+}
+__device__ __forceinline__ float max_abs4(float m, const f32x4 v) { // NaN do not count
+  // two instructions; the compiler quiets every operand of fmaxf first, eight more
+  asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(m) : "v"(v.x), "v"(v.y));
+  asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(m) : "v"(v.z), "v"(v.w));
+  return m;
 }
 
 // work of workgroup number n of a large-tile round launch of one tile; BB: samples of a workgroup tile (128 or 64)
@@ -1644,8 +1658,9 @@ __device__ __forceinline__ float max_abs4(float m, const f32x4 v) {
 //           rows hold k * step, k is what is staged, and the step multiplies the finished sum.  3 exact products of 8 x 8
 //           bits per element against the one rounded input k * step of the fp32 pipe;
 //   XP = 3  three for any other input, of whose nine products the three below 2^-24 of the whole are left out.
-// Sums are kept in fp32 as before, in chains an eighth as long.  A stage with a value outside the range in which the
-// parts and their products are safe (infinities among them, whose parts would be NaN) is multiplied on the fp32 pipe.
+// Sums are kept in fp32 as before, in chains an eighth as long.  A tile with a value outside the range in which the
+// parts and their products are safe (infinities among them, whose parts would be NaN) is multiplied again on the fp32
+// pipe; choosing the pipe stage by stage inside the loop cost a copy of all accumulators per stage.
 // LAZY (calls with speculate = 0): nothing is quantized ahead; the last workgroup of a sample tile writes the rows of
 // the samples that go on.  The other instantiations always quantize ahead, as their callers ask for.
 template <int WT, int BB, int WO, int XP, bool LAZY>
@@ -1664,7 +1679,7 @@ __device__ __forceinline__ void mvm_big_workgroup(const MvmArgs &a, const int ro
   __shared__ int sh_b[BB];
   __shared__ float sh_scale[BB];
   __shared__ int sh_last;
-  __shared__ int sh_slow[2]; // the last stage in this buffer that the fp32 pipe has to multiply
+  __shared__ int sh_slow; // whether the fp32 pipe has to multiply this tile
 
   const int n_act = (round > 0) ? a.st.count[round] : a.m_batch;
   if (n_act < min_active) return; // this round is run by the 32 x 32 kernel
@@ -1705,92 +1720,70 @@ __device__ __forceinline__ void mvm_big_workgroup(const MvmArgs &a, const int ro
   const int wt_k = t / (OT / 4);
   const int wt_col = (t % (OT / 4)) * 4;
   const int wt_o = tile_o * OT + wt_col; // WT = 1: first of this thread's four outputs
+  // a thread whose four outputs reach past the last one reads the last four of the row and moves them into place (what
+  // it then holds for outputs that do not exist is never used)
+  const int wt_shift = wt_o - min(wt_o, a.O - 4);
+  const bool wt_ragged = tile_o * OT + OT > a.O && (a.O & 3) != 0; // the same for the whole workgroup
+  const float *wt_src = a.w + (long)wt_k * a.w_ld + (wt_o - wt_shift);
+  const long wt_step = (long)WROWS * a.w_ld; // from one of the thread's rows to the next
 
   auto gload = [&](int s, f32x4 (&gx)[XJ], f32x4 (&gw)[WJ]) __attribute__((always_inline)) {
     const int k0 = s * BKS;
 #pragma unroll
     for (int j = 0; j < XJ; ++j) gx[j] = *reinterpret_cast<const f32x4 *>(x_src[j] + k0);
-    if (WT == 0) {
+    if (k0 + BKS <= K) {
+#pragma unroll
+      for (int j = 0; j < WJ; ++j) {
+        if (WT == 0) gw[j] = *reinterpret_cast<const f32x4_unaligned *>(w_src[j] + k0 + st_col);
+        else gw[j] = *reinterpret_cast<const f32x4_unaligned *>(wt_src + (long)k0 * a.w_ld + j * wt_step);
+      }
+    } else if (WT == 0) {
       const int kc = k0 + st_col;
-      if (kc + 4 <= K) {
 #pragma unroll
-        for (int j = 0; j < WJ; ++j) gw[j] = *reinterpret_cast<const f32x4_unaligned *>(w_src[j] + kc);
-      } else {
+      for (int j = 0; j < WJ; ++j) {
 #pragma unroll
-        for (int j = 0; j < WJ; ++j) {
-          f32x4 z;
-          z.x = (kc < K) ? w_src[j][kc] : 0.0f;
-          z.y = (kc + 1 < K) ? w_src[j][kc + 1] : 0.0f;
-          z.z = (kc + 2 < K) ? w_src[j][kc + 2] : 0.0f;
-          z.w = 0.0f;
-          gw[j] = z;
-        }
+        for (int e = 0; e < 4; ++e) gw[j][e] = (kc + e < K) ? w_src[j][kc + e] : 0.0f;
       }
     } else {
 #pragma unroll
       for (int j = 0; j < WJ; ++j) {
-        const int k = min(k0 + wt_k + WROWS * j, K - 1); // rows past K meet the zero padding of the inputs
-        const float *row = a.w + (long)k * a.w_ld;
-        if (wt_o + 4 <= a.O) {
-          gw[j] = *reinterpret_cast<const f32x4_unaligned *>(row + wt_o);
-        } else {
-          f32x4 z;
-          z.x = (wt_o < a.O) ? row[wt_o] : 0.0f;
-          z.y = (wt_o + 1 < a.O) ? row[wt_o + 1] : 0.0f;
-          z.z = (wt_o + 2 < a.O) ? row[wt_o + 2] : 0.0f;
-          z.w = 0.0f;
-          gw[j] = z;
-        }
+        const int over = max(k0 + wt_k + WROWS * j - (K - 1), 0); // rows past K meet the zero padding of the inputs
+        gw[j] = *reinterpret_cast<const f32x4_unaligned *>(wt_src + (long)(k0 - over) * a.w_ld + j * wt_step);
       }
     }
   };
   // k * step times 1 / step is k up to a few units in the 24th bit: rounding to bf16 returns k itself
   const float inv_step = XP == 1 ? 1.0f / a.x_step : 1.0f;
   constexpr float SAFE = XP == 1 ? 0x1p100f : 0x1p60f; // parts and products stay finite below it
-  auto lds_store = [&](int s, const f32x4 (&gx)[XJ], const f32x4 (&gw)[WJ]) __attribute__((always_inline)) {
-    const int buf = s & 1;
+  auto lds_store = [&](int buf, const f32x4 (&gx)[XJ], const f32x4 (&gw)[WJ]) __attribute__((always_inline)) {
     float m = 0.0f;
 #pragma unroll
     for (int j = 0; j < XJ; ++j) {
       __bf16 *dst = &lds_x[buf][0][big_x_offset((t >> 3) + 32 * j, (t & 7) >> 1) + (t & 1) * 4];
       if (XP == 1) {
-        *reinterpret_cast<bf16x4 *>(dst) = __builtin_convertvector(gx[j] * inv_step, bf16x4);
+        const f32x4 k = gx[j] * inv_step;
+        *reinterpret_cast<u32x2 *>(dst) = u32x2{pack_bf16(k.x, k.y), pack_bf16(k.z, k.w)};
       } else {
-        bf16x4 hi, mid, lo;
+        u32x2 hi, mid, lo;
         split_bf16(gx[j], hi, mid, lo);
-        *reinterpret_cast<bf16x4 *>(dst) = hi;
-        *reinterpret_cast<bf16x4 *>(dst + BB * BKS) = mid;
-        *reinterpret_cast<bf16x4 *>(dst + 2 * BB * BKS) = lo;
+        *reinterpret_cast<u32x2 *>(dst) = hi;
+        *reinterpret_cast<u32x2 *>(dst + BB * BKS) = mid;
+        *reinterpret_cast<u32x2 *>(dst + 2 * BB * BKS) = lo;
         m = max_abs4(m, gx[j]);
       }
     }
 #pragma unroll
     for (int j = 0; j < WJ; ++j) {
-      m = max_abs4(m, gw[j]);
+      f32x4 w = gw[j];
+      if (WT == 1 && wt_ragged && wt_shift > 0) w = {wt_shift == 1 ? w.y : (wt_shift == 2 ? w.z : w.w), wt_shift == 1 ? w.z : w.w, w.w, w.w};
+      m = max_abs4(m, w);
       if (WT == 0) {
-        *reinterpret_cast<f32x4 *>(&lds_w[buf][big_lds_offset((t >> 3) + 32 * j, t & 7)]) = gw[j];
+        *reinterpret_cast<f32x4 *>(&lds_w[buf][big_lds_offset((t >> 3) + 32 * j, t & 7)]) = w;
       } else {
-        *reinterpret_cast<f32x4 *>(&lds_w[buf][(wt_k + WROWS * j) * WPITCH + wt_col]) = gw[j];
+        *reinterpret_cast<f32x4 *>(&lds_w[buf][(wt_k + WROWS * j) * WPITCH + wt_col]) = w;
       }
     }
-    if (!(m < SAFE)) {
-      sh_slow[buf] = s;
-      if (XP == 3) { // rounded up, the upper part of a value at the end of the range would be infinite: cut it off instead
-#pragma unroll
-        for (int j = 0; j < XJ; ++j) {
-          __bf16 *dst = &lds_x[buf][0][big_x_offset((t >> 3) + 32 * j, (t & 7) >> 1) + (t & 1) * 4];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const float v = gx[j][e];
-            const float hi = fabsf(v) < __builtin_inff() ? __uint_as_float(__float_as_uint(v) & 0xffff0000u) : v;
-            const __bf16 mid = (__bf16)(v - hi);
-            dst[e] = (__bf16)hi;
-            dst[BB * BKS + e] = mid;
-            dst[2 * BB * BKS + e] = (__bf16)(v - hi - (float)mid);
-          }
-        }
-      }
-    }
+    if (!(m < SAFE)) sh_slow = 1;
   };
 
   floatx16 acc[NB];
@@ -1829,12 +1822,12 @@ __device__ __forceinline__ void mvm_big_workgroup(const MvmArgs &a, const int ro
 #pragma unroll
         for (int p = 0; p < XP; ++p) x[nb][p] = read_x(buf, p, j, nb);
       }
-      bf16x4 h0, m0, l0, h1, m1, l1;
+      u32x2 h0, m0, l0, h1, m1, l1;
       split_bf16(read_w(buf, 2 * j), h0, m0, l0);
       split_bf16(read_w(buf, 2 * j + 1), h1, m1, l1);
-      const bf16x8 w[3] = {__builtin_shufflevector(h0, h1, 0, 1, 2, 3, 4, 5, 6, 7),
-                           __builtin_shufflevector(m0, m1, 0, 1, 2, 3, 4, 5, 6, 7),
-                           __builtin_shufflevector(l0, l1, 0, 1, 2, 3, 4, 5, 6, 7)};
+      const bf16x8 w[3] = {__builtin_bit_cast(bf16x8, u32x4{h0.x, h0.y, h1.x, h1.y}),
+                           __builtin_bit_cast(bf16x8, u32x4{m0.x, m0.y, m1.x, m1.y}),
+                           __builtin_bit_cast(bf16x8, u32x4{l0.x, l0.y, l1.x, l1.y})};
 #pragma unroll
       for (int p = 0; p < XP; ++p) {
 #pragma unroll
@@ -1847,26 +1840,8 @@ __device__ __forceinline__ void mvm_big_workgroup(const MvmArgs &a, const int ro
       }
     }
   };
-  auto compute_fp32 = [&](int buf) __attribute__((always_inline)) { // the parts of an input add up to it again
-#pragma unroll 1
-    for (int e = 0; e < 16; ++e) {
-      const int k = h * 16 + e;
-      const float w = WT ? lds_w[buf][k * WPITCH + wo * 32 + r] : lds_w[buf][big_lds_offset(wo * 32 + r, k >> 2) + (k & 3)];
-#pragma unroll
-      for (int nb = 0; nb < NB; ++nb) {
-        float x = 0.0f;
-#pragma unroll
-        for (int p = XP - 1; p >= 0; --p) {
-          const float part = (float)lds_x[buf][p][big_x_offset(wb * (BB / WB) + nb * 32 + r, k >> 3) + (k & 7)];
-          x = (p == 0 && !(fabsf(part) < __builtin_inff())) ? part : x + part; // an infinity's lower parts are NaN
-        }
-        acc[nb] = __builtin_amdgcn_mfma_f32_32x32x2f32(w, x, acc[nb], 0, 0, 0);
-      }
-    }
-  };
-
   const int stages = a.k_pad / BKS;
-  if (t < 2) sh_slow[t] = -1;
+  if (t == 0) sh_slow = 0;
   __syncthreads();
   {
     f32x4 gx[XJ], gw[WJ];
@@ -1876,10 +1851,33 @@ __device__ __forceinline__ void mvm_big_workgroup(const MvmArgs &a, const int ro
     for (int s = 0; s < stages; ++s) {
       const bool next = s + 1 < stages;
       if (next) gload(s + 1, gx, gw);
-      if (__builtin_expect(__builtin_amdgcn_readfirstlane(sh_slow[s & 1]) == s, 0)) compute_fp32(s & 1);
-      else compute(s & 1);
-      if (next) lds_store(s + 1, gx, gw);
+      compute(s & 1);
+      if (next) lds_store((s + 1) & 1, gx, gw);
       __syncthreads();
+    }
+  }
+  float x_step = XP == 1 ? a.x_step : 1.0f;
+  if (sh_slow) { // a value out of the range of the parts: this tile again on the fp32 pipe, straight from memory
+    x_step = 1.0f; // the rows hold k * step
+    const int o = min(tile_o * OT + wo * 32 + r, a.O - 1);
+    const float *w_first = a.w + (WT ? (long)o : (long)o * a.w_ld);
+    const long w_next = WT ? (long)a.w_ld : 1;
+    const float *x_first[NB];
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+      const int slot = min(tile_b * BB + wb * (BB / WB) + nb * 32 + r, n_act - 1);
+      x_first[nb] = xq + (long)((round > 0) ? pick2(a.st.row, round & 1)[slot] : slot) * a.k_pad;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[nb][e] = 0.0f;
+    }
+#pragma unroll 1
+    for (int k0 = 0; k0 < K; k0 += 2) {
+      const int k = k0 + h;
+      const float w = k < K ? w_first[k * w_next] : 0.0f;
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) {
+        acc[nb] = __builtin_amdgcn_mfma_f32_32x32x2f32(w, k < K ? x_first[nb][k] : 0.0f, acc[nb], 0, 0, 0);
+      }
     }
   }
 
@@ -1903,7 +1901,7 @@ __device__ __forceinline__ void mvm_big_workgroup(const MvmArgs &a, const int ro
         const int o0 = tile_o * OT + wo * 32 + g * 8 + h * 4;
         float v[4];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) v[q] = XP == 1 ? sums[4 * g + q] * a.x_step : sums[4 * g + q];
+        for (int q = 0; q < 4; ++q) v[q] = XP == 1 ? sums[4 * g + q] * x_step : sums[4 * g + q];
         int up = 0, lo = 0;
         if (o0 < a.O) mvm_finish_outputs(a, round, b_out, fin_out, o0, v, up, lo);
         up_max = max(up_max, up);
@@ -1971,13 +1969,13 @@ __device__ __forceinline__ void mvm_big_workgroup(const MvmArgs &a, const int ro
 }
 
 template <int WT, int BB, int WO, int XP, bool LAZY>
-__global__ __launch_bounds__(256, 2) void k_mvm_big(MvmArgs a, int min_active) {
+__global__ __launch_bounds__(256, XP == 1 && BB == 64 ? 3 : 2) void k_mvm_big(MvmArgs a, int min_active) {
   mvm_big_workgroup<WT, BB, WO, XP, LAZY>(a, a.round, (int)blockIdx.x, min_active);
 }
 
 // several tiles in one launch (round 0): a tile that is not run by this kernel has no workgroups in the table
 template <int WT, int BB, int XP>
-__global__ __launch_bounds__(256, 2) void k_mvm_big_group(MvmGroup g, int round) {
+__global__ __launch_bounds__(256, XP == 1 && BB == 64 ? 3 : 2) void k_mvm_big_group(MvmGroup g, int round) {
   int t = 0;
   while (t + 1 < g.n && (int)blockIdx.x >= g.start[t + 1]) ++t;
   const MvmArgs &a = g.args[t];
@@ -2510,8 +2508,8 @@ void launch_mvm_init_group(const MvmGroup &g, int max_k, hipStream_t s) {
 constexpr int TAIL_GRID = 1024; // workgroups of a later-round launch when the full grid would be larger
 
 // workgroups of a large-tile launch with sample tiles of `bb` samples
-static int big_workgroups(const MvmArgs &a, int bb) {
-  const int tiles_o = (a.O + 127) / 128, tiles_b = (a.m_batch + bb - 1) / bb;
+static int big_workgroups(const MvmArgs &a, int bb, int ot = 128) {
+  const int tiles_o = (a.O + ot - 1) / ot, tiles_b = (a.m_batch + bb - 1) / bb;
   return 8 * tiles_o * ((tiles_b + 7) / 8);
 }
 
@@ -2547,21 +2545,6 @@ void launch_mvm_big_group(const MvmGroup &g, int total_workgroups, int bb, bool 
 #undef RPU_LAUNCH_BIG
 }
 
-// samples of a round from which the large-tile kernel takes over, 0 when a call of this shape never uses it: it
-// needs outputs for a whole 128-wide tile and enough half tiles for every second CU
-static int big_threshold(int m_batch, int O) {
-  // measured on the 1024 x 1024 tile: the half tiles overtake the 32 x 32 kernel at about 1500 samples (backward 70
-  // against 88 us at 1536, 74 against 113 us at 2000; at 1024 the 32 x 32 kernel still leads, 63 against 68 us)
-  constexpr int big_min = 1536;
-  // narrower tiles (the patches of a convolution): part of the 128 outputs of a tile are idle, but a staged operand
-  // byte still meets four times the multiply-adds of the 32 x 32 kernel
-  constexpr int narrow_min_batch = 16384, narrow_min_outputs = 33;
-  if (m_batch < big_min || O < narrow_min_outputs || (O < 128 && m_batch < narrow_min_batch)) return 0;
-  const int tiles_o = (O + 127) / 128, tiles_b = (m_batch + 63) / 64;
-  if (8 * tiles_o * ((tiles_b + 7) / 8) < 128) return 0;
-  return big_min;
-}
-
 static int current_device_cus() {
   static int cus[64] = {0};
   int dev = 0;
@@ -2572,6 +2555,17 @@ static int current_device_cus() {
     cus[dev] = n;
   }
   return cus[dev];
+}
+
+// Samples of a round from which the large-tile kernel takes over, 0 when a call of this shape never uses it: as many as
+// give every CU a 64 x 64 tile.  Measured against the 32 x 32 kernel (us, large / small): 1024 x 1024 backward, 1024
+// samples 42 / 46, 512 samples 41 / 28; 512 x 512 backward, 2048 samples 29 / 35, 1024 samples 27 / 21; 768 -> 2304,
+// 1024 samples 61 / 95; 784 -> 256, 2048 samples 51 / 44, 4096 samples 60 / 69; 1024 -> 128, 4096 samples 62 / 50.
+static int big_threshold(int m_batch, int O) {
+  if (O < 33) return 0; // most of a tile's outputs would be idle
+  const int tiles_o = (O + 63) / 64, n_cus = current_device_cus();
+  const int from = 64 * ((n_cus + tiles_o - 1) / tiles_o);
+  return m_batch >= from ? from : 0;
 }
 
 bool mvm_uses_large_tiles(int m_batch, int O) { return big_threshold(m_batch, O) > 0; }
@@ -2720,16 +2714,24 @@ void launch_mvm_round(const MvmArgs &a_in, hipStream_t s) {
   if (a.round > 0 && !a.speculate) a.big_from = 0;
   if (a.big_from > 0) {
     const bool lazy = !a.transposed && !a.speculate && a.max_rounds > 1;
-    const bool narrow = a.O <= 64; // see mvm_big_workgroup, WO
-    const int bb = narrow ? 128 : mvm_big_sample_tile(big_workgroups(a, 128), current_device_cus());
-    const dim3 big_grid(big_workgroups(a, bb));
+    // outputs x samples of a workgroup tile.  Narrow tiles: 64 x 128 (see mvm_big_workgroup, WO).  Fewer than three tiles
+    // of 64 x 64 per CU: those (1024 x 1024, 2048 samples backward 47 us against 53 with 128 x 64 and 73 with 128 x 128;
+    // 768 -> 2304, 1024 samples 61 against 63 and 104); from there on the wider tiles stage less for the same products
+    // (1024 x 1024, 4096 samples 71, 67 and 79 us; 768 -> 2304, 2048 samples 85, 81 and 110).
+    const int n_cus = current_device_cus();
+    const bool sparse = a.O > 64 && big_workgroups(a, 64, 64) < 3 * n_cus;
+    const int ot = a.O <= 64 || sparse ? 64 : 128;
+    const int bb = sparse ? 64 : (ot == 64 ? 128 : mvm_big_sample_tile(big_workgroups(a, 128), n_cus));
+    const dim3 big_grid(big_workgroups(a, bb, ot));
     const int min_active = a.round > 0 ? a.big_from : 0;
 #define RPU_LAUNCH_BIG(WT, BB, WO, XP, LAZY) \
   hipLaunchKernelGGL((k_mvm_big<WT, BB, WO, XP, LAZY>), big_grid, dim3(256), 0, s, a, min_active)
 #define RPU_PICK_BIG(WT, XP) \
   do { \
-    if (narrow && lazy) RPU_LAUNCH_BIG(WT, 128, 2, XP, true); \
-    else if (narrow) RPU_LAUNCH_BIG(WT, 128, 2, XP, false); \
+    if (ot == 64 && bb == 128 && lazy) RPU_LAUNCH_BIG(WT, 128, 2, XP, true); \
+    else if (ot == 64 && bb == 128) RPU_LAUNCH_BIG(WT, 128, 2, XP, false); \
+    else if (ot == 64 && lazy) RPU_LAUNCH_BIG(WT, 64, 2, XP, true); \
+    else if (ot == 64) RPU_LAUNCH_BIG(WT, 64, 2, XP, false); \
     else if (bb == 128 && lazy) RPU_LAUNCH_BIG(WT, 128, 4, XP, true); \
     else if (bb == 128) RPU_LAUNCH_BIG(WT, 128, 4, XP, false); \
     else if (lazy) RPU_LAUNCH_BIG(WT, 64, 4, XP, true); \

@@ -10,9 +10,10 @@ from aihwkit_amd.rpu_base import tiles
 
 pytestmark = pytest.mark.gpu
 
-# tile edges of 64 and 128 outputs and 64 and 128 samples, contraction stages of 32, each with a remainder
-SHAPES = [(33, 64, 16384), (65, 65, 16400), (433, 48, 16500), (31, 129, 1536), (160, 130, 1601), (513, 257, 2049),
-          (1024, 128, 8193), (96, 1000, 8192)]
+# workgroup tiles of 64 x 128, 64 x 64, 128 x 64 and 128 x 128 outputs x samples, contraction stages of 32, each with a
+# remainder; at least one 64 x 64 tile per CU, or the 32 x 32 kernel runs the call
+SHAPES = [(33, 64, 16384), (65, 65, 16400), (433, 48, 16500), (31, 129, 5505), (160, 1003, 1601), (513, 257, 3401),
+          (1024, 128, 8193), (1001, 1000, 4100), (96, 1000, 8192)]
 
 
 def _tile(x_size, d_size, io, w):
@@ -66,7 +67,7 @@ def test_quantized_products_against_64_bit_sums(gpu_device, x_size, d_size, batc
         _close(got, q @ axis, np.abs(q) @ np.abs(axis), 4 * width + 16)
 
 
-@pytest.mark.parametrize("x_size,d_size,batch", [(100, 50, 16500), (256, 256, 2048), (300, 300, 8192)])
+@pytest.mark.parametrize("x_size,d_size,batch", [(100, 50, 16500), (256, 256, 4100), (300, 300, 12000)])
 def test_values_out_of_the_range_of_the_parts(gpu_device, x_size, d_size, batch):
     """Infinities, NaN and values near the end of the fp32 range give what fp32 products give."""
     rng = np.random.default_rng(1)
