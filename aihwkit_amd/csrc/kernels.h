@@ -72,6 +72,8 @@ struct MvmArgs {
   long out_sb, out_so; // output element (b, o) at out[b * out_sb + o * out_so]
   int m_batch;
   int K, O;       // contraction length and number of outputs
+  int in_one;     // 1: the last of the K inputs of a sample is the constant 1 and not stored (bias column; forward)
+  int out_drop;   // 1: the last of the O outputs is not stored (bias column; backward)
   int k_pad;      // K rounded up to the step of the contraction kernel (mvm_k_pad)
   float x_step;   // > 0: the quantized inputs are multiples of this step, at most 256 of them (mvm_input_step); 0: any values
   float *xq[2];   // ping-pong scratch [rows][k_pad]: DAC-quantized inputs, zero padded (rows: see MvmState::row)

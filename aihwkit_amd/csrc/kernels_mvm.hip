@@ -101,6 +101,11 @@ __device__ __forceinline__ MvmGatherRow mvm_gather_row(const MvmArgs &a, int b) 
   return MvmGatherRow{a.in + (long)n * a.in_gs - 2, a.in_index + (long)(b - n * a.in_group) * a.K};
 }
 
+// element k of a sample whose stored elements start at `row`
+__device__ __forceinline__ float mvm_input(const MvmArgs &a, const float *__restrict__ row, int k) {
+  return a.in_one && k == a.K - 1 ? 1.0f : row[(long)k * a.in_sk];
+}
+
 // quantized copy of sample b's input row into row `slot` of a scratch matrix, by `width` threads of which
 // this one is number t
 __device__ __forceinline__ void write_dac_row(const MvmArgs &a, int b, int slot, float scale, int round, float *dst,
@@ -111,7 +116,7 @@ __device__ __forceinline__ void write_dac_row(const MvmArgs &a, int b, int slot,
   for (int k = t; k < a.k_pad; k += width) {
     float v = 0.0f;
     if (k < a.K) {
-      v = row[(long)k * a.in_sk];
+      v = mvm_input(a, row, k);
       if (!a.io.perfect) v = dac_value(v, scale, a.io, a.key, a.call, round, b, k);
     }
     out[k] = v;
@@ -195,6 +200,7 @@ __device__ __forceinline__ void mvm_finish_outputs(const MvmArgs &a, int round, 
   lo = 0;
   float *out_p = a.out + (long)b * a.out_sb + (long)o0 * a.out_so;
   long out_so = a.out_so;
+  const int o_end = a.O - a.out_drop; // outputs that are stored (rows kept aside: out_drop is 0)
   if (out_rows) { // results kept aside, sample-major: [m_batch][O]
     out_p = out_rows + (long)b * a.O + o0;
     out_so = 1;
@@ -202,7 +208,7 @@ __device__ __forceinline__ void mvm_finish_outputs(const MvmArgs &a, int round, 
   if (a.io.perfect) {
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      if (o0 + q < a.O) {
+      if (o0 + q < o_end) {
         float res = a.alpha * v[q];
         if (a.beta != 0.0f) res += a.beta * out_p[(long)q * out_so];
         out_p[(long)q * out_so] = res;
@@ -214,18 +220,18 @@ __device__ __forceinline__ void mvm_finish_outputs(const MvmArgs &a, int round, 
   if (fin == 0.0f) { // zero input: the reference short-cuts to a zero output
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      if (o0 + q < a.O) out_p[(long)q * out_so] = 0.0f;
+      if (o0 + q < o_end) out_p[(long)q * out_so] = 0.0f;
     }
     return;
   }
 
   mvm_adc_values(a, round, b, fin, o0, v, up, lo, pre, post);
-  if (out_so == 1 && (o0 + 3) < a.O && ((((uintptr_t)out_p) & 15) == 0)) {
+  if (out_so == 1 && (o0 + 3) < o_end && ((((uintptr_t)out_p) & 15) == 0)) {
     *reinterpret_cast<float4 *>(out_p) = make_float4(v[0], v[1], v[2], v[3]);
   } else {
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      if (o0 + q < a.O) out_p[(long)q * out_so] = v[q];
+      if (o0 + q < o_end) out_p[(long)q * out_so] = v[q];
     }
   }
 }
@@ -720,7 +726,7 @@ __device__ __forceinline__ void mvm_init_sample(const MvmArgs &a, int b, int t, 
 #pragma unroll
     for (int i = 0; i < KEEP; ++i) {
       const int k = t + i * SUB;
-      xk[i] = (k < a.K) ? row[(long)k * a.in_sk] : 0.0f;
+      xk[i] = (k < a.K) ? mvm_input(a, row, k) : 0.0f;
     }
   }
   float nm = 1.0f;
@@ -744,7 +750,7 @@ __device__ __forceinline__ void mvm_init_sample(const MvmArgs &a, int b, int t, 
       }
     } else {
       for (int k = t; k < a.K; k += SUB) {
-        const float x = row[(long)k * a.in_sk];
+        const float x = mvm_input(a, row, k);
         amax = fmaxf(amax, fabsf(x));
         vmax = fmaxf(vmax, x);
         ps += x > 0.0f ? x : 0.0f;
@@ -1029,7 +1035,7 @@ __device__ __forceinline__ void mvm_prepare_next_rows(const MvmArgs &a, int roun
       const int k = k0 + 32 * u + kq;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        xv[u][i] = (k < k_hi && sc[i] != 0.0f && k < a.K) ? in[(long)bt[i] * a.in_sb + (long)k * a.in_sk] : 0.0f;
+        xv[u][i] = (k < k_hi && sc[i] != 0.0f && k < a.K) ? mvm_input(a, in + (long)bt[i] * a.in_sb, k) : 0.0f;
       }
     }
 #pragma unroll
@@ -1599,7 +1605,7 @@ __device__ __forceinline__ void big_prepare_next_rows(const MvmArgs &a, int roun
 #pragma unroll
     for (int i = 0; i < RPT; ++i) {
       const int row = rq * RPT + i;
-      xv[i] = (sh_scale[row] != 0.0f && k < a.K) ? in[(long)sh_b[row] * a.in_sb + (long)k * a.in_sk] : 0.0f;
+      xv[i] = (sh_scale[row] != 0.0f && k < a.K) ? mvm_input(a, in + (long)sh_b[row] * a.in_sb, k) : 0.0f;
     }
 #pragma unroll
     for (int i = 0; i < RPT; ++i) {

@@ -810,23 +810,28 @@ struct Tile {
     a.small_tiles_only = side ? 1 : 0;
 
     // the x side carries the optional bias column: input of forward, output of backward
+    // (the bias column is made and dropped by the kernels that read the input and store the output; a pass with terms
+    // before the ADC, whose kernels read whole rows, goes through a widened copy)
+    const bool widened = bias && side;
     float *final_out = out;
     if (!transposed) {
-      if (bias) {
+      if (widened) {
         s_bias.ensure((size_t)B * X);
         launch_make_bias(in, s_bias.p, B, X, in_trans ? 1 : 0, s);
         a.in = s_bias.p; a.in_sb = X; a.in_sk = 1;
       } else {
-        a.in = in; a.in_sb = in_trans ? 1 : X; a.in_sk = in_trans ? B : 1;
+        a.in = in; a.in_sb = in_trans ? 1 : X - (bias ? 1 : 0); a.in_sk = in_trans ? B : 1;
+        a.in_one = bias ? 1 : 0;
       }
       a.out = out; a.out_sb = out_trans ? 1 : D; a.out_so = out_trans ? B : 1;
     } else {
       a.in = in; a.in_sb = in_trans ? 1 : D; a.in_sk = in_trans ? B : 1;
-      if (bias) {
+      if (widened) {
         s_bias.ensure((size_t)B * X);
         a.out = s_bias.p; a.out_sb = X; a.out_so = 1;
       } else {
-        a.out = out; a.out_sb = out_trans ? 1 : X; a.out_so = out_trans ? B : 1;
+        a.out = out; a.out_sb = out_trans ? 1 : X - (bias ? 1 : 0); a.out_so = out_trans ? B : 1;
+        a.out_drop = bias ? 1 : 0;
       }
     }
 
@@ -962,7 +967,7 @@ struct Tile {
         }
       }
     }
-    if (transposed && bias) launch_drop_bias(s_bias.p, final_out, B, X, out_trans ? 1 : 0, s);
+    if (transposed && widened) launch_drop_bias(s_bias.p, final_out, B, X, out_trans ? 1 : 0, s);
     RPU_HIP_CHECK(hipGetLastError());
     last_stream = s;
     if (!transposed && !w_other) last_forward_batch = B;
