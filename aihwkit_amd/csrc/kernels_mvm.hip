@@ -2724,8 +2724,10 @@ void launch_mvm_round(const MvmArgs &a_in, hipStream_t s) {
     // of 64 x 64 per CU: those (1024 x 1024, 2048 samples backward 47 us against 53 with 128 x 64 and 73 with 128 x 128;
     // 768 -> 2304, 1024 samples 61 against 63 and 104); from there on the wider tiles stage less for the same products
     // (1024 x 1024, 4096 samples 71, 67 and 79 us; 768 -> 2304, 2048 samples 85, 81 and 110).
+    // Contractions of one or two stages are all ADC stage and stores: the tile with the most workgroups per CU (five of
+    // 64 x 64 against two of 128 x 128; 433 x 48 convolution tile, 131072 patches: training step 1438 -> 1369 us).
     const int n_cus = current_device_cus();
-    const bool sparse = a.O > 64 && big_workgroups(a, 64, 64) < 3 * n_cus;
+    const bool sparse = a.O > 64 && (big_workgroups(a, 64, 64) < 3 * n_cus || a.k_pad <= 2 * BKS);
     const int ot = a.O <= 64 || sparse ? 64 : 128;
     const int bb = sparse ? 64 : (ot == 64 ? 128 : mvm_big_sample_tile(big_workgroups(a, 128), n_cus));
     const dim3 big_grid(big_workgroups(a, bb, ot));
