@@ -1128,9 +1128,10 @@ __global__ __launch_bounds__(256, ((C > 1 || DEEP) ? 4 : 8)) void k_update_pulse
 // in blocks of STREAM_PASSES passes, each stage one block behind the one before it, one barrier per block.  Which lanes
 // fire in a pass and which go down are 64-bit lane masks (k_update_lines_stream), 64 passes of them to a load (lane p
 // fetches those of pass p), spread to the wave by v_readlane.
-// A factor of zero leaves w where it is -- bit for bit, unless w is outside its bounds or a parameter is not finite: such
-// a wave selects by the factor's bits instead.  Passes, noise bytes and the arithmetic of a step are those of
-// PulsedRows: same weights, bit for bit.
+// With multiplicative noise (and constant steps) a factor of zero leaves w where it is, unless w is outside its bounds or
+// a parameter is not finite; such a wave, and every wave of a device with additive noise, whose step
+// w + slope w + scale f has a term without a factor, selects by the factor's bits instead.  Passes, noise bytes and the
+// arithmetic of a step are those of PulsedRows: same weights.
 // 433 x 48 tile, 131 072 samples, 21 000 passes a row: 1973 -> 493 us (55 cycles a pass; draw and steps take 45 each on
 // their own, the seven waves of a workgroup share four SIMDs).
 template <int PARTS> struct PulseStream {
@@ -1353,8 +1354,10 @@ __device__ __forceinline__ void pulse_stream_steps(const UpdateArgs &a, const SH
                                                    const PulseCell<KIND> &cp, float &w, const int block, const int blocks,
                                                    const int lane) {
   const unsigned slots = plane_slots(a);
+  // where a factor of zero leaves w alone: not with additive noise, whose slope term has no factor; w within its bounds
   const float big = fmaxf(fmaxf(fabsf(cp.slope_up), fabsf(cp.slope_dn)), fmaxf(fabsf(cp.scale_up), fabsf(cp.scale_dn)));
-  const bool by_bits = __any(!(w >= cp.lo && w <= cp.hi && big < 1e15f && fabsf(w) < 1e15f));
+  const bool by_bits = (KIND != RPU_DEVICE_CONSTANT_STEP && !MULT) ||
+                       __any(!(w >= cp.lo && w <= cp.hi && big < 1e15f && fabsf(w) < 1e15f));
   __syncthreads();
   if (pulse_stream_over(sh, 0)) return;
   uint32_t lo = 0u, hi = 0u, lo_next, hi_next;

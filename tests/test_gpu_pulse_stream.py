@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 import torch
 
+from aihwkit_amd.rpu_base import devices as dv
 from helpers import constant_step, make_meta, soft_bounds
 
 pytestmark = pytest.mark.gpu
@@ -19,20 +20,31 @@ def _tile(x_size, d_size, dev):
     return tile
 
 
+def _additive(dw_min_std):
+    """A linear-step device whose noise is added to the step: a step without its factor still has the slope term."""
+    dev = dv.LinearStepResistiveDeviceParameter()
+    for name, value in dict(gamma_up=0.4, gamma_down=0.2, mult_noise=False, dw_min_std=dw_min_std, construction_seed=5,
+                            enforce_consistency=True).items():
+        setattr(dev, name, value)
+    return dev
+
+
 # blocks of 64 columns and a rest, one and two teams to a workgroup (more than 256 blocks in all), a chunk that is not
 # full, batches with almost no pulse; lr sets the longest bit line: 1, 3, 7 and 31 (the last walked pulse by pulse)
 @pytest.mark.parametrize("x_size,d_size,batch,lr,sparse", [
     (5, 3, 1024, 0.0005, False), (64, 2, 1056, 0.02, False), (65, 4, 1500, 0.05, False), (129, 100, 1025, 0.004, False),
     (200, 7, 4100, 0.0005, True), (250, 5, 2048, 0.6, False), (433, 48, 2100, 0.02, False), (70, 260, 1030, 0.02, True)])
-@pytest.mark.parametrize("kind", ["soft_bounds", "constant_step", "quiet"])
+@pytest.mark.parametrize("kind", ["soft_bounds", "constant_step", "quiet", "additive", "additive_quiet"])
 def test_pipelined_pulse_loop_equals_the_plain_one(x_size, d_size, batch, lr, sparse, kind):
     from aihwkit_amd.rpu_base.tiles import TileGroup
     if kind == "soft_bounds":
         dev = soft_bounds(construction_seed=5)
     elif kind == "constant_step":
         dev = constant_step(construction_seed=5)
-    else:
+    elif kind == "quiet":
         dev = soft_bounds(construction_seed=5, dw_min_std=0.0)
+    else:
+        dev = _additive(0.3 if kind == "additive" else 0.0)
     gen = torch.Generator("cuda").manual_seed(batch + x_size)
     x = torch.rand(batch, x_size, generator=gen, device="cuda") * 2 - 1
     d = torch.randn(batch, d_size, generator=gen, device="cuda") * 0.05
