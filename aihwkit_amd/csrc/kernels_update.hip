@@ -1354,10 +1354,12 @@ __device__ __forceinline__ void pulse_stream_steps(const UpdateArgs &a, const SH
                                                    const PulseCell<KIND> &cp, float &w, const int block, const int blocks,
                                                    const int lane) {
   const unsigned slots = plane_slots(a);
-  // where a factor of zero leaves w alone: not with additive noise, whose slope term has no factor; w within its bounds
-  const float big = fmaxf(fmaxf(fabsf(cp.slope_up), fabsf(cp.slope_dn)), fmaxf(fabsf(cp.scale_up), fabsf(cp.scale_dn)));
+  // where a factor of zero leaves w alone: not with additive noise, whose slope term has no factor; w within its bounds;
+  // slope * w + scale finite all along (compared one by one: a maximum would lose a NaN)
+  const auto tame = [](float v) { return fabsf(v) < 1e15f; };
   const bool by_bits = (KIND != RPU_DEVICE_CONSTANT_STEP && !MULT) ||
-                       __any(!(w >= cp.lo && w <= cp.hi && big < 1e15f && fabsf(w) < 1e15f));
+                       __any(!(w >= cp.lo && w <= cp.hi && tame(cp.lo) && tame(cp.hi) && tame(cp.slope_up) &&
+                               tame(cp.slope_dn) && tame(cp.scale_up) && tame(cp.scale_dn)));
   __syncthreads();
   if (pulse_stream_over(sh, 0)) return;
   uint32_t lo = 0u, hi = 0u, lo_next, hi_next;

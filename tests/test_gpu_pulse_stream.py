@@ -90,3 +90,32 @@ def test_pipelined_pulse_loop_with_weights_outside_their_bounds(storage_mode):
     assert torch.equal(results[0], results[1])
     assert bool((results[0][:, ::15] == 2.5).all())   # no x pulse: untouched
     assert float(results[0][:, 3].max()) < 2.5
+
+
+@pytest.mark.parametrize("name,value", [("slope_up", float("nan")), ("dwmin_down", float("inf")), ("max_bound", float("inf"))])
+def test_pipelined_pulse_loop_with_parameters_that_are_not_finite(name, value):
+    """Cross-points with such a parameter, or none, follow the plain loop; the ones without a pulse stay as they are."""
+    from aihwkit_amd.rpu_base import tiles
+    from aihwkit_amd.rpu_base.tiles import TileGroup
+    x_size, d_size, batch = 130, 6, 1200
+    host = make_meta(desired_bl=31).create_array(x_size, d_size, soft_bounds(construction_seed=5))
+    hidden = host.get_hidden_parameters()
+    hidden[host.get_hidden_parameter_names().index(name), :, ::3] = value
+    host.set_hidden_parameters(hidden)
+    start = torch.from_numpy(np.random.default_rng(3).uniform(-0.4, 0.4, (d_size, x_size)).astype(np.float32))
+    host.set_weights(start)
+    gen = torch.Generator("cuda").manual_seed(1)
+    x = torch.rand(batch, x_size, generator=gen, device="cuda") * 2 - 1
+    x[:, ::5] = 0.0
+    d = torch.randn(batch, d_size, generator=gen, device="cuda") * 0.05
+    one, other = tiles.CudaAnalogTile(host), tiles.CudaAnalogTile(host)
+    before = one.get_weights()
+    for tile in (one, other):
+        tile.set_seed(17)
+        tile.set_learning_rate(0.01)
+    one.update(x, d, False)
+    TileGroup([other]).update([x], [d])
+    mine, theirs = one.get_weights().numpy(), other.get_weights().numpy()
+    assert np.array_equal(mine, theirs, equal_nan=True)
+    assert np.array_equal(mine[:, ::5], before.numpy()[:, ::5], equal_nan=True)
+    assert not np.array_equal(mine, before.numpy(), equal_nan=True)
