@@ -1,0 +1,86 @@
+"""The native calls on torch tensors (csrc/torch_calls.cpp) leave tensors without a storage of their own -- inside a
+function transform or a tracer -- to the general path, which raises; they used to end the process.  Each case runs in a
+process of its own, all calls on tensors that claim to be on a GPU."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+SCRIPT = """
+import struct, sys
+import torch
+from torch._subclasses.fake_tensor import FakeTensorMode
+from aihwkit_amd._cabi import torch_calls
+from helpers import constant_step, make_meta
+
+transform = sys.argv[1]
+m, sizes = torch_calls(), struct.pack("=ii", 8, 4)
+tile = make_meta().create_array(8, 4, constant_step())
+tile.set_learning_rate(0.01)
+h = tile._h.value
+
+CALLS = {
+    "forward": lambda x, d: m.forward(h, x, 8, 4, False, False, False, False, True),
+    "backward": lambda x, d: m.backward(h, d, 4, 8, False, False, False, False, True),
+    "update": lambda x, d: m.update(h, x, d, 8, 4, False, False, False, False, True),
+    "group_forward": lambda x, d: m.group_forward(0, sizes, [x], None, False, True),
+    "group_backward": lambda x, d: m.group_backward(0, sizes, [d], None, False, True),
+    "group_update": lambda x, d: m.group_update(0, sizes, [x], [d], True),
+}
+
+def f(x, d):
+    for name, call in CALLS.items():
+        print(name, flush=True)
+        assert call(x, d) is None
+    return x + 1
+
+with FakeTensorMode():
+    x, d = (torch.empty(3, 2, n, device="cuda") for n in (8, 4))
+    assert x.is_cuda
+    if transform == "vmap":
+        torch.vmap(f)(x, d)
+    elif transform == "vjp":
+        torch.func.vjp(f, x[0], d[0])
+    elif transform == "jvp":
+        torch.func.jvp(f, (x[0], d[0]), (x[1], d[1]))
+    else:
+        f(x[0], d[0])
+print("done")
+"""
+
+
+@pytest.mark.parametrize("transform", ["vmap", "vjp", "jvp", "none"])
+def test_tensors_without_storage_are_left_to_the_general_path(transform):
+    env = dict(os.environ, PYTHONPATH=os.pathsep.join([ROOT, os.path.join(ROOT, "tests")]))
+    run = subprocess.run([sys.executable, "-c", SCRIPT, transform], env=env, capture_output=True, text=True, timeout=240)
+    assert run.returncode == 0 and run.stdout.strip().endswith("done"), run.stdout + run.stderr[-1500:]
+
+
+def _tile(x_size, d_size):
+    import torch
+
+    from aihwkit_amd.rpu_base import tiles
+    from helpers import constant_step, make_meta, noise_free_io
+    host = make_meta(noise_free_io(), noise_free_io()).create_array(x_size, d_size, constant_step(construction_seed=1))
+    host.set_weights(torch.full((d_size, x_size), 0.25))
+    tile = tiles.CudaAnalogTile(host)
+    tile.set_learning_rate(0.01)
+    return tile
+
+
+@pytest.mark.gpu
+def test_calls_inside_a_function_transform_raise():
+    import torch
+
+    from aihwkit_amd.rpu_base.tiles import TileGroup
+    tile = _tile(8, 4)
+    group = TileGroup([tile])
+    x, d = torch.ones(3, 2, 8, device="cuda"), torch.ones(3, 2, 4, device="cuda")
+    for call in (lambda x, d: tile.forward(x), lambda x, d: tile.backward(d), lambda x, d: tile.update(x, d, False),
+                 lambda x, d: group.forward([x])[0], lambda x, d: group.backward([d])[0], lambda x, d: group.update([x], [d])):
+        with pytest.raises(RuntimeError):
+            torch.vmap(call)(x, d)
+    assert tile.forward(x[0]).shape == (2, 4)
