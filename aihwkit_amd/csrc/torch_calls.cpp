@@ -177,8 +177,9 @@ struct Operands {
   int64_t batch = -1;
 };
 
-// pointers and row strides of a list of matrices [batch][size of tile i]; false: not the plain case
-template <typename Size> bool operands(PyObject *list, Py_ssize_t n, int64_t batch, Size size, Operands &o) {
+// pointers and row strides of a list of matrices [batch][size of tile i] (WRITTEN: a pointer to write through, for which a
+// copy-on-write tensor makes its copy); false: not the plain case
+template <bool WRITTEN, typename Size> bool operands(PyObject *list, Py_ssize_t n, int64_t batch, Size size, Operands &o) {
   if (!PyList_Check(list) || PyList_GET_SIZE(list) != n) return false;
   o.tensors.reserve(n);
   o.ptr.reserve(n);
@@ -190,7 +191,7 @@ template <typename Size> bool operands(PyObject *list, Py_ssize_t n, int64_t bat
     if (o.batch < 0) o.batch = t->size(0);
     if (t->size(0) != o.batch || t->size(1) != size(i)) return false;
     o.tensors.push_back(*t);
-    o.ptr.push_back(data(*t));
+    o.ptr.push_back(WRITTEN ? out_data(*t) : data(*t));
     o.ld.push_back(o.batch > 1 ? (long)t->stride(0) : (long)size(i));
   }
   return n > 0 && o.batch >= 0 && o.batch <= 0x7fffffff;
@@ -201,7 +202,7 @@ template <bool FORWARD> PyObject *group_product(PyObject *const *a, Py_ssize_t n
   if (nargs != 6) return PyErr_Format(PyExc_TypeError, "6 arguments expected"), nullptr;
   const GroupSizes sz(a[1]);
   Operands in, out;
-  if (!operands(a[2], sz.n, -1, [&](Py_ssize_t i) { return FORWARD ? sz.x(i) : sz.d(i); }, in)) Py_RETURN_NONE;
+  if (!operands<false>(a[2], sz.n, -1, [&](Py_ssize_t i) { return FORWARD ? sz.x(i) : sz.d(i); }, in)) Py_RETURN_NONE;
   const auto out_size = [&](Py_ssize_t i) { return FORWARD ? sz.d(i) : sz.x(i); };
   THPObjectPtr result;
   if (a[3] == Py_None) {
@@ -225,7 +226,7 @@ template <bool FORWARD> PyObject *group_product(PyObject *const *a, Py_ssize_t n
   } else {
     Py_RETURN_NONE;
   }
-  if (!operands(result.get(), sz.n, in.batch, out_size, out)) Py_RETURN_NONE;
+  if (!operands<true>(result.get(), sz.n, in.batch, out_size, out)) Py_RETURN_NONE;
   rpu_group_t *g = static_cast<rpu_group_t *>(pointer(a[0]));
   const hipStream_t s = stream_of(in.tensors[0]);
   const bool is_test = truth(a[4]);
@@ -251,8 +252,8 @@ PyObject *group_update_checked(PyObject *const *a, Py_ssize_t n) {
   if (n != 5) return PyErr_Format(PyExc_TypeError, "5 arguments expected"), nullptr;
   const GroupSizes sz(a[1]);
   Operands x, d;
-  if (!operands(a[2], sz.n, -1, [&](Py_ssize_t i) { return sz.x(i); }, x)) Py_RETURN_NONE;
-  if (!operands(a[3], sz.n, x.batch, [&](Py_ssize_t i) { return sz.d(i); }, d)) Py_RETURN_NONE;
+  if (!operands<false>(a[2], sz.n, -1, [&](Py_ssize_t i) { return sz.x(i); }, x)) Py_RETURN_NONE;
+  if (!operands<false>(a[3], sz.n, x.batch, [&](Py_ssize_t i) { return sz.d(i); }, d)) Py_RETURN_NONE;
   rpu_group_t *g = static_cast<rpu_group_t *>(pointer(a[0]));
   const hipStream_t s = stream_of(x.tensors[0]);
   const bool ok = call(

@@ -84,3 +84,18 @@ def test_calls_inside_a_function_transform_raise():
         with pytest.raises(RuntimeError):
             torch.vmap(call)(x, d)
     assert tile.forward(x[0]).shape == (2, 4)
+
+
+@pytest.mark.gpu
+def test_outputs_that_share_their_memory_until_written():
+    """A lazily cloned output tensor gets its copy before a group writes to it: the tensor it was cloned from stays."""
+    import torch
+
+    from aihwkit_amd.rpu_base.tiles import TileGroup
+    group = TileGroup([_tile(8, 4)])
+    x, d = torch.ones(2, 8, device="cuda"), torch.ones(2, 4, device="cuda")
+    for call, inputs, size in ((group.forward, [x], 4), (group.backward, [d], 8)):
+        first = torch.full((2, size), 7.0, device="cuda")
+        out = torch._lazy_clone(first)
+        call(inputs, outs=[out])
+        assert bool((first == 7.0).all()) and bool((out != 7.0).all())
