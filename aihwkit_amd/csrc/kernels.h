@@ -298,6 +298,7 @@ struct UpdateArgs {
   float *prob_b; // [B] probability scale of x
   uint32_t *x_words; // [B][X] packed pulse words: written where bit lines are longer than seven pulses, else only their
   uint32_t *d_words; // [B][D] bit planes (launch_words_from_planes makes them for the inspection hook)
+  int keep_words;    // 1: the words are written whatever the bit lines (not with x_lane_masks)
   // bit lines beyond 31 pulses: a sample takes words_per_sample consecutive rows of words (and bit positions in the
   // planes); m_batch then counts those rows, bl / prob_a / prob_b / x / d stay per sample (row r belongs to sample
   // r / words_per_sample and holds its pulse slots 31 (r % words_per_sample) + 1 ..).  0 or 1: one row per sample.

@@ -332,7 +332,7 @@ __device__ __forceinline__ void update_lines_block(const UpdateArgs &a, const in
   const float P = b_ok ? (is_x ? a.prob_b[sample] : a.prob_a[sample]) : 0.0f;
   const int K = b_ok ? min(max(a.bl[sample] - 31 * wrow, 0), 31) : 0;
   const int kmax = a.kmax[a.kmax_slot], slots = kmax + 1;
-  const bool keep_words = kmax > UPDATE_PLANES_ONLY_KMAX;
+  const bool keep_words = a.keep_words || kmax > UPDATE_PLANES_ONLY_KMAX;
   uint32_t *planes = is_x ? a.x_planes : a.d_planes;
   const int c0 = 2 * by;
   for (int el = wave; el < LINES_E; el += 4) {

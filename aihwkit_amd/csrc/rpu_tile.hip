@@ -1526,7 +1526,7 @@ struct Tile {
     last_update_pulse = pulse_type;
     last_bl = a.bl; last_a = a.prob_a; last_b = a.prob_b;
     last_update = a;
-    last_in_planes = pulse_type == RPU_PULSE_STOCHASTIC_COMPRESSED;
+    last_in_planes = pulse_type == RPU_PULSE_STOCHASTIC_COMPRESSED && !a.keep_words;
   }
 
   void pulsed_update_on(const DeviceView &dv, const UpdatePar &up, float lr, const float *xin, long x_sb, long x_sj,
@@ -1549,6 +1549,8 @@ struct Tile {
         row_major_pulse_loop(a);
         a.wt_src = d_w.p; // the launch of the pulse trains makes the row-major copy
       }
+      // the static block belongs to all tiles of the GPU: its words are made now, a later inspection only reads them
+      a.keep_words = ws ? 1 : 0;
       // (pulse counters and write noise read the bit planes; the static block is laid out for planes)
       a.x_lane_masks = (!ws && !aggregated && !counting && !(dv.w == d_wp.p && persistent()) && update_takes_stream(a)) ? 1 : 0;
       launch_update_lines(a, s);

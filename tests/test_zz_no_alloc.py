@@ -110,3 +110,28 @@ def test_update_without_allocation_refuses_what_does_not_fit():
     long_tile.set_update_without_allocation(True)
     with pytest.raises(RuntimeError, match="at most 31 pulses"):
         long_tile.update(xg[:8, :40].contiguous(), dg[:8, :30].contiguous(), False, False, False, False)
+
+
+def test_inspecting_one_tile_leaves_the_shared_scratch_to_the_others():
+    """All tiles of a GPU share the static array: reading the pulse words of one tile, or updating it with words, writes
+    nothing there, so the words that another tile's later update left stay."""
+    meta, dev = config2()
+    _, other = pair(meta, dev, 200, 131)      # its words lie where the bit planes of the smaller tile are
+    ref, noa = pair(meta, dev, 70, 40)
+    rng = np.random.default_rng(4)
+
+    def lines(batch, x_size, d_size):
+        return (torch.from_numpy(rng.uniform(-1, 1, (batch, x_size)).astype(np.float32)).cuda(),
+                torch.from_numpy((0.05 * rng.standard_normal((batch, d_size))).astype(np.float32)).cuda())
+
+    x1, d1 = lines(150, 200, 131)
+    x2, d2 = lines(37, 70, 40)
+    words = [torch.zeros(8, n, dtype=torch.int32, device="cuda") for n in (200, 131)]
+    for look in (lambda: other.get_update_words(150), lambda: other.update_with_words(*words)):
+        other.update(x1, d1, False)
+        ref.update(x2, d2, False)
+        noa.update(x2, d2, False)
+        look()
+        for u, v in zip(ref.get_update_words(37), noa.get_update_words(37)):
+            assert torch.equal(u, v)
+        assert torch.equal(ref.get_weights(), noa.get_weights())
