@@ -811,8 +811,8 @@ struct Tile {
 
     // the x side carries the optional bias column: input of forward, output of backward
     // (the bias column is made and dropped by the kernels that read the input and store the output; a pass with terms
-    // before the ADC, whose kernels read whole rows, goes through a widened copy)
-    const bool widened = bias && side;
+    // before the ADC, whose kernels read whole rows, goes through a widened copy, and so does one without any other input)
+    const bool widened = bias && (side || X == 1);
     float *final_out = out;
     if (!transposed) {
       if (widened) {
