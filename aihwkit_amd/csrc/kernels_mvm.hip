@@ -1658,14 +1658,20 @@ __device__ __forceinline__ int big_x_offset(int row, int chunk) {
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-__device__ __forceinline__ uint32_t pack_bf16(float lower, float upper) { // both rounded to nearest even
-  uint32_t p;
-  asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(p) : "v"(lower), "v"(upper));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+
+// Both rounded to nearest even, by an instruction that the compiler chooses: an MFMA must not read a register sooner than two
+// wait states after a vector instruction wrote it, and the compiler does not see that in assembly text (the second register
+// of an operand that was converted one instruction before came out stale).  The empty text keeps it from rounding the
+// value a second time where the halves are widened again.
+__device__ __forceinline__ uint32_t pack_bf16(float lower, float upper) {
+  uint32_t p = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{lower, upper}, bf16x2));
+  asm("" : "+v"(p));
   return p;
 }
 // v = hi + mid + lo with every part rounded to bf16: 3 x 8 bits hold the 24 of a float, so the sum is exact (above
-// 2^-110; the low part of a smaller value may drop out).  On the packed pairs: written with conversions of the single
-// parts, the compiler rounds every value a second time before it widens it again.
+// 2^-110; the low part of a smaller value may drop out).
 __device__ __forceinline__ void split_bf16(const f32x4 v, u32x2 &hi, u32x2 &mid, u32x2 &lo) {
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
