@@ -176,7 +176,8 @@ int mvm_round_workgroups(const MvmArgs &a);            // workgroups of a round 
 // counts its workgroups (mvm_big_workgroups; 0 for the other tiles).
 int mvm_big_workgroups(const MvmArgs &a, int bb);
 // bb: samples of a workgroup tile, 128 or 64 (mvm_big_sample_tile: by the workgroups the launch would have with 128)
-int mvm_big_sample_tile(int workgroups_128, int n_cus);
+// stepped: the inputs of the launch are whole numbers of DAC steps (MvmArgs::x_step)
+int mvm_big_sample_tile(int workgroups_128, int n_cus, bool stepped);
 float mvm_input_step(const IoDev &io);
 // w_oc: how the tiles of the launch address their weights (MvmArgs::w_oc; the same for all of them)
 void launch_mvm_big_group(const MvmGroup &g, int total_workgroups, int bb, bool w_oc, bool stepped, hipStream_t s);

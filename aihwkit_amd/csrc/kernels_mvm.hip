@@ -1707,6 +1707,7 @@ template <int WT, int BB, int WO, int XP, bool LAZY>
 __device__ __forceinline__ void mvm_big_workgroup(const MvmArgs &a, const int round, const int n, const int min_active) {
   static_assert(BB == 128 || BB == 64, "sample tile of 128 or 64");
   static_assert(WO == 4 || WO == 2, "two or four waves along the outputs");
+  static_assert(XP == 1 || BB == 64 || WO == 2, "one workgroup per CU");
   constexpr int OT = 32 * WO;            // outputs of a workgroup tile
   constexpr int WB = 4 / WO;             // waves along the samples
   constexpr int NB = BB / 32 / WB;       // 32-sample blocks per wave
@@ -2560,8 +2561,11 @@ int mvm_big_workgroups(const MvmArgs &a, int bb) { return a.O >= 128 ? big_workg
 // multiply-adds per byte staged), otherwise its idle CUs cost more than that (384 workgroups occupy half of the CUs
 // twice as long as the other half) and tiles of 64 samples, three to a CU, fill the chip more evenly.  Measured on
 // the 1024 x 1024 tile: batch 8192 and 16384 (exactly one and two rounds) are 7 .. 12 % faster with 128, every other
-// batch between 2048 and 20480 with 64 (up to 35 % at 2048, 18 % at 10240).
-int mvm_big_sample_tile(int workgroups_128, int n_cus) {
+// batch between 2048 and 20480 with 64 (up to 35 % at 2048, 18 % at 10240).  Inputs in three parts (not `stepped`): 64
+// always; with 128 the staged planes take 80 KB, so a CU would hold one workgroup, four waves, and not two (1024 x 1024,
+// forward without noise: batch 8192 145 us against 140, 16384 278 against 270; backward the same within 1 us).
+int mvm_big_sample_tile(int workgroups_128, int n_cus, bool stepped) {
+  if (!stepped) return 64;
   const int slots = 2 * n_cus;
   const int rounds = (workgroups_128 + slots - 1) / slots;
   const int idle = rounds * slots - workgroups_128;
@@ -2570,18 +2574,14 @@ int mvm_big_sample_tile(int workgroups_128, int n_cus) {
 
 void launch_mvm_big_group(const MvmGroup &g, int total_workgroups, int bb, bool w_oc, bool stepped, hipStream_t s) {
   const dim3 grid(total_workgroups);
-#define RPU_LAUNCH_BIG(WT, BB) \
+#define RPU_LAUNCH_BIG(BB, XP) \
   do { \
-    if (stepped) hipLaunchKernelGGL((k_mvm_big_group<WT, BB, 1>), grid, dim3(256), 0, s, g, 0); \
-    else hipLaunchKernelGGL((k_mvm_big_group<WT, BB, 3>), grid, dim3(256), 0, s, g, 0); \
+    if (w_oc) hipLaunchKernelGGL((k_mvm_big_group<1, BB, XP>), grid, dim3(256), 0, s, g, 0); \
+    else hipLaunchKernelGGL((k_mvm_big_group<0, BB, XP>), grid, dim3(256), 0, s, g, 0); \
   } while (0)
-  if (bb == 128) {
-    if (w_oc) RPU_LAUNCH_BIG(1, 128);
-    else RPU_LAUNCH_BIG(0, 128);
-  } else {
-    if (w_oc) RPU_LAUNCH_BIG(1, 64);
-    else RPU_LAUNCH_BIG(0, 64);
-  }
+  if (!stepped) RPU_LAUNCH_BIG(64, 3);
+  else if (bb == 128) RPU_LAUNCH_BIG(128, 1);
+  else RPU_LAUNCH_BIG(64, 1);
 #undef RPU_LAUNCH_BIG
 }
 
@@ -2763,19 +2763,20 @@ void launch_mvm_round(const MvmArgs &a_in, hipStream_t s) {
     const int n_cus = current_device_cus();
     const bool sparse = a.O > 64 && (big_workgroups(a, 64, 64) < 3 * n_cus || a.k_pad <= 2 * BKS);
     const int ot = a.O <= 64 || sparse ? 64 : 128;
-    const int bb = sparse ? 64 : (ot == 64 ? 128 : mvm_big_sample_tile(big_workgroups(a, 128), n_cus));
+    const int bb = sparse ? 64 : (ot == 64 ? 128 : mvm_big_sample_tile(big_workgroups(a, 128), n_cus, a.x_step > 0.0f));
     const dim3 big_grid(big_workgroups(a, bb, ot));
     const int min_active = a.round > 0 ? a.big_from : 0;
 #define RPU_LAUNCH_BIG(WT, BB, WO, XP, LAZY) \
   hipLaunchKernelGGL((k_mvm_big<WT, BB, WO, XP, LAZY>), big_grid, dim3(256), 0, s, a, min_active)
 #define RPU_PICK_BIG(WT, XP) \
   do { \
+    constexpr int WIDE = XP == 1 ? 128 : 64; /* mvm_big_sample_tile */ \
     if (ot == 64 && bb == 128 && lazy) RPU_LAUNCH_BIG(WT, 128, 2, XP, true); \
     else if (ot == 64 && bb == 128) RPU_LAUNCH_BIG(WT, 128, 2, XP, false); \
     else if (ot == 64 && lazy) RPU_LAUNCH_BIG(WT, 64, 2, XP, true); \
     else if (ot == 64) RPU_LAUNCH_BIG(WT, 64, 2, XP, false); \
-    else if (bb == 128 && lazy) RPU_LAUNCH_BIG(WT, 128, 4, XP, true); \
-    else if (bb == 128) RPU_LAUNCH_BIG(WT, 128, 4, XP, false); \
+    else if (bb == 128 && lazy) RPU_LAUNCH_BIG(WT, WIDE, 4, XP, true); \
+    else if (bb == 128) RPU_LAUNCH_BIG(WT, WIDE, 4, XP, false); \
     else if (lazy) RPU_LAUNCH_BIG(WT, 64, 4, XP, true); \
     else RPU_LAUNCH_BIG(WT, 64, 4, XP, false); \
   } while (0)

@@ -564,7 +564,7 @@ struct Tile {
     s_tiledone.ensure((size_t)32 * ((n + 31) / 32));
   }
 
-  IoDev io_dev(const IOPar &io) const {
+  static IoDev io_dev(const IOPar &io) {
     IoDev d;
     d.inp_res = io.p.inp_res; d.inp_bound = io.p.inp_bound; d.inp_noise = io.p.inp_noise; d.inp_asym = io.p.inp_asymmetry;
     d.out_res = io.p.out_res; d.out_bound = io.p.out_bound; d.out_noise = io.p.out_noise; d.out_asym = io.p.out_asymmetry;
@@ -2704,6 +2704,7 @@ static int group_mvm(rpu_group_t *group, const float *const *x_dev, const long *
     // a batch of 1024 or more on tiles at least 128 outputs wide: the large-tile kernel runs round 0 of those tiles,
     // if the group has enough of its workgroups to fill the chip
     int big_total = 0, big_bb = 128;
+    bool all_stepped = true; // of the tiles on the large-tile kernel (MvmArgs::x_step)
     if (m_batch >= 1024) {
       if (group->cu_count == 0) {
         hipDeviceProp_t prop;
@@ -2717,14 +2718,15 @@ static int group_mvm(rpu_group_t *group, const float *const *x_dev, const long *
         shape.m_batch = m_batch;
         total_128 += mvm_big_workgroups(shape, 128);
         total_64 += mvm_big_workgroups(shape, 64);
+        const Tile &t = group->tiles[i]->t;
+        if (shape.O >= 128 && mvm_input_step(Tile::io_dev(transposed ? t.bio : t.fio)) <= 0.0f) all_stepped = false;
       }
-      big_bb = mvm_big_sample_tile(total_128, group->cu_count);
+      big_bb = mvm_big_sample_tile(total_128, group->cu_count, all_stepped);
       big_total = big_bb == 128 ? total_128 : total_64;
     }
     // with the half tiles, one workgroup on every second CU already beats the 32 x 32 kernel
     const bool use_big = big_total >= (big_bb == 128 ? 256 : 128);
     bool all_big = use_big;
-    bool all_stepped = true; // of the tiles on the large-tile kernel (MvmArgs::x_step)
     // per tile: arguments of a plain forward call (row-major x [m_batch][x_size], y [m_batch][d_size])
     std::vector<MvmArgs> args(n);
     std::vector<int> depth(n), mode(n);
@@ -2745,7 +2747,6 @@ static int group_mvm(rpu_group_t *group, const float *const *x_dev, const long *
       if (a.in_sb < in_size || a.out_sb < out_size) throw RpuError("A row stride is shorter than the row.");
       a.big_from = big ? -1 : 0;
       if (!big) all_big = false;
-      else if (a.x_step <= 0.0f) all_stepped = false;
       mvm_round_variant(a, depth[i], mode[i]);
       rounds = std::max(rounds, a.max_rounds);
       args[i] = a;
