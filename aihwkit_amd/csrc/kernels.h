@@ -178,7 +178,7 @@ int mvm_big_workgroups(const MvmArgs &a, int bb);
 // bb: samples of a workgroup tile, 128 or 64 (mvm_big_sample_tile: by the workgroups the launch would have with 128)
 // stepped: the inputs of the launch are whole numbers of DAC steps (MvmArgs::x_step)
 int mvm_big_sample_tile(int workgroups_128, int n_cus, bool stepped);
-float mvm_input_step(const IoDev &io);
+float mvm_input_step(const IoDev &io, int K);
 // w_oc: how the tiles of the launch address their weights (MvmArgs::w_oc; the same for all of them)
 void launch_mvm_big_group(const MvmGroup &g, int total_workgroups, int bb, bool w_oc, bool stepped, hipStream_t s);
 void mvm_round_variant(const MvmArgs &a, int &prefetch_depth, int &weight_mode);

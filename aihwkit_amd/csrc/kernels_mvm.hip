@@ -1585,8 +1585,9 @@ __global__ __launch_bounds__(256) void k_mvm_round(MvmArgs a) {
 // from L2 feeds 64 multiply-adds instead of 16.
 // On the fp32 matrix pipe, which set the pace before, a round of 16384 samples on a 1024 x 1024 tile took 316 us
 // (backward), the four linear layers of a 768-wide transformer block 69 + 34 + 80 + 69 us at 1024 tokens; with the split
-// operands 164 us and 49 + 30 + 54 + 50 us.  Error against 64-bit sums (relative, 1024 terms): 5.7e-7 before, 3.1e-7 with
-// quantized inputs, 4.9e-7 with any other.  Same per-sample state, lists, epilogue and random streams as the 32 x 32 kernel: a round
+// operands 164 us and 49 + 30 + 54 + 50 us.  Error against 64-bit sums (relative): of 16 / 32 / 256 / 1024 terms 0.76 / 1.05
+// / 2.9 / 5.7e-7 on the fp32 pipe, 0.65 / 0.79 / 1.6 / 3.1e-7 with quantized inputs, 0.29 / 0.35 / 0.80 / 1.7e-7 with any
+// other.  Same per-sample state, lists, epilogue and random streams as the 32 x 32 kernel: a round
 // may be run by either (the launcher picks by the number of samples in the round).
 // WT = 0: weights contiguous along k (forward), 1: contiguous along the outputs (backward, W read in place).
 
@@ -1697,10 +1698,12 @@ __device__ __forceinline__ float max_abs4(float m, const f32x4 v) { // NaN do no
 //   XP = 1  one for an input that the DAC has rounded to a multiple k of its step, |k| <= 256 (MvmArgs::x_step): the
 //           rows hold k * step, k is what is staged, and the step multiplies the finished sum.  3 exact products of 8 x 8
 //           bits per element against the one rounded input k * step of the fp32 pipe;
-//   XP = 3  three for any other input, of whose nine products the three below 2^-24 of the whole are left out.
-// Sums are kept in fp32 as before, in chains an eighth as long.  A tile with a value outside the range in which the
-// parts and their products are safe (infinities among them, whose parts would be NaN) is multiplied again on the fp32
-// pipe; choosing the pipe stage by stage inside the loop cost a copy of all accumulators per stage.
+//   XP = 3  three for any other input: nine products, of which the one of the two low parts (2^-36 of the whole) is left
+//           out.  The sums of the seven that correct the product of the high parts are added to it at the end: a sum
+//           of n terms is then rounded n / 16 times where it counts, against n / 2 times on the fp32 pipe.
+// Sums are kept in fp32 as before, in chains an eighth as long (XP = 1) or shorter.  A tile with a value outside the range
+// in which the parts and their products are safe (infinities among them, whose parts would be NaN) is multiplied again on
+// the fp32 pipe; choosing the pipe stage by stage inside the loop cost a copy of all accumulators per stage.
 // LAZY (calls with speculate = 0): nothing is quantized ahead; the last workgroup of a sample tile writes the rows of
 // the samples that go on.  The other instantiations always quantize ahead, as their callers ask for.
 template <int WT, int BB, int WO, int XP, bool LAZY>
@@ -1827,11 +1830,11 @@ __device__ __forceinline__ void mvm_big_workgroup(const MvmArgs &a, const int ro
     if (!(m < SAFE)) sh_slow = 1;
   };
 
-  floatx16 acc[NB];
+  floatx16 acc[NB], low[XP == 3 ? NB : 1];
 #pragma unroll
   for (int i = 0; i < NB; ++i) {
 #pragma unroll
-    for (int e = 0; e < 16; ++e) acc[i][e] = 0.0f;
+    for (int e = 0; e < 16; ++e) acc[i][e] = low[XP == 3 ? i : 0][e] = 0.0f;
   }
 
   // lane (r, h) multiplies k = 16 h .. 16 h + 15 of a stage, eight values per MFMA: the order of k within a stage does
@@ -1869,13 +1872,18 @@ __device__ __forceinline__ void mvm_big_workgroup(const MvmArgs &a, const int ro
       const bf16x8 w[3] = {__builtin_bit_cast(bf16x8, u32x4{h0.x, h0.y, h1.x, h1.y}),
                            __builtin_bit_cast(bf16x8, u32x4{m0.x, m0.y, m1.x, m1.y}),
                            __builtin_bit_cast(bf16x8, u32x4{l0.x, l0.y, l1.x, l1.y})};
+      // part q of a weight with part p of an input
 #pragma unroll
-      for (int p = 0; p < XP; ++p) {
+      for (int i = 0; i < (XP == 1 ? 3 : 4); ++i) {
+        const int n = XP == 1 ? i : 3 - i;
 #pragma unroll
-        for (int q = 0; q + p < 3; ++q) {
+        for (int q = 0; q <= min(n, 2); ++q) {
+          const int p = n - q;
+          if (p >= XP) continue;
 #pragma unroll
           for (int nb = 0; nb < NB; ++nb) {
-            acc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[q], x[nb][p], acc[nb], 0, 0, 0);
+            floatx16 &sum = XP == 3 && n > 0 ? low[XP == 3 ? nb : 0] : acc[nb];
+            sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[q], x[nb][p < XP ? p : 0], sum, 0, 0, 0);
           }
         }
       }
@@ -1898,6 +1906,10 @@ __device__ __forceinline__ void mvm_big_workgroup(const MvmArgs &a, const int ro
     }
   }
   float x_step = XP == 1 ? a.x_step : 1.0f;
+  if (XP == 3) {
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) acc[nb] += low[XP == 3 ? nb : 0];
+  }
   if (sh_slow) { // a value out of the range of the parts: this tile again on the fp32 pipe, straight from memory
     x_step = 1.0f; // the rows hold k * step
     const int o = min(tile_o * OT + wo * 32 + r, a.O - 1);
@@ -2460,9 +2472,11 @@ int mvm_max_rounds(const IoDev &io) {
 
 // The DAC step if every quantized input is a multiple k of it with |k| <= 256 up to rounding (a bf16 holds those k), 0
 // otherwise: no input noise or asymmetry on top, and an input range that is itself a multiple of the step, because
-// values beyond it are clipped to the range.
-float mvm_input_step(const IoDev &io) {
-  if (io.perfect || !(io.inp_res > 0.0f) || io.inp_noise > 0.0f || io.inp_asym != 0.0f) return 0.0f;
+// values beyond it are clipped to the range.  Sums of fewer than 16 terms take three parts: the step that multiplies the
+// finished sum is a rounding of its own (relative error of 2 / 4 / 8 terms: 6.7 / 6.3 / 5.9e-8 with one part, 2.5 / 4.0 /
+// 5.7e-8 on the fp32 pipe), and with one stage to multiply they cost the same.
+float mvm_input_step(const IoDev &io, int K) {
+  if (K < 16 || io.perfect || !(io.inp_res > 0.0f) || io.inp_noise > 0.0f || io.inp_asym != 0.0f) return 0.0f;
   const double steps = (double)io.inp_bound / (double)io.inp_res;
   if (!(steps >= 1.0 && steps < 256.5) || std::fabs(steps - std::rint(steps)) > 1e-6 * steps) return 0.0f;
   if (!(io.inp_res > 0x1p-60f && io.inp_res < 0x1p60f)) return 0.0f;

@@ -598,7 +598,7 @@ struct Tile {
     a.transposed = transposed ? 1 : 0;
     mvm_set_weights(a, w_other ? w_other : wdev(), w_ld(), xd);
     a.io = io_dev(io);
-    a.x_step = mvm_input_step(a.io);
+    a.x_step = mvm_input_step(a.io, K);
     a.alpha = io.p.out_scale; a.beta = 0.0f;
     a.key = key(); a.call = call++;
     a.st.next_scale[0] = s_nsc0.p; a.st.next_scale[1] = s_nsc1.p;
@@ -2719,7 +2719,7 @@ static int group_mvm(rpu_group_t *group, const float *const *x_dev, const long *
         total_128 += mvm_big_workgroups(shape, 128);
         total_64 += mvm_big_workgroups(shape, 64);
         const Tile &t = group->tiles[i]->t;
-        if (shape.O >= 128 && mvm_input_step(Tile::io_dev(transposed ? t.bio : t.fio)) <= 0.0f) all_stepped = false;
+        if (shape.O >= 128 && mvm_input_step(Tile::io_dev(transposed ? t.bio : t.fio), transposed ? t.D : t.X) <= 0.0f) all_stepped = false;
       }
       big_bb = mvm_big_sample_tile(total_128, group->cu_count, all_stepped);
       big_total = big_bb == 128 ? total_128 : total_64;

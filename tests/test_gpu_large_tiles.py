@@ -88,3 +88,40 @@ def test_values_out_of_the_range_of_the_parts(gpu_device, x_size, d_size, batch)
     with np.errstate(all="ignore"):
         bound = (x_size + 2) * 2.0 ** -24 * (np.abs(x.astype(np.float64)) @ np.abs(w.astype(np.float64)).T)
         assert np.all((np.abs(got.astype(np.float64) - want) <= bound + 1e-37)[fine])
+
+
+def _chain(x, w):
+    """x w^T as multiply-adds of two terms at a time in fp32, as the fp32 matrix pipe makes it."""
+    x, w = x.astype(np.float64), w.astype(np.float64)
+    if x.shape[1] % 2:
+        x, w = np.pad(x, ((0, 0), (0, 1))), np.pad(w, ((0, 0), (0, 1)))
+    acc = np.zeros((x.shape[0], w.shape[0]), np.float32)
+    for k in range(0, x.shape[1], 2):
+        acc = (acc + (np.outer(x[:, k], w[:, k]) + np.outer(x[:, k + 1], w[:, k + 1]))).astype(np.float32)
+    return acc
+
+
+@pytest.mark.parametrize("stepped", [False, True])
+@pytest.mark.parametrize("terms", [1, 2, 3, 5, 8, 15, 16, 17, 27, 32, 33, 64, 433, 1024])
+def test_no_further_from_64_bit_sums_than_a_chain_in_fp32(gpu_device, terms, stepped):
+    """Root mean square error over 256 x 64 outputs; the two that are compared are each known to 1 / sqrt(2 * 16384)."""
+    rng = np.random.default_rng(terms)
+    out_size, batch, steps = 64, 16384, 63
+    io = noise_free_io(inp_res=1.0 / (2 * steps) if stepped else -1.0)
+    io.out_res, io.out_bound, io.is_perfect = -1.0, float("inf"), not stepped
+    w = rng.uniform(-0.6, 0.6, (out_size, terms)).astype(np.float32)
+    x = rng.uniform(-1.0, 1.0, (batch, terms)).astype(np.float32)
+    want_x = x.astype(np.float64)
+    if stepped:
+        x[:, 0] = 1.0  # meets the range
+        step = np.float32(2.0 * np.float32(1.0 / (2 * steps)))
+        want_x = np.rint(x / step).astype(np.float64) * float(step)
+        x = want_x.astype(np.float32)
+    some = slice(0, batch, batch // 256)
+    want = want_x[some] @ w.T.astype(np.float64)
+    chain = np.sqrt(np.mean((_chain(x[some], w) - want) ** 2))
+    forward = _tile(terms, out_size, io, w).forward(torch.from_numpy(x).cuda())
+    backward = _tile(out_size, terms, io, np.ascontiguousarray(w.T)).backward(torch.from_numpy(x).cuda())
+    for got in (forward, backward):
+        error = np.sqrt(np.mean((got[some].double().cpu().numpy() - want) ** 2))
+        assert error <= 1.04 * chain
