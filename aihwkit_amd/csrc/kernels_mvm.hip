@@ -1678,8 +1678,9 @@ template <bool STAGED> __device__ __forceinline__ uint32_t pack_bf16(float lower
   asm("" : "+v"(p));
   return p;
 }
-// v = hi + mid + lo with every part rounded to bf16: 3 x 8 bits hold the 24 of a float, so the sum is exact (above
-// 2^-110; the low part of a smaller value may drop out).
+// v = hi + mid + lo with every part rounded to bf16: 3 x 8 bits hold the 24 of a float, so the sum is exact where the last
+// bit of v is one that a bf16 can have, 2^-133.  The last bit of a float may be 2^-149: the kernel splits 2^16 times the
+// value.
 template <bool STAGED> __device__ __forceinline__ void split_bf16(const f32x4 v, u32x2 &hi, u32x2 &mid, u32x2 &lo) {
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
@@ -1805,7 +1806,8 @@ __device__ __forceinline__ void mvm_big_workgroup(const MvmArgs &a, const int ro
   };
   // k * step times 1 / step is k up to a few units in the 24th bit: rounding to bf16 returns k itself
   const float inv_step = XP == 1 ? 1.0f / a.x_step : 1.0f;
-  constexpr float SAFE = XP == 1 ? 0x1p100f : 0x1p60f; // parts and products stay finite below it
+  constexpr float LIFT = 0x1p16f; // the operands in parts are this times their value (split_bf16)
+  constexpr float SAFE = XP == 1 ? 0x1p84f : 0x1p44f; // parts and products stay finite below it
   auto lds_store = [&](int buf, const f32x4 (&gx)[XJ], const f32x4 (&gw)[WJ]) __attribute__((always_inline)) {
     float m = 0.0f;
 #pragma unroll
@@ -1816,7 +1818,7 @@ __device__ __forceinline__ void mvm_big_workgroup(const MvmArgs &a, const int ro
         *reinterpret_cast<u32x2 *>(dst) = u32x2{pack_bf16<true>(k.x, k.y), pack_bf16<true>(k.z, k.w)};
       } else {
         u32x2 hi, mid, lo;
-        split_bf16<true>(gx[j], hi, mid, lo);
+        split_bf16<true>(gx[j] * LIFT, hi, mid, lo);
         *reinterpret_cast<u32x2 *>(dst) = hi;
         *reinterpret_cast<u32x2 *>(dst + BB * BKS) = mid;
         *reinterpret_cast<u32x2 *>(dst + 2 * BB * BKS) = lo;
@@ -1828,6 +1830,7 @@ __device__ __forceinline__ void mvm_big_workgroup(const MvmArgs &a, const int ro
       f32x4 w = gw[j];
       if (WT == 1 && wt_ragged && wt_shift > 0) w = {wt_shift == 1 ? w.y : (wt_shift == 2 ? w.z : w.w), wt_shift == 1 ? w.z : w.w, w.w, w.w};
       m = max_abs4(m, w);
+      w *= LIFT;
       if (WT == 0) {
         *reinterpret_cast<f32x4 *>(&lds_w[buf][big_lds_offset((t >> 3) + 32 * j, t & 7)]) = w;
       } else {
@@ -1912,13 +1915,13 @@ __device__ __forceinline__ void mvm_big_workgroup(const MvmArgs &a, const int ro
       __syncthreads();
     }
   }
-  float x_step = XP == 1 ? a.x_step : 1.0f;
+  float unit = XP == 1 ? a.x_step / LIFT : 1.0f / (LIFT * LIFT); // of the sums
   if (XP == 3) {
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) acc[nb] += low[XP == 3 ? nb : 0];
   }
   if (sh_slow) { // a value out of the range of the parts: this tile again on the fp32 pipe, straight from memory
-    x_step = 1.0f; // the rows hold k * step
+    unit = 1.0f; // the rows hold k * step, and nothing is lifted
     const int o = min(tile_o * OT + wo * 32 + r, a.O - 1);
     const float *w_first = a.w + (WT ? (long)o : (long)o * a.w_ld);
     const long w_next = WT ? (long)a.w_ld : 1;
@@ -1961,7 +1964,7 @@ __device__ __forceinline__ void mvm_big_workgroup(const MvmArgs &a, const int ro
         const int o0 = tile_o * OT + wo * 32 + g * 8 + h * 4;
         float v[4];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) v[q] = XP == 1 ? sums[4 * g + q] * x_step : sums[4 * g + q];
+        for (int q = 0; q < 4; ++q) v[q] = sums[4 * g + q] * unit;
         int up = 0, lo = 0;
         if (o0 < a.O) mvm_finish_outputs(a, round, b_out, fin_out, o0, v, up, lo);
         up_max = max(up_max, up);

@@ -125,3 +125,22 @@ def test_no_further_from_64_bit_sums_than_a_chain_in_fp32(gpu_device, terms, ste
     for got in (forward, backward):
         error = np.sqrt(np.mean((got[some].double().cpu().numpy() - want) ** 2))
         assert error <= 1.04 * chain
+
+
+@pytest.mark.parametrize("small", ["weights", "inputs", "weights of quantized inputs"])
+@pytest.mark.parametrize("x_size,d_size,batch", [(40, 64, 16500), (433, 48, 16500), (513, 257, 3401)])
+def test_values_near_the_lower_end_of_the_range(gpu_device, x_size, d_size, batch, small):
+    """An operand times 2^-120 gives 2^-120 times the result: the operands keep all their bits (multiples of 2^-144).
+    Where the result and its scaling are below the range of normal floats, each is rounded to a multiple of 2^-149."""
+    rng = np.random.default_rng(x_size)
+    quantized = small == "weights of quantized inputs"
+    io = noise_free_io(inp_res=1.0 / 126 if quantized else -1.0)
+    io.out_res, io.out_bound, io.is_perfect = -1.0, float("inf"), not quantized
+    w = (rng.integers(-2 ** 23, 2 ** 23, (d_size, x_size)) * 2.0 ** -24).astype(np.float32)
+    tiny = np.float32(2.0 ** -120)
+    normal, low = _tile(x_size, d_size, io, w), _tile(x_size, d_size, io, w if small == "inputs" else w * tiny)
+    for call, width in (("forward", x_size), ("backward", d_size)):
+        v = torch.from_numpy((rng.integers(-2 ** 23, 2 ** 23, (batch, width)) * 2.0 ** -24).astype(np.float32)).cuda()
+        want = getattr(normal, call)(v).double()
+        got = getattr(low, call)(v * float(tiny) if small == "inputs" else v).double() * 2.0 ** 120
+        assert float((got - want).abs().max()) <= 4 * 2.0 ** -30
