@@ -2482,13 +2482,14 @@ int mvm_max_rounds(const IoDev &io) {
 
 // The DAC step if every quantized input is a multiple k of it with |k| <= 256 up to rounding (a bf16 holds those k), 0
 // otherwise: no input noise or asymmetry on top, and an input range that is itself a multiple of the step, because
-// values beyond it are clipped to the range.  Sums of fewer than 16 terms take three parts: the step that multiplies the
+// values beyond it are clipped to the range (2^-23: what the roundings of a step and of its product with the range leave
+// of a whole number).  Sums of fewer than 16 terms take three parts: the step that multiplies the
 // finished sum is a rounding of its own (relative error of 2 / 4 / 8 terms: 6.7 / 6.3 / 5.9e-8 with one part, 2.5 / 4.0 /
 // 5.7e-8 on the fp32 pipe), and with one stage to multiply they cost the same.
 float mvm_input_step(const IoDev &io, int K) {
   if (K < 16 || io.perfect || !(io.inp_res > 0.0f) || io.inp_noise > 0.0f || io.inp_asym != 0.0f) return 0.0f;
   const double steps = (double)io.inp_bound / (double)io.inp_res;
-  if (!(steps >= 1.0 && steps < 256.5) || std::fabs(steps - std::rint(steps)) > 1e-6 * steps) return 0.0f;
+  if (!(steps >= 1.0 && steps < 256.5) || std::fabs(steps - std::rint(steps)) > 0x1p-23 * steps) return 0.0f;
   if (!(io.inp_res > 0x1p-60f && io.inp_res < 0x1p60f)) return 0.0f;
   return io.inp_res;
 }

@@ -144,3 +144,18 @@ def test_values_near_the_lower_end_of_the_range(gpu_device, x_size, d_size, batc
         want = getattr(normal, call)(v).double()
         got = getattr(low, call)(v * float(tiny) if small == "inputs" else v).double() * 2.0 ** 120
         assert float((got - want).abs().max()) <= 4 * 2.0 ** -30
+
+
+@pytest.mark.parametrize("terms", [16, 64])
+def test_a_range_that_is_nearly_a_multiple_of_the_step(gpu_device, terms):
+    """63 steps reach 5e-7 beyond the range: the inputs that meet it are the range, not 63 steps."""
+    rng = np.random.default_rng(terms)
+    io = noise_free_io(inp_res=float(np.float32((1.0 + 5e-7) / 126)))
+    io.out_res, io.out_bound = -1.0, float("inf")
+    step = 2.0 * float(np.float32(io.inp_res))
+    assert 3e-7 < 63 * step - 1.0 < 1e-6
+    w = rng.uniform(-0.6, 0.6, (64, terms)).astype(np.float32)
+    x = np.where(rng.random((16384, terms)) < 0.5, -1.0, 1.0).astype(np.float32)
+    got = _tile(terms, 64, io, w).forward(torch.from_numpy(x).cuda())[::64].double().cpu().numpy()
+    want, chain = x[::64] @ w.T.astype(np.float64), _chain(x[::64], w)
+    assert np.sqrt(np.mean((got - want) ** 2)) <= 1.04 * np.sqrt(np.mean((chain - want) ** 2))
