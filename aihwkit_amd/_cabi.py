@@ -7,6 +7,7 @@ there is no Python or CPU fallback for the tile computations.
 import ctypes as C
 import os
 import threading
+import warnings
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "lib", "librpu_amd.so")
@@ -238,12 +239,21 @@ def lib():
     return _lib
 
 
+class _GeneralPath:
+    """Stands in for the native module where that is missing: every call answers None, which sends the Python tiles to
+    their general path (the same C entry points through ctypes)."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
 _torch_calls = None
 
 
 def torch_calls():
-    """The native module behind the compute calls on torch tensors (``csrc/torch_calls.cpp``), loaded once.  Raises if it
-    has not been built; torch must have been imported."""
+    """The native module behind the compute calls on torch tensors (``csrc/torch_calls.cpp``), loaded once; torch must have
+    been imported.  It is host code that saves time around each call: without it (it needs torch's headers to be built) the
+    tiles compute all the same."""
     global _torch_calls
     if _torch_calls is None:
         import importlib.machinery
@@ -251,12 +261,15 @@ def torch_calls():
 
         lib()
         path = os.path.join(_HERE, "lib", "rpu_torch.so")
-        if not os.path.exists(path):
-            raise RuntimeError(f"{path} is missing: build it with `make -C aihwkit_amd/csrc`.")
         loader = importlib.machinery.ExtensionFileLoader("rpu_torch", path)
         spec = importlib.util.spec_from_file_location("rpu_torch", path, loader=loader)
-        module = importlib.util.module_from_spec(spec)
-        loader.exec_module(module)
+        try:
+            module = importlib.util.module_from_spec(spec)
+            loader.exec_module(module)
+        except ImportError as error:
+            warnings.warn(f"The native calls on torch tensors could not be loaded ({error}); calls take longer without them. "
+                          "Build them with `make -C aihwkit_amd/csrc`.", RuntimeWarning, stacklevel=3)
+            module = _GeneralPath()
         _torch_calls = module
     return _torch_calls
 

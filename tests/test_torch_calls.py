@@ -99,3 +99,51 @@ def test_outputs_that_share_their_memory_until_written():
         out = torch._lazy_clone(first)
         call(inputs, outs=[out])
         assert bool((first == 7.0).all()) and bool((out != 7.0).all())
+
+
+@pytest.fixture
+def without_native_calls(monkeypatch, tmp_path):
+    """No module at the place where it is looked for."""
+    from aihwkit_amd import _cabi
+    _cabi.lib()
+    monkeypatch.setattr(_cabi, "_torch_calls", None)
+    monkeypatch.setattr(_cabi, "_HERE", str(tmp_path))
+    with pytest.warns(RuntimeWarning, match="make -C"):
+        _cabi.torch_calls()
+
+
+def test_tiles_take_the_general_path_without_the_native_calls(without_native_calls):
+    import torch
+
+    from helpers import constant_step, make_meta
+    from aihwkit_amd.rpu_base.tiles import CudaAnalogTile
+    tile = make_meta().create_array(8, 4, constant_step())  # on the host: the GPU tile's methods get as far as the tensors
+    tile._update_without_allocation = False
+    x, d = torch.ones(3, 8), torch.ones(3, 4)
+    for call in (lambda: CudaAnalogTile.forward(tile, x), lambda: CudaAnalogTile.backward(tile, d),
+                 lambda: CudaAnalogTile.update(tile, x, d, False)):
+        with pytest.raises(RuntimeError, match="x_input|d_input"):  # the words of that path for tensors on the CPU
+            call()
+
+
+@pytest.mark.gpu
+def test_results_without_the_native_calls(without_native_calls, monkeypatch):
+    import torch
+
+    from aihwkit_amd import _cabi
+    from aihwkit_amd.rpu_base.tiles import TileGroup
+
+    def results():
+        tile, other = _tile(40, 24), _tile(40, 24)
+        group = TileGroup([other])
+        g = torch.Generator("cuda").manual_seed(3)
+        x, d = (torch.rand(7, n, generator=g, device="cuda") - 0.5 for n in (40, 24))
+        tile.update(x, d, False)
+        group.update([x], [d])
+        return [tile.forward(x), tile.backward(d), tile.get_weights()] + group.forward([x]) + group.backward([d])
+
+    general = results()
+    monkeypatch.undo()
+    assert not isinstance(_cabi.torch_calls(), _cabi._GeneralPath)
+    for a, b in zip(general, results()):
+        assert torch.equal(torch.as_tensor(a), torch.as_tensor(b))
