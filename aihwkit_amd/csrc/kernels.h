@@ -171,6 +171,7 @@ bool mvm_group_can_merge_rest(const MvmGroup &g, int weight_mode);
 int mvm_group_rest_resident_limit(int weight_mode); // workgroups of k_mvm_rest_group that the GPU holds at once
 void launch_mvm_rest_group(const MvmGroup &g, int weight_mode, int round_first, int rounds, int workgroups, int *seen,
                            hipStream_t s);
+int current_device_cus(); // compute units of the calling thread's GPU
 int mvm_round_workgroups(const MvmArgs &a);            // workgroups of a round launch for this tile
 // Large-tile (128 x 128) variant for round 0 of a group: args[t].big_from < 0 marks the tiles it runs, start[]
 // counts its workgroups (mvm_big_workgroups; 0 for the other tiles).

@@ -31,6 +31,7 @@
 //   *_group        the same kernels over the tiles of a group in one launch.
 #include "kernels.h"
 
+#include <atomic>
 #include <cmath>
 #include <mutex>
 
@@ -2610,8 +2611,8 @@ void launch_mvm_big_group(const MvmGroup &g, int total_workgroups, int bb, bool 
 #undef RPU_LAUNCH_BIG
 }
 
-static int current_device_cus() {
-  static int cus[64] = {0};
+int current_device_cus() {
+  static std::atomic<int> cus[64];
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
   if (cus[dev] == 0) {

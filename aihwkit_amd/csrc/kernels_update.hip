@@ -2003,10 +2003,10 @@ static int update_pulsed_columns(const UpdateArgs &a) {
 
 // Whether the pulse loop of this call runs as a pipeline of waves (k_update_pulsed_stream): a batch that fills the
 // pipeline, on a tile with at most one wave of cross-points per SIMD (with more, the plain loop's waves overlap each
-// other and its fewer instructions per pass count: 25 against 40).
+// other and its fewer instructions per pass count: 25 against 40).  A CU has four SIMDs.
 bool update_takes_stream(const UpdateArgs &a) {
   return update_pulsed_columns(a) == 1 && a.n_chunks >= 32 && a.m_batch < (1 << 23) &&
-         (long)((a.x_size + 63) / 64) * a.d_size <= 1024;
+         (long)((a.x_size + 63) / 64) * a.d_size <= 4L * current_device_cus();
 }
 template <bool NOISE, int PARTS> static void launch_update_pulsed_stream(const UpdateArgs &a, hipStream_t s) {
   const dim3 grid(((a.x_size + 63) / 64 + PARTS - 1) / PARTS, a.d_size), block(64 * (1 + 3 * PARTS));
@@ -2025,7 +2025,7 @@ void launch_update_pulsed(const UpdateArgs &a, hipStream_t s) {
     // two teams to a workgroup where single ones would be more than the CUs: seven waves on a CU's four SIMDs, evenly
     // over the chip, instead of two workgroups on some CUs and one on the others
     const bool noise = a.dev.dw_min_std > 0.0f;
-    if ((long)((a.x_size + 63) / 64) * a.d_size <= 256) {
+    if ((long)((a.x_size + 63) / 64) * a.d_size <= current_device_cus()) {
       if (noise) launch_update_pulsed_stream<true, 1>(a, s);
       else launch_update_pulsed_stream<false, 1>(a, s);
     } else {

@@ -2724,8 +2724,8 @@ static int group_mvm(rpu_group_t *group, const float *const *x_dev, const long *
       big_bb = mvm_big_sample_tile(total_128, group->cu_count, all_stepped);
       big_total = big_bb == 128 ? total_128 : total_64;
     }
-    // with the half tiles, one workgroup on every second CU already beats the 32 x 32 kernel
-    const bool use_big = big_total >= (big_bb == 128 ? 256 : 128);
+    // one workgroup per CU; with the half tiles, one on every second CU already beats the 32 x 32 kernel
+    const bool use_big = big_total > 0 && big_total >= (big_bb == 128 ? group->cu_count : group->cu_count / 2);
     bool all_big = use_big;
     // per tile: arguments of a plain forward call (row-major x [m_batch][x_size], y [m_batch][d_size])
     std::vector<MvmArgs> args(n);
