@@ -390,13 +390,13 @@ def main() -> int:
         tile_b.set_profiling(False)
         fl = 2.0 * x_size * d_size * big
         other = {
-            "forward_batch_16384": {"kernel": "k_mvm_big<0> (all rounds of a call)", "kernel_ms": prof_fb["mvm_round"][0],
+            "forward_batch_16384": {"kernel": "k_mvm_big<0, 128, 4, 1, false> (all rounds of a call)", "kernel_ms": prof_fb["mvm_round"][0],
                                     "mean_bm_rounds": rounds_b,
                                     "useful_tflops": fl / (prof_fb["mvm_round"][0] * 1e-3) / 1e12,
                                     "frac_of_mfma_peak_useful": fl / (prof_fb["mvm_round"][0] * 1e-3) / 1e12 / SPLIT_MFMA_PEAK_TFLOPS,
                                     "frac_of_mfma_peak_executed": rounds_b * fl / (prof_fb["mvm_round"][0] * 1e-3) / 1e12
                                     / SPLIT_MFMA_PEAK_TFLOPS},
-            "backward_batch_16384": {"kernel": "k_mvm_big<1>", "kernel_ms": prof_bb["mvm_round"][0],
+            "backward_batch_16384": {"kernel": "k_mvm_big<1, 128, 4, 1, false>", "kernel_ms": prof_bb["mvm_round"][0],
                                      "tflops": fl / (prof_bb["mvm_round"][0] * 1e-3) / 1e12,
                                      "frac_of_mfma_peak": fl / (prof_bb["mvm_round"][0] * 1e-3) / 1e12 / SPLIT_MFMA_PEAK_TFLOPS},
         }

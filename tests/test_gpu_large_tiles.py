@@ -23,11 +23,16 @@ def _tile(x_size, d_size, io, w):
     return tiles.CudaAnalogTile(host)
 
 
-def _close(got, want, terms, lengths):
+def _close(got, want, terms, lengths, n=None):
     """A sum of n products in fp32 is off by at most (n + 2) half units of the sum of the absolute products; random signs
-    leave far less than a quarter of that bound."""
+    leave far less than a quarter of that bound.  Over all sums: n / 2 roundings of sums no larger than the last one, each
+    off by 2^-24 / sqrt(3) of it (root mean square), and two more of the operand and of the result.  A lost low part would
+    show: 2^-18 of every product."""
+    error = np.abs(got.double().cpu().numpy() - want)
     bound = 0.25 * (lengths + 2) * 2.0 ** -24 * terms + 1e-37
-    assert np.all(np.abs(got.double().cpu().numpy() - want) <= bound)
+    assert np.all(error <= bound)
+    roundings = (lengths if n is None else n) / 2 + 2
+    assert np.sqrt(np.mean(error ** 2)) <= 2.0 ** -24 * np.sqrt(roundings / 3 * np.mean(want ** 2))
 
 
 @pytest.mark.parametrize("scale", [0.3, 1e-12, 1e10])
@@ -64,7 +69,7 @@ def test_quantized_products_against_64_bit_sums(gpu_device, x_size, d_size, batc
         q = np.clip(np.rint(v / step), -steps, steps).astype(np.float64) * float(step)
         got = call(torch.from_numpy(v).cuda())
         # the reference's own rounding of k * step and of the clipped range: one half unit per product
-        _close(got, q @ axis, np.abs(q) @ np.abs(axis), 4 * width + 16)
+        _close(got, q @ axis, np.abs(q) @ np.abs(axis), 4 * width + 16, width)
 
 
 @pytest.mark.parametrize("x_size,d_size,batch", [(100, 50, 16500), (256, 256, 4100), (300, 300, 12000)])
