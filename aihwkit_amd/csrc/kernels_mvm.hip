@@ -1586,7 +1586,7 @@ __global__ __launch_bounds__(256) void k_mvm_round(MvmArgs a) {
 // from L2 feeds 64 multiply-adds instead of 16.
 // On the fp32 matrix pipe, which set the pace before, a round of 16384 samples on a 1024 x 1024 tile took 316 us
 // (backward), the four linear layers of a 768-wide transformer block 69 + 34 + 80 + 69 us at 1024 tokens; with the split
-// operands 164 us and 49 + 30 + 54 + 50 us.  Error against 64-bit sums (relative): of 16 / 32 / 256 / 1024 terms 0.76 / 1.05
+// operands 153 us and 45 + 27 + 44 + 48 us.  Error against 64-bit sums (relative): of 16 / 32 / 256 / 1024 terms 0.76 / 1.05
 // / 2.9 / 5.7e-7 on the fp32 pipe, 0.65 / 0.79 / 1.6 / 3.1e-7 with quantized inputs, 0.29 / 0.35 / 0.80 / 1.7e-7 with any
 // other.  Same per-sample state, lists, epilogue and random streams as the 32 x 32 kernel: a round
 // may be run by either (the launcher picks by the number of samples in the round).
@@ -2589,7 +2589,8 @@ int mvm_big_workgroups(const MvmArgs &a, int bb) { return a.O >= 128 ? big_workg
 // the 1024 x 1024 tile: batch 8192 and 16384 (exactly one and two rounds) are 7 .. 12 % faster with 128, every other
 // batch between 2048 and 20480 with 64 (up to 35 % at 2048, 18 % at 10240).  Inputs in three parts (not `stepped`): 64
 // always; with 128 the staged planes take 80 KB, so a CU would hold one workgroup, four waves, and not two (1024 x 1024,
-// forward without noise: batch 8192 145 us against 140, 16384 278 against 270; backward the same within 1 us).
+// forward without noise, one sum per output: batch 8192 145 us against 140, 16384 278 against 270; backward the same
+// within 1 us), and the corrections' sums another 64 registers.
 int mvm_big_sample_tile(int workgroups_128, int n_cus, bool stepped) {
   if (!stepped) return 64;
   const int slots = 2 * n_cus;

@@ -1133,7 +1133,8 @@ __global__ __launch_bounds__(256, ((C > 1 || DEEP) ? 4 : 8)) void k_update_pulse
 // w + slope w + scale f has a term without a factor, selects by the factor's bits instead.  Passes, noise bytes and the
 // arithmetic of a step are those of PulsedRows: same weights.
 // 433 x 48 tile, 131 072 samples, 21 000 passes a row: 1973 -> 493 us (55 cycles a pass; draw and steps take 45 each on
-// their own, the seven waves of a workgroup share four SIMDs).
+// their own, the seven waves of a workgroup share four SIMDs).  Instructions per pass and 64 columns: 22, of which 18
+// vector ones, against 33 and 18 in the plain loop.
 template <int PARTS> struct PulseStream {
   float tbl[CTOC_LEVELS]; // first: its offset goes into the reads
   float4 fac[PARTS][3][16][64]; // [team][block modulo 3][four passes][column]
@@ -2002,8 +2003,10 @@ static int update_pulsed_columns(const UpdateArgs &a) {
 }
 
 // Whether the pulse loop of this call runs as a pipeline of waves (k_update_pulsed_stream): a batch that fills the
-// pipeline, on a tile with at most one wave of cross-points per SIMD (with more, the plain loop's waves overlap each
-// other and its fewer instructions per pass count: 25 against 40).  A CU has four SIMDs.
+// pipeline, on a tile with at most one wave of cross-points per SIMD (a CU has four).  Pulse loop of 433 columns and
+// 65536 samples, plain / pipeline: 16 rows 3016 / 624 us, 48 rows 3014 / 748, 96 rows 2954 / 1455, 144 rows 3105 / 2144.
+// Beyond that the plain loop's waves overlap each other: 256 rows 3051 / 2804; with 2048 samples 115 / 122, and the masks
+// take 9 us more to make than the planes.  (160 rows: 3095 / 2152 and 114 / 92; such tiles keep the plain loop.)
 bool update_takes_stream(const UpdateArgs &a) {
   return update_pulsed_columns(a) == 1 && a.n_chunks >= 32 && a.m_batch < (1 << 23) &&
          (long)((a.x_size + 63) / 64) * a.d_size <= 4L * current_device_cus();
