@@ -164,3 +164,25 @@ def test_a_range_that_is_nearly_a_multiple_of_the_step(gpu_device, terms):
     got = _tile(terms, 64, io, w).forward(torch.from_numpy(x).cuda())[::64].double().cpu().numpy()
     want, chain = x[::64] @ w.T.astype(np.float64), _chain(x[::64], w)
     assert np.sqrt(np.mean((got - want) ** 2)) <= 1.04 * np.sqrt(np.mean((chain - want) ** 2))
+
+
+@pytest.mark.parametrize("shapes,batch,perfect", [([(12, 160), (300, 256)], 4096, False),    # a tile of few terms among others
+                                                  ([(200, 512)] * 4, 4100, True),             # two rounds of square tiles' work
+                                                  ([(15, 128), (16, 131), (64, 300)], 8200, False)])
+def test_grouped_products_in_three_parts_against_64_bit_sums(gpu_device, shapes, batch, perfect):
+    rng = np.random.default_rng(len(shapes))
+    steps = 63
+    io = noise_free_io(inp_res=-1.0 if perfect else 1.0 / (2 * steps))
+    io.out_res, io.out_bound, io.is_perfect = -1.0, float("inf"), perfect
+    step = 2.0 * float(np.float32(1.0 / (2 * steps)))
+    weights = [rng.uniform(-0.6, 0.6, (d, x)).astype(np.float32) for x, d in shapes]
+    group = tiles.TileGroup([_tile(x, d, io, w) for (x, d), w in zip(shapes, weights)])
+    inputs = []
+    for x, _ in shapes:
+        v = (rng.integers(-steps, steps + 1, (batch, x)) * step).astype(np.float32)
+        v[:, 0] = 1.0  # meets the range
+        inputs.append(v)
+    for got, v, w in zip(group.forward([torch.from_numpy(v).cuda() for v in inputs]), inputs, weights):
+        q = v.astype(np.float64) if perfect else np.rint(v / step) * step
+        w64 = w.astype(np.float64)
+        _close(got, q @ w64.T, np.abs(q) @ np.abs(w64).T, 4 * w.shape[1] + 16, w.shape[1])
