@@ -312,7 +312,10 @@ struct UpdateArgs {
   uint32_t *d_planes;
   // 1: the x lines are kept as 64-bit lane masks instead (bit lines of up to seven pulses): bit l of word
   // ((row of words * ceil(x_size / 64) + block) * slots + k) is slot k of element 64 block + l, k = slots - 1 its sign
+  // 2: those masks in the order in which k_update_pulsed_masks reads them, x_mask_columns columns to a lane (spans of 64
+  // x_mask_columns elements, see pulse_mask_spans): [row of words][span][slot][sign of the d line][fires | steps down][column]
   int x_lane_masks;
+  int x_mask_columns;
   int n_chunks;    // ceil(m_batch / 32)
   int *row_cost;   // [d_size] work of the pulse loop on each d row of this call (zeroed by the prepare kernel, summed by
                    // the kernel that makes the d pulse trains); null: not kept
@@ -342,6 +345,8 @@ int update_pulsed_variant(const UpdateArgs &a);
 bool update_reads_row_cost(const UpdateArgs &a); // by its shape: whether the pulse loop of this call looks at row_cost
 int update_pulsed_workgroups(const UpdateArgs &a);
 bool update_takes_stream(const UpdateArgs &a); // by its shape: the call may set x_lane_masks (launch_update_lines, launch_update_pulsed)
+int update_mask_columns(const UpdateArgs &a);  // by its shape: the call may set x_lane_masks = 2 with these x_mask_columns; 0: not
+size_t update_mask_words(const UpdateArgs &a, int columns); // 64-bit words that such a call needs at x_planes
 void launch_update_pulsed_group(const UpdateGroup &g, int variant, int total_workgroups, hipStream_t s);
 
 // tables of the update kernels on the current device (once per GPU; blocking copy, no allocation)

@@ -259,6 +259,13 @@ __device__ __forceinline__ uint32_t pulse_word(const UpdateArgs &a, bool is_x, i
   return word;
 }
 
+// Lane masks of the x lines for k_update_pulsed_masks: a span is the 64 C columns of one of its waves -- four waves share
+// 256 C columns, and column c of a wave's lanes lies 256 c behind the first.
+__host__ __device__ __forceinline__ int pulse_mask_spans(int x_size, int columns) {
+  return 4 * ((x_size + 256 * columns - 1) / (256 * columns));
+}
+template <int C> __device__ __forceinline__ int pulse_mask_column(int span, int c) { return ((span >> 2) * C + c) * 256 + (span & 3) * 64; }
+
 // longest bit line of a batch whose packed words are not written: only the loop for longer ones reads them
 constexpr int UPDATE_PLANES_ONLY_KMAX = 7;
 
@@ -371,12 +378,10 @@ __device__ __forceinline__ void update_lines_block(const UpdateArgs &a, const in
 }
 
 // Row-major copy a.w of the [x_size][d_size] matrix a.wt_src for the pulse loop, 32 x 32 tiles through LDS: made by
-// workgroups that the launch of the pulse trains carries beyond its own (`first` .. of blockIdx.x), so that it costs no
-// launch of its own and runs beside that kernel's work.
-__device__ __forceinline__ void update_copy_weights(const UpdateArgs &a, int first, float (*tile)[33]) {
+// the `workers` workgroups that the launch of the pulse trains carries beyond its own, so that it costs no launch of its
+// own and runs beside that kernel's work (me: number of this one among them).
+__device__ __forceinline__ void update_copy_weights(const UpdateArgs &a, int me, int workers, float (*tile)[33]) {
   const int tiles_j = (a.x_size + 31) / 32, tiles_i = (a.d_size + 31) / 32;
-  const int workers = ((int)gridDim.x - first) * (int)gridDim.y;
-  const int me = ((int)blockIdx.x - first) * (int)gridDim.y + (int)blockIdx.y;
   const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5; // 8 rows of 32 per pass
   for (int t = me; t < tiles_j * tiles_i; t += workers) {
     const int j0 = (t / tiles_i) * 32, i0 = (t % tiles_i) * 32;
@@ -402,7 +407,7 @@ __global__ __launch_bounds__(256) void k_update_lines(UpdateArgs a) {
   const int own = (a.x_size + LINES_E - 1) / LINES_E + (a.d_size + LINES_E - 1) / LINES_E;
   if ((int)blockIdx.x >= own) { // only launched with a.wt_src set
     __shared__ float tile[32][33];
-    update_copy_weights(a, own, tile);
+    update_copy_weights(a, ((int)blockIdx.x - own) * (int)gridDim.y + (int)blockIdx.y, ((int)gridDim.x - own) * (int)gridDim.y, tile);
     return;
   }
   update_lines_block<LINES_E, IN_PLACE>(a, (int)blockIdx.x, (int)blockIdx.y, vals, wt);
@@ -419,7 +424,9 @@ __global__ __launch_bounds__(256) void k_update_lines_stream(UpdateArgs a) {
   const int blocks_x = (a.x_size + 63) / 64, blocks_d = (a.d_size + 15) / 16;
   const int bx = (int)blockIdx.x, by = (int)blockIdx.y;
   if (bx >= blocks_x + blocks_d) { // only launched with a.wt_src set
-    update_copy_weights(a, blocks_x + blocks_d, reinterpret_cast<float (*)[33]>(&vals[0][0]));
+    const int own = blocks_x + blocks_d;
+    update_copy_weights(a, (bx - own) * (int)gridDim.y + by, ((int)gridDim.x - own) * (int)gridDim.y,
+                        reinterpret_cast<float (*)[33]>(&vals[0][0]));
     return;
   }
   const int kmax = a.kmax[a.kmax_slot];
@@ -475,6 +482,102 @@ __global__ __launch_bounds__(256) void k_update_lines_stream(UpdateArgs a) {
       mine = lane == k ? m : mine;
     }
     if (lane <= kmax) reinterpret_cast<unsigned long long *>(a.x_planes)[((long)b * blocks_x + bx) * (kmax + 1) + lane] = mine;
+  }
+}
+
+// The pulse trains as k_update_pulsed_masks reads them (UpdateArgs::x_lane_masks = 2): for every row of words b, the 64 C
+// columns that a wave of that kernel owns and each slot k, once for either sign of the d line, C lane masks of the
+// columns that fire and C of those that step down, next to each other: all that a pass needs in one scalar load.  A wave
+// makes those of one row of words at a time; 16384 samples of 1024 + 1024 lines: 133 us, 148 as planes.  Workgroups in one dimension: the x lines (`rows_per_wave` rows of words to a wave),
+// the d lines (64 samples x 16 elements, bit planes), the copy of the weights.  Random numbers as in k_update_lines.
+template <int C>
+__global__ __launch_bounds__(256) void k_update_lines_masks(UpdateArgs a, int rows_per_wave) {
+  __shared__ float vals[64][17];
+  __shared__ uint32_t wt[64][17];
+  const int kmax = a.kmax[a.kmax_slot];
+  const int spans = pulse_mask_spans(a.x_size, C), sample_tiles = (a.m_batch + 63) / 64;
+  const int row_tiles = (a.m_batch + 4 * rows_per_wave - 1) / (4 * rows_per_wave);
+  const int n_x = spans * row_tiles, tiles_x = (a.x_size + 15) / 16, tiles_d = (a.d_size + 15) / 16, n_d = tiles_d * sample_tiles;
+  const int wg = (int)blockIdx.x;
+  if (wg >= n_x + n_d) { // only launched with a.wt_src set
+    update_copy_weights(a, wg - n_x - n_d, (int)gridDim.x - n_x - n_d, reinterpret_cast<float (*)[33]>(&vals[0][0]));
+    return;
+  }
+  if (wg >= n_x) {
+    update_lines_block<16, false>(a, tiles_x + (wg - n_x) % tiles_d, (wg - n_x) / tiles_d, vals, wt);
+    return;
+  }
+  if (kmax > UPDATE_PLANES_ONLY_KMAX) { // planes and words, as k_update_lines leaves them
+    for (int q = wg; q < tiles_x * sample_tiles; q += n_x) {
+      update_lines_block<16, false>(a, q % tiles_x, q / tiles_x, vals, wt);
+      __syncthreads();
+    }
+    return;
+  }
+  const int lane = (int)threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int span = wg % spans, b0 = ((wg / spans) * 4 + wave) * rows_per_wave;
+  const int b1 = min(b0 + rows_per_wave, a.m_batch);
+  if (b0 >= b1) return;
+  const int wps = max(a.words_per_sample, 1);
+  // lane l < 4 kmax: slot l / 4, sign of the d line (l / 2) & 1, columns that fire (even) or step down (odd)
+  const int my_slot = lane >> 2;
+  const bool my_dir = lane & 1, my_turn = (lane >> 1) & 1;
+  unsigned long long *out = reinterpret_cast<unsigned long long *>(a.x_planes) + (long)span * kmax * 4 * C + (lane >> 1) * 2 * C + (lane & 1) * C;
+  int e[C];
+  const float *x[C];
+  PhiloxFirst first[C];
+  float v[C];
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    e[c] = pulse_mask_column<C>(span, c) + lane;
+    x[c] = a.x + (long)min(e[c], a.x_size - 1) * a.x_sj; // elements behind the end of the line never fire
+    v[c] = x[c][(long)(wps > 1 ? b0 / wps : b0) * a.x_sb];
+    first[c] = philox_first((uint32_t)e[c], a.call, RNG_PULSE_X, a.key);
+  }
+  for (int b = b0; b < b1; ++b) {
+    const int sample = wps > 1 ? b / wps : b, wrow = wps > 1 ? b - sample * wps : 0;
+    const int K = min(max(a.bl[sample] - 31 * wrow, 0), 31);
+    const float P = a.prob_b[sample];
+    const PhiloxSecond second = philox_second((uint32_t)sample, a.call, a.key);
+    float now[C];
+#pragma unroll
+    for (int c = 0; c < C; ++c) now[c] = v[c];
+    if (b + 1 < b1) { // on their way while this row is worked out
+      const int next = wps > 1 ? (b + 1) / wps : b + 1;
+#pragma unroll
+      for (int c = 0; c < C; ++c) v[c] = x[c][(long)next * a.x_sb];
+    }
+    unsigned long long mine[C];
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      const bool ok = e[c] < a.x_size;
+      if (K <= 4 && wrow == 0 && a.up.res <= 0.0f) { // pulse_word, slot by slot
+        const float PP = ok ? fabsf(now[c]) * P : 0.0f, most = PP * 16777216.0f;
+        const unsigned long long sg = K > 0 ? __ballot(PP != 0.0f && !(now[c] > 0.0f)) : 0ull;
+        mine[c] = my_turn ? ~sg : sg;
+        const Philox4 r = philox_finish(first[c], second, a.key, K > 2);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          if (k >= kmax) break;
+          const unsigned long long m = k < K ? __ballot(most > (float)(r.v[k] >> 8)) : 0ull;
+          mine[c] = (!my_dir && my_slot == k) ? m : mine[c];
+        }
+        for (int k = 4; k < kmax; ++k) mine[c] = (!my_dir && my_slot == k) ? 0ull : mine[c];
+      } else {
+        const uint32_t word = ok ? pulse_word(a, true, e[c], sample, now[c], P, K, wrow) : 0u;
+        const unsigned long long sg = __ballot(word & 1u);
+        mine[c] = my_turn ? ~sg : sg;
+        for (int k = 0; k < kmax; ++k) {
+          const unsigned long long m = __ballot((word >> (k + 1)) & 1u);
+          mine[c] = (!my_dir && my_slot == k) ? m : mine[c];
+        }
+      }
+    }
+    if (lane < 4 * kmax) {
+      unsigned long long *o = out + (long)b * spans * kmax * 4 * C;
+#pragma unroll
+      for (int c = 0; c < C; ++c) o[c] = mine[c];
+    }
   }
 }
 
@@ -682,6 +785,15 @@ __global__ __launch_bounds__(256) void k_words_from_planes(UpdateArgs a) {
     const int b = (int)(idx / per), el = (int)(idx % per);
     const bool is_x = el < a.x_size;
     const int e = is_x ? el : el - a.x_size, size = is_x ? a.x_size : a.d_size;
+    if (is_x && a.x_lane_masks == 2) {
+      const int cols = a.x_mask_columns, spans = pulse_mask_spans(a.x_size, cols);
+      const int span = (e / (256 * cols)) * 4 + ((e >> 6) & 3), c = (e >> 8) % cols;
+      const unsigned long long *m = reinterpret_cast<const unsigned long long *>(a.x_planes) + ((long)b * spans + span) * kmax * 4 * cols + c;
+      uint32_t word = kmax > 0 ? (uint32_t)(m[cols] >> (e & 63)) & 1u : 0u;
+      for (int k = 0; k < kmax; ++k) word |= ((uint32_t)(m[(long)k * 4 * cols] >> (e & 63)) & 1u) << (k + 1);
+      a.x_words[(long)b * size + e] = word;
+      continue;
+    }
     if (is_x && a.x_lane_masks) {
       const unsigned long long *m = reinterpret_cast<const unsigned long long *>(a.x_planes) +
                                     ((long)b * ((a.x_size + 63) / 64) + (e >> 6)) * slots;
@@ -1418,21 +1530,18 @@ __global__ __launch_bounds__(64 * (1 + 3 * PARTS)) void k_update_pulsed_stream(U
   }
 }
 
-// The same pulse loop with the rows dealt out by their work.  The time a row takes follows its number of d pulses, which
+// Rows dealt out by their work.  The time a row takes follows its number of d pulses, which
 // varies by several percent between rows, and a CU holds four rows at a time: whichever CU draws four long ones sets
 // the kernel's time.  Here a workgroup of 1024 threads fills a CU and takes four rows, one per 256 threads, chosen so
 // that every workgroup has the same work: workgroup n (on XCD n % 8) belongs to the band of d_size / 8 consecutive rows
 // of its XCD, ranks the band's rows by a.row_cost (ties by row number: every workgroup of the band finds the same
 // order) and takes, as number s of the band's S = d_size / 32 workgroups, the ranks s, 2 S - 1 - s, 2 S + s and
 // 4 S - 1 - s.  Rows of a band in one L2 also keep the strided stores of UpdateArgs::w_out together.
-// For four columns per lane, rows of at most 1024 columns, d_size a multiple of 256 (bands of whole groups of 32 rows).  Which row a group of threads works
-// on changes nothing in the result of the row.
+// For four columns per lane, rows of at most 1024 columns, d_size a multiple of 256 (bands of whole groups of 32 rows).
+// Which row a group of threads works on changes nothing in the result of the row.
 constexpr int BALANCED_MAX_BAND = 1024;
-template <int KIND, bool MULT, bool NOISE>
-__global__ __launch_bounds__(1024) void k_update_pulsed_balanced(UpdateArgs a) {
-  __shared__ float tbl[CTOC_LEVELS];
-  __shared__ int cost[BALANCED_MAX_BAND];
-  __shared__ int order[BALANCED_MAX_BAND];
+// the row of this thread, the same for the 256 threads that share it; cost, order: BALANCED_MAX_BAND words in LDS each
+__device__ __forceinline__ int balanced_row(const UpdateArgs &a, int *cost, int *order) {
   const int band = a.d_size >> 3, per_band = band >> 2;
   const int xcd = (int)blockIdx.x & 7, s = (int)blockIdx.x >> 3;
   const int row0 = xcd * band;
@@ -1469,9 +1578,301 @@ __global__ __launch_bounds__(1024) void k_update_pulsed_balanced(UpdateArgs a) {
   __syncthreads();
   const int g = (int)threadIdx.x >> 8;
   const int rank = (g & 1) ? (g + 1) * per_band - 1 - s : g * per_band + s;
-  // the same for the 256 threads of a row: kept in a scalar register, like a row number taken from the grid
-  const int row = __builtin_amdgcn_readfirstlane(row0 + order[rank]);
+  // kept in a scalar register, like a row number taken from the grid
+  return __builtin_amdgcn_readfirstlane(row0 + order[rank]);
+}
+
+// the plain pulse loop with the rows dealt out by their work
+template <int KIND, bool MULT, bool NOISE>
+__global__ __launch_bounds__(1024) void k_update_pulsed_balanced(UpdateArgs a) {
+  __shared__ float tbl[CTOC_LEVELS];
+  __shared__ int cost[BALANCED_MAX_BAND];
+  __shared__ int order[BALANCED_MAX_BAND];
+  const int row = balanced_row(a, cost, order);
   update_pulsed_row<KIND, MULT, NOISE, 4, false>(a, 0, row, tbl, (int)threadIdx.x & 255);
+}
+
+// ---- the pulse loop on lane masks -----------------------------------------------------------------------------------
+// Tiles whose waves fill the SIMDs are bound by the issue of vector instructions, so here a pass has as few of them as
+// it can.  Which lanes fire and which step down are 64-bit masks of the C columns of a wave (k_update_lines_masks), one
+// scalar load for a pass, and go into EXEC: a step is a multiply-add with the upward parameters by all lanes, the same
+// with the downward ones by those that go down, then multiply-add and clip by those that fire -- four vector
+// instructions per column.  The passes of 64 samples are listed ahead in LDS by the wave itself, as offsets of their
+// masks; one v_readlane gives the offset of a pass, its masks and noise factors are fetched a pass ahead.  The factors
+// 1 + std * quantile stand in LDS once for every lane of a wave, so that a read meets no other lane's bank (random
+// reads of one copy cost 6.3 cycles of the LDS pipe each, these two) and byte q of the generator's output becomes an
+// address by a single v_perm_b32.  Passes, noise bytes and the arithmetic of a step are those of PulsedRows: same weights.
+// 1024 x 1024, four columns per lane: 28.4 vector instructions per pass against 46.5, of which 16 are the steps, 10 the
+// factors; they now fill all of the issue slots.  Pulse loop of 16384 samples 2371 -> 1424 us, of 256 samples 51.5 -> 36.4.
+// (One pass at a time instead of two: 1684 us, the scalar loads then arrive late.)
+template <bool NOISE> struct PulseMasks {
+  float tbl[NOISE ? CTOC_LEVELS : 1][64];
+  uint32_t list[16][256]; // per wave: offsets of the masks of the passes of 64 samples (32 where kmax > 3)
+};
+
+template <int C> struct PassMasks;
+typedef uint32_t mask_words16 __attribute__((ext_vector_type(16)));
+typedef uint32_t mask_words8 __attribute__((ext_vector_type(8)));
+template <> struct PassMasks<4> { typedef mask_words16 type; };
+template <> struct PassMasks<2> { typedef mask_words8 type; };
+
+template <int KIND, bool MULT, int NK, bool NOISE, int C> struct MaskedRows {
+  typedef typename PassMasks<C>::type Masks;
+  static constexpr unsigned SAMPLES = NK <= 3 ? 64 : 32; // listed at a time: at most 64 * 3 or 32 * 7 passes
+  static constexpr unsigned LIST = 256;                  // entries of `list`
+  const UpdateArgs &a;
+  float (&w)[C];
+  const PulseCell<KIND> (&cp)[C];
+  const char *tbl;
+  uint32_t *list;
+  const int lane;
+  const uint32_t lane4;
+  uint32_t s0 = 1u, s1 = 0u;
+
+  __device__ __forceinline__ MaskedRows(const UpdateArgs &a_, float (&w_)[C], const PulseCell<KIND> (&cp_)[C], const char *tbl_,
+                                        uint32_t *list_, int lane_)
+      : a(a_), w(w_), cp(cp_), tbl(tbl_), list(list_), lane(lane_), lane4((uint32_t)lane_ << 2) {}
+
+  // the factors of the next pass, as PulsedRows::draw
+  __device__ __forceinline__ void draw(float (&f)[C]) {
+    if (!NOISE) return;
+    const uint32_t r = s0 + s1;
+    s1 ^= s0;
+    s0 = __builtin_amdgcn_bitop3_b32(__builtin_rotateleft32(s0, 26), s1, s1 << 9, 0x96);
+    s1 = __builtin_rotateleft32(s1, 13);
+#pragma unroll
+    for (int c = 0; c < C; ++c) // byte c of r over the lane's offset: 256 bytes to a table entry
+      f[c] = *reinterpret_cast<const float *>(tbl + __builtin_amdgcn_perm(r, lane4, 0x0c0c0000u | ((4u + (unsigned)c) << 8)));
+  }
+
+  static __device__ __forceinline__ unsigned long long mask_of(const Masks &m, int word) {
+    return ((unsigned long long)m[2 * word + 1] << 32) | m[2 * word];
+  }
+
+  // The masks and factors have arrived; whatever is loaded next is not waited for here.
+  static __device__ __forceinline__ void arrived(Masks &m, float (&f)[C]) {
+    asm volatile("" : "+s"(m));
+    if (NOISE) {
+#pragma unroll
+      for (int c = 0; c < C; ++c) asm volatile("" : "+v"(f[c]));
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+
+  // One pass.  EXEC is all ones here (whole waves, uniform control flow) and is so again afterwards.
+  __device__ __forceinline__ void step(const Masks &m, const float (&f)[C]) {
+    float t[C];
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      if (KIND == RPU_DEVICE_CONSTANT_STEP) t[c] = __builtin_amdgcn_inverse_ballot_w64(mask_of(m, C + c)) ? cp[c].scale_dn : cp[c].scale_up;
+      else t[c] = __builtin_fmaf(cp[c].slope_up, w[c], MULT ? cp[c].scale_up : w[c]);
+    }
+// column n: t with the downward parameters; then the step w + t f (constant steps, multiplicative noise) or t + scale f
+#define RPU_DOWN(n) "s_mov_b64 exec, %[g" #n "]\n\tv_fma_f32 %[t" #n "], %[s" #n "], %[w" #n "], %[c" #n "]\n\t"
+#define RPU_FIRE(n) "s_mov_b64 exec, %[m" #n "]\n\tv_fma_f32 %[w" #n "], %[t" #n "], %[f" #n "], %[w" #n "]\n\tv_med3_f32 %[w" #n "], %[w" #n "], %[l" #n "], %[h" #n "]\n\t"
+#define RPU_FIRE_ADD(n) "s_mov_b64 exec, %[m" #n "]\n\tv_fma_f32 %[w" #n "], %[c" #n "], %[f" #n "], %[t" #n "]\n\tv_med3_f32 %[w" #n "], %[w" #n "], %[l" #n "], %[h" #n "]\n\t"
+#define RPU_ALL "s_mov_b64 exec, -1"
+#define RPU_OUT(n) [t##n] "+&v"(t[n]), [w##n] "+&v"(w[n])
+#define RPU_IN(n) [f##n] "v"(NOISE ? f[n] : 1.0f), [l##n] "v"(cp[n].lo), [h##n] "v"(cp[n].hi), [m##n] "s"(mask_of(m, n))
+#define RPU_IN_DN(n) RPU_IN(n), [s##n] "v"(cp[n].slope_dn), [c##n] "v"(cp[n].scale_dn), [g##n] "s"(mask_of(m, C + n))
+#define RPU_IN_ADD(n) RPU_IN(n), [s##n] "v"(cp[n].slope_dn), [c##n] "v"(scale[n]), [g##n] "s"(mask_of(m, C + n))
+#define RPU_DOWN_ADD(n) "s_mov_b64 exec, %[g" #n "]\n\tv_fma_f32 %[t" #n "], %[s" #n "], %[w" #n "], %[w" #n "]\n\t"
+#define RPU_STEP(DO4, DO2, IN)                                                                                          \
+  if constexpr (C == 4) asm volatile(DO4 RPU_ALL : RPU_OUT(0), RPU_OUT(1), RPU_OUT(2), RPU_OUT(3) : IN(0), IN(1), IN(2), IN(3)); \
+  else asm volatile(DO2 RPU_ALL : RPU_OUT(0), RPU_OUT(1) : IN(0), IN(1))
+    if constexpr (KIND == RPU_DEVICE_CONSTANT_STEP) {
+      RPU_STEP(RPU_FIRE(0) RPU_FIRE(1) RPU_FIRE(2) RPU_FIRE(3), RPU_FIRE(0) RPU_FIRE(1), RPU_IN);
+    } else if constexpr (MULT) {
+      RPU_STEP(RPU_DOWN(0) RPU_DOWN(1) RPU_DOWN(2) RPU_DOWN(3) RPU_FIRE(0) RPU_FIRE(1) RPU_FIRE(2) RPU_FIRE(3),
+               RPU_DOWN(0) RPU_DOWN(1) RPU_FIRE(0) RPU_FIRE(1), RPU_IN_DN);
+    } else {
+      float scale[C];
+#pragma unroll
+      for (int c = 0; c < C; ++c) scale[c] = __builtin_amdgcn_inverse_ballot_w64(mask_of(m, C + c)) ? cp[c].scale_dn : cp[c].scale_up;
+      RPU_STEP(RPU_DOWN_ADD(0) RPU_DOWN_ADD(1) RPU_DOWN_ADD(2) RPU_DOWN_ADD(3) RPU_FIRE_ADD(0) RPU_FIRE_ADD(1) RPU_FIRE_ADD(2) RPU_FIRE_ADD(3),
+               RPU_DOWN_ADD(0) RPU_DOWN_ADD(1) RPU_FIRE_ADD(0) RPU_FIRE_ADD(1), RPU_IN_ADD);
+    }
+#undef RPU_DOWN
+#undef RPU_DOWN_ADD
+#undef RPU_FIRE
+#undef RPU_FIRE_ADD
+#undef RPU_ALL
+#undef RPU_OUT
+#undef RPU_IN
+#undef RPU_IN_DN
+#undef RPU_IN_ADD
+#undef RPU_STEP
+  }
+
+  __device__ __forceinline__ void run(const unsigned cell, const int i, const int span, const int spans, const int kmax) {
+    typedef const __attribute__((address_space(4))) char *Bytes;
+    const unsigned pair = 2u * C * 8u;                       // bytes of a pass: the masks of the columns that fire, and go down
+    const unsigned row_bytes = (unsigned)(spans * kmax) * 2u * pair;
+    const Bytes masks = (Bytes)(uintptr_t)a.x_planes + (size_t)(span * kmax) * 2u * pair;
+    const unsigned ds = (unsigned)a.d_size, slots = (unsigned)kmax + 1u, n_chunks = (unsigned)a.n_chunks;
+    const uint32_t lr_mask = a.lr < 0.0f ? 0xffffffffu : 0u;
+    if (NOISE) {
+      const Philox4 r = philox4x32_10(cell, 0u, a.call, RNG_CTOC, a.key.k0, a.key.k1);
+      s0 = r.v[0] | 1u; // as PulsedRows::run
+      s1 = r.v[1];
+    }
+    // the d line's planes of a list's samples: lane (slot, chunk of the list)
+    constexpr unsigned CHUNKS = SAMPLES / 32;
+    auto load_d = [&](unsigned chunk) {
+      const unsigned ch = chunk + (unsigned)lane % CHUNKS, slot = (unsigned)lane / CHUNKS;
+      return (slot < slots && ch < n_chunks) ? a.d_planes[(size_t)(ch * slots + slot) * ds + (unsigned)i] : 0u;
+    };
+    auto d_bits = [&](uint32_t v, int slot) -> unsigned long long {
+      const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)v, slot * (int)CHUNKS);
+      const uint32_t hi = CHUNKS > 1 ? (uint32_t)__builtin_amdgcn_readlane((int)v, slot * (int)CHUNKS + 1) : 0u;
+      return ((unsigned long long)hi << 32) | lo;
+    };
+    // Two passes at a time: their masks and factors are fetched while the two before them are worked on, so that a fetch has
+    // two passes to arrive in.  The list goes on behind passes of the samples before that were too few for four.
+    float f0[C], f1[C], g0[C], g1[C];
+    draw(f0);
+    draw(f1);
+    auto fetch = [&](uint32_t e, int p) { return *(const __attribute__((address_space(4))) Masks *)(masks + (unsigned)__builtin_amdgcn_readlane((int)e, p)); };
+    uint32_t d_now = load_d(0u);
+    unsigned chunk = 0u, listed = 0u;
+    while (chunk < n_chunks) {
+      // the passes of the next samples, until there are enough to be worth a walk
+      do {
+        const uint32_t dv = d_now;
+        d_now = load_d(chunk + CHUNKS);
+        unsigned pos = listed, passes = 0u;
+        unsigned long long fire[NK];
+#pragma unroll
+        for (int k = 0; k < NK; ++k) {
+          fire[k] = k < kmax ? d_bits(dv, k) : 0ull;
+          pos = __builtin_amdgcn_mbcnt_hi((uint32_t)(fire[k] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)fire[k], pos));
+          passes += (unsigned)__popcll(fire[k]);
+        }
+        if (passes != 0u) {
+          // a sample whose d line is positive (lr > 0) steps down where x has the same sign
+          const unsigned long long turn = ~d_bits(dv, kmax) ^ (((unsigned long long)lr_mask << 32) | lr_mask);
+          const unsigned off = (32u * chunk + (unsigned)lane) * row_bytes + (__builtin_amdgcn_inverse_ballot_w64(turn) ? pair : 0u);
+#pragma unroll
+          for (int k = 0; k < NK; ++k) {
+            if (__builtin_amdgcn_inverse_ballot_w64(fire[k])) {
+              list[pos] = off + (unsigned)k * 2u * pair;
+              ++pos;
+            }
+          }
+          listed += passes;
+        }
+        chunk += CHUNKS;
+      } while (chunk < n_chunks && listed + SAMPLES * NK <= LIST);
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      const unsigned walked = listed & ~3u;
+      if (walked) {
+        const uint32_t head = list[lane & 3];
+        Masks a0 = fetch(head, 0), a1 = fetch(head, 1);
+        for (unsigned p0 = 0; p0 < walked; p0 += 64u) {
+          const int n = (int)min(64u, walked - p0);
+          const uint32_t e = list[min(p0 + 2u + (unsigned)lane, listed - 1u)]; // of the pass two further on
+          for (int p = 0; p < n; p += 4) {
+            arrived(a0, f0);
+            arrived(a1, f1);
+            Masks b0 = fetch(e, p), b1 = fetch(e, p + 1);
+            draw(g0);
+            draw(g1);
+            __builtin_amdgcn_sched_barrier(0);
+            step(a0, f0);
+            step(a1, f1);
+            arrived(b0, g0);
+            arrived(b1, g1);
+            a0 = fetch(e, p + 2); // behind the last pass: any entry
+            a1 = fetch(e, p + 3);
+            draw(f0);
+            draw(f1);
+            __builtin_amdgcn_sched_barrier(0);
+            step(b0, g0);
+            step(b1, g1);
+          }
+        }
+        // what is left moves to the front
+        const uint32_t rest = list[min(walked + (unsigned)lane, (unsigned)LIST - 1u)];
+        __builtin_amdgcn_wave_barrier();
+        listed -= walked;
+        if ((unsigned)lane < listed) list[lane] = rest;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+      }
+    }
+    const uint32_t last = list[lane & 3];
+    for (unsigned p = 0; p < listed; ++p) { // at most three
+      Masks m = fetch(last, (int)p);
+      arrived(m, f0);
+      step(m, f0);
+#pragma unroll
+      for (int c = 0; c < C; ++c) f0[c] = f1[c];
+      draw(f1);
+    }
+  }
+};
+
+// A workgroup of 256 R threads takes R units, a unit being 256 C columns of one d row, four waves.  dealt: four rows to a
+// workgroup by their work (balanced_row).
+template <int KIND, bool MULT, bool NOISE, int C>
+__global__ __launch_bounds__(1024) void k_update_pulsed_masks(UpdateArgs a, int dealt) {
+  __shared__ __attribute__((aligned(16))) PulseMasks<NOISE> sh;
+  const int tid = (int)threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int kmax = a.kmax[a.kmax_slot];
+  if (NOISE && kmax <= UPDATE_PLANES_ONLY_KMAX) {
+    for (int t = tid; t < CTOC_LEVELS * 16; t += (int)blockDim.x) {
+      const float f = __builtin_fmaf(a.dev.dw_min_std, g_ctoc_xi[t >> 4], 1.0f);
+      reinterpret_cast<float4 *>(&sh.tbl[0][0])[t] = make_float4(f, f, f, f);
+    }
+    __syncthreads();
+  }
+  const int groups = (a.x_size + 256 * C - 1) / (256 * C), per_wg = (int)blockDim.x >> 8;
+  int i, g = 0;
+  if (C == 4 && dealt) {
+    static_assert(sizeof(sh.list) >= 2 * BALANCED_MAX_BAND * sizeof(int), "the ranking goes where the lists will be");
+    int *cost = reinterpret_cast<int *>(&sh.list[0][0]);
+    i = balanced_row(a, cost, cost + BALANCED_MAX_BAND);
+    __syncthreads();
+  } else {
+    int wg = (int)blockIdx.x;
+    // stores along a column of a matrix whose rows run the other way: consecutive rows on one XCD (see k_update_pulsed)
+    if (a.w_out && (gridDim.x & 7u) == 0u) wg = (wg & 7) * ((int)gridDim.x >> 3) + (wg >> 3);
+    const int unit = wg * per_wg + (wave >> 2);
+    if (unit >= groups * a.d_size) return;
+    i = unit / groups;
+    g = unit % groups;
+  }
+  const int span = 4 * g + (wave & 3);
+  int j[C];
+  bool valid[C];
+  unsigned cell[C];
+  PulseCell<KIND> cp[C];
+  float w[C];
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    const int jt = pulse_mask_column<C>(span, c) + lane;
+    valid[c] = jt < a.x_size;
+    j[c] = valid[c] ? jt : a.x_size - 1;
+    cell[c] = (unsigned)i * (unsigned)a.x_size + (unsigned)j[c];
+    cp[c].load(a.dev, cell[c]);
+    w[c] = a.w[cell[c]];
+  }
+  const char *tbl = reinterpret_cast<const char *>(&sh.tbl[0][0]);
+  if (kmax <= 3) {
+    MaskedRows<KIND, MULT, 3, NOISE, C>(a, w, cp, tbl, sh.list[wave], lane).run(cell[0], i, span, 4 * groups, kmax);
+  } else if (kmax <= UPDATE_PLANES_ONLY_KMAX) {
+    MaskedRows<KIND, MULT, 7, NOISE, C>(a, w, cp, tbl, sh.list[wave], lane).run(cell[0], i, span, 4 * groups, kmax);
+  } else {
+#pragma unroll
+    for (int c = 0; c < C; ++c) w[c] = pulsed_gather<KIND, MULT>(a, w[c], cp[c], cell[c], i, j[c], valid[c], kmax);
+  }
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    if (!valid[c]) continue;
+    if (a.w_out) a.w_out[(long)i * a.wo_si + (long)j[c] * a.wo_sj] = w[c]; // see UpdateArgs::w_out
+    else a.w[cell[c]] = w[c];
+  }
 }
 
 // Several tiles in one launch (same device kind, noise and columns per lane): start[t] .. start[t + 1] are the
@@ -1904,6 +2305,18 @@ void launch_update_lines(const UpdateArgs &a, hipStream_t s) {
     extra = (extra + sample_tiles - 1) / sample_tiles;
   }
   const bool in_place = a.x_index || a.d_group;
+  if (a.x_lane_masks == 2) {
+    // rows of words per wave: more of them share what a column's generator keeps, as long as sixteen waves are left to a CU
+    // (16384 x 1024, 1 / 2 / 8 rows: 156 / 142 / 133 us)
+    const unsigned spans = (unsigned)pulse_mask_spans(a.x_size, a.x_mask_columns);
+    const long waves = (long)spans * a.m_batch;
+    const int per_wave = (int)std::max(1L, std::min(8L, waves / (16L * current_device_cus())));
+    const unsigned row_tiles = (unsigned)((a.m_batch + 4 * per_wave - 1) / (4 * per_wave));
+    const dim3 grid(spans * row_tiles + (unsigned)((a.d_size + 15) / 16) * sample_tiles + extra * sample_tiles);
+    if (a.x_mask_columns == 4) hipLaunchKernelGGL(k_update_lines_masks<4>, grid, dim3(256), 0, s, a, per_wave);
+    else hipLaunchKernelGGL(k_update_lines_masks<2>, grid, dim3(256), 0, s, a, per_wave);
+    return;
+  }
   if (a.x_lane_masks) {
     const dim3 grid((a.x_size + 63) / 64 + (a.d_size + 15) / 16 + extra, sample_tiles);
     if (in_place) hipLaunchKernelGGL(k_update_lines_stream<true>, grid, dim3(256), 0, s, a);
@@ -2011,6 +2424,40 @@ bool update_takes_stream(const UpdateArgs &a) {
   return update_pulsed_columns(a) == 1 && a.n_chunks >= 32 && a.m_batch < (1 << 23) &&
          (long)((a.x_size + 63) / 64) * a.d_size <= 4L * current_device_cus();
 }
+// Columns per lane of the pulse loop on lane masks (k_update_pulsed_masks), 0: not for this call.  Its launches cost about
+// 4 us more than those on bit planes (a table of 64 KB, masks instead of planes), which a pass has to earn back, and a wave
+// on its own takes as long for a pass as before: it wants batch and units (256 columns per lane of a row) together.
+// Pulse trains and pulse loop of a call, planes / masks, us, soft bounds: 1024 x 1024 64 samples 30.2 / 29.0, 256 63 / 48,
+// 4096 648 / 396; 700 x 700 128 34 / 32, 1024 152 / 110; 512 x 512 128 24.9 / 25.1, 256 36.9 / 33.3; 512 x 256 256 33.4 /
+// 33.7; without noise 1024 x 1024 256 45 / 37, 700 x 700 128 27.0 / 26.6, 512 x 256 4096 228 / 240.
+int update_mask_columns(const UpdateArgs &a) {
+  const int cols = update_pulsed_columns(a);
+  const long spans = pulse_mask_spans(a.x_size, cols), units = spans / 4 * a.d_size, cus = current_device_cus();
+  // (bit lines beyond seven pulses are walked as before, from planes and words: no use for lines that are all longer)
+  if (cols == 1 || a.x_index || a.d_group || !(a.up.update_bl_management || a.up.desired_bl <= UPDATE_PLANES_ONLY_KMAX) || 64L * cols * spans * a.m_batch > (1L << 30)) return 0; // offsets of masks in 32 bits
+  return a.m_batch >= 128 && units * a.m_batch >= 512 * cus && units > (a.dev.dw_min_std > 0.0f ? cus : 2 * cus - 1) ? cols : 0;
+}
+// 64-bit words of the masks of a call whose longest bit line has seven pulses
+size_t update_mask_words(const UpdateArgs &a, int columns) {
+  return (size_t)a.m_batch * (size_t)pulse_mask_spans(a.x_size, columns) * UPDATE_PLANES_ONLY_KMAX * 4u * (size_t)columns;
+}
+template <bool NOISE, int C> static void launch_update_pulsed_masks(const UpdateArgs &a, hipStream_t s) {
+  const long units = (long)((a.x_size + 256 * C - 1) / (256 * C)) * a.d_size;
+  // Units of a workgroup.  With noise its table lets two workgroups share a CU: one or two of equal size hold the units of
+  // a CU.  Without one there is nothing to share.
+  const long per_cu = (units + current_device_cus() - 1) / current_device_cus();
+  const long per_wg = !NOISE ? 1 : per_cu <= 4 ? per_cu : std::min(4L, (per_cu + 1) / 2);
+  const int dealt = update_pulsed_balanced(a, C) ? 1 : 0;
+  const long rows = dealt ? 4 : per_wg;
+  const dim3 grid((unsigned)((units + rows - 1) / rows)), block((unsigned)(256 * rows));
+  if (a.dev.kind == RPU_DEVICE_CONSTANT_STEP) {
+    hipLaunchKernelGGL((k_update_pulsed_masks<RPU_DEVICE_CONSTANT_STEP, true, NOISE, C>), grid, block, 0, s, a, dealt);
+  } else if (a.dev.ls_mult_noise) {
+    hipLaunchKernelGGL((k_update_pulsed_masks<RPU_DEVICE_LINEAR_STEP, true, NOISE, C>), grid, block, 0, s, a, dealt);
+  } else {
+    hipLaunchKernelGGL((k_update_pulsed_masks<RPU_DEVICE_LINEAR_STEP, false, NOISE, C>), grid, block, 0, s, a, dealt);
+  }
+}
 template <bool NOISE, int PARTS> static void launch_update_pulsed_stream(const UpdateArgs &a, hipStream_t s) {
   const dim3 grid(((a.x_size + 63) / 64 + PARTS - 1) / PARTS, a.d_size), block(64 * (1 + 3 * PARTS));
   if (a.dev.kind == RPU_DEVICE_CONSTANT_STEP) {
@@ -2024,6 +2471,16 @@ template <bool NOISE, int PARTS> static void launch_update_pulsed_stream(const U
 
 void launch_update_pulsed(const UpdateArgs &a, hipStream_t s) {
   const int cols = update_pulsed_columns(a);
+  if (a.x_lane_masks == 2) {
+    if (a.dev.dw_min_std > 0.0f) {
+      if (cols == 4) launch_update_pulsed_masks<true, 4>(a, s);
+      else launch_update_pulsed_masks<true, 2>(a, s);
+    } else {
+      if (cols == 4) launch_update_pulsed_masks<false, 4>(a, s);
+      else launch_update_pulsed_masks<false, 2>(a, s);
+    }
+    return;
+  }
   if (a.x_lane_masks) {
     // two teams to a workgroup where single ones would be more than the CUs: seven waves on a CU's four SIMDs, evenly
     // over the chip, instead of two workgroups on some CUs and one on the others

@@ -56,6 +56,61 @@ RPU_HD Philox4 philox4x32_10(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3,
   return out;
 }
 
+// The same function of a counter whose words 2 and 3 are the same for many calls, in parts that can be kept between
+// calls: what word 0 alone decides in the first three rounds (three of their six products), what word 1 alone does (one),
+// and the rest.  philox4x32_10(c0, c1, c2, c3) == philox_finish(philox_first(c0, c2, c3), philox_second(c1, c2)).
+struct PhiloxFirst {
+  uint32_t lo, m1, hi, q3;
+};
+struct PhiloxSecond {
+  uint32_t m2, m3;
+};
+constexpr uint32_t PHILOX_M0 = 0xD2511F53u, PHILOX_M1 = 0xCD9E8D57u, PHILOX_W0 = 0x9E3779B9u, PHILOX_W1 = 0xBB67AE85u;
+RPU_HD uint32_t philox_xor3(uint32_t a, uint32_t b, uint32_t c) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_amdgcn_bitop3_b32(a, b, c, 0x96);
+#else
+  return a ^ b ^ c;
+#endif
+}
+RPU_HD PhiloxFirst philox_first(uint32_t c0, uint32_t c2, uint32_t c3, PhiloxKey key) {
+  const uint64_t p0 = (uint64_t)PHILOX_M0 * c0;
+  const uint64_t p1 = (uint64_t)PHILOX_M1 * philox_xor3((uint32_t)(p0 >> 32), c3, key.k1);
+  const uint64_t p2 = (uint64_t)PHILOX_M0 * philox_xor3((uint32_t)(p1 >> 32), PHILOX_M1 * c2, key.k0 + PHILOX_W0);
+  return {(uint32_t)p0, (uint32_t)p1 ^ (key.k0 + 2u * PHILOX_W0), (uint32_t)(p2 >> 32), (uint32_t)p2};
+}
+RPU_HD PhiloxSecond philox_second(uint32_t c1, uint32_t c2, PhiloxKey key) {
+  const uint64_t p = (uint64_t)PHILOX_M0 * philox_xor3((uint32_t)(((uint64_t)PHILOX_M1 * c2) >> 32), c1, key.k0);
+  return {(uint32_t)(p >> 32) ^ (key.k1 + PHILOX_W1), (uint32_t)p ^ (key.k1 + 2u * PHILOX_W1)};
+}
+// words 0 and 1, and with `all` words 2 and 3 (a product more)
+RPU_HD Philox4 philox_finish(const PhiloxFirst &f, const PhiloxSecond &s, PhiloxKey key, bool all = true) {
+  const uint64_t p = (uint64_t)PHILOX_M1 * (f.lo ^ s.m2);
+  uint32_t c0 = (uint32_t)(p >> 32) ^ f.m1, c1 = (uint32_t)p, c2 = f.hi ^ s.m3, c3 = f.q3;
+  uint32_t k0 = key.k0 + 3u * PHILOX_W0, k1 = key.k1 + 3u * PHILOX_W1;
+#pragma unroll
+  for (int r = 3; r < 9; ++r) {
+    const uint64_t p0 = (uint64_t)PHILOX_M0 * c0, p1 = (uint64_t)PHILOX_M1 * c2;
+    c0 = philox_xor3((uint32_t)(p1 >> 32), c1, k0);
+    c2 = philox_xor3((uint32_t)(p0 >> 32), c3, k1);
+    c1 = (uint32_t)p1;
+    c3 = (uint32_t)p0;
+    k0 += PHILOX_W0;
+    k1 += PHILOX_W1;
+  }
+  Philox4 out;
+  const uint64_t p1 = (uint64_t)PHILOX_M1 * c2;
+  out.v[0] = philox_xor3((uint32_t)(p1 >> 32), c1, k0);
+  out.v[1] = (uint32_t)p1;
+  out.v[2] = out.v[3] = 0u;
+  if (all) {
+    const uint64_t p0 = (uint64_t)PHILOX_M0 * c0;
+    out.v[2] = philox_xor3((uint32_t)(p0 >> 32), c3, k1);
+    out.v[3] = (uint32_t)p0;
+  }
+  return out;
+}
+
 // what a draw is used for; part of the counter so that streams never overlap
 enum RngPurpose : uint32_t {
   RNG_OUT_NOISE = 1,  // ADC output noise

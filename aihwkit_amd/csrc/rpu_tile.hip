@@ -1552,7 +1552,17 @@ struct Tile {
       // the static block belongs to all tiles of the GPU: its words are made now, a later inspection only reads them
       a.keep_words = ws ? 1 : 0;
       // (pulse counters and write noise read the bit planes; the static block is laid out for planes)
-      a.x_lane_masks = (!ws && !aggregated && !counting && !(dv.w == d_wp.p && persistent()) && update_takes_stream(a)) ? 1 : 0;
+      a.x_lane_masks = 0;
+      if (!ws && !aggregated && !counting && !(dv.w == d_wp.p && persistent())) {
+        if (update_takes_stream(a)) {
+          a.x_lane_masks = 1;
+        } else if (const int columns = update_mask_columns(a)) {
+          a.x_lane_masks = 2;
+          a.x_mask_columns = columns;
+          u_xpl.ensure(2 * update_mask_words(a, columns));
+          a.x_planes = u_xpl.p;
+        }
+      }
       launch_update_lines(a, s);
       prof_mark(s, "update_lines");
       if (counting) count_pulses(a, false, s);

@@ -1,0 +1,83 @@
+"""The pulse loop of tiles with several columns per lane runs on lane masks (k_update_pulsed_masks) where batch and rows are
+many enough (update_mask_columns).  A group call runs the plain pulse loop on the same pulse trains and noise streams, so
+both leave the same weights, bit for bit."""
+import pytest
+import torch
+
+from helpers import constant_step, soft_bounds
+from test_gpu_pulse_stream import _additive, _tile
+
+pytestmark = pytest.mark.gpu
+
+
+def _device(kind):
+    if kind == "soft_bounds":
+        return soft_bounds(construction_seed=5)
+    if kind == "constant_step":
+        return constant_step(construction_seed=5)
+    if kind == "quiet":
+        return soft_bounds(construction_seed=5, dw_min_std=0.0)
+    return _additive(0.3 if kind == "additive" else 0.0)
+
+
+def _data(x_size, d_size, batch, sparse):
+    gen = torch.Generator("cuda").manual_seed(batch + x_size)
+    x = torch.rand(batch, x_size, generator=gen, device="cuda") * 2 - 1
+    d = torch.randn(batch, d_size, generator=gen, device="cuda") * 0.05
+    if sparse:
+        d[torch.rand(batch, generator=gen, device="cuda") < sparse] = 0.0
+    return x, d
+
+
+# four and two columns per lane; a span of columns that is full, one more than full, mostly behind the row's end; rows that
+# are dealt out by their work (1024 x 1024) and units that do not fill the last workgroup; chunks that are not full; lr sets
+# the longest bit line: 1, 3, 7 and 31 (the last walked pulse by pulse); rows with hardly a pass
+@pytest.mark.parametrize("x_size,d_size,batch,lr,sparse", [
+    (1024, 1024, 130, 0.01, 0), (1024, 515, 300, 0.05, 0), (1025, 515, 257, 0.0005, 0), (1024, 1024, 129, 0.6, 0),
+    (513, 301, 512, 0.02, 0), (257, 601, 260, 0.05, 0), (512, 513, 1000, 0.0005, 0.99), (700, 333, 450, 0.02, 0.9),
+    (520, 512, 200, 0.6, 0)])
+@pytest.mark.parametrize("kind", ["soft_bounds", "constant_step", "quiet", "additive", "additive_quiet"])
+def test_pulse_loop_on_lane_masks_equals_the_plain_one(x_size, d_size, batch, lr, sparse, kind):
+    from aihwkit_amd.rpu_base.tiles import TileGroup
+    x, d = _data(x_size, d_size, batch, sparse)
+    one, other = (_tile(x_size, d_size, _device(kind)) for _ in range(2))
+    start = one.get_weights()
+    for tile in (one, other):
+        tile.set_learning_rate(lr)
+    group = TileGroup([other])
+    for call in range(2):
+        if call:  # lines along the batch
+            one.update(x.t().contiguous(), d.t().contiguous(), False, True, True)
+        else:
+            one.update(x, d, False)
+        group.update([x], [d])
+    assert torch.equal(one.get_weights(), other.get_weights())
+    assert not torch.equal(one.get_weights(), start)
+    for mine, theirs in zip(one.get_update_words(batch), other.get_update_words(batch)):
+        assert torch.equal(mine, theirs)
+
+
+def test_pulse_loop_on_lane_masks_with_weights_outside_their_bounds(storage_mode):
+    """They are cut back by the first pulse and not before; a negative learning rate turns the direction."""
+    from aihwkit_amd.rpu_base.tiles import TileGroup
+    x_size, d_size, batch = 600, 400, 300
+    x, d = _data(x_size, d_size, batch, 0)
+    x[:, ::5] = 0.0
+    results = []
+    for grouped in (False, True):
+        tile = _tile(x_size, d_size, _device("soft_bounds"))
+        if storage_mode == "xd_shared":
+            w = tile._shared_weights.t()
+        else:
+            w = torch.empty(d_size, x_size, device="cuda")
+            tile.set_shared_weights_row_major(w)
+        w[:, ::3] = 2.5
+        tile.set_learning_rate(-0.01)
+        if grouped:
+            TileGroup([tile]).update([x], [d])
+        else:
+            tile.update(x, d, False)
+        results.append(w.clone())
+    assert torch.equal(results[0], results[1])
+    assert bool((results[0][:, ::15] == 2.5).all())   # no x pulse: untouched
+    assert float(results[0][:, 3].max()) < 2.5
