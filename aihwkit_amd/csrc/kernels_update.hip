@@ -296,6 +296,16 @@ __host__ __device__ __forceinline__ int pulse_mask_spans(int x_size, int columns
 }
 template <int C> __device__ __forceinline__ int pulse_mask_column(int span, int c) { return ((span >> 2) * C + c) * 256 + (span & 3) * 64; }
 
+// Whether a call's pulses can be drawn slot by slot (pulse_slot): bit lines of at most four pulses, one row of words per
+// sample, no discretized probabilities.  What pulse_word draws then, without the packed word, and with the rounds of the
+// generator that only the element or only the sample decides done once (15 to 16 wide products a draw instead of 18 to 20,
+// which are most of these kernels' time): pulse trains of 131072 samples of 433 + 48 lines 224 -> 189 us.
+__device__ __forceinline__ bool pulses_by_slot(const UpdateArgs &a, int kmax) {
+  return kmax <= 4 && a.words_per_sample <= 1 && a.up.res <= 0.0f;
+}
+// pulse in a slot from its random word: PP > u32_to_uniform(rnd), both sides 2^24 times as large
+__device__ __forceinline__ bool pulse_slot(uint32_t rnd, float PP_2_24) { return PP_2_24 > (float)(rnd >> 8); }
+
 // longest bit line of a batch whose packed words are not written: only the loop for longer ones reads them
 constexpr int UPDATE_PLANES_ONLY_KMAX = 7;
 
@@ -362,7 +372,7 @@ __device__ __forceinline__ void update_lines_block(const UpdateArgs &a, const in
     }
   }
   __syncthreads();
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int b = b0 + lane; // row of words
   const bool b_ok = b < a.m_batch;
   const int sample = wps > 1 ? b / wps : b, wrow = wps > 1 ? b - sample * wps : 0;
@@ -372,6 +382,36 @@ __device__ __forceinline__ void update_lines_block(const UpdateArgs &a, const in
   const bool keep_words = a.keep_words || kmax > UPDATE_PLANES_ONLY_KMAX;
   uint32_t *planes = is_x ? a.x_planes : a.d_planes;
   const int c0 = 2 * by;
+  if (!keep_words && pulses_by_slot(a, kmax)) {
+    // the element is the same for all lanes: its share of the generator is scalar work, the sample's is done once
+    const PhiloxSecond second = philox_second((uint32_t)sample, a.call, a.key);
+    for (int el = wave; el < LINES_E; el += 4) {
+      const int e = e0 + el;
+      if (e >= size) break; // wave-uniform
+      const float v = vals[lane][el], PP = fabsf(v) * P, most = PP * 16777216.0f;
+      const Philox4 r = philox_finish(philox_first((uint32_t)e, a.call, is_x ? RNG_PULSE_X : RNG_PULSE_D, a.key), second, a.key, kmax > 2);
+      unsigned long long any = 0ull;
+      int passes = 0;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        if (k >= kmax) break;
+        const unsigned long long m = __ballot(k < K && pulse_slot(r.v[k], most));
+        any |= m;
+        passes += __popcll(m);
+        if (lane == 0) {
+          planes[((long)c0 * slots + k) * size + e] = (uint32_t)m;
+          if (c0 + 1 < a.n_chunks) planes[((long)(c0 + 1) * slots + k) * size + e] = (uint32_t)(m >> 32);
+        }
+      }
+      if (!is_x && a.row_cost && lane == 0 && passes) atomicAdd(&a.row_cost[e], 9 * passes + 4 * __popcll(any));
+      const unsigned long long sg = __ballot(K > 0 && PP != 0.0f && !(v > 0.0f));
+      if (lane == 0) {
+        planes[((long)c0 * slots + kmax) * size + e] = (uint32_t)sg;
+        if (c0 + 1 < a.n_chunks) planes[((long)(c0 + 1) * slots + kmax) * size + e] = (uint32_t)(sg >> 32);
+      }
+    }
+    return;
+  }
   for (int el = wave; el < LINES_E; el += 4) {
     const int e = e0 + el;
     if (e >= size) break; // wave-uniform
@@ -473,7 +513,7 @@ __global__ __launch_bounds__(256) void k_update_lines_stream(UpdateArgs a) {
     }
     return;
   }
-  const int lane = (int)threadIdx.x & 63, wave = (int)threadIdx.x >> 6;
+  const int lane = (int)threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int e0 = bx * 64, b0 = by * 64;
   const int wps = max(a.words_per_sample, 1);
   if (IN_PLACE && a.x_index) { // lanes along the patches, as in update_lines_block
@@ -500,6 +540,26 @@ __global__ __launch_bounds__(256) void k_update_lines_stream(UpdateArgs a) {
   }
   __syncthreads();
   const int e = e0 + lane;
+  unsigned long long *masks = reinterpret_cast<unsigned long long *>(a.x_planes) + (long)bx * (kmax + 1) + lane;
+  if (pulses_by_slot(a, kmax)) {
+    const PhiloxFirst first = philox_first((uint32_t)e, a.call, RNG_PULSE_X, a.key);
+    for (int i = 0; i < 16; ++i) {
+      const int b = b0 + wave * 16 + i;
+      if (b >= a.m_batch) break; // wave-uniform
+      const int K = a.bl[b];
+      const float v = vals[wave * 16 + i][lane], PP = e < a.x_size ? fabsf(v) * a.prob_b[b] : 0.0f, most = PP * 16777216.0f;
+      const Philox4 r = philox_finish(first, philox_second((uint32_t)b, a.call, a.key), a.key, K > 2);
+      unsigned long long mine = K > 0 ? __ballot(PP != 0.0f && !(v > 0.0f)) : 0ull; // lane kmax keeps the signs
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        if (k >= kmax) break;
+        const unsigned long long m = k < K ? __ballot(pulse_slot(r.v[k], most)) : 0ull;
+        mine = lane == k ? m : mine;
+      }
+      if (lane <= kmax) masks[(long)b * blocks_x * (kmax + 1)] = mine;
+    }
+    return;
+  }
   for (int i = 0; i < 16; ++i) {
     const int b = b0 + wave * 16 + i;
     if (b >= a.m_batch) break; // wave-uniform
@@ -511,7 +571,7 @@ __global__ __launch_bounds__(256) void k_update_lines_stream(UpdateArgs a) {
       const unsigned long long m = __ballot((word >> (k + 1)) & 1u);
       mine = lane == k ? m : mine;
     }
-    if (lane <= kmax) reinterpret_cast<unsigned long long *>(a.x_planes)[((long)b * blocks_x + bx) * (kmax + 1) + lane] = mine;
+    if (lane <= kmax) masks[(long)b * blocks_x * (kmax + 1)] = mine;
   }
 }
 
@@ -549,6 +609,7 @@ __global__ __launch_bounds__(256) void k_update_lines_masks(UpdateArgs a, int ro
   const int b1 = min(b0 + rows_per_wave, a.m_batch);
   if (b0 >= b1) return;
   const int wps = max(a.words_per_sample, 1);
+  const bool by_slot = pulses_by_slot(a, kmax);
   // lane l < 4 kmax: slot l / 4, sign of the d line (l / 2) & 1, columns that fire (even) or step down (odd)
   const int my_slot = lane >> 2;
   const bool my_dir = lane & 1, my_turn = (lane >> 1) & 1;
@@ -581,7 +642,7 @@ __global__ __launch_bounds__(256) void k_update_lines_masks(UpdateArgs a, int ro
 #pragma unroll
     for (int c = 0; c < C; ++c) {
       const bool ok = e[c] < a.x_size;
-      if (K <= 4 && wrow == 0 && a.up.res <= 0.0f) { // pulse_word, slot by slot
+      if (by_slot) {
         const float PP = ok ? fabsf(now[c]) * P : 0.0f, most = PP * 16777216.0f;
         const unsigned long long sg = K > 0 ? __ballot(PP != 0.0f && !(now[c] > 0.0f)) : 0ull;
         mine[c] = my_turn ? ~sg : sg;
@@ -589,10 +650,9 @@ __global__ __launch_bounds__(256) void k_update_lines_masks(UpdateArgs a, int ro
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
           if (k >= kmax) break;
-          const unsigned long long m = k < K ? __ballot(most > (float)(r.v[k] >> 8)) : 0ull;
+          const unsigned long long m = k < K ? __ballot(pulse_slot(r.v[k], most)) : 0ull;
           mine[c] = (!my_dir && my_slot == k) ? m : mine[c];
         }
-        for (int k = 4; k < kmax; ++k) mine[c] = (!my_dir && my_slot == k) ? 0ull : mine[c];
       } else {
         const uint32_t word = ok ? pulse_word(a, true, e[c], sample, now[c], P, K, wrow) : 0u;
         const unsigned long long sg = __ballot(word & 1u);
