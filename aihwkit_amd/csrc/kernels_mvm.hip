@@ -1699,6 +1699,18 @@ __device__ __forceinline__ float max_abs4(float m, const f32x4 v) { // NaN do no
   return m;
 }
 
+// LDS of a large-tile workgroup (mvm_big_workgroup)
+template <int WT, int BB, int WO, int XP> struct BigLds {
+  static constexpr int WPITCH = 32 * WO + 4; // floats per staged k-row of an output-contiguous weight tile
+  __attribute__((aligned(16))) __bf16 x[2][XP][BB * BKS];
+  __attribute__((aligned(16))) float w[2][WT ? BKS * WPITCH : 32 * WO * BROW];
+  int hits[2 * BB];
+  int b[BB];
+  float scale[BB];
+  int last;
+  int slow; // whether the fp32 pipe has to multiply this tile
+};
+
 // work of workgroup number n of a large-tile round launch of one tile; BB: samples of a workgroup tile (128 or 64)
 // WO: waves along the outputs, 32 outputs each: 4, or 2 for tiles of at most 64 outputs (the other two waves then take
 // the second half of the samples instead of outputs that do not exist).
@@ -1716,7 +1728,8 @@ __device__ __forceinline__ float max_abs4(float m, const f32x4 v) { // NaN do no
 // LAZY (calls with speculate = 0): nothing is quantized ahead; the last workgroup of a sample tile writes the rows of
 // the samples that go on.  The other instantiations always quantize ahead, as their callers ask for.
 template <int WT, int BB, int WO, int XP, bool LAZY>
-__device__ __forceinline__ void mvm_big_workgroup(const MvmArgs &a, const int round, const int n, const int min_active) {
+__device__ __forceinline__ void mvm_big_workgroup(const MvmArgs &a, const int round, const int n, const int min_active,
+                                                  BigLds<WT, BB, WO, XP> &sh) {
   static_assert(BB == 128 || BB == 64, "sample tile of 128 or 64");
   static_assert(WO == 4 || WO == 2, "two or four waves along the outputs");
   static_assert(XP == 1 || BB == 64 || WO == 2, "one workgroup per CU");
@@ -1725,14 +1738,12 @@ __device__ __forceinline__ void mvm_big_workgroup(const MvmArgs &a, const int ro
   constexpr int NB = BB / 32 / WB;       // 32-sample blocks per wave
   constexpr int XJ = BB / 32;            // staged sample rows per thread
   constexpr int WJ = OT / 32;            // staged chunks of weights per thread
-  constexpr int WPITCH = OT + 4;         // floats per staged k-row of an output-contiguous weight tile
-  __shared__ __attribute__((aligned(16))) __bf16 lds_x[2][XP][BB * BKS];
-  __shared__ __attribute__((aligned(16))) float lds_w[2][WT ? BKS * WPITCH : OT * BROW];
-  __shared__ int sh_hits[2 * BB];
-  __shared__ int sh_b[BB];
-  __shared__ float sh_scale[BB];
-  __shared__ int sh_last;
-  __shared__ int sh_slow; // whether the fp32 pipe has to multiply this tile
+  constexpr int WPITCH = BigLds<WT, BB, WO, XP>::WPITCH;
+  auto &lds_x = sh.x;
+  auto &lds_w = sh.w;
+  int *const sh_hits = sh.hits, *const sh_b = sh.b;
+  float *const sh_scale = sh.scale;
+  int &sh_last = sh.last, &sh_slow = sh.slow;
 
   const int n_act = (round > 0) ? a.st.count[round] : a.m_batch;
   if (n_act < min_active) return; // this round is run by the 32 x 32 kernel
@@ -2034,7 +2045,56 @@ __device__ __forceinline__ void mvm_big_workgroup(const MvmArgs &a, const int ro
 
 template <int WT, int BB, int WO, int XP, bool LAZY>
 __global__ __launch_bounds__(256, XP == 1 && BB == 64 ? 3 : 2) void k_mvm_big(MvmArgs a, int min_active) {
-  mvm_big_workgroup<WT, BB, WO, XP, LAZY>(a, a.round, (int)blockIdx.x, min_active);
+  __shared__ BigLds<WT, BB, WO, XP> sh;
+  mvm_big_workgroup<WT, BB, WO, XP, LAZY>(a, a.round, (int)blockIdx.x, min_active, sh);
+}
+
+// k_mvm_rounds_rest for a call whose rounds have more workgroups than the GPU holds at once, or run on the large tiles, or
+// gather their rows: one workgroup per CU walks the tiles that a round lists.  In a 768 -> 2304 step of 1024 samples that
+// lists nothing, eight launches of 2 to 5 us (large-tile and 32 x 32 kernel, four rounds) become one of 5 us.  A round that
+// does list samples runs on the kernel that its own launch would run it on (XP > 0: large tiles from a.big_from samples on;
+// the sum of an output does not depend on the tile's shape), so results are the same bits; on a few hundred workgroups it
+// takes longer, once: the next call is launched by what this one listed.
+template <int WMODE, int XP>
+__global__ __launch_bounds__(256, 2) void k_mvm_rest_walk(MvmArgs a) {
+  constexpr int WT = WMODE == 1 ? 1 : 0;
+  typedef BigLds<WT, 64, 2, XP ? XP : 1> Big;
+  constexpr size_t RED = sizeof(float) * WAVES * 16 * 64, STAGE = sizeof(float) * WAVES * 2 * TILE * LDS_ROW;
+  __shared__ __attribute__((aligned(16))) unsigned char lds[RED + STAGE > sizeof(Big) ? RED + STAGE : sizeof(Big)];
+  float (*red)[16][64] = reinterpret_cast<float (*)[16][64]>(lds);
+  float *stage = reinterpret_cast<float *>(lds + RED);
+  if (a.dual.on == 2) {
+    const int all = workgroups_for(a.O, a.m_batch);
+    for (int n = blockIdx.x; n < all; n += gridDim.x) mvm_dual_select(a, n);
+  }
+  const RoundWait wt = round_wait_of(a.st.count, a.dual.seen, a.wait_spins, a.wait_extra);
+  for (int r = a.round; r < a.max_rounds; ++r) {
+    const int n_act = __hip_atomic_load(&a.st.count[r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    mvm_note_round(a, r, n_act, r == a.round && a.dual.on == 2);
+    if (n_act == 0) return; // the same for every workgroup
+    if (r > a.round && !mvm_device_barrier(&a.st.count[MVM_ARRIVE_BASE + 4 * r + 2], (int)gridDim.x, wt, r)) return;
+    const bool large = XP != 0 && runs_on_large_tiles(a, r, n_act);
+    if constexpr (XP != 0) {
+      if (large) {
+        const int total = 8 * ((a.O + 63) / 64) * (((n_act + 63) / 64 + 7) / 8);
+        for (int n = blockIdx.x; n < total; n += gridDim.x) {
+          mvm_big_workgroup<WT, 64, 2, XP, false>(a, r, n, 0, *reinterpret_cast<Big *>(lds));
+          __syncthreads(); // LDS is reused by the next tile
+        }
+      }
+    }
+    const int total = large ? 0 : workgroups_for(a.O, n_act);
+    for (int n = blockIdx.x; n < total; n += gridDim.x) {
+      if (a.in_index) {
+        int tile_o, tile_b;
+        if (tile_of(a, n, n_act, tile_o, tile_b)) mvm_gather_tile_rows(a, r, tile_b, n_act);
+      }
+      mvm_round_workgroup<1, WMODE>(a, r, n, n_act, red, stage);
+      __syncthreads(); // LDS is reused by the next tile
+    }
+    if (r + 1 == a.max_rounds) return;
+    if (!mvm_arrive(&a.st.count[MVM_ARRIVE_BASE + 4 * r], (int)gridDim.x, wt, r)) return;
+  }
 }
 
 // several tiles in one launch (round 0): a tile that is not run by this kernel has no workgroups in the table
@@ -2044,7 +2104,8 @@ __global__ __launch_bounds__(256, XP == 1 && BB == 64 ? 3 : 2) void k_mvm_big_gr
   while (t + 1 < g.n && (int)blockIdx.x >= g.start[t + 1]) ++t;
   const MvmArgs &a = g.args[t];
   if (round > 0 && round >= a.max_rounds) return;
-  mvm_big_workgroup<WT, BB, 4, XP, false>(a, round, (int)blockIdx.x - g.start[t], 0);
+  __shared__ BigLds<WT, BB, 4, XP> sh;
+  mvm_big_workgroup<WT, BB, 4, XP, false>(a, round, (int)blockIdx.x - g.start[t], 0, sh);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -2703,7 +2764,23 @@ static int mvm_rest_depth(const MvmArgs &a) {
   return (weight_mode(a) == 1 && depth == 4) ? 2 : depth;
 }
 
+// whether the launch of the rounds expected empty walks its tiles (k_mvm_rest_walk) instead of having a workgroup for each
+static bool mvm_rest_walks(const MvmArgs &a) {
+  return a.in_index || (!a.small_tiles_only && big_threshold(a.m_batch, a.O) > 0) || mvm_round_workgroups(a) > current_device_cus();
+}
+
+typedef void (*RestWalk)(MvmArgs);
+// a.big_from as launch_mvm_round sets it: some round of the call may run on the large tiles
+static RestWalk mvm_rest_walk_kernel(const MvmArgs &a) {
+  const int mode = weight_mode(a);
+  if (a.big_from == 0) return mode == 0 ? k_mvm_rest_walk<0, 0> : (mode == 1 ? k_mvm_rest_walk<1, 0> : k_mvm_rest_walk<2, 0>);
+  if (a.x_step > 0.0f) return mode == 0 ? k_mvm_rest_walk<0, 1> : (mode == 1 ? k_mvm_rest_walk<1, 1> : k_mvm_rest_walk<2, 1>);
+  return mode == 0 ? k_mvm_rest_walk<0, 3> : (mode == 1 ? k_mvm_rest_walk<1, 3> : k_mvm_rest_walk<2, 3>);
+}
+
 int mvm_rest_resident_limit(const MvmArgs &a) {
+  // a walking launch has one workgroup per CU, all variants of it less than half of a CU's registers and LDS
+  if (mvm_rest_walks(a)) return resident_workgroups(k_mvm_rest_walk<1, 3>);
   static std::mutex m;
   static int limit[64][3][3] = {};
   int dev = 0;
@@ -2749,10 +2826,8 @@ int mvm_group_rest_resident_limit(int mode) {
 // CUs at that moment (a second stream) can make a wait run out; that is reported (see RoundWait), never passed over.
 bool mvm_can_merge_rest(const MvmArgs &a, int resident_limit) {
   if (a.io.perfect || a.io.bound_management == RPU_BM_NONE || a.max_rounds < 3 || a.transposed) return false;
-  // gathered input: the rows of a further round are written by k_mvm_round_tail alone, one launch per round
-  if (a.pre_add || a.skip_if_zero || a.nm_phase || a.in_index) return false;
-  if (!a.small_tiles_only && big_threshold(a.m_batch, a.O) > 0) return false;
-  return mvm_round_workgroups(a) <= resident_limit;
+  if (a.pre_add || a.skip_if_zero || a.nm_phase) return false;
+  return mvm_rest_walks(a) ? resident_limit > 0 : mvm_round_workgroups(a) <= resident_limit;
 }
 
 void launch_mvm_dual(const MvmArgs &a_in, hipStream_t s) {
@@ -2779,6 +2854,12 @@ void launch_mvm_round(const MvmArgs &a_in, hipStream_t s) {
   // calls that quantize nothing ahead expect few samples in a further round: the 32 x 32 kernels take them all, and
   // the round is one launch
   if (a.round > 0 && !a.speculate) a.big_from = 0;
+  if (a.rest_in_one && mvm_rest_walks(a)) {
+    const dim3 grid((unsigned)std::min(mvm_round_workgroups(a), current_device_cus()));
+    const RestWalk kernel = mvm_rest_walk_kernel(a);
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, a);
+    return;
+  }
   if (a.big_from > 0) {
     const bool lazy = !a.transposed && !a.speculate && a.max_rounds > 1;
     // outputs x samples of a workgroup tile.  Narrow tiles: 64 x 128 (see mvm_big_workgroup, WO).  Fewer than three tiles

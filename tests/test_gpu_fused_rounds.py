@@ -360,3 +360,33 @@ def test_worst_case_second_round_on_a_fresh_tile_matches_the_oracle(gpu_device):
         y = gpu.forward(xin).cpu().numpy()
         assert np.array_equal(gpu.get_bm_rounds(batch).numpy(), rounds), mode
         assert np.array_equal(y, want), mode
+
+
+@pytest.mark.parametrize("shape", [(160, 1100, 1030), (64, 80, 9000), (100, 700, 500)])
+def test_large_calls_share_one_launch_for_the_later_rounds(gpu_device, shape):
+    """Calls whose rounds run on the large tiles (rows quantized ahead, and written by the last workgroup of a sample tile),
+    or have more workgroups than the GPU holds: quiet inputs, then saturating ones that the one launch does not expect,
+    then quiet ones again.  All sums are exact, so every kernel gives the same bits."""
+    x_size, d_size, batch = shape
+    rng = np.random.default_rng(d_size)
+    io = noise_free_io(inp_res=1 / 64.0, out_res=1 / 256.0, out_bound=2.0, noise_management=NM.NONE, bound_management=BM.Iterative)
+    w = (rng.integers(-32, 33, (d_size, x_size)) / 64.0).astype(F)
+    host, _orc, _ = build_pair(make_meta(io, noise_free_io()), soft_bounds(construction_seed=3, w_max_dtod=0.0, w_min_dtod=0.0),
+                               x_size, d_size, gpu=False)
+    host.set_weights(torch.from_numpy(w))
+    loud = (rng.integers(-64, 65, (batch, x_size)) / 64.0).astype(F)
+    quiet = (rng.integers(-1, 2, (batch, x_size)) / 64.0).astype(F)
+    results = []
+    for mode in (0, 2, -1):
+        gpu = tiles.CudaAnalogTile(host)
+        gpu.set_fused_rounds(mode)
+        outs = []
+        for x in [quiet] * 3 + [loud] * 2 + [quiet] * 2:
+            y = gpu.forward(torch.from_numpy(x).cuda()).cpu().numpy()
+            outs.append((y, gpu.get_bm_rounds(batch).numpy().copy()))
+        results.append(outs)
+    assert results[0][0][1].max() == 1 and results[0][3][1].max() >= 3
+    for other in results[1:]:
+        for (y0, r0), (y1, r1) in zip(results[0], other):
+            assert np.array_equal(r0, r1)
+            assert np.array_equal(y0, y1)
