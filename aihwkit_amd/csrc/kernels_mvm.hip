@@ -1748,11 +1748,12 @@ __device__ __forceinline__ void mvm_big_workgroup(const MvmArgs &a, const int ro
   const int n_act = (round > 0) ? a.st.count[round] : a.m_batch;
   if (n_act < min_active) return; // this round is run by the 32 x 32 kernel
   // workgroup n runs on XCD n % 8: an XCD walks the output tiles of one sample tile after the other, so a tile of
-  // quantized inputs (the large operand) enters one L2 only and the small weight matrix is what every XCD streams
-  const int tiles_o = (a.O + OT - 1) / OT;
-  const int tile_o = (n >> 3) % tiles_o;
-  const int tile_b = ((n >> 3) / tiles_o) * 8 + (n & 7);
-  if (tile_b * BB >= n_act) return;
+  // quantized inputs (the large operand) enters one L2 only (two where XCDs share a sample tile, an eighth of the tiles to
+  // each) and the small weight matrix is what every XCD streams
+  const int tiles_o = (a.O + OT - 1) / OT, tiles = tiles_o * ((n_act + BB - 1) / BB), share = (tiles + 7) >> 3;
+  const int tile = (n & 7) * share + (n >> 3);
+  if ((n >> 3) >= share || tile >= tiles) return;
+  const int tile_b = tile / tiles_o, tile_o = tile - tile_b * tiles_o;
   const bool more_rounds = round + 1 < a.max_rounds;
   if (more_rounds && !LAZY && !(round == 0 && a.rows_ahead_in_init)) {
     big_prepare_next_rows<BB>(a, round, tile_o, tiles_o, tile_b, n_act, sh_b, sh_scale);
@@ -2076,7 +2077,7 @@ __global__ __launch_bounds__(256, 2) void k_mvm_rest_walk(MvmArgs a) {
     const bool large = XP != 0 && runs_on_large_tiles(a, r, n_act);
     if constexpr (XP != 0) {
       if (large) {
-        const int total = 8 * ((a.O + 63) / 64) * (((n_act + 63) / 64 + 7) / 8);
+        const int total = 8 * ((((a.O + 63) / 64) * ((n_act + 63) / 64) + 7) / 8);
         for (int n = blockIdx.x; n < total; n += gridDim.x) {
           mvm_big_workgroup<WT, 64, 2, XP, false>(a, r, n, 0, *reinterpret_cast<Big *>(lds));
           __syncthreads(); // LDS is reused by the next tile
@@ -2638,7 +2639,7 @@ constexpr int TAIL_GRID = 1024; // workgroups of a later-round launch when the f
 // workgroups of a large-tile launch with sample tiles of `bb` samples
 static int big_workgroups(const MvmArgs &a, int bb, int ot = 128) {
   const int tiles_o = (a.O + ot - 1) / ot, tiles_b = (a.m_batch + bb - 1) / bb;
-  return 8 * tiles_o * ((tiles_b + 7) / 8);
+  return 8 * ((tiles_o * tiles_b + 7) / 8);
 }
 
 int mvm_big_workgroups(const MvmArgs &a, int bb) { return a.O >= 128 ? big_workgroups(a, bb) : 0; }
