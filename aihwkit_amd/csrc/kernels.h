@@ -420,8 +420,9 @@ void launch_device_drift(float *w, float *prev, float *w0, float *t, const float
 
 // per-row statistic of the first n_cols columns: largest absolute value, or sum of squares
 void launch_row_stat(const float *w, const MatLayout &lay, int n_cols, int sum_squares, float *row_out, hipStream_t s);
-// out[0] = largest of v[0..n-1] when positive, else 1
-void launch_max_or_one(const float *v, int n, float *out, hipStream_t s);
+// the largest absolute values of abs_max_parts() parts of the first n_cols columns
+void launch_abs_max_parts(const float *w, const MatLayout &lay, int n_cols, float *parts, hipStream_t s);
+size_t abs_max_parts();
 // WeightRemapper::apply (weight_remapper.cpp:19-190): from the row statistic in row_stat the per-row factors
 // mul / div and the new scales; then w[i][j] = w[i][j] * mul[i] / div[i]
 struct RemapDev {
@@ -431,13 +432,13 @@ struct RemapDev {
 void launch_remap(float *w, float *scales, float *row_stat, float *mul, float *div, const MatLayout &lay,
                   const RemapDev &p, hipStream_t s);
 
-// WeightModifier::apply (weight_modifier.cpp:28-224): out = modified copy of w; amax_dev == null: assumed_wmax
+// WeightModifier::apply (weight_modifier.cpp:28-224): out = modified copy of w; amax_parts == null: assumed_wmax
 struct ModifierDev {
   int type, sto_round, copy_last_column, n_coeffs;
   float std_dev, res, dorefa_clip, pdrop, g_max, assumed_wmax;
   float coeffs[8];
 };
-void launch_modify(float *out, const float *w, const ModifierDev &p, const float *amax_dev, PhiloxKey key, uint32_t call,
+void launch_modify(float *out, const float *w, const ModifierDev &p, const float *amax_parts, PhiloxKey key, uint32_t call,
                    const MatLayout &lay, hipStream_t s);
 
 // adds the coincidences of the batch to the per-cross-point counters: pos where the signs of x and d agree,

@@ -251,12 +251,33 @@ __device__ __forceinline__ float block_max(float v, float *sh) {
   return r;
 }
 
-__global__ __launch_bounds__(256) void k_max_or_one(const float *v, int n, float *out) {
+// Largest absolute values of ABS_MAX_PARTS parts of a matrix, the first n_cols columns of it (all of them, or all but the
+// last).  Read in memory order, 16 bytes a load, whichever way the matrix is stored: a 768 x 2304 tile kept as
+// [x_size][d_size] took 13 us row by row (strided reads), and 5 more for a launch that put the rows together; 4 us here,
+// and the kernel that needs the value takes the largest part itself.
+constexpr int ABS_MAX_PARTS = 512;
+__global__ __launch_bounds__(256) void k_abs_max_parts(const float *w, MatLayout lay, int n_cols, float *parts) {
   __shared__ float sh[4];
+  // the last column is the end of the memory of a [x_size][d_size] matrix
+  const bool skip = n_cols < lay.x_size && !lay.xd;
+  const size_t n = lay.xd ? (size_t)n_cols * lay.d_size : lay.size();
+  const size_t first = blockIdx.x * (size_t)blockDim.x + threadIdx.x, stride = (size_t)gridDim.x * blockDim.x;
   float m = 0.0f;
-  for (int i = threadIdx.x; i < n; i += blockDim.x) m = fmaxf(m, v[i]);
+  if (skip) {
+    for (size_t i = first; i < n; i += stride) {
+      if (lay.col_of(i) < n_cols) m = fmaxf(m, fabsf(w[i]));
+    }
+  } else {
+    const size_t n4 = ((uintptr_t)w & 15) == 0 ? n >> 2 : 0;
+    const float4 *w4 = reinterpret_cast<const float4 *>(w);
+    for (size_t i = first; i < n4; i += stride) {
+      const float4 v = w4[i];
+      m = fmaxf(fmaxf(m, fmaxf(fabsf(v.x), fabsf(v.y))), fmaxf(fabsf(v.z), fabsf(v.w)));
+    }
+    for (size_t i = 4 * n4 + first; i < n; i += stride) m = fmaxf(m, fabsf(w[i]));
+  }
   m = block_max(m, sh);
-  if (threadIdx.x == 0) *out = m > 0.0f ? m : 1.0f;
+  if (threadIdx.x == 0) parts[blockIdx.x] = m;
 }
 
 // One workgroup: the per-row factors of a remap and the new scales.  The weights then become w * mul / div, which
@@ -326,9 +347,17 @@ __device__ __forceinline__ float discretize(float v, float res, int sto_round, f
 
 // WeightModifier::apply (weight_modifier.cpp:28-224).  One Philox call per element: words 0, 1 give the normal
 // draw, word 2 the stochastic rounding, word 3 the dropped connections.
-__global__ __launch_bounds__(256) void k_modify(float *out, const float *w, ModifierDev p, const float *amax_dev,
+__global__ __launch_bounds__(256) void k_modify(float *out, const float *w, ModifierDev p, const float *amax_parts,
                                                  PhiloxKey key, uint32_t call, MatLayout lay, size_t n) {
-  const float amax = amax_dev ? *amax_dev : p.assumed_wmax;
+  float amax = p.assumed_wmax;
+  if (amax_parts) { // the largest weight, one when all are zero
+    float m = 0.0f;
+#pragma unroll
+    for (int i = 0; i < ABS_MAX_PARTS / 64; ++i) m = fmaxf(m, amax_parts[64 * i + (threadIdx.x & 63)]);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
+    amax = m > 0.0f ? m : 1.0f;
+  }
   for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
     float v = w[i];
     if (p.copy_last_column && lay.col_of(i) == lay.x_size - 1) {
@@ -446,9 +475,10 @@ void launch_row_stat(const float *w, const MatLayout &lay, int n_cols, int sum_s
   hipLaunchKernelGGL(k_row_stat, dim3(lay.d_size), dim3(256), 0, s, w, lay, n_cols, sum_squares, row_out);
 }
 
-void launch_max_or_one(const float *v, int n, float *out, hipStream_t s) {
-  hipLaunchKernelGGL(k_max_or_one, dim3(1), dim3(256), 0, s, v, n, out);
+void launch_abs_max_parts(const float *w, const MatLayout &lay, int n_cols, float *parts, hipStream_t s) {
+  hipLaunchKernelGGL(k_abs_max_parts, dim3(ABS_MAX_PARTS), dim3(256), 0, s, w, lay, n_cols, parts);
 }
+size_t abs_max_parts() { return ABS_MAX_PARTS; }
 
 void launch_remap(float *w, float *scales, float *row_stat, float *mul, float *div, const MatLayout &lay,
                   const RemapDev &p, hipStream_t s) {
@@ -458,10 +488,10 @@ void launch_remap(float *w, float *scales, float *row_stat, float *mul, float *d
   hipLaunchKernelGGL(k_remap_apply, dim3(grid_for(n)), dim3(256), 0, s, w, mul, div, lay, n);
 }
 
-void launch_modify(float *out, const float *w, const ModifierDev &p, const float *amax_dev, PhiloxKey key, uint32_t call,
+void launch_modify(float *out, const float *w, const ModifierDev &p, const float *amax_parts, PhiloxKey key, uint32_t call,
                    const MatLayout &lay, hipStream_t s) {
   const size_t n = lay.size();
-  hipLaunchKernelGGL(k_modify, dim3(grid_for(n)), dim3(256), 0, s, out, w, p, amax_dev, key, call, lay, n);
+  hipLaunchKernelGGL(k_modify, dim3(grid_for(n)), dim3(256), 0, s, out, w, p, amax_parts, key, call, lay, n);
 }
 
 void launch_write_noise_all(float *w_apparent, const float *w_persistent, float noise_std, PhiloxKey key, uint32_t call,

@@ -1307,14 +1307,13 @@ struct Tile {
     p.std_dev = q.std_dev; p.res = q.res; p.dorefa_clip = q.dorefa_clip; p.pdrop = q.pdrop; p.g_max = q.g_max;
     p.assumed_wmax = q.assumed_wmax;
     for (int c = 0; c < q.n_coeffs; ++c) p.coeffs[c] = q.coeffs[c];
-    const float *amax_dev = nullptr;
+    const float *amax_parts = nullptr;
     if (q.rel_to_actual_wmax && q.type != RPU_MODIFIER_COPY) {
-      s_rowstat.ensure(3 * (size_t)D + 1);
-      launch_row_stat(d_w.p, layout(), q.copy_last_column ? X - 1 : X, 0, s_rowstat.p, s);
-      launch_max_or_one(s_rowstat.p, D, s_rowstat.p + 3 * (size_t)D, s);
-      amax_dev = s_rowstat.p + 3 * (size_t)D;
+      s_rowstat.ensure(abs_max_parts());
+      launch_abs_max_parts(d_w.p, layout(), q.copy_last_column ? X - 1 : X, s_rowstat.p, s);
+      amax_parts = s_rowstat.p;
     }
-    launch_modify(d_fbw.p, d_w.p, p, amax_dev, key(), call++, layout(), s);
+    launch_modify(d_fbw.p, d_w.p, p, amax_parts, key(), call++, layout(), s);
     RPU_HIP_CHECK(hipGetLastError());
     last_stream = s;
   }
