@@ -125,6 +125,9 @@ struct MvmArgs {
   const int *in_index_lines;
   int in_group;
   long in_gs;
+  int *few;      // calls of k_mvm_few: [7][m_batch] counters and saturation marks, zero between calls
+  int *few_seen; // host-visible: few_call of the last call in which a sample needed a second round, and of the last call
+  int few_call;
 };
 
 // weight operand of a call: the matrix at w with rows of `ld` elements, stored [d_size][x_size] (xd_storage = false) or
@@ -183,6 +186,15 @@ float mvm_input_step(const IoDev &io, int K);
 // w_oc: how the tiles of the launch address their weights (MvmArgs::w_oc; the same for all of them)
 void launch_mvm_big_group(const MvmGroup &g, int total_workgroups, int bb, bool w_oc, bool stepped, hipStream_t s);
 void mvm_round_variant(const MvmArgs &a, int &prefetch_depth, int &weight_mode);
+
+// Small batches: everything from the noise management to the last bound-management round in one launch (k_mvm_few).
+// a.few is needed where a.max_rounds > 1.  rounds: 1, or 3 to work out rounds 0 to 2 together (a.dual.buf[1], buf[2]),
+// for calls whose samples are expected to need them; same results.
+bool mvm_few(const MvmArgs &a, bool training_tile); // whether a call takes that launch
+int mvm_few_variant(const MvmArgs *const *calls, int n); // blocks of a launch of n calls; the results do not depend on it
+int mvm_few_workgroups(const MvmArgs &a, int variant);
+void launch_mvm_few(const MvmArgs &a, int variant, int rounds, hipStream_t s);
+void launch_mvm_few_group(const MvmGroup &g, int variant, int rounds, bool w_oc, int max_k, int total_workgroups, hipStream_t s);
 
 // Fused convolution forward (unfold + noisy MVM with its bound-management rounds) for tiles of at most 32 outputs:
 // images [n_images][image_size], idx_t the transposed index matrix [patches][x_size], out [n_images][d_size][patches].

@@ -196,7 +196,8 @@ struct Tile {
   // round 2; the host-visible pair (samples of the last call that needed round 1, its batch) that the choice between
   // the fused and the separate launches is made from (fused_rounds: -1 by those values, 0 never, 1 .. 3 as forced)
   DevBuf<float> s_dual0, s_dual1, s_dual2, s_xq2;
-  DevBuf<int> s_dsel, s_dhit1, s_dhit2;
+  DevBuf<int> s_dsel, s_dhit1, s_dhit2, s_few;
+  int few_calls = 0; // see few_args
   int *seen_host = nullptr, *seen_dev = nullptr;
   int rest_from = 0, rest_quiet = 0; // the last round that listed samples in the recent calls, and calls since it did
   int fused_rounds = -1;
@@ -411,7 +412,7 @@ struct Tile {
   void release_all() {
     d_w.release(); d_wmax.release(); d_wmin.release(); d_sup.release(); d_sdown.release();
     d_slup.release(); d_sldown.release();
-    s_dual0.release(); s_dual1.release(); s_dual2.release(); s_xq2.release(); s_dsel.release(); s_dhit1.release();
+    s_dual0.release(); s_dual1.release(); s_dual2.release(); s_xq2.release(); s_dsel.release(); s_dhit1.release(); s_few.release();
     s_dhit2.release();
     if (seen_host) {
       (void)hipHostFree(seen_host);
@@ -585,6 +586,38 @@ struct Tile {
     if (m_batch == 0) return false;
     if (!p0 || !p1) throw RpuError("Null device pointer.");
     return true;
+  }
+
+  // What a call of k_mvm_few needs beyond mvm_args: few_counters(a) counters and saturation marks, zero between calls, and
+  // few_rows(a) floats for the results of rounds 1 and 2 (whether or not this call works on three rounds at once: the next
+  // one may, and be captured).  `seen`: host-visible numbers of the last call (of this tile or group) in which a sample went
+  // on to a second round and of the last call that has ended.  Returns the rounds to work out together (launch_mvm_few).
+  static size_t few_counters(const MvmArgs &a) { return a.max_rounds > 1 ? 7 * (size_t)a.m_batch : 0; }
+  static size_t few_rows(const MvmArgs &a) { return a.max_rounds > 2 ? 2 * (size_t)a.m_batch * a.O : 0; }
+  static void ensure_few(DevBuf<int> &counters, size_t n_counters, DevBuf<float> &rows, size_t n_rows, hipStream_t s) {
+    if (counters.n < n_counters) {
+      counters.ensure(n_counters);
+      launch_fill(reinterpret_cast<float *>(counters.p), 0.0f, n_counters, s); // all-zero bits
+    }
+    rows.ensure(n_rows);
+  }
+  int few_args(MvmArgs &a, int *counters, float *rows, int call_number, const volatile int *seen_host, int *seen_dev) const {
+    a.few = counters;
+    a.few_seen = seen_dev;
+    a.few_call = call_number;
+    if (a.max_rounds < 3) return 1;
+    a.dual.buf[1] = rows;
+    a.dual.buf[2] = rows + (size_t)a.m_batch * a.O;
+    if (fused_rounds >= 0) return fused_rounds & 1 ? 3 : 1;
+    return seen_host[1] - seen_host[0] <= 8 ? 3 : 1;
+  }
+  bool training_tile() const { return dev.pulsed() || is_transfer(); }
+  // words 0 to 3: the launches of the rounds, 4 and 5: few_args
+  void ensure_seen() {
+    if (seen_host) return;
+    RPU_HIP_CHECK(hipHostMalloc((void **)&seen_host, 6 * sizeof(int), hipHostMallocMapped));
+    for (int i = 0; i < 6; ++i) seen_host[i] = 0; // until the first calls say otherwise
+    RPU_HIP_CHECK(hipHostGetDevicePointer((void **)&seen_dev, seen_host, 0));
   }
 
   // shared driver of forward (transposed = 0) and backward (transposed = 1)
@@ -857,7 +890,18 @@ struct Tile {
     }
 
     prof_begin(s);
-    if (io.perfect) {
+    const bool running = io.p.noise_management == RPU_NM_AVERAGE_ABS_MAX || io.p.noise_management == RPU_NM_AVERAGE_ABS_MAX_SINGLE_VALUE;
+    if (!side && !gather && !running && mvm_few(a, training_tile())) {
+      int together = 1;
+      if (a.max_rounds > 1) {
+        ensure_seen();
+        ensure_few(s_few, few_counters(a), s_dual1, few_rows(a), s);
+        together = few_args(a, s_few.p, s_dual1.p, few_calls++, seen_host + 4, seen_dev + 4);
+      }
+      const MvmArgs *call = &a;
+      launch_mvm_few(a, mvm_few_variant(&call, 1), together, s);
+      prof_mark(s, "mvm_few");
+    } else if (io.perfect) {
       a.round = 0;
       launch_mvm_init(a, s);
       prof_mark(s, "mvm_init");
@@ -881,11 +925,7 @@ struct Tile {
       int fused = 0;      // rounds of the fused launch: 2, or 3 where the recent calls listed samples for round 2
       int merge_from = 0; // > 0: the rounds from this one on run as one launch
       if (!transposed && !w_other && !side && io.p.bound_management != RPU_BM_NONE && fused_rounds != 0) {
-        if (!seen_host) {
-          RPU_HIP_CHECK(hipHostMalloc((void **)&seen_host, 4 * sizeof(int), hipHostMallocMapped));
-          seen_host[0] = seen_host[1] = seen_host[2] = seen_host[3] = 0;
-          RPU_HIP_CHECK(hipHostGetDevicePointer((void **)&seen_dev, seen_host, 0));
-        }
+        ensure_seen();
         a.dual.seen = seen_dev;
         const int needed = *(volatile int *)&seen_host[0], of = *(volatile int *)&seen_host[1];
         const int last_listed = *(volatile int *)&seen_host[2];
@@ -2453,6 +2493,9 @@ struct rpu_group {
   MvmArgs *h_args = nullptr; // pinned staging
   int *h_start = nullptr;
   hipEvent_t copied = nullptr;
+  DevBuf<int> few_counters; // see Tile::few_args
+  DevBuf<float> few_rows;
+  int few_calls = 0;
   // host-visible pairs (any tile listed a sample for round 1, batch), one per kernel variant of the group's last call:
   // the next call runs the rounds after round 0 in one launch where nothing was listed
   int *seen_host = nullptr, *seen_dev = nullptr;
@@ -2487,6 +2530,8 @@ struct rpu_group {
         d_ustart.release();
         d_args.release();
         d_start.release();
+        few_counters.release();
+        few_rows.release();
         for (auto &b : first_rows) b.release();
       } catch (...) {
       }
@@ -2738,7 +2783,15 @@ static int group_mvm(rpu_group_t *group, const float *const *x_dev, const long *
     bool all_big = use_big;
     // per tile: arguments of a plain forward call (row-major x [m_batch][x_size], y [m_batch][d_size])
     std::vector<MvmArgs> args(n);
-    std::vector<int> depth(n), mode(n);
+    std::vector<int> depth(n), mode(n), few(n), few_rounds(n, 1);
+    if (!group->seen_host) {
+      RPU_HIP_CHECK(hipHostMalloc((void **)&group->seen_host, (2 * kSeenPairs + 3) * sizeof(int), hipHostMallocMapped));
+      for (int i = 0; i < 2 * kSeenPairs + 3; ++i) group->seen_host[i] = 0; // until the first calls say otherwise
+      RPU_HIP_CHECK(hipHostGetDevicePointer((void **)&group->seen_dev, group->seen_host, 0));
+      hipDeviceProp_t prop;
+      RPU_HIP_CHECK(hipGetDeviceProperties(&prop, group->device_id));
+      group->cu_count = prop.multiProcessorCount;
+    }
     int rounds = 1;
     bool storage_xd = false;
     for (int i = 0; i < n; ++i) {
@@ -2757,10 +2810,30 @@ static int group_mvm(rpu_group_t *group, const float *const *x_dev, const long *
       a.big_from = big ? -1 : 0;
       if (!big) all_big = false;
       mvm_round_variant(a, depth[i], mode[i]);
+      // (the test hook of the waits is about the other launches; the large-tile kernel takes all of its tiles through the
+      // lists and marks that the init kernel sets up)
+      few[i] = !big && !group->wait_spins_hook && !group->wait_extra_hook && mvm_few(a, t.training_tile()) ? 1 : 0;
       rounds = std::max(rounds, a.max_rounds);
       args[i] = a;
       t.last_stream = s;
       if (!transposed) t.last_forward_batch = m_batch;
+    }
+    {
+      size_t counters = 0, rows = 0;
+      for (int i = 0; i < n; ++i) {
+        counters += few[i] ? Tile::few_counters(args[i]) : 0;
+        rows += few[i] ? Tile::few_rows(args[i]) : 0;
+      }
+      Tile::ensure_few(group->few_counters, counters, group->few_rows, rows, s);
+      ++group->few_calls;
+      counters = rows = 0;
+      for (int i = 0; i < n; ++i) {
+        if (!few[i]) continue;
+        few_rounds[i] = group->tiles[i]->t.few_args(args[i], group->few_counters.p + counters, group->few_rows.p + rows, group->few_calls,
+                                                    group->seen_host + 2 * kSeenPairs + 1, group->seen_dev + 2 * kSeenPairs + 1);
+        counters += Tile::few_counters(args[i]);
+        rows += Tile::few_rows(args[i]);
+      }
     }
     // Tiles that quantize the same input the same way (the column blocks of a layer that was split over several
     // tiles) share the rows of rounds 0 and 1: one of them writes the rows, all of them read them.  Rows of later
@@ -2787,7 +2860,7 @@ static int group_mvm(rpu_group_t *group, const float *const *x_dev, const long *
                                 ((std::isinf(p.out_bound) && std::isinf(q.out_bound)) || p.out_bound == q.out_bound)))));
       };
       std::vector<int> first_of; // first tile of each set
-      std::vector<int> set_of(n, -1), members;
+      std::vector<int> set_of(n, -1), members, readers, writer; // readers: members that run on quantized rows in memory
       for (int i = 0; i < n; ++i) {
         if (!shares(args[i])) continue;
         for (size_t c = 0; c < first_of.size() && set_of[i] < 0; ++c) {
@@ -2797,8 +2870,13 @@ static int group_mvm(rpu_group_t *group, const float *const *x_dev, const long *
           set_of[i] = (int)first_of.size();
           first_of.push_back(i);
           members.push_back(0);
+          readers.push_back(0);
+          writer.push_back(-1);
         }
         ++members[set_of[i]];
+        if (few[i]) continue; // (quantizes the rows for itself, the same way)
+        ++readers[set_of[i]];
+        if (writer[set_of[i]] < 0) writer[set_of[i]] = i;
       }
       if (group->first_rows.size() < 2 * first_of.size()) group->first_rows.resize(2 * first_of.size());
       group->shared_sets = group->shared_tiles = 0;
@@ -2810,25 +2888,38 @@ static int group_mvm(rpu_group_t *group, const float *const *x_dev, const long *
       }
       for (int i = 0; i < n; ++i) {
         const int c = set_of[i];
-        if (c < 0 || members[c] < 2) continue;
+        if (c < 0 || readers[c] < 2 || few[i]) continue;
         MvmArgs &a = args[i];
         DevBuf<float> &r0 = group->first_rows[2 * c], &r1 = group->first_rows[2 * c + 1];
         r0.ensure((size_t)m_batch * a.k_pad);
         if (a.max_rounds > 1) r1.ensure((size_t)m_batch * a.k_pad);
         a.xq_first[0] = r0.p;
         a.xq_first[1] = a.max_rounds > 1 ? r1.p : nullptr;
-        a.xq_first_writer = first_of[c] == i ? 1 : 0;
+        a.xq_first_writer = writer[c] == i ? 1 : 0;
       }
     }
-    // tiles that share a kernel variant sit next to each other
+    // tiles that share a kernel variant sit next to each other, first those that run in one launch (k_mvm_few)
     std::vector<int> order(n);
     for (int i = 0; i < n; ++i) order[i] = i;
-    std::stable_sort(order.begin(), order.end(),
-                     [&](int a, int b) { return depth[a] * 4 + mode[a] < depth[b] * 4 + mode[b]; });
+    std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
+      if (few[a] != few[b]) return few[a] > few[b];
+      return depth[a] * 4 + mode[a] < depth[b] * 4 + mode[b];
+    });
     struct Segment { int first, count, depth, mode, start_offset, workgroups; };
     std::vector<Segment> segments;
     int cursor = 0; // position in h_start
-    for (int i = 0; i < n;) {
+    std::vector<const MvmArgs *> few_calls;
+    while ((int)few_calls.size() < n && few[order[few_calls.size()]]) few_calls.push_back(&args[order[few_calls.size()]]);
+    const int n_few = (int)few_calls.size(), few_variant = mvm_few_variant(few_calls.data(), n_few);
+    int few_workgroups = 0, few_max_k = 0, few_together = 3; // a launch has one form; the buffers of three rounds serve one
+    for (int i = 0; i < n_few; ++i) {
+      group->h_start[cursor++] = few_workgroups;
+      few_workgroups += mvm_few_workgroups(*few_calls[i], few_variant);
+      few_max_k = std::max(few_max_k, few_calls[i]->K);
+      few_together = std::min(few_together, few_rounds[order[i]]);
+    }
+    if (n_few) group->h_start[cursor++] = few_workgroups;
+    for (int i = n_few; i < n;) {
       Segment seg{i, 0, depth[order[i]], mode[order[i]], cursor, 0};
       int wg = 0;
       int j = i;
@@ -2856,18 +2947,22 @@ static int group_mvm(rpu_group_t *group, const float *const *x_dev, const long *
     RPU_HIP_CHECK(hipMemcpyAsync(group->d_start.p, group->h_start, (size_t)cursor * sizeof(int), hipMemcpyHostToDevice, s));
     RPU_HIP_CHECK(hipEventRecord(group->copied, s));
 
-    MvmGroup all{group->d_args.p, nullptr, n, m_batch};
-    int max_k = 0;
-    for (int i = 0; i < n; ++i) max_k = std::max(max_k, args[i].K);
-    launch_mvm_init_group(all, max_k, s);
-    if (!group->seen_host) {
-      RPU_HIP_CHECK(hipHostMalloc((void **)&group->seen_host, (2 * kSeenPairs + 1) * sizeof(int), hipHostMallocMapped));
-      for (int i = 0; i < 2 * kSeenPairs + 1; ++i) group->seen_host[i] = 0;
-      RPU_HIP_CHECK(hipHostGetDevicePointer((void **)&group->seen_dev, group->seen_host, 0));
-      hipDeviceProp_t prop;
-      RPU_HIP_CHECK(hipGetDeviceProperties(&prop, group->device_id));
-      group->cu_count = prop.multiProcessorCount;
+    if (n_few) {
+      MvmGroup g{group->d_args.p, group->d_start.p, n_few, m_batch};
+      launch_mvm_few_group(g, few_variant, few_together, transposed != storage_xd, few_max_k, few_workgroups, s);
     }
+    if (n_few == n) { // nothing was listed for a later launch: what the pairs say of this call
+      for (int k = 0; k < kSeenPairs; ++k) {
+        *(volatile int *)&group->seen_host[2 * k] = 0;
+        *(volatile int *)&group->seen_host[2 * k + 1] = m_batch;
+      }
+      RPU_HIP_CHECK(hipGetLastError());
+      return;
+    }
+    MvmGroup all{group->d_args.p + n_few, nullptr, n - n_few, m_batch};
+    int max_k = 0;
+    for (int i = n_few; i < n; ++i) max_k = std::max(max_k, args[order[i]].K);
+    launch_mvm_init_group(all, max_k, s);
     std::vector<bool> merged(segments.size(), false);
     for (int r = 0; r < rounds; ++r) {
       if (use_big && r == 0) {

@@ -1,0 +1,80 @@
+"""Small batches run noise management, conversion, contraction and all bound-management rounds in one launch (k_mvm_few).
+Exact-arithmetic setting: outputs and round counts equal the oracle's bit for bit, whatever the blocks of the launch."""
+import numpy as np
+import pytest
+import torch
+
+from aihwkit_amd.rpu_base import devices as dv
+from aihwkit_amd.rpu_base import tiles
+from helpers import build_pair, constant_step, make_meta, noise_free_io
+
+pytestmark = pytest.mark.gpu
+F = np.float32
+NM, BM = dv.NoiseManagementType, dv.BoundManagementType
+
+
+def grid(rng, top, shape, unit):
+    return (rng.integers(-top, top + 1, shape) / unit).astype(F)
+
+
+def exact_pair(rng, x_size, d_size, out_bound, w_top, seed=1):
+    f_io = noise_free_io(inp_res=1 / 64.0, out_res=1 / 512.0, noise_management=NM.AbsMax, bound_management=BM.Iterative,
+                         out_bound=out_bound)
+    b_io = noise_free_io(inp_res=1 / 64.0, out_res=1 / 512.0, noise_management=NM.Max)
+    dev = constant_step(w_max_dtod=0.0, w_min_dtod=0.0, w_max=1.0, w_min=-1.0, construction_seed=seed)
+    host, orc, _ = build_pair(make_meta(f_io, b_io), dev, x_size, d_size, gpu=False)
+    w = grid(rng, w_top, (d_size, x_size), 64.0)
+    host.set_weights(torch.from_numpy(w))
+    orc.set_weights(w)
+    return host, orc
+
+
+# x_size, d_size, batch, bias: lengths on both sides of a load (64 inputs), of a block (16, 32, 64 outputs; 1, 2, 4 samples),
+# of eight blocks of outputs, one workgroup for a sample, the longest rows; the last ones take the larger blocks
+@pytest.mark.parametrize("x_size,d_size,batch,bias", [
+    (1, 1, 1, False), (2, 3, 2, True), (63, 15, 3, False), (64, 16, 1, False), (65, 17, 5, True), (130, 128, 1, False),
+    (257, 129, 2, False), (2048, 33, 3, False), (2048, 257, 16, False), (300, 512, 7, True), (200, 65, 101, False),
+    (96, 257, 130, False), (129, 10, 1027, False)])
+def test_small_calls_equal_the_oracle(gpu_device, x_size, d_size, batch, bias):
+    rng = np.random.default_rng(x_size * 1000 + d_size)
+    host, orc = exact_pair(rng, x_size, d_size, 1.0, 16)
+    x = grid(rng, 64, (batch, x_size - int(bias)), 64.0)
+    x *= rng.choice([0.0, 1 / 64.0, 1.0, 1.0], (batch, 1)).astype(F) if batch > 2 else F(1.0)
+    x[:, : x.shape[1] // 2] *= rng.choice([0.0, 1.0], (batch, 1)).astype(F)
+    d = grid(rng, 64, (batch, d_size), 64.0)
+    y_o, g_o = orc.forward(x, bias), orc.backward(d, bias)
+    rounds = orc.bm_rounds(batch)
+    for mode in (0, 1, -1):                          # rounds one by one, rounds 0 to 2 together, by the calls before
+        gpu = tiles.CudaAnalogTile(host)
+        gpu.set_fused_rounds(mode)
+        for _ in range(2):                           # the second call finds the counters and marks of the first
+            gpu.set_profiling(True)
+            y = gpu.forward(torch.from_numpy(x).cuda(), bias).cpu().numpy()
+            assert [name for name, _ms in gpu.get_profile()][1:] == ["mvm_few"]
+            gpu.set_profiling(False)
+            assert np.array_equal(y, y_o)
+            assert np.array_equal(gpu.get_bm_rounds(batch).numpy(), rounds)
+            assert np.array_equal(gpu.backward(torch.from_numpy(d).cuda(), bias).cpu().numpy(), g_o)
+
+
+# batch, shapes: small calls next to others that share their input's quantized rows; next to tiles of the large-tile kernel
+@pytest.mark.parametrize("batch,shapes", [
+    (128, [(257, 16), (257, 512), (257, 33), (257, 600), (64, 16)]),
+    (1024, [(40, 130)] * 8 + [(64, 256)] * 2 + [(64, 40), (64, 30), (33, 20)]),
+    (5, [(130, 16), (130, 200), (2048, 40), (1, 1)])])
+def test_groups_with_small_calls_equal_the_oracle(gpu_device, batch, shapes):
+    rng = np.random.default_rng(batch)
+    pairs = [exact_pair(rng, x, d, 2.0, 32, seed=k + 1) for k, (x, d) in enumerate(shapes)]
+    grouped = [tiles.CudaAnalogTile(host) for host, _ in pairs]
+    group = tiles.TileGroup(grouped)
+    by_size = {x: grid(rng, 64, (batch, x), 64.0) for x, _ in shapes}
+    ds = [grid(rng, 64, (batch, d), 64.0) for _, d in shapes]
+    x_dev = {n: torch.from_numpy(x).cuda() for n, x in by_size.items()}
+    for _ in range(2):
+        got = group.forward([x_dev[x] for x, _ in shapes])
+        rounds = [t.get_bm_rounds(batch).numpy().copy() for t in grouped]
+        back = group.backward([torch.from_numpy(d).cuda() for d in ds])
+        for (x, _), (_, orc), r, y, d, g in zip(shapes, pairs, rounds, got, ds, back):
+            assert np.array_equal(y.cpu().numpy(), orc.forward(by_size[x]))
+            assert np.array_equal(r, orc.bm_rounds(batch))
+            assert np.array_equal(g.cpu().numpy(), orc.backward(d))
