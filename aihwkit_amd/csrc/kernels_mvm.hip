@@ -3401,7 +3401,7 @@ void launch_mvm_round(const MvmArgs &a_in, hipStream_t s) {
 #undef RPU_LAUNCH_ROUND
 }
 
-// Whether a call runs as k_mvm_few: a function of the tile, its IO settings and the batch, so that a tile takes the same sums
+// The largest batch whose calls run as k_mvm_few: a function of the tile and its IO settings, so that a tile takes the same sums
 // on its own and in a group (whose workgroups read every weight once per block of samples, all tiles at a time: that, and not
 // the single call, sets the limits).  us, the other launches / one:
 //   forward, weights that saturate round 0: 512 x 512, 1 sample 27.5 / 13.3, 32 27 / 19, 100 (26 M multiply-adds) 27 / 27, 200
@@ -3410,15 +3410,15 @@ void launch_mvm_round(const MvmArgs &a_in, hipStream_t s) {
 //   layers of tiles of at most 512 x 512: 768 -> 2304, 8 tokens 27.3 / 25.3, 16 (2.8 M a tile) 27.1 / 26.0, 32 28 / 37;
 //   3072 x 3072, 8 tokens (2.1 M) 54 / 53, 16 56 / 68
 // Inference tiles come in such groups, training tiles mostly do not.
-bool mvm_few(const MvmArgs &a, bool training_tile) {
+int mvm_few_batch(const MvmArgs &a, bool training_tile) {
   const IoDev &io = a.io;
   const int nm = io.noise_management;
-  if (io.perfect || a.in_index || a.pre_add || a.skip_if_zero || a.nm_phase || a.small_tiles_only || a.K > 2048 || a.K <= a.in_one) return false;
-  if (nm != RPU_NM_NONE && nm != RPU_NM_CONSTANT && nm != RPU_NM_ABS_MAX && nm != RPU_NM_MAX) return false;
-  if (io.bound_management != RPU_BM_NONE && (io.bound_management != RPU_BM_ITERATIVE || a.transposed)) return false;
+  if (io.perfect || a.in_index || a.pre_add || a.skip_if_zero || a.nm_phase || a.small_tiles_only || a.K > 2048 || a.K <= a.in_one) return 0;
+  if (nm != RPU_NM_NONE && nm != RPU_NM_CONSTANT && nm != RPU_NM_ABS_MAX && nm != RPU_NM_MAX) return 0;
+  if (io.bound_management != RPU_BM_NONE && (io.bound_management != RPU_BM_ITERATIVE || a.transposed)) return 0;
   const long per_cu = !training_tile ? 12288 : (a.max_rounds > 1 ? 51200 : 102400); // multiply-adds
   // (a sample takes a load of 64 inputs by 16 outputs at least: a long batch on a tiny tile is not a small call)
-  return (long)((a.K + 63) & ~63) * ((a.O + 15) & ~15) * a.m_batch <= per_cu * current_device_cus();
+  return (int)(per_cu * current_device_cus() / ((long)((a.K + 63) & ~63) * ((a.O + 15) & ~15)));
 }
 // the variant of a launch of such calls: the smallest blocks of samples and outputs with at most two workgroups to a CU
 int mvm_few_variant(const MvmArgs *const *calls, int n) {

@@ -588,12 +588,14 @@ struct Tile {
     return true;
   }
 
-  // What a call of k_mvm_few needs beyond mvm_args: few_counters(a) counters and saturation marks, zero between calls, and
-  // few_rows(a) floats for the results of rounds 1 and 2 (whether or not this call works on three rounds at once: the next
-  // one may, and be captured).  `seen`: host-visible numbers of the last call (of this tile or group) in which a sample went
-  // on to a second round and of the last call that has ended.  Returns the rounds to work out together (launch_mvm_few).
-  static size_t few_counters(const MvmArgs &a) { return a.max_rounds > 1 ? 7 * (size_t)a.m_batch : 0; }
-  static size_t few_rows(const MvmArgs &a) { return a.max_rounds > 2 ? 2 * (size_t)a.m_batch * a.O : 0; }
+  // What a call of k_mvm_few needs beyond mvm_args: few_counters() counters and saturation marks, zero between calls, and
+  // few_rows() floats for the results of rounds 1 and 2 (whether or not this call works on three rounds at once: the next
+  // one may, and be captured).  A larger call on the other launches makes room for its largest small call as well, so that a
+  // program that warmed up on it can capture any smaller one; `batch` is that of the small call.  `seen`: host-visible
+  // numbers of the last call (of this tile or group) in which a sample went on to a second round and of the last call that
+  // has ended.  Returns the rounds to work out together (launch_mvm_few).
+  static size_t few_counters(const MvmArgs &a, int batch) { return a.max_rounds > 1 ? 7 * (size_t)batch : 0; }
+  static size_t few_rows(const MvmArgs &a, int batch) { return a.max_rounds > 2 ? 2 * (size_t)batch * a.O : 0; }
   static void ensure_few(DevBuf<int> &counters, size_t n_counters, DevBuf<float> &rows, size_t n_rows, hipStream_t s) {
     if (counters.n < n_counters) {
       counters.ensure(n_counters);
@@ -891,11 +893,14 @@ struct Tile {
 
     prof_begin(s);
     const bool running = io.p.noise_management == RPU_NM_AVERAGE_ABS_MAX || io.p.noise_management == RPU_NM_AVERAGE_ABS_MAX_SINGLE_VALUE;
-    if (!side && !gather && !running && mvm_few(a, training_tile())) {
+    const int few_batch = side || gather || running ? 0 : std::min(B, mvm_few_batch(a, training_tile()));
+    if (few_batch > 0 && a.max_rounds > 1) {
+      ensure_seen();
+      ensure_few(s_few, few_counters(a, few_batch), s_dual1, few_rows(a, few_batch), s);
+    }
+    if (few_batch == B) {
       int together = 1;
       if (a.max_rounds > 1) {
-        ensure_seen();
-        ensure_few(s_few, few_counters(a), s_dual1, few_rows(a), s);
         together = few_args(a, s_few.p, s_dual1.p, few_calls++, seen_host + 4, seen_dev + 4);
       }
       const MvmArgs *call = &a;
@@ -2783,7 +2788,7 @@ static int group_mvm(rpu_group_t *group, const float *const *x_dev, const long *
     bool all_big = use_big;
     // per tile: arguments of a plain forward call (row-major x [m_batch][x_size], y [m_batch][d_size])
     std::vector<MvmArgs> args(n);
-    std::vector<int> depth(n), mode(n), few(n), few_rounds(n, 1);
+    std::vector<int> depth(n), mode(n), few(n), few_batch(n), few_rounds(n, 1);
     if (!group->seen_host) {
       RPU_HIP_CHECK(hipHostMalloc((void **)&group->seen_host, (2 * kSeenPairs + 3) * sizeof(int), hipHostMallocMapped));
       for (int i = 0; i < 2 * kSeenPairs + 3; ++i) group->seen_host[i] = 0; // until the first calls say otherwise
@@ -2812,7 +2817,8 @@ static int group_mvm(rpu_group_t *group, const float *const *x_dev, const long *
       mvm_round_variant(a, depth[i], mode[i]);
       // (the test hook of the waits is about the other launches; the large-tile kernel takes all of its tiles through the
       // lists and marks that the init kernel sets up)
-      few[i] = !big && !group->wait_spins_hook && !group->wait_extra_hook && mvm_few(a, t.training_tile()) ? 1 : 0;
+      few_batch[i] = std::min(m_batch, mvm_few_batch(a, t.training_tile()));
+      few[i] = !big && !group->wait_spins_hook && !group->wait_extra_hook && few_batch[i] == m_batch ? 1 : 0;
       rounds = std::max(rounds, a.max_rounds);
       args[i] = a;
       t.last_stream = s;
@@ -2821,8 +2827,8 @@ static int group_mvm(rpu_group_t *group, const float *const *x_dev, const long *
     {
       size_t counters = 0, rows = 0;
       for (int i = 0; i < n; ++i) {
-        counters += few[i] ? Tile::few_counters(args[i]) : 0;
-        rows += few[i] ? Tile::few_rows(args[i]) : 0;
+        counters += Tile::few_counters(args[i], few_batch[i]);
+        rows += Tile::few_rows(args[i], few_batch[i]);
       }
       Tile::ensure_few(group->few_counters, counters, group->few_rows, rows, s);
       ++group->few_calls;
@@ -2831,8 +2837,8 @@ static int group_mvm(rpu_group_t *group, const float *const *x_dev, const long *
         if (!few[i]) continue;
         few_rounds[i] = group->tiles[i]->t.few_args(args[i], group->few_counters.p + counters, group->few_rows.p + rows, group->few_calls,
                                                     group->seen_host + 2 * kSeenPairs + 1, group->seen_dev + 2 * kSeenPairs + 1);
-        counters += Tile::few_counters(args[i]);
-        rows += Tile::few_rows(args[i]);
+        counters += Tile::few_counters(args[i], m_batch);
+        rows += Tile::few_rows(args[i], m_batch);
       }
     }
     // Tiles that quantize the same input the same way (the column blocks of a layer that was split over several
