@@ -495,6 +495,7 @@ void launch_lines_to_images(float *images, const float *lines_major, int n_image
 // [n][d][p] -> [(n, p)][d]
 void launch_ndp_to_bd(float *bd, const float *ndp, int n_images, int d_size, int patches, hipStream_t s);
 void launch_fill(float *p, float value, size_t n, hipStream_t s);
+void launch_upload(void *dst, const void *pinned, size_t words, hipStream_t s); // words of eight bytes
 
 // n_vec unit vectors of length `size`: row v is e_((start + v) % size)
 void launch_unit_vectors(float *out, int n_vec, int size, int start, hipStream_t s);

@@ -205,6 +205,13 @@ __global__ void k_fill(float *p, float value, size_t n) {
   for (size_t idx = blockIdx.x * (size_t)blockDim.x + threadIdx.x; idx < n; idx += (size_t)gridDim.x * blockDim.x) p[idx] = value;
 }
 
+// Arguments of a grouped call from pinned host memory: words the host may rewrite for the next call, so every load goes
+// to the host (no cache of the GPU keeps them).
+__global__ __launch_bounds__(256) void k_upload(unsigned long long *dst, const unsigned long long *src, unsigned n) {
+  const unsigned i = blockIdx.x * 256u + threadIdx.x;
+  if (i < n) dst[i] = __hip_atomic_load(src + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 int grid_of(size_t n) {
   size_t blocks = (n + 255) / 256;
   if (blocks > 4096) blocks = 4096;
@@ -311,6 +318,11 @@ void launch_ndp_to_bd(float *bd, const float *ndp, int n_images, int d_size, int
 
 void launch_fill(float *p, float value, size_t n, hipStream_t s) {
   hipLaunchKernelGGL(k_fill, dim3(grid_of(n)), dim3(256), 0, s, p, value, n);
+}
+
+void launch_upload(void *dst, const void *pinned, size_t words, hipStream_t s) {
+  hipLaunchKernelGGL(k_upload, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, s, (unsigned long long *)dst,
+                     (const unsigned long long *)pinned, (unsigned)words);
 }
 
 void launch_mean_abs(const float *v, size_t n, float *out, hipStream_t s) {

@@ -75,6 +75,32 @@ template <typename T> struct DevBuf {
   }
 };
 
+// What a grouped call's kernels read: workgroup tables and the tiles' argument blocks, put together in pinned memory and
+// uploaded by one launch.  Two hipMemcpyAsync are two launches of 3.8 us each with 2 to 3 us of host time more.
+template <class A> struct GroupArgs {
+  DevBuf<unsigned long long> dev;
+  char *host = nullptr, *host_on_dev = nullptr;
+  size_t table_words = 0; // of eight bytes, before the argument blocks
+  static_assert(sizeof(A) % 8 == 0 && alignof(A) <= 16, "argument blocks are uploaded in words of eight bytes");
+  void make(size_t n_args, size_t n_table) {
+    table_words = (n_table + 3) / 4 * 2;
+    const size_t words = table_words + n_args * (sizeof(A) / 8);
+    dev.ensure(words);
+    RPU_HIP_CHECK(hipHostMalloc((void **)&host, 8 * words, hipHostMallocMapped));
+    RPU_HIP_CHECK(hipHostGetDevicePointer((void **)&host_on_dev, host, 0));
+  }
+  int *table() { return reinterpret_cast<int *>(host); }
+  A *args() { return reinterpret_cast<A *>(host + 8 * table_words); }
+  const int *dev_table() const { return reinterpret_cast<const int *>(dev.p); }
+  const A *dev_args() const { return reinterpret_cast<const A *>(dev.p + table_words); }
+  void upload(size_t n_args, hipStream_t s) { launch_upload(dev.p, host_on_dev, table_words + n_args * (sizeof(A) / 8), s); }
+  void release() {
+    if (host) (void)hipHostFree(host);
+    host = nullptr;
+    dev.release();
+  }
+};
+
 class DeviceGuard {
 public:
   explicit DeviceGuard(int device) {
@@ -2493,10 +2519,7 @@ int rpu_tile_set_extra(rpu_tile_t *tile, const int64_t *values_host, int count) 
 struct rpu_group {
   std::vector<rpu_tile *> tiles;
   int device_id = -1;
-  DevBuf<MvmArgs> d_args;
-  DevBuf<int> d_start;
-  MvmArgs *h_args = nullptr; // pinned staging
-  int *h_start = nullptr;
+  GroupArgs<MvmArgs> mvm_args;
   hipEvent_t copied = nullptr;
   DevBuf<int> few_counters; // see Tile::few_args
   DevBuf<float> few_rows;
@@ -2513,10 +2536,7 @@ struct rpu_group {
   std::vector<DevBuf<float>> first_rows;
   int shared_sets = 0, shared_tiles = 0; // of the last call
   // grouped update: the tiles' argument blocks and the workgroup tables of its launches
-  DevBuf<UpdateArgs> d_uargs;
-  DevBuf<int> d_ustart;
-  UpdateArgs *h_uargs = nullptr; // pinned staging
-  int *h_ustart = nullptr;
+  GroupArgs<UpdateArgs> update_args;
   std::mutex mutex;
   ~rpu_group() {
     if (device_id >= 0) {
@@ -2526,15 +2546,9 @@ struct rpu_group {
           (void)hipEventSynchronize(copied);
           (void)hipEventDestroy(copied);
         }
-        if (h_args) (void)hipHostFree(h_args);
-        if (h_start) (void)hipHostFree(h_start);
         if (seen_host) (void)hipHostFree(seen_host);
-        if (h_uargs) (void)hipHostFree(h_uargs);
-        if (h_ustart) (void)hipHostFree(h_ustart);
-        d_uargs.release();
-        d_ustart.release();
-        d_args.release();
-        d_start.release();
+        update_args.release();
+        mvm_args.release();
         few_counters.release();
         few_rows.release();
         for (auto &b : first_rows) b.release();
@@ -2562,10 +2576,7 @@ int rpu_group_create(rpu_group_t **out, rpu_tile_t *const *tiles, int n_tiles) {
     }
     DeviceGuard dg(g->device_id);
     const size_t n = (size_t)n_tiles;
-    g->d_args.ensure(n);
-    g->d_start.ensure(3 * n + 4);
-    RPU_HIP_CHECK(hipHostMalloc((void **)&g->h_args, n * sizeof(MvmArgs), hipHostMallocDefault));
-    RPU_HIP_CHECK(hipHostMalloc((void **)&g->h_start, (3 * n + 4) * sizeof(int), hipHostMallocDefault));
+    g->mvm_args.make(n, 3 * n + 4);
     RPU_HIP_CHECK(hipEventCreateWithFlags(&g->copied, hipEventDisableTiming));
     *out = g.release();
   });
@@ -2583,15 +2594,12 @@ int rpu_group_update_strided(rpu_group_t *group, const float *const *x_dev, cons
     DeviceGuard dg(group->device_id);
     hipStream_t s = (hipStream_t)stream;
     const int n = (int)group->tiles.size();
-    if (!group->h_uargs) {
+    if (!group->update_args.host) {
       // per tile the arguments of the kernels that make the lines and, after those of all tiles, the view that the
       // cross-point kernels take (the same, or with x and d exchanged for a tile that stores [x_size][d_size])
-      group->d_uargs.ensure(2 * (size_t)n);
-      group->d_ustart.ensure(2 * (size_t)n + 16);
-      RPU_HIP_CHECK(hipHostMalloc((void **)&group->h_uargs, 2 * (size_t)n * sizeof(UpdateArgs), hipHostMallocDefault));
-      RPU_HIP_CHECK(hipHostMalloc((void **)&group->h_ustart, (2 * (size_t)n + 16) * sizeof(int), hipHostMallocDefault));
+      group->update_args.make(2 * (size_t)n, 2 * (size_t)n + 16);
     }
-    // the staging buffers may still feed the copy of the previous call
+    // the pinned memory may still feed the upload of the previous call
     RPU_HIP_CHECK(hipEventSynchronize(group->copied));
     ensure_update_tables();
 
@@ -2635,41 +2643,41 @@ int rpu_group_update_strided(rpu_group_t *group, const float *const *x_dev, cons
     long lines_blocks_16 = 0;
     for (int i = 0; i < m; ++i) lines_blocks_16 += update_lines_blocks(args[i], true);
     const bool wide_lines = lines_blocks_16 * ((m_batch + 63) / 64) >= 256;
+    int *const table = group->update_args.table();
     int cursor = 0, blocks = 0;
     const int lines_offset = cursor;
     for (int i = 0; i < m; ++i) {
-      group->h_ustart[cursor++] = blocks;
+      table[cursor++] = blocks;
       blocks += update_lines_blocks(args[order[i]], wide_lines);
     }
-    group->h_ustart[cursor++] = blocks;
+    table[cursor++] = blocks;
     struct Segment { int first, count, variant, start_offset, workgroups; };
     std::vector<Segment> segments;
     for (int i = 0; i < m;) {
       Segment seg{i, 0, variant[order[i]], cursor, 0};
       int wg = 0, j = i;
       for (; j < m && variant[order[j]] == seg.variant; ++j) {
-        group->h_ustart[cursor++] = wg;
+        table[cursor++] = wg;
         wg += update_pulsed_workgroups(views[order[j]]);
       }
-      group->h_ustart[cursor++] = wg;
+      table[cursor++] = wg;
       seg.count = j - i;
       seg.workgroups = wg;
       segments.push_back(seg);
       i = j;
     }
     for (int i = 0; i < m; ++i) {
-      group->h_uargs[i] = args[order[i]];
-      group->h_uargs[m + i] = views[order[i]];
+      group->update_args.args()[i] = args[order[i]];
+      group->update_args.args()[m + i] = views[order[i]];
     }
-    RPU_HIP_CHECK(hipMemcpyAsync(group->d_uargs.p, group->h_uargs, 2 * (size_t)m * sizeof(UpdateArgs), hipMemcpyHostToDevice, s));
-    RPU_HIP_CHECK(hipMemcpyAsync(group->d_ustart.p, group->h_ustart, (size_t)cursor * sizeof(int), hipMemcpyHostToDevice, s));
+    group->update_args.upload(2 * (size_t)m, s);
     RPU_HIP_CHECK(hipEventRecord(group->copied, s));
 
-    UpdateGroup all{group->d_uargs.p, group->d_ustart.p + lines_offset, m, m_batch};
+    UpdateGroup all{group->update_args.dev_args(), group->update_args.dev_table() + lines_offset, m, m_batch};
     launch_update_prepare_group(all, s);
     launch_update_lines_group(all, wide_lines, blocks, s);
     for (const Segment &seg : segments) {
-      UpdateGroup g{group->d_uargs.p + m + seg.first, group->d_ustart.p + seg.start_offset, seg.count, m_batch};
+      UpdateGroup g{group->update_args.dev_args() + m + seg.first, group->update_args.dev_table() + seg.start_offset, seg.count, m_batch};
       launch_update_pulsed_group(g, seg.variant, seg.workgroups, s);
     }
     RPU_HIP_CHECK(hipGetLastError());
@@ -2757,7 +2765,7 @@ static int group_mvm(rpu_group_t *group, const float *const *x_dev, const long *
         return;
       }
     }
-    // the staging buffers may still feed the copy of the previous call
+    // the pinned memory may still feed the upload of the previous call
     RPU_HIP_CHECK(hipEventSynchronize(group->copied));
 
     // a batch of 1024 or more on tiles at least 128 outputs wide: the large-tile kernel runs round 0 of those tiles,
@@ -2913,48 +2921,48 @@ static int group_mvm(rpu_group_t *group, const float *const *x_dev, const long *
     });
     struct Segment { int first, count, depth, mode, start_offset, workgroups; };
     std::vector<Segment> segments;
-    int cursor = 0; // position in h_start
+    int *const table = group->mvm_args.table();
+    int cursor = 0; // position in the table
     std::vector<const MvmArgs *> few_calls;
     while ((int)few_calls.size() < n && few[order[few_calls.size()]]) few_calls.push_back(&args[order[few_calls.size()]]);
     const int n_few = (int)few_calls.size(), few_variant = mvm_few_variant(few_calls.data(), n_few);
     int few_workgroups = 0, few_max_k = 0, few_together = 3; // a launch has one form; the buffers of three rounds serve one
     for (int i = 0; i < n_few; ++i) {
-      group->h_start[cursor++] = few_workgroups;
+      table[cursor++] = few_workgroups;
       few_workgroups += mvm_few_workgroups(*few_calls[i], few_variant);
       few_max_k = std::max(few_max_k, few_calls[i]->K);
       few_together = std::min(few_together, few_rounds[order[i]]);
     }
-    if (n_few) group->h_start[cursor++] = few_workgroups;
+    if (n_few) table[cursor++] = few_workgroups;
     for (int i = n_few; i < n;) {
       Segment seg{i, 0, depth[order[i]], mode[order[i]], cursor, 0};
       int wg = 0;
       int j = i;
       for (; j < n && depth[order[j]] == seg.depth && mode[order[j]] == seg.mode; ++j) {
-        group->h_start[cursor++] = wg;
+        table[cursor++] = wg;
         wg += mvm_round_workgroups(args[order[j]]);
       }
-      group->h_start[cursor++] = wg;
+      table[cursor++] = wg;
       seg.count = j - i;
       seg.workgroups = wg;
       segments.push_back(seg);
       i = j;
     }
-    const int big_offset = cursor; // table of the large-tile launch over all tiles, in the order of d_args
+    const int big_offset = cursor; // table of the large-tile launch over all tiles, in the order of the arguments
     if (use_big) {
       int wg = 0;
       for (int i = 0; i < n; ++i) {
-        group->h_start[cursor++] = wg;
+        table[cursor++] = wg;
         if (args[order[i]].big_from != 0) wg += mvm_big_workgroups(args[order[i]], big_bb);
       }
-      group->h_start[cursor++] = wg;
+      table[cursor++] = wg;
     }
-    for (int i = 0; i < n; ++i) group->h_args[i] = args[order[i]];
-    RPU_HIP_CHECK(hipMemcpyAsync(group->d_args.p, group->h_args, (size_t)n * sizeof(MvmArgs), hipMemcpyHostToDevice, s));
-    RPU_HIP_CHECK(hipMemcpyAsync(group->d_start.p, group->h_start, (size_t)cursor * sizeof(int), hipMemcpyHostToDevice, s));
+    for (int i = 0; i < n; ++i) group->mvm_args.args()[i] = args[order[i]];
+    group->mvm_args.upload((size_t)n, s);
     RPU_HIP_CHECK(hipEventRecord(group->copied, s));
 
     if (n_few) {
-      MvmGroup g{group->d_args.p, group->d_start.p, n_few, m_batch};
+      MvmGroup g{group->mvm_args.dev_args(), group->mvm_args.dev_table(), n_few, m_batch};
       launch_mvm_few_group(g, few_variant, few_together, transposed != storage_xd, few_max_k, few_workgroups, s);
     }
     if (n_few == n) { // nothing was listed for a later launch: what the pairs say of this call
@@ -2965,21 +2973,21 @@ static int group_mvm(rpu_group_t *group, const float *const *x_dev, const long *
       RPU_HIP_CHECK(hipGetLastError());
       return;
     }
-    MvmGroup all{group->d_args.p + n_few, nullptr, n - n_few, m_batch};
+    MvmGroup all{group->mvm_args.dev_args() + n_few, nullptr, n - n_few, m_batch};
     int max_k = 0;
     for (int i = n_few; i < n; ++i) max_k = std::max(max_k, args[order[i]].K);
     launch_mvm_init_group(all, max_k, s);
     std::vector<bool> merged(segments.size(), false);
     for (int r = 0; r < rounds; ++r) {
       if (use_big && r == 0) {
-        MvmGroup g{group->d_args.p, group->d_start.p + big_offset, n, m_batch};
+        MvmGroup g{group->mvm_args.dev_args(), group->mvm_args.dev_table() + big_offset, n, m_batch};
         launch_mvm_big_group(g, big_total, big_bb, transposed != storage_xd, all_stepped, s);
         if (all_big) continue;
       }
       for (size_t k = 0; k < segments.size(); ++k) {
         const Segment &seg = segments[k];
         if (merged[k]) continue;
-        MvmGroup g{group->d_args.p + seg.first, group->d_start.p + seg.start_offset, seg.count, m_batch};
+        MvmGroup g{group->mvm_args.dev_args() + seg.first, group->mvm_args.dev_table() + seg.start_offset, seg.count, m_batch};
         int *seen = k < (size_t)kSeenPairs ? group->seen_dev + 2 * k : nullptr;
         // the last call of this group listed nothing for round 1: one launch for all rounds after round 0
         const int rest_wgs = (r == 1 && rounds >= 3) ? std::min(256, mvm_group_rest_resident_limit(seg.mode)) : 0;
