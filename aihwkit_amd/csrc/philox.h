@@ -136,16 +136,18 @@ enum RngPurpose : uint32_t {
 RPU_HD float u32_to_uniform(uint32_t r) { return (float)(r >> 8) * (1.0f / 16777216.0f); }
 
 #if defined(__HIPCC__)
-// Box-Muller on two 32-bit words: two independent N(0,1).
+// Box-Muller on two 32-bit words: two independent N(0,1).  The hardware's logarithm is that to base 2 and its sine takes
+// turns, so the factors 2 ln 2 and 2 pi cost no rounding of their own; the square root is the hardware's (1 ulp).  Error
+// against 64 bits over 2^24 pairs, root mean square / largest: 6.1e-8 / 8.8e-7; with a correctly rounded root of -2 ln u
+// and an angle in radians 1.3e-7 / 2.2e-6, and some thirty instructions more in an ADC stage of four outputs (131072 x 48
+// outputs of 433 terms: 156 -> 139 us; 256-sample step of a 1024 x 1024 tile 116.4 -> 113.5).
 __device__ __forceinline__ void box_muller(uint32_t r0, uint32_t r1, float &n0, float &n1) {
   // u in (0, 1]: never log(0)
   const float u = ((float)(r0 >> 8) + 1.0f) * (1.0f / 16777216.0f);
   const float t = (float)(r1 >> 8) * (1.0f / 16777216.0f); // turns
-  const float rad = __fsqrt_rn(-2.0f * __logf(u));
-  float s, c;
-  __sincosf(6.283185307179586f * t, &s, &c);
-  n0 = rad * c;
-  n1 = rad * s;
+  const float rad = __builtin_amdgcn_sqrtf(-1.3862943611198906f * __builtin_amdgcn_logf(u)); // -2 ln u
+  n0 = rad * __builtin_amdgcn_cosf(t);
+  n1 = rad * __builtin_amdgcn_sinf(t);
 }
 
 // Box-Muller on one 32-bit word: radius from the high 16 bits (mid-point rule, so the discrete
