@@ -58,11 +58,12 @@ def test_small_calls_equal_the_oracle(gpu_device, x_size, d_size, batch, bias):
             assert np.array_equal(gpu.backward(torch.from_numpy(d).cuda(), bias).cpu().numpy(), g_o)
 
 
-# batch, shapes: small calls next to others that share their input's quantized rows; next to tiles of the large-tile kernel
+# batch, shapes: small calls next to others that share their input's quantized rows; next to tiles of the large-tile kernel;
+# the largest blocks with the longest rows, which take the most LDS
 @pytest.mark.parametrize("batch,shapes", [
     (128, [(257, 16), (257, 512), (257, 33), (257, 600), (64, 16)]),
     (1024, [(40, 130)] * 8 + [(64, 256)] * 2 + [(64, 40), (64, 30), (33, 20)]),
-    (5, [(130, 16), (130, 200), (2048, 40), (1, 1)])])
+    (5, [(130, 16), (130, 200), (2048, 40), (1, 1)]), (16, [(2048, 300)] * 13)])
 def test_groups_with_small_calls_equal_the_oracle(gpu_device, batch, shapes):
     rng = np.random.default_rng(batch)
     pairs = [exact_pair(rng, x, d, 2.0, 32, seed=k + 1) for k, (x, d) in enumerate(shapes)]
