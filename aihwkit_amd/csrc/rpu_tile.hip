@@ -640,6 +640,14 @@ struct Tile {
     return seen_host[1] - seen_host[0] <= 8 ? 3 : 1;
   }
   bool training_tile() const { return dev.pulsed() || is_transfer(); }
+  // Whether the outputs of a call lie among the inputs of one: the workgroups of k_mvm_few read their inputs while others
+  // store outputs; the other launches have quantized the inputs of round 0 before the first output is stored.
+  static bool writes_into(const MvmArgs &from, const MvmArgs &to) {
+    const long in_last = (long)(to.m_batch - 1) * to.in_sb + (long)(to.K - to.in_one - 1) * to.in_sk;
+    const long out_last = (long)(from.m_batch - 1) * from.out_sb + (long)(from.O - from.out_drop - 1) * from.out_so;
+    const uintptr_t in = (uintptr_t)to.in, out = (uintptr_t)from.out;
+    return out <= in + sizeof(float) * in_last && in <= out + sizeof(float) * out_last;
+  }
   // words 0 to 3: the launches of the rounds, 4 and 5: few_args
   void ensure_seen() {
     if (seen_host) return;
@@ -924,7 +932,7 @@ struct Tile {
       ensure_seen();
       ensure_few(s_few, few_counters(a, few_batch), s_dual1, few_rows(a, few_batch), s);
     }
-    if (few_batch == B) {
+    if (few_batch == B && !writes_into(a, a)) {
       int together = 1;
       if (a.max_rounds > 1) {
         together = few_args(a, s_few.p, s_dual1.p, few_calls++, seen_host + 4, seen_dev + 4);
@@ -2831,6 +2839,11 @@ static int group_mvm(rpu_group_t *group, const float *const *x_dev, const long *
       args[i] = a;
       t.last_stream = s;
       if (!transposed) t.last_forward_batch = m_batch;
+    }
+    for (int i = 0; i < n * n; ++i) {
+      if (!Tile::writes_into(args[i / n], args[i % n])) continue;
+      few.assign(n, 0);
+      break;
     }
     {
       size_t counters = 0, rows = 0;

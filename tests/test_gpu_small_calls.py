@@ -1,5 +1,7 @@
 """Small batches run noise management, conversion, contraction and all bound-management rounds in one launch (k_mvm_few).
 Exact-arithmetic setting: outputs and round counts equal the oracle's bit for bit, whatever the blocks of the launch."""
+import ctypes as C
+
 import numpy as np
 import pytest
 import torch
@@ -101,3 +103,24 @@ def test_small_calls_after_larger_ones_allocate_nothing(gpu_device, grouped):
         x = grid(rng, 64, (batch, 300), 64.0)
         assert np.array_equal(forward(torch.from_numpy(x).cuda()).cpu().numpy(), orc.forward(x))
     assert lib().rpu_device_allocation_count() == before
+
+
+# outputs that lie over the inputs of the call (of another tile of the group): the inputs are read before anything is stored
+@pytest.mark.parametrize("size,batch", [(200, 7), (64, 3)])
+def test_small_calls_onto_their_own_input_equal_the_oracle(gpu_device, size, batch):
+    rng = np.random.default_rng(size)
+    host, orc = exact_pair(rng, size, size, 8.0, 16)
+    gpu, other = tiles.CudaAnalogTile(host), tiles.CudaAnalogTile(host)
+    x = grid(rng, 64, (batch, size), 64.0)
+    want = orc.forward(x)
+    assert np.any(want) and orc.bm_rounds(batch).max() == 1   # a second round reads the inputs again
+    buf = torch.from_numpy(x).cuda()
+    stream = torch.cuda.current_stream().cuda_stream
+    assert lib().rpu_tile_forward(gpu._h, buf.data_ptr(), buf.data_ptr(), batch, 0, 0, 0, 0, stream) == 0
+    assert np.array_equal(buf.cpu().numpy(), want)
+    first, second = torch.from_numpy(x).cuda(), torch.from_numpy(x).cuda()
+    group = tiles.TileGroup([gpu, other])
+    ins = (C.c_void_p * 2)(first.data_ptr(), second.data_ptr())
+    outs = (C.c_void_p * 2)(second.data_ptr(), first.data_ptr())
+    assert lib().rpu_group_forward(group._g, ins, outs, batch, 0, stream) == 0
+    assert np.array_equal(first.cpu().numpy(), want) and np.array_equal(second.cpu().numpy(), want)
