@@ -35,12 +35,12 @@ SPLIT_MFMA_PEAK_TFLOPS = 2500.0 / 3  # dense bf16 matrix, three products per ele
 # FETCH_SIZE / WRITE_SIZE are KiB per dispatch; a device copy of 64 MiB in the same runs reads FETCH_SIZE = 32782 and
 # WRITE_SIZE = 65536, so FETCH_SIZE is scaled by 2.0 and WRITE_SIZE by 1.0.
 PMC_TRAFFIC_BYTES = {
-    "k_update_pulsed": (15063 * 2.0 + 4096 * 1.0) * 1024,
+    "k_update_pulsed": (16615 * 2.0 + 4096 * 1.0) * 1024,  # k_update_pulsed_masks
     "k_mvm_round": (6851 * 2.0 + 2115 * 1.0) * 1024,  # a round over all 256 samples
     # the launches of a forward call whose rounds 0 to 2 share one launch: k_mvm_dual<0, 3>, then k_mvm_rounds_rest
     "forward_fused_3": ((14557 + 586) * 2.0 + (3157 + 1024) * 1.0) * 1024,
 }
-PMC_SOURCE = {"k_update_pulsed": "profiles/k_update_pulsed_config2.txt", "k_mvm_round": "profiles/k_mvm_round_config2.txt",
+PMC_SOURCE = {"k_update_pulsed": "profiles/k_update_pulsed_masks_config2.txt", "k_mvm_round": "profiles/k_mvm_round_config2.txt",
               "forward_fused_3": "profiles/k_mvm_dual_config2.txt"}
 
 
