@@ -240,6 +240,13 @@ def main() -> int:
         out["_bracket"] = (bracket, 1)
         return out
 
+    def contraction(prof):
+        # (ms, launches) of a call's contraction: its round launches, or the one launch that runs a small batch
+        return prof["mvm_few"] if "mvm_few" in prof else prof["mvm_round"]
+
+    def backward_kernel(prof):
+        return "k_mvm_few (whole call)" if "mvm_few" in prof else "k_mvm_round"
+
     n = max(args.steps, 10)
     # forward / backward alone, on the initial weights (they do not change the tile)
     ms_forward = time_calls(lambda: tile.forward(xg, False, False, False, False, True), n)
@@ -322,20 +329,20 @@ def main() -> int:
             "ms_per_step": msx_step,
             "update": {"ms_per_call": msx_u, "kernels_ms": {k: v[0] for k, v in px_u.items()}},
             "forward": {"ms_per_call": msx_f, "gflops": fl / (msx_f * 1e-3) / 1e9, "mean_bm_rounds": rounds_x,
-                        "kernels_ms": {k: v[0] for k, v in px_f.items()}, "round_launches": px_f["mvm_round"][1]},
+                        "kernels_ms": {k: v[0] for k, v in px_f.items()}, "round_launches": contraction(px_f)[1]},
             "backward": {"ms_per_call": msx_b, "gflops": fl / (msx_b * 1e-3) / 1e9,
                          "kernels_ms": {k: v[0] for k, v in px_b.items()}},
             "roofline": {"kernel": "k_update_pulsed", "bound": "hbm", "achieved": ubytes / (px_u["update_pulsed"][0] * 1e-3) / 1e9,
                          "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": ubytes / (px_u["update_pulsed"][0] * 1e-3) / 1e9 / HBM_PEAK_GBS,
                          "traffic": None, "algorithmic_bytes": ubytes, "kernel_ms": px_u["update_pulsed"][0]},
             "roofline_forward": {"kernel": "all round launches of a call", "bound": "mfma",
-                                 "achieved": fl / (px_f["mvm_round"][0] * 1e-3) / 1e12, "peak": FP32_MFMA_PEAK_TFLOPS,
-                                 "unit": "TFLOP/s", "frac": fl / (px_f["mvm_round"][0] * 1e-3) / 1e12 / FP32_MFMA_PEAK_TFLOPS,
-                                 "kernel_ms": px_f["mvm_round"][0]},
-            "roofline_backward": {"kernel": "k_mvm_round", "bound": "mfma",
-                                  "achieved": fl / (px_b["mvm_round"][0] * 1e-3) / 1e12, "peak": FP32_MFMA_PEAK_TFLOPS,
-                                  "unit": "TFLOP/s", "frac": fl / (px_b["mvm_round"][0] * 1e-3) / 1e12 / FP32_MFMA_PEAK_TFLOPS,
-                                  "kernel_ms": px_b["mvm_round"][0]},
+                                 "achieved": fl / (contraction(px_f)[0] * 1e-3) / 1e12, "peak": FP32_MFMA_PEAK_TFLOPS,
+                                 "unit": "TFLOP/s", "frac": fl / (contraction(px_f)[0] * 1e-3) / 1e12 / FP32_MFMA_PEAK_TFLOPS,
+                                 "kernel_ms": contraction(px_f)[0]},
+            "roofline_backward": {"kernel": backward_kernel(px_b), "bound": "mfma",
+                                  "achieved": fl / (contraction(px_b)[0] * 1e-3) / 1e12, "peak": FP32_MFMA_PEAK_TFLOPS,
+                                  "unit": "TFLOP/s", "frac": fl / (contraction(px_b)[0] * 1e-3) / 1e12 / FP32_MFMA_PEAK_TFLOPS,
+                                  "kernel_ms": contraction(px_b)[0]},
         }
         del tile_x
 
@@ -418,11 +425,11 @@ def main() -> int:
     flops_per_call = 2.0 * x_size * d_size * batch
     update_bytes = bytes_per_device * x_size * d_size + 4.0 * (x_size + d_size) * batch
     k_update_ms = prof_update["update_pulsed"][0]
-    k_fwd_ms = prof_forward["mvm_round"][0]   # all round launches of one forward call
-    fused_forward = prof_forward["mvm_round"][1] < 5 and args.config == 2  # rounds 0 and 1 ran as one launch
-    fused_3 = fused_forward and prof_forward["mvm_round"][1] == 2           # rounds 0 to 2, then one launch for the rest
+    k_fwd_ms = contraction(prof_forward)[0]   # all round launches of one forward call
+    fused_forward = contraction(prof_forward)[1] < 5 and args.config == 2  # rounds 0 and 1 ran as one launch
+    fused_3 = fused_forward and contraction(prof_forward)[1] == 2           # rounds 0 to 2, then one launch for the rest
     fwd_traffic = "forward_fused_3" if fused_3 else ("k_mvm_round" if args.config == 2 and not fused_forward else None)
-    k_bwd_ms = prof_backward["mvm_round"][0]
+    k_bwd_ms = contraction(prof_backward)[0]
 
     out = {
         "metric": "pulsed-update Gdevice-updates/s + noisy fwd GFLOP/s, 1024^2 tile, 1 MI355X",
@@ -445,7 +452,7 @@ def main() -> int:
                    "pulses_per_call": pulses, "pulses_per_cross_point": pulses / (x_size * d_size)},
         "forward": {"ms_per_call": ms_forward, "gflops": flops_per_call / (ms_forward * 1e-3) / 1e9,
                     "mean_bm_rounds": float(rounds.mean()), "kernels_ms": {k: v[0] for k, v in prof_forward.items()},
-                    "round_launches": prof_forward["mvm_round"][1],
+                    "round_launches": contraction(prof_forward)[1],
                     "note": "with most samples in a second round the tile runs rounds 0 and 1 as one launch (round 2 as well "
                             "when its recent calls listed samples for it), with none the rounds after round 0 as one "
                             "launch (rpu_tile_set_fused_rounds, default: by what its last calls needed); same outputs"},
@@ -459,6 +466,7 @@ def main() -> int:
                                         "WRITE_SIZE), not measured in this run") if args.config == 2 else None,
                      "algorithmic_bytes": update_bytes, "kernel_ms": k_update_ms},
         "roofline_forward": {"kernel": "k_mvm_dual + k_mvm_rounds_rest (all rounds of a call)" if fused_forward
+                             else "k_mvm_few (whole call)" if "mvm_few" in prof_forward
                              else "k_mvm_round (all rounds of a call)", "bound": "mfma",
                              "achieved": flops_per_call / (k_fwd_ms * 1e-3) / 1e12, "peak": FP32_MFMA_PEAK_TFLOPS,
                              "unit": "TFLOP/s", "frac": flops_per_call / (k_fwd_ms * 1e-3) / 1e12 / FP32_MFMA_PEAK_TFLOPS,
@@ -466,7 +474,7 @@ def main() -> int:
                              "traffic_source": ("constant from " + PMC_SOURCE[fwd_traffic] + ", not measured in this run")
                              if fwd_traffic else None,
                              "algorithmic_flops": flops_per_call, "kernel_ms": k_fwd_ms},
-        "roofline_backward": {"kernel": "k_mvm_round", "bound": "mfma",
+        "roofline_backward": {"kernel": backward_kernel(prof_backward), "bound": "mfma",
                               "achieved": flops_per_call / (k_bwd_ms * 1e-3) / 1e12, "peak": FP32_MFMA_PEAK_TFLOPS,
                               "unit": "TFLOP/s", "frac": flops_per_call / (k_bwd_ms * 1e-3) / 1e12 / FP32_MFMA_PEAK_TFLOPS,
                               "kernel_ms": k_bwd_ms},
