@@ -128,6 +128,7 @@ struct MvmArgs {
   int *few;      // calls of k_mvm_few: [7][m_batch] counters and saturation marks, zero between calls
   int *few_seen; // host-visible: few_call of the last call in which a sample needed a second round, and of the last call
   int few_call;
+  int cus; // compute units of the tile's GPU: the rules of a launch ask for them several times (a query of the runtime each)
 };
 
 // weight operand of a call: the matrix at w with rows of `ld` elements, stored [d_size][x_size] (xd_storage = false) or

@@ -3217,9 +3217,11 @@ static int mvm_rest_depth(const MvmArgs &a) {
   return (weight_mode(a) == 1 && depth == 4) ? 2 : depth;
 }
 
+static int cus_of(const MvmArgs &a) { return a.cus > 0 ? a.cus : current_device_cus(); }
+
 // whether the launch of the rounds expected empty walks its tiles (k_mvm_rest_walk) instead of having a workgroup for each
 static bool mvm_rest_walks(const MvmArgs &a) {
-  return a.in_index || (!a.small_tiles_only && big_threshold(a.m_batch, a.O) > 0) || mvm_round_workgroups(a) > current_device_cus();
+  return a.in_index || (!a.small_tiles_only && big_threshold(a.m_batch, a.O) > 0) || mvm_round_workgroups(a) > cus_of(a);
 }
 
 typedef void (*RestWalk)(MvmArgs);
@@ -3233,18 +3235,20 @@ static RestWalk mvm_rest_walk_kernel(const MvmArgs &a) {
 
 int mvm_rest_resident_limit(const MvmArgs &a) {
   // a walking launch has one workgroup per CU, all variants of it less than half of a CU's registers and LDS
-  if (mvm_rest_walks(a)) return resident_workgroups(k_mvm_rest_walk<1, 3>);
+  const bool walks = mvm_rest_walks(a);
   static std::mutex m;
-  static int limit[64][3][3] = {};
+  static int limit[64][3][3] = {}, walk_limit[64] = {}; // (a query of the runtime takes microseconds: asked once)
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
   const int mode = weight_mode(a);
   const int depth = mvm_rest_depth(a);
   const int di = depth == 4 ? 2 : (depth == 2 ? 1 : 0);
   std::lock_guard<std::mutex> lock(m);
-  int &v = limit[dev][di][mode];
+  int &v = walks ? walk_limit[dev] : limit[dev][di][mode];
   if (v == 0) {
-    if (mode == 0) {
+    if (walks) {
+      v = resident_workgroups(k_mvm_rest_walk<1, 3>);
+    } else if (mode == 0) {
       v = depth == 4 ? resident_workgroups(k_mvm_rounds_rest<4, 0>)
                      : (depth == 2 ? resident_workgroups(k_mvm_rounds_rest<2, 0>) : resident_workgroups(k_mvm_rounds_rest<1, 0>));
     } else if (mode == 1) { // the deepest prefetch is not built for this addressing (mvm_rest_depth)
@@ -3308,7 +3312,7 @@ void launch_mvm_round(const MvmArgs &a_in, hipStream_t s) {
   // the round is one launch
   if (a.round > 0 && !a.speculate) a.big_from = 0;
   if (a.rest_in_one && mvm_rest_walks(a)) {
-    const dim3 grid((unsigned)std::min(mvm_round_workgroups(a), current_device_cus()));
+    const dim3 grid((unsigned)std::min(mvm_round_workgroups(a), cus_of(a)));
     const RestWalk kernel = mvm_rest_walk_kernel(a);
     hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, a);
     return;
@@ -3418,7 +3422,7 @@ int mvm_few_batch(const MvmArgs &a, bool training_tile) {
   if (io.bound_management != RPU_BM_NONE && (io.bound_management != RPU_BM_ITERATIVE || a.transposed)) return 0;
   const long per_cu = !training_tile ? 12288 : (a.max_rounds > 1 ? 51200 : 102400); // multiply-adds
   // (a sample takes a load of 64 inputs by 16 outputs at least: a long batch on a tiny tile is not a small call)
-  return (int)(per_cu * current_device_cus() / ((long)((a.K + 63) & ~63) * ((a.O + 15) & ~15)));
+  return (int)(per_cu * cus_of(a) / ((long)((a.K + 63) & ~63) * ((a.O + 15) & ~15)));
 }
 // the variant of a launch of such calls: the smallest blocks of samples and outputs with at most two workgroups to a CU
 int mvm_few_variant(const MvmArgs *const *calls, int n) {

@@ -224,6 +224,7 @@ struct Tile {
   DevBuf<float> s_dual0, s_dual1, s_dual2, s_xq2;
   DevBuf<int> s_dsel, s_dhit1, s_dhit2, s_few;
   int few_calls = 0; // see few_args
+  int cus = 0;       // MvmArgs::cus
   int *seen_host = nullptr, *seen_dev = nullptr;
   int rest_from = 0, rest_quiet = 0; // the last round that listed samples in the recent calls, and calls since it did
   int fused_rounds = -1;
@@ -663,6 +664,8 @@ struct Tile {
     const int O = transposed ? X : D;
     ensure_mvm_scratch(B);
     MvmArgs a{};
+    if (cus == 0) cus = current_device_cus(); // under the caller's DeviceGuard
+    a.cus = cus;
     a.x_size = X; a.d_size = D; a.m_batch = B; a.K = K; a.O = O;
     a.transposed = transposed ? 1 : 0;
     mvm_set_weights(a, w_other ? w_other : wdev(), w_ld(), xd);
