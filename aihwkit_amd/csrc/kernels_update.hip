@@ -168,37 +168,50 @@ __device__ __forceinline__ void update_prepare_sample(const UpdateArgs &a, const
 }
 
 // The lines of the indexed interface read in place, for long batches.  A workgroup of 16 waves owns 64 patches, one per
-// lane, of four images; wave w takes the elements j = w (mod 16) of both lines, and the waves meet in LDS.  Neighbouring
-// lanes read neighbouring patches -- the line-major index, the gradient tensor and (mostly) the image elements are runs of
-// a row for every load of a wave -- and an index entry is read once for the four images.  131072 patches of 433 + 48
-// elements: 110 us with one thread per sample, a chain of loads, -> 43 us.
+// lane, of NI images; wave w takes the elements j = w (mod 16) of both lines, and the waves meet in LDS.
+// NI = 4: neighbouring lanes read neighbouring patches of an image -- the line-major index, the gradient tensor and (mostly)
+// the image elements are runs of a row for every load of a wave -- and an index entry is read once for the four images.
+// 131072 patches of 433 + 48 elements: 110 us with one thread per sample, a chain of loads, -> 43 us.
+// NI = 1: the 64 patches follow each other across images, for images of so few patches that most lanes would have none.
+template <int NI>
 __global__ __launch_bounds__(1024) void k_update_prepare_in_place(UpdateArgs a) {
-  constexpr int NI = 4;
+  constexpr int UX = NI == 1 ? 8 : 4; // index entries in flight
   __shared__ float sh_max[2][NI][16][64];
   if (a.row_cost) {
     for (int i = (int)(blockIdx.x * 1024u + threadIdx.x); i < a.d_size; i += (int)(gridDim.x * 1024u)) a.row_cost[i] = 0;
   }
   const int lane = (int)threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-  const int P = a.x_group, blocks_p = (P + 63) / 64;
-  const int n0 = (int)(blockIdx.x / (unsigned)blocks_p) * NI, p = (int)(blockIdx.x % (unsigned)blocks_p) * 64 + lane;
-  const bool live = p < P;
-  const int images = min(NI, a.m_batch / P - n0);
+  const int P = a.x_group;
+  int n0, p, images = 1; // lane's first image and its patch
+  bool live;
+  if (NI == 1) {
+    const int b = (int)blockIdx.x * 64 + lane;
+    live = b < a.m_batch;
+    n0 = min(b, a.m_batch - 1) / P;
+    p = min(b, a.m_batch - 1) - n0 * P;
+  } else {
+    const int blocks_p = (P + 63) / 64;
+    n0 = (int)(blockIdx.x / (unsigned)blocks_p) * NI;
+    p = (int)(blockIdx.x % (unsigned)blocks_p) * 64 + lane;
+    live = p < P;
+    images = min(NI, a.m_batch / P - n0);
+  }
   float xm[NI] = {}, dm[NI] = {};
   if (a.up.update_management || a.up.update_bl_management) {
     const int *idx = a.x_index_lines + min(p, P - 1);
     const float *image = a.x + (long)n0 * a.x_gs - 2;
-    for (int j0 = wave; j0 < a.x_size; j0 += 64) { // sixteen loads in flight
-      int at[4];
+    for (int j0 = wave; j0 < a.x_size; j0 += 16 * UX) {
+      int at[UX];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) at[u] = (j0 + 16 * u < a.x_size) ? idx[(long)(j0 + 16 * u) * P] : 0;
-      float v[4][NI];
+      for (int u = 0; u < UX; ++u) at[u] = (j0 + 16 * u < a.x_size) ? idx[(long)(j0 + 16 * u) * P] : 0;
+      float v[UX][NI];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
+      for (int u = 0; u < UX; ++u) {
 #pragma unroll
         for (int i = 0; i < NI; ++i) v[u][i] = (at[u] > 1 && i < images) ? image[at[u] + (long)i * a.x_gs] : (float)min(at[u], 1);
       }
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
+      for (int u = 0; u < UX; ++u) {
 #pragma unroll
         for (int i = 0; i < NI; ++i) xm[i] = fmaxf(xm[i], fabsf(v[u][i]));
       }
@@ -2371,8 +2384,15 @@ int grid_for(long total) {
 void launch_update_prepare(const UpdateArgs &a, hipStream_t s) {
   const int longest = a.x_size > a.d_size ? a.x_size : a.d_size;
   if (a.x_index_lines && a.d_group && a.m_batch >= 4096) {
+    // images of fewer patches than lanes: this kernel, 4096 / 65536 samples, us: 144 -> 32 elements, 1 patch per image (four
+    // images a workgroup) 25.7 / 235, (patches that follow each other) 14 / 45; 432 -> 48, 4 patches 25 / 139, 21 / 60, 16
+    // patches 16 / 47, 11 / 25, 49 patches 33 / 37, 13 / 43.  One thread per sample: 21 / 60, 41 / 80, 41 / 66, 47 / 72
+    if (a.x_group < 64) {
+      hipLaunchKernelGGL(k_update_prepare_in_place<1>, dim3((a.m_batch + 63) / 64), dim3(1024), 0, s, a);
+      return;
+    }
     const unsigned images = (unsigned)(a.m_batch / a.x_group), blocks = (unsigned)((a.x_group + 63) / 64) * ((images + 3) / 4);
-    hipLaunchKernelGGL(k_update_prepare_in_place, dim3(blocks), dim3(1024), 0, s, a);
+    hipLaunchKernelGGL(k_update_prepare_in_place<4>, dim3(blocks), dim3(1024), 0, s, a);
     return;
   }
   if (longest > 1024 || a.m_batch <= 1024) {

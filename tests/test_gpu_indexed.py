@@ -309,8 +309,16 @@ def test_gathered_forward_runs_every_round_whatever_the_launch_mode(gpu_device, 
          pulse="StochasticCompressed"),
     dict(c_in=3, hw=(11, 10), kernel=(3, 3), stride=(1, 1), padding=(1, 1), n=5, c_out=20, device="constant", bl=31,
          pulse="DeterministicImplicit"),
-    # 4800 samples: the per-sample maxima come from the kernel with one thread per sample
+    # 4800 samples: the maxima of 64 patches of four images come from a workgroup, here of three
     dict(c_in=3, hw=(40, 40), kernel=(3, 3), stride=(1, 1), padding=(1, 1), n=3, c_out=20, device="soft", bl=31,
+         pulse="StochasticCompressed"),
+    # 4140, 4101 and 4158 samples of 9, 1 and 63 patches per image: maxima of 64 patches that follow each other, whichever
+    # images they are of
+    dict(c_in=2, hw=(9, 9), kernel=(5, 5), stride=(2, 2), padding=(0, 0), n=460, c_out=33, device="constant", bl=31,
+         pulse="StochasticCompressed"),
+    dict(c_in=15, hw=(3, 3), kernel=(3, 3), stride=(1, 1), padding=(0, 0), n=4101, c_out=17, device="soft", bl=31,
+         pulse="StochasticCompressed"),
+    dict(c_in=3, hw=(9, 11), kernel=(3, 3), stride=(1, 1), padding=(0, 0), n=66, c_out=40, device="soft", bl=31,
          pulse="StochasticCompressed"),
 ])
 def test_pulsed_update_reads_patches_and_gradients_in_place(gpu_device, case):
