@@ -199,6 +199,7 @@ SYMBOLS = {
     "rpu_tile_get_update_words": (C.c_int, [_P, _P, _P, _P, C.c_int]),
     "rpu_tile_get_update_words_per_sample": (C.c_int, [_P, _P]),
     "rpu_tile_set_fused_rounds": (C.c_int, [_P, C.c_int]),
+    "rpu_tile_set_small_calls": (C.c_int, [_P, C.c_int]),
     "rpu_tile_set_round_wait_test_hook": (C.c_int, [_P, C.c_int, C.c_int]),
     "rpu_group_set_round_wait_test_hook": (C.c_int, [_P, C.c_int, C.c_int]),
     "rpu_tile_get_update_ab": (C.c_int, [_P, _P, _P, C.c_int]),

@@ -224,6 +224,7 @@ struct Tile {
   DevBuf<float> s_dual0, s_dual1, s_dual2, s_xq2;
   DevBuf<int> s_dsel, s_dhit1, s_dhit2, s_few;
   int few_calls = 0; // see few_args
+  bool small_calls = true; // rpu_tile_set_small_calls
   int cus = 0;       // MvmArgs::cus
   int *seen_host = nullptr, *seen_dev = nullptr;
   int rest_from = 0, rest_quiet = 0; // the last round that listed samples in the recent calls, and calls since it did
@@ -640,7 +641,8 @@ struct Tile {
     if (fused_rounds >= 0) return fused_rounds & 1 ? 3 : 1;
     return seen_host[1] - seen_host[0] <= 8 ? 3 : 1;
   }
-  bool training_tile() const { return dev.pulsed() || is_transfer(); }
+  // the largest batch whose calls take k_mvm_few, 0: none do
+  int small_call_batch(const MvmArgs &a) const { return small_calls ? mvm_few_batch(a, dev.pulsed() || is_transfer()) : 0; }
   // Whether the outputs of a call lie among the inputs of one: the workgroups of k_mvm_few read their inputs while others
   // store outputs; the other launches have quantized the inputs of round 0 before the first output is stored.
   static bool writes_into(const MvmArgs &from, const MvmArgs &to) {
@@ -930,7 +932,7 @@ struct Tile {
 
     prof_begin(s);
     const bool running = io.p.noise_management == RPU_NM_AVERAGE_ABS_MAX || io.p.noise_management == RPU_NM_AVERAGE_ABS_MAX_SINGLE_VALUE;
-    const int few_batch = side || gather || running ? 0 : std::min(B, mvm_few_batch(a, training_tile()));
+    const int few_batch = side || gather || running ? 0 : std::min(B, small_call_batch(a));
     if (few_batch > 0 && a.max_rounds > 1) {
       ensure_seen();
       ensure_few(s_few, few_counters(a, few_batch), s_dual1, few_rows(a, few_batch), s);
@@ -2836,7 +2838,7 @@ static int group_mvm(rpu_group_t *group, const float *const *x_dev, const long *
       mvm_round_variant(a, depth[i], mode[i]);
       // (the test hook of the waits is about the other launches; the large-tile kernel takes all of its tiles through the
       // lists and marks that the init kernel sets up)
-      few_batch[i] = std::min(m_batch, mvm_few_batch(a, t.training_tile()));
+      few_batch[i] = std::min(m_batch, t.small_call_batch(a));
       few[i] = !big && !group->wait_spins_hook && !group->wait_extra_hook && few_batch[i] == m_batch ? 1 : 0;
       rounds = std::max(rounds, a.max_rounds);
       args[i] = a;
@@ -2981,11 +2983,7 @@ static int group_mvm(rpu_group_t *group, const float *const *x_dev, const long *
       MvmGroup g{group->mvm_args.dev_args(), group->mvm_args.dev_table(), n_few, m_batch};
       launch_mvm_few_group(g, few_variant, few_together, transposed != storage_xd, few_max_k, few_workgroups, s);
     }
-    if (n_few == n) { // nothing was listed for a later launch: what the pairs say of this call
-      for (int k = 0; k < kSeenPairs; ++k) {
-        *(volatile int *)&group->seen_host[2 * k] = 0;
-        *(volatile int *)&group->seen_host[2 * k + 1] = m_batch;
-      }
+    if (n_few == n) { // says nothing about the launches that the pairs choose
       RPU_HIP_CHECK(hipGetLastError());
       return;
     }
@@ -3125,6 +3123,7 @@ int rpu_tile_clone(rpu_tile_t **out, const rpu_tile_t *src_c) {
     t.update_variant = s.update_variant;
     t.update_variant_samples = s.update_variant_samples;
     t.fused_rounds = s.fused_rounds;
+    t.small_calls = s.small_calls;
     if (s.is_transfer()) {
       t.tr = std::make_unique<TransferPar>(*s.tr);
       t.update_idx = s.update_idx;
@@ -3577,6 +3576,14 @@ int rpu_tile_set_fused_rounds(rpu_tile_t *tile, int mode) {
     std::lock_guard<std::mutex> lock(tile->t.mutex);
     tile->t.fused_rounds = mode;
     tile->t.merged_off = false; // an explicit choice re-arms the merged launches after a reported time-out
+  });
+}
+
+int rpu_tile_set_small_calls(rpu_tile_t *tile, int enable) {
+  return guarded([&] {
+    if (!tile) throw RpuError("null tile");
+    std::lock_guard<std::mutex> lock(tile->t.mutex);
+    tile->t.small_calls = enable != 0;
   });
 }
 

@@ -528,6 +528,11 @@ class _CudaTileMixin:
         first launch as well, 0 = one launch per round, -1 (default) = the tile decides by what its recent calls needed.  Outputs and round counts do not depend on it."""
         check(lib().rpu_tile_set_fused_rounds(self._h, int(mode)))
 
+    def set_small_calls(self, enable: bool = True) -> None:
+        """Whether small batches may run as one launch (default).  ``False``: the launches of larger batches, whose sums are
+        added in another order, serve every batch."""
+        check(lib().rpu_tile_set_small_calls(self._h, int(enable)))
+
     def set_round_wait_test_hook(self, spin_limit: int = 0, extra_arrivals: int = 0) -> None:
         """For the test of the time-out path of the merged-round launches only: shorten their bounded waits to
         ``spin_limit`` polls and make them expect ``extra_arrivals`` workgroups more than the launch has."""

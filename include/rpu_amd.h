@@ -695,6 +695,11 @@ int rpu_tile_set_extra(rpu_tile_t *tile, const int64_t *values_host, int count);
  * the shortcut).  Tile groups report the same way at their next call. */
 int rpu_tile_set_fused_rounds(rpu_tile_t *tile, int mode);
 
+/* No counterpart in the reference.  A call of a small batch runs noise management, conversions, contraction and all
+ * bound-management rounds in one launch, whose sums are added in another order than those of the launches for larger
+ * batches.  enable = 0: the tile (alone and in a group) keeps to the latter for every batch. */
+int rpu_tile_set_small_calls(rpu_tile_t *tile, int enable);
+
 /* No counterpart in the reference; for the test of the time-out path above only.  spin_limit > 0 shortens the bounded
  * waits of the tile's (or group's) merged-round launches to that many polls, extra_arrivals = 1 makes every wait expect
  * one workgroup more than the launch has, so that it runs out while every workgroup still leaves its kernel normally.

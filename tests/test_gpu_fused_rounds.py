@@ -309,6 +309,7 @@ def test_a_group_reports_a_wait_that_runs_out(gpu_device):
         host.set_weights(torch.from_numpy(w))
         orc.set_weights(w)
         grouped.append(tiles.CudaAnalogTile(host))
+        grouped[-1].set_small_calls(False)                        # these run no rounds in launches of their own
         oracles.append(orc)
     group = tiles.TileGroup(grouped)
     sizes = [t.get_x_size() for t in grouped]
@@ -332,6 +333,40 @@ def test_a_group_reports_a_wait_that_runs_out(gpu_device):
     for xs in (loud, quiet, quiet, loud):                         # one launch per round from now on: exact again
         for y, orc, x in zip(run(xs), oracles, xs):
             assert np.array_equal(y, orc.forward(x))
+
+
+def test_calls_in_one_launch_leave_what_the_others_know(gpu_device):
+    """Forward calls of a group that list samples for round 1, with backward calls between them that run as one launch
+    (k_mvm_few) and list nothing: the next forward call must still expect work in round 1 and not choose the launch for
+    rounds that are expected empty.  That launch would run into the shortened wait, and the call after it fail."""
+    from helpers import constant_step
+    rng = np.random.default_rng(6)
+    batch, sizes = 120, ((64, 64), (130, 96))
+    grouped, oracles = [], []
+    for k, (x_size, d_size) in enumerate(sizes):
+        f_io = noise_free_io(inp_res=1 / 128.0, out_res=1 / 512.0, noise_management=NM.AbsMax,
+                             bound_management=BM.Iterative, out_bound=2.0)
+        dev = constant_step(w_max_dtod=0.0, w_min_dtod=0.0, w_max=1.0, w_min=-1.0, construction_seed=k + 1)
+        host, orc, _ = build_pair(make_meta(f_io, noise_free_io()), dev, x_size, d_size, gpu=False)
+        w = (rng.integers(-60, 61, (d_size, x_size)) / 64.0).astype(F)
+        host.set_weights(torch.from_numpy(w))
+        orc.set_weights(w)
+        grouped.append(tiles.CudaAnalogTile(host))
+        oracles.append(orc)
+    group = tiles.TileGroup(grouped)
+    xs = [(rng.integers(-64, 65, (batch, n)) / 64.0).astype(F) for n, _ in sizes]
+    ds = [torch.from_numpy((rng.integers(-64, 65, (batch, n)) / 64.0).astype(F)).cuda() for _, n in sizes]
+    for _ in range(2):
+        for t in grouped:
+            t.set_small_calls(False)
+        group.set_round_wait_test_hook(2000, 1)
+        got = group.forward([torch.from_numpy(x).cuda() for x in xs])
+        for y, orc, x in zip(got, oracles, xs):
+            assert np.array_equal(y.cpu().numpy(), orc.forward(x)) and orc.bm_rounds(batch).max() >= 2
+        for t in grouped:
+            t.set_small_calls(True)
+        group.set_round_wait_test_hook(0, 0)                      # (the hook keeps to the launches that wait)
+        group.backward(ds)
 
 
 def test_worst_case_second_round_on_a_fresh_tile_matches_the_oracle(gpu_device):
