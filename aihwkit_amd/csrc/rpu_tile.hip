@@ -2892,9 +2892,9 @@ static int group_mvm(rpu_group_t *group, const float *const *x_dev, const long *
                                 ((std::isinf(p.out_bound) && std::isinf(q.out_bound)) || p.out_bound == q.out_bound)))));
       };
       std::vector<int> first_of; // first tile of each set
-      std::vector<int> set_of(n, -1), members, readers, writer; // readers: members that run on quantized rows in memory
+      std::vector<int> set_of(n, -1), members;
       for (int i = 0; i < n; ++i) {
-        if (!shares(args[i])) continue;
+        if (few[i] || !shares(args[i])) continue; // (few: quantizes the rows for itself, the same way)
         for (size_t c = 0; c < first_of.size() && set_of[i] < 0; ++c) {
           if (same_rows(args[i], args[first_of[c]])) set_of[i] = (int)c;
         }
@@ -2902,13 +2902,8 @@ static int group_mvm(rpu_group_t *group, const float *const *x_dev, const long *
           set_of[i] = (int)first_of.size();
           first_of.push_back(i);
           members.push_back(0);
-          readers.push_back(0);
-          writer.push_back(-1);
         }
         ++members[set_of[i]];
-        if (few[i]) continue; // (quantizes the rows for itself, the same way)
-        ++readers[set_of[i]];
-        if (writer[set_of[i]] < 0) writer[set_of[i]] = i;
       }
       if (group->first_rows.size() < 2 * first_of.size()) group->first_rows.resize(2 * first_of.size());
       group->shared_sets = group->shared_tiles = 0;
@@ -2920,14 +2915,14 @@ static int group_mvm(rpu_group_t *group, const float *const *x_dev, const long *
       }
       for (int i = 0; i < n; ++i) {
         const int c = set_of[i];
-        if (c < 0 || readers[c] < 2 || few[i]) continue;
+        if (c < 0 || members[c] < 2) continue;
         MvmArgs &a = args[i];
         DevBuf<float> &r0 = group->first_rows[2 * c], &r1 = group->first_rows[2 * c + 1];
         r0.ensure((size_t)m_batch * a.k_pad);
         if (a.max_rounds > 1) r1.ensure((size_t)m_batch * a.k_pad);
         a.xq_first[0] = r0.p;
         a.xq_first[1] = a.max_rounds > 1 ? r1.p : nullptr;
-        a.xq_first_writer = writer[c] == i ? 1 : 0;
+        a.xq_first_writer = first_of[c] == i ? 1 : 0;
       }
     }
     // tiles that share a kernel variant sit next to each other, first those that run in one launch (k_mvm_few)

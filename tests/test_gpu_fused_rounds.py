@@ -177,6 +177,7 @@ def test_tiles_of_a_split_layer_share_their_quantized_input(gpu_device, batch, o
             host.set_weights(torch.from_numpy(w))
             orc.set_weights(w)
             grouped.append(tiles.CudaAnalogTile(host))
+            grouped[-1].set_small_calls(False)       # those quantize the rows for themselves
             oracles.append(orc)
             where.append((bi, i0, n_in, o0, n_out))
             o0 += n_out
@@ -225,6 +226,8 @@ def test_shared_input_rows_leave_noisy_results_unchanged(gpu_device):
         host.set_weights(torch.from_numpy(rng.uniform(-0.4, 0.4, (70 + 10 * k, n_in)).astype(F)))
         alone.append(tiles.CudaAnalogTile(host))
         grouped.append(tiles.CudaAnalogTile(host))
+        for t in (alone[-1], grouped[-1]):
+            t.set_small_calls(False)                 # those quantize the rows for themselves
     group = tiles.TileGroup(grouped)
     for call in range(3):
         x = torch.from_numpy((rng.uniform(-1, 1, (batch, n_in)) * rng.choice([0.05, 1.0], (batch, 1))).astype(F)).cuda()

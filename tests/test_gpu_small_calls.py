@@ -84,6 +84,22 @@ def test_groups_with_small_calls_equal_the_oracle(gpu_device, batch, shapes):
             assert np.array_equal(g.cpu().numpy(), orc.backward(d))
 
 
+def test_small_calls_share_no_quantized_rows(gpu_device):
+    """Tiles with the same input: a call in one launch writes no rows that they could share, the other launches do."""
+    rng = np.random.default_rng(4)
+    grouped = [tiles.CudaAnalogTile(exact_pair(rng, 96, 40, 2.0, 32)[0]) for _ in range(3)]
+    group = tiles.TileGroup(grouped)
+    x = torch.from_numpy(grid(rng, 64, (5, 96), 64.0)).cuda()
+    small = group.forward([x] * 3)
+    assert group.get_shared_input_sets() == (0, 0)
+    for t in grouped:
+        t.set_small_calls(False)
+    other = group.forward([x] * 3)
+    assert group.get_shared_input_sets() == (1, 3)
+    for y, z in zip(small, other):
+        assert torch.equal(y, z)
+
+
 # a program that has warmed up on its largest batch captures smaller ones: they find their scratch there
 @pytest.mark.parametrize("grouped", [False, True])
 def test_small_calls_after_larger_ones_allocate_nothing(gpu_device, grouped):
