@@ -191,7 +191,9 @@ void mvm_round_variant(const MvmArgs &a, int &prefetch_depth, int &weight_mode);
 // Small batches: everything from the noise management to the last bound-management round in one launch (k_mvm_few).
 // a.few is needed where a.max_rounds > 1.  rounds: 1, or 3 to work out rounds 0 to 2 together (a.dual.buf[1], buf[2]),
 // for calls whose samples are expected to need them; same results.
-int mvm_few_batch(const MvmArgs &a, bool training_tile); // the largest batch whose calls take that launch, 0: none do
+int mvm_few_batch(const MvmArgs &a); // the largest batch whose calls take that launch, 0: none do
+int mvm_few_blocks(int O);
+int mvm_few_group_batch(long blocks);
 int mvm_few_variant(const MvmArgs *const *calls, int n); // blocks of a launch of n calls; the results do not depend on it
 int mvm_few_workgroups(const MvmArgs &a, int variant);
 void launch_mvm_few(const MvmArgs &a, int variant, int rounds, hipStream_t s);

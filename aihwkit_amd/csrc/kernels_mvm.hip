@@ -3405,25 +3405,32 @@ void launch_mvm_round(const MvmArgs &a_in, hipStream_t s) {
 #undef RPU_LAUNCH_ROUND
 }
 
-// The largest batch whose calls run as k_mvm_few: a function of the tile and its IO settings, so that a tile takes the same sums
-// on its own and in a group (whose workgroups read every weight once per block of samples, all tiles at a time: that, and not
-// the single call, sets the limits).  us, the other launches / one:
-//   forward, weights that saturate round 0: 512 x 512, 1 sample 27.5 / 13.3, 32 27 / 19, 100 (26 M multiply-adds) 27 / 27, 200
-//   28 / 31; 785 -> 256, 64 samples 40 / 22; 129 -> 10, 64 16.4 / 7.0; 1024 x 1024, 32 36 / 29, 64 37 / 39
-//   backward: 512 x 512, 1 sample 14.8 / 8.2, 100 14.1 / 11.0, 200 14.3 / 12.5; 785 -> 256, 200 (40 M) 14.4 / 20.4
-//   layers of tiles of at most 512 x 512: 768 -> 2304, 8 tokens 27.3 / 25.3, 16 (2.8 M a tile) 27.1 / 26.0, 32 28 / 37;
-//   3072 x 3072, 8 tokens (2.1 M) 54 / 53, 16 56 / 68
-// Inference tiles come in such groups, training tiles mostly do not.
-int mvm_few_batch(const MvmArgs &a, bool training_tile) {
+// Blocks of the largest kind (four samples by 64 outputs) that a call launches for four of its samples
+int mvm_few_blocks(int O) { return MvmFew<false, 4, 64, 1>::workgroups(O, 4); }
+
+// The largest batch whose calls run as k_mvm_few.  A second set of blocks on a CU that holds two doubles the launch: the GPU
+// has to hold all of them at once.  us, the other launches / one, at that line and beyond: 160 -> 100, backward, 600 samples
+// 11.4 / 9.9, 800 11.7 / 15.5; 64 -> 32, 1000 17.0 / 7.8, 3000 16.7 / 17.5, backward 6000 11.5 / 21.7; 64 -> 2048, 64 17.4 /
+// 16.6, 100 18.3 / 23.4; layers of tiles of at most 512 x 512, 768 -> 2304, 24 tokens 52 / 35, 32 28 / 32; 24 tiles of 300 x
+// 300, 16 tokens 33 / 26, 24 33 / 39; 24 of 130 x 125, 64 tokens 28.5 / 32.7 (mvm_few_group_batch).
+// Within it the multiply-adds, weights that saturate round 0 (the last workgroup of a sample runs the rounds from 3 on alone):
+//   forward: 512 x 512, 1 sample 27.5 / 13.3, 50 (13 M) 26.7 / 18.2, 100 26.9 / 26.0, 160 27.7 / 28.5; 1024 x 1024, 24 35.4 /
+//   26.4, 64 36.0 / 37.5; 1500 x 1500, 16 46 / 34, 32 (72 M) 47 / 69; the line is drawn well before the first loss
+//   backward: 512 x 512, 100 14.0 / 10.6, 256 (67 M) 14.3 / 12.2; 1024 x 1024, 64 (67 M) 17.4 / 14.9, 128 17.6 / 17.5; 1500 x
+//   1500, 64 (144 M) 30.0 / 34.6
+int mvm_few_batch(const MvmArgs &a) {
   const IoDev &io = a.io;
   const int nm = io.noise_management;
   if (io.perfect || a.in_index || a.pre_add || a.skip_if_zero || a.nm_phase || a.small_tiles_only || a.K > 2048 || a.K <= a.in_one) return 0;
   if (nm != RPU_NM_NONE && nm != RPU_NM_CONSTANT && nm != RPU_NM_ABS_MAX && nm != RPU_NM_MAX) return 0;
   if (io.bound_management != RPU_BM_NONE && (io.bound_management != RPU_BM_ITERATIVE || a.transposed)) return 0;
-  const long per_cu = !training_tile ? 12288 : (a.max_rounds > 1 ? 51200 : 102400); // multiply-adds
+  const long per_cu = a.max_rounds > 1 ? 51200 : 262144; // multiply-adds
   // (a sample takes a load of 64 inputs by 16 outputs at least: a long batch on a tiny tile is not a small call)
-  return (int)(per_cu * cus_of(a) / ((long)((a.K + 63) & ~63) * ((a.O + 15) & ~15)));
+  const long most = per_cu * cus_of(a) / ((long)((a.K + 63) & ~63) * ((a.O + 15) & ~15));
+  return (int)std::min(most, 4L * (2 * cus_of(a) / mvm_few_blocks(a.O)));
 }
+// The same for a group of tiles whose calls have `blocks` blocks for four samples, all tiles taken together.
+int mvm_few_group_batch(long blocks) { return (int)(4 * (2L * current_device_cus() / blocks)); }
 // the variant of a launch of such calls: the smallest blocks of samples and outputs with at most two workgroups to a CU
 int mvm_few_variant(const MvmArgs *const *calls, int n) {
   for (int v = 0; v < 3; ++v) {

@@ -10,6 +10,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <climits>
 #include <cmath>
 #include <cstring>
 #include <memory>
@@ -225,6 +226,9 @@ struct Tile {
   DevBuf<int> s_dsel, s_dhit1, s_dhit2, s_few;
   int few_calls = 0; // see few_args
   bool small_calls = true; // rpu_tile_set_small_calls
+  // largest batch that the groups of this tile run as k_mvm_few, forward and backward: so does the tile in calls of its own,
+  // whose sums are then those of a call of the group
+  int group_batch[2] = {INT_MAX, INT_MAX};
   int cus = 0;       // MvmArgs::cus
   int *seen_host = nullptr, *seen_dev = nullptr;
   int rest_from = 0, rest_quiet = 0; // the last round that listed samples in the recent calls, and calls since it did
@@ -642,7 +646,9 @@ struct Tile {
     return seen_host[1] - seen_host[0] <= 8 ? 3 : 1;
   }
   // the largest batch whose calls take k_mvm_few, 0: none do
-  int small_call_batch(const MvmArgs &a) const { return small_calls ? mvm_few_batch(a, dev.pulsed() || is_transfer()) : 0; }
+  int small_call_batch(const MvmArgs &a) const {
+    return small_calls ? std::min(mvm_few_batch(a), group_batch[a.transposed]) : 0;
+  }
   // Whether the outputs of a call lie among the inputs of one: the workgroups of k_mvm_few read their inputs while others
   // store outputs; the other launches have quantized the inputs of round 0 before the first output is stored.
   static bool writes_into(const MvmArgs &from, const MvmArgs &to) {
@@ -2551,6 +2557,39 @@ struct rpu_group {
   // grouped update: the tiles' argument blocks and the workgroup tables of its launches
   GroupArgs<UpdateArgs> update_args;
   std::mutex mutex;
+  // whether the tile runs a call of the group in launches of its own (see group_mvm)
+  static bool runs_alone(const IOPar &io) {
+    return Tile::has_pre_adc_terms(io) || (!io.perfect && (io.p.noise_management == RPU_NM_AVERAGE_ABS_MAX ||
+                                                           io.p.noise_management == RPU_NM_AVERAGE_ABS_MAX_SINGLE_VALUE));
+  }
+  // The tiles of a group take the one launch of small batches together or not at all: next to the other launches it would
+  // come on top.
+  void limit_small_calls() {
+    for (int transposed = 0; transposed < 2; ++transposed) {
+      int batch = INT_MAX;
+      long blocks = 0;
+      bool alone = false;
+      for (rpu_tile *tile : tiles) {
+        const Tile &t = tile->t;
+        const IOPar &io = transposed ? t.bio : t.fio;
+        MvmArgs a{};
+        a.K = transposed ? t.D : t.X;
+        a.O = transposed ? t.X : t.D;
+        a.transposed = transposed;
+        a.io = Tile::io_dev(io);
+        a.max_rounds = io.perfect ? 0 : mvm_max_rounds(a.io);
+        alone = alone || runs_alone(io);
+        batch = std::min(batch, mvm_few_batch(a));
+        blocks += mvm_few_blocks(a.O);
+      }
+      if (alone) continue;
+      batch = std::min(batch, mvm_few_group_batch(blocks));
+      for (rpu_tile *tile : tiles) {
+        std::lock_guard<std::mutex> lock(tile->t.mutex);
+        tile->t.group_batch[transposed] = std::min(tile->t.group_batch[transposed], batch);
+      }
+    }
+  }
   ~rpu_group() {
     if (device_id >= 0) {
       try {
@@ -2588,6 +2627,7 @@ int rpu_group_create(rpu_group_t **out, rpu_tile_t *const *tiles, int n_tiles) {
       g->tiles.push_back(tiles[i]);
     }
     DeviceGuard dg(g->device_id);
+    g->limit_small_calls();
     const size_t n = (size_t)n_tiles;
     g->mvm_args.make(n, 3 * n + 4);
     RPU_HIP_CHECK(hipEventCreateWithFlags(&g->copied, hipEventDisableTiming));
@@ -2755,10 +2795,7 @@ static int group_mvm(rpu_group_t *group, const float *const *x_dev, const long *
       bool one_by_one = false;
       for (int i = 0; i < n && !one_by_one; ++i) {
         const Tile &t = group->tiles[i]->t;
-        const IOPar &gio = transposed ? t.bio : t.fio;
-        one_by_one = Tile::has_pre_adc_terms(gio) ||
-                     (!gio.perfect && (gio.p.noise_management == RPU_NM_AVERAGE_ABS_MAX ||
-                                       gio.p.noise_management == RPU_NM_AVERAGE_ABS_MAX_SINGLE_VALUE));
+        one_by_one = rpu_group::runs_alone(transposed ? t.bio : t.fio);
       }
       if (one_by_one) {
         for (int i = 0; i < n; ++i) {

@@ -9,7 +9,7 @@ import torch
 from aihwkit_amd._cabi import lib
 from aihwkit_amd.rpu_base import devices as dv
 from aihwkit_amd.rpu_base import tiles
-from helpers import build_pair, constant_step, make_meta, noise_free_io
+from helpers import build_pair, constant_step, io_params, make_meta, noise_free_io
 
 pytestmark = pytest.mark.gpu
 F = np.float32
@@ -62,14 +62,17 @@ def test_small_calls_equal_the_oracle(gpu_device, x_size, d_size, batch, bias):
 
 # batch, shapes: small calls next to others that share their input's quantized rows; next to tiles of the large-tile kernel;
 # the largest blocks with the longest rows, which take the most LDS
-@pytest.mark.parametrize("batch,shapes", [
-    (128, [(257, 16), (257, 512), (257, 33), (257, 600), (64, 16)]),
-    (1024, [(40, 130)] * 8 + [(64, 256)] * 2 + [(64, 40), (64, 30), (33, 20)]),
-    (5, [(130, 16), (130, 200), (2048, 40), (1, 1)]), (16, [(2048, 300)] * 13)])
-def test_groups_with_small_calls_equal_the_oracle(gpu_device, batch, shapes):
+@pytest.mark.parametrize("batch,shapes,others", [
+    (128, [(257, 16), (257, 512), (257, 33), (257, 600), (64, 16)], ()),
+    (60, [(257, 16), (257, 512), (257, 33), (257, 600), (64, 16)], (1, 3)),
+    (1024, [(40, 130)] * 8 + [(64, 256)] * 2 + [(64, 40), (64, 30), (33, 20)], ()),
+    (5, [(130, 16), (130, 200), (2048, 40), (1, 1)], ()), (16, [(2048, 300)] * 13, ())])
+def test_groups_with_small_calls_equal_the_oracle(gpu_device, batch, shapes, others):
     rng = np.random.default_rng(batch)
     pairs = [exact_pair(rng, x, d, 2.0, 32, seed=k + 1) for k, (x, d) in enumerate(shapes)]
     grouped = [tiles.CudaAnalogTile(host) for host, _ in pairs]
+    for k in others:
+        grouped[k].set_small_calls(False)
     group = tiles.TileGroup(grouped)
     by_size = {x: grid(rng, 64, (batch, x), 64.0) for x, _ in shapes}
     ds = [grid(rng, 64, (batch, d), 64.0) for _, d in shapes]
@@ -82,6 +85,53 @@ def test_groups_with_small_calls_equal_the_oracle(gpu_device, batch, shapes):
             assert np.array_equal(y.cpu().numpy(), orc.forward(by_size[x]))
             assert np.array_equal(r, orc.bm_rounds(batch))
             assert np.array_equal(g.cpu().numpy(), orc.backward(d))
+
+
+# 40 tiles with one block of outputs each, of four samples: twelve of those to a tile fill the GPU (two to a CU).  With noise,
+# so that a sum in another order would show in the bits of some output; a shared input, so that the other launches show too
+@pytest.mark.parametrize("mixed", [False, True])
+def test_groups_take_one_launch_up_to_what_the_gpu_holds(gpu_device, mixed):
+    rng = np.random.default_rng(9)
+    io = dict(inp_res=1 / 127.0, out_res=-1.0, out_noise=0.1, noise_management=NM.AbsMax)
+    meta = make_meta(io_params(bound_management=BM.Iterative, out_bound=4.0, **io), io_params(**io))
+    sizes = [(96, 64)] * 39 + [(96, 1800 if mixed else 64)]     # alone, the large one takes other launches from 70 samples on
+    grouped = []
+    for k, (x_size, d_size) in enumerate(sizes):
+        host, _orc, _ = build_pair(meta, constant_step(construction_seed=k + 1), x_size, d_size, gpu=False)
+        host.set_weights(torch.from_numpy(rng.uniform(-0.5, 0.5, (d_size, x_size)).astype(F)))
+        grouped.append(tiles.CudaAnalogTile(host))
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+
+    def one_launch(tile, x):
+        tile.set_profiling(True)
+        y = tile.forward(x, False)
+        names = [name for name, _ms in tile.get_profile()][1:]
+        tile.set_profiling(False)
+        return y, names == ["mvm_few"]
+
+    blocks = 39 + (32 if mixed else 1)                           # 1800 outputs: 29 blocks, an eighth of them to each XCD
+    largest = 4 * (2 * cus // blocks)
+    before = torch.from_numpy(rng.uniform(-1, 1, (largest + 1, 96)).astype(F)).cuda()
+    assert one_launch(grouped[0], before)[1]                     # a tile of no group: up to its own limit
+    group = tiles.TileGroup(grouped)
+    for batch in (largest, largest + 1):
+        x = torch.from_numpy(rng.uniform(-1, 1, (batch, 96)).astype(F)).cuda()
+        for k, t in enumerate(grouped):
+            t.set_seed(100 + k)
+        got = group.forward([x] * len(grouped))
+        assert group.get_shared_input_sets() == ((0, 0) if batch == largest else (1, 40))
+        for k, (t, y) in enumerate(zip(grouped, got)):
+            t.set_seed(100 + k)
+            alone, small = one_launch(t, x)
+            assert small == (batch == largest)
+            assert torch.equal(alone, y)                         # the same sums as in the call of the group
+        d = [torch.from_numpy(rng.uniform(-1, 1, (batch, n)).astype(F)).cuda() for _, n in sizes]
+        for k, t in enumerate(grouped):
+            t.set_seed(200 + k)
+        back = group.backward(d)
+        for k, (t, g, v) in enumerate(zip(grouped, d, back)):
+            t.set_seed(200 + k)
+            assert torch.equal(t.backward(g, False), v)
 
 
 def test_small_calls_share_no_quantized_rows(gpu_device):
