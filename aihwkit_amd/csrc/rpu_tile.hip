@@ -102,6 +102,76 @@ template <class A> struct GroupArgs {
   }
 };
 
+// Bytes that a call reads or writes: [begin, end), and where pitch > 0 only `width` bytes of each of its rows, which begin
+// `pitch` apart (a column slice of a larger matrix).
+struct Place {
+  uintptr_t begin, end;
+  size_t pitch, width;
+  Place(const float *p, int rows, long row_stride, int columns, long column_stride) {
+    begin = end = (uintptr_t)p;
+    if (rows > 0 && columns > 0) end += sizeof(float) * ((rows - 1) * row_stride + (columns - 1) * column_stride + 1);
+    width = sizeof(float) * (size_t)std::max(columns, 0);
+    pitch = rows > 1 && column_stride == 1 && row_stride >= columns ? sizeof(float) * (size_t)row_stride : 0;
+  }
+  static Place read_by(const MvmArgs &a) { return Place(a.in, a.m_batch, a.in_sb, a.K - a.in_one, a.in_sk); }
+  static Place written_by(const MvmArgs &a) { return Place(a.out, a.m_batch, a.out_sb, a.O - a.out_drop, a.out_so); }
+};
+// The union of some places, in the order of addresses: whether another one meets it is a binary search.  Slices of one matrix
+// that interleave are told apart where all places have the same pitch.
+class Places {
+public:
+  void clear() {
+    spans.clear();
+    columns.clear();
+    pitch = 0;
+    sorted = false;
+  }
+  void add(const Place &p) {
+    if (p.begin == p.end) return;
+    if (spans.empty()) pitch = p.pitch;
+    else if (pitch != p.pitch) pitch = 0;
+    spans.push_back({p.begin, p.end});
+    if (pitch) add_columns(p, [&](size_t from, size_t to) { columns.push_back({from, to}); });
+    sorted = false;
+  }
+  bool meets(const Place &p) {
+    if (!sorted) {
+      merge(spans);
+      if (pitch) merge(columns);
+      sorted = true;
+    }
+    if (p.begin == p.end || !meets(spans, p.begin, p.end)) return false;
+    if (pitch == 0 || p.pitch != pitch) return true;
+    bool met = false;
+    add_columns(p, [&](size_t from, size_t to) { met = met || meets(columns, from, to); });
+    return met;
+  }
+
+private:
+  typedef std::vector<std::pair<uintptr_t, uintptr_t>> Spans;
+  Spans spans, columns;
+  size_t pitch = 0;
+  bool sorted = false;
+  template <class F> static void add_columns(const Place &p, F f) {
+    const size_t from = p.begin % p.pitch, to = from + p.width;
+    f(from, std::min(to, p.pitch));
+    if (to > p.pitch) f(0, to - p.pitch);
+  }
+  static void merge(Spans &s) {
+    std::sort(s.begin(), s.end());
+    size_t n = 0;
+    for (size_t i = 1; i < s.size(); ++i) {
+      if (s[i].first <= s[n].second) s[n].second = std::max(s[n].second, s[i].second);
+      else s[++n] = s[i];
+    }
+    s.resize(s.empty() ? 0 : n + 1);
+  }
+  static bool meets(const Spans &s, uintptr_t from, uintptr_t to) {
+    const auto after = std::lower_bound(s.begin(), s.end(), std::make_pair(to, (uintptr_t)0)); // the first that begins at or behind `to`
+    return after != s.begin() && (after - 1)->second > from;
+  }
+};
+
 class DeviceGuard {
 public:
   explicit DeviceGuard(int device) {
@@ -649,13 +719,14 @@ struct Tile {
   int small_call_batch(const MvmArgs &a) const {
     return small_calls ? std::min(mvm_few_batch(a), group_batch[a.transposed]) : 0;
   }
-  // Whether the outputs of a call lie among the inputs of one: the workgroups of k_mvm_few read their inputs while others
-  // store outputs; the other launches have quantized the inputs of round 0 before the first output is stored.
-  static bool writes_into(const MvmArgs &from, const MvmArgs &to) {
-    const long in_last = (long)(to.m_batch - 1) * to.in_sb + (long)(to.K - to.in_one - 1) * to.in_sk;
-    const long out_last = (long)(from.m_batch - 1) * from.out_sb + (long)(from.O - from.out_drop - 1) * from.out_so;
-    const uintptr_t in = (uintptr_t)to.in, out = (uintptr_t)from.out;
-    return out <= in + sizeof(float) * in_last && in <= out + sizeof(float) * out_last;
+  // Whether the outputs of a call lie among its inputs: the workgroups of k_mvm_few read their inputs while others store
+  // outputs; the other launches have quantized the inputs of round 0 before the first output is stored.
+  static bool writes_into_its_input(const MvmArgs &a) {
+    const Place in = Place::read_by(a), out = Place::written_by(a);
+    if (out.begin >= in.end || in.begin >= out.end) return false;
+    Places p;
+    p.add(in);
+    return p.meets(out);
   }
   // words 0 to 3: the launches of the rounds, 4 and 5: few_args
   void ensure_seen() {
@@ -943,7 +1014,7 @@ struct Tile {
       ensure_seen();
       ensure_few(s_few, few_counters(a, few_batch), s_dual1, few_rows(a, few_batch), s);
     }
-    if (few_batch == B && !writes_into(a, a)) {
+    if (few_batch == B && !writes_into_its_input(a)) {
       int together = 1;
       if (a.max_rounds > 1) {
         together = few_args(a, s_few.p, s_dual1.p, few_calls++, seen_host + 4, seen_dev + 4);
@@ -2543,6 +2614,7 @@ struct rpu_group {
   DevBuf<int> few_counters; // see Tile::few_args
   DevBuf<float> few_rows;
   int few_calls = 0;
+  Places inputs; // of the last call, kept for its memory
   // host-visible pairs (any tile listed a sample for round 1, batch), one per kernel variant of the group's last call:
   // the next call runs the rounds after round 0 in one launch where nothing was listed
   int *seen_host = nullptr, *seen_dev = nullptr;
@@ -2882,10 +2954,14 @@ static int group_mvm(rpu_group_t *group, const float *const *x_dev, const long *
       t.last_stream = s;
       if (!transposed) t.last_forward_batch = m_batch;
     }
-    for (int i = 0; i < n * n; ++i) {
-      if (!Tile::writes_into(args[i / n], args[i % n])) continue;
-      few.assign(n, 0);
-      break;
+    if (std::find(few.begin(), few.end(), 1) != few.end()) { // (see Tile::writes_into_its_input)
+      group->inputs.clear();
+      for (const MvmArgs &a : args) group->inputs.add(Place::read_by(a));
+      for (int i = 0; i < n; ++i) {
+        if (!few[i] || !group->inputs.meets(Place::written_by(args[i]))) continue;
+        few.assign(n, 0);
+        break;
+      }
     }
     {
       size_t counters = 0, rows = 0;

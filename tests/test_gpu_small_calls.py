@@ -190,3 +190,24 @@ def test_small_calls_onto_their_own_input_equal_the_oracle(gpu_device, size, bat
     outs = (C.c_void_p * 2)(second.data_ptr(), first.data_ptr())
     assert lib().rpu_group_forward(group._g, ins, outs, batch, 0, stream) == 0
     assert np.array_equal(first.cpu().numpy(), want) and np.array_equal(second.cpu().numpy(), want)
+
+
+# input and outputs as column slices of one matrix: their rows interleave, but no element is both; then outputs that begin on
+# the last column of the input, which every tile has to read before any stores.  (The tiles that take the one launch quantize
+# their rows for themselves, the others share them.)
+@pytest.mark.parametrize("over,sets", [(0, (0, 0)), (1, (1, 2))])
+def test_small_calls_on_interleaved_columns(gpu_device, over, sets):
+    rng = np.random.default_rng(12)
+    batch, x_size, outs = 7, 96, (64, 33)
+    pairs = [exact_pair(rng, x_size, d, 8.0 if over else 2.0, 16, seed=k + 1) for k, d in enumerate(outs)]
+    group = tiles.TileGroup([tiles.CudaAnalogTile(host) for host, _ in pairs])
+    buf = torch.from_numpy(grid(rng, 64, (batch, 4 + x_size + sum(outs) + 5), 64.0)).cuda()
+    x = buf[:, 4:4 + x_size]
+    want = [orc.forward(x.cpu().numpy().copy()) for _, orc in pairs]
+    assert not over or max(orc.bm_rounds(batch).max() for _, orc in pairs) == 1   # a second round reads the inputs again
+    at = 4 + x_size - over
+    ys = [buf[:, at:at + outs[0]], buf[:, at + outs[0]:at + sum(outs)]]
+    group.forward([x, x], outs=ys)
+    assert group.get_shared_input_sets() == sets
+    for y, w in zip(ys, want):
+        assert np.array_equal(y.cpu().numpy(), w)
