@@ -293,8 +293,9 @@ struct Tile {
   // round 2; the host-visible pair (samples of the last call that needed round 1, its batch) that the choice between
   // the fused and the separate launches is made from (fused_rounds: -1 by those values, 0 never, 1 .. 3 as forced)
   DevBuf<float> s_dual0, s_dual1, s_dual2, s_xq2;
-  DevBuf<int> s_dsel, s_dhit1, s_dhit2, s_few;
+  DevBuf<int> s_dsel, s_dhit1, s_dhit2;
   int few_calls = 0; // see few_args
+  bool few_cleared = false; // whether few_counters has cleared them
   bool small_calls = true; // rpu_tile_set_small_calls
   // largest batch that the groups of this tile run as k_mvm_few, forward and backward: so does the tile in calls of its own,
   // whose sums are then those of a call of the group
@@ -514,7 +515,7 @@ struct Tile {
   void release_all() {
     d_w.release(); d_wmax.release(); d_wmin.release(); d_sup.release(); d_sdown.release();
     d_slup.release(); d_sldown.release();
-    s_dual0.release(); s_dual1.release(); s_dual2.release(); s_xq2.release(); s_dsel.release(); s_dhit1.release(); s_few.release();
+    s_dual0.release(); s_dual1.release(); s_dual2.release(); s_xq2.release(); s_dsel.release(); s_dhit1.release();
     s_dhit2.release();
     if (seen_host) {
       (void)hipHostFree(seen_host);
@@ -529,7 +530,7 @@ struct Tile {
     last_bl = nullptr; last_a = last_b = nullptr; last_update = UpdateArgs{}; last_in_planes = false;
     t_unit.release(); t_read.release();
     i_ref.release(); i_prog.release(); i_nu_plus.release(); i_nu_minus.release(); i_scalar.release(); i_absmax.release();
-    has_reference = programmed = false;
+    has_reference = programmed = few_cleared = false;
     x_idx.release(); x_idx_t.release(); x_fold_ptr.release(); x_fold_off.release(); fold_image_size = -1;
     x_mat.release(); d_mat.release();
     d_decay.release(); d_diff.release(); d_rbias.release(); s_clip.release();
@@ -630,6 +631,7 @@ struct Tile {
     device_id = target;
     cu_count = 0;
     try {
+      make_counts();
       if (is_transfer()) {
         for (auto &sl : slots) sl->upload(size(), true);
         if (!tr->fully_hidden) {
@@ -646,7 +648,6 @@ struct Tile {
         }
         upload_params();
       }
-      s_count.ensure(MVM_COUNT_WORDS);
       ensure_update_tables();
     } catch (...) {
       release_all();
@@ -690,28 +691,43 @@ struct Tile {
     return true;
   }
 
-  // What a call of k_mvm_few needs beyond mvm_args: few_counters() counters and saturation marks, zero between calls, and
-  // few_rows() floats for the results of rounds 1 and 2 (whether or not this call works on three rounds at once: the next
-  // one may, and be captured).  A larger call on the other launches makes room for its largest small call as well, so that a
-  // program that warmed up on it can capture any smaller one; `batch` is that of the small call.  `seen`: host-visible
-  // numbers of the last call (of this tile or group) in which a sample went on to a second round and of the last call that
-  // has ended.  Returns the rounds to work out together (launch_mvm_few).
-  static size_t few_counters(const MvmArgs &a, int batch) { return a.max_rounds > 1 ? 7 * (size_t)batch : 0; }
-  static size_t few_rows(const MvmArgs &a, int batch) { return a.max_rounds > 2 ? 2 * (size_t)batch * a.O : 0; }
-  static void ensure_few(DevBuf<int> &counters, size_t n_counters, DevBuf<float> &rows, size_t n_rows, hipStream_t s) {
-    if (counters.n < n_counters) {
-      counters.ensure(n_counters);
-      launch_fill(reinterpret_cast<float *>(counters.p), 0.0f, n_counters, s); // all-zero bits
-    }
-    rows.ensure(n_rows);
+  // What a call of k_mvm_few needs beyond mvm_args.  Seven counters and saturation marks per sample, zero between calls: room
+  // for the tile's largest small forward call stands behind the counts of the rounds from the start, so that neither a larger
+  // call nor a captured one has to make any.  The results of rounds 1 and 2 go where the other launches keep quantized rows,
+  // which mvm_args makes large enough.  `seen`: host-visible numbers of the last call (of this tile or group) in which a
+  // sample went on to a second round and of the last call that has ended.  Returns the rounds to work out together
+  // (launch_mvm_few).
+  void make_counts() {
+    MvmArgs a{};
+    a.K = X;
+    a.O = D;
+    a.io = io_dev(fio);
+    a.max_rounds = fio.perfect ? 0 : mvm_max_rounds(a.io);
+    s_count.ensure(MVM_COUNT_WORDS + (a.max_rounds > 1 ? 7 * (size_t)mvm_few_batch(a) : 0));
   }
-  int few_args(MvmArgs &a, int *counters, float *rows, int call_number, const volatile int *seen_host, int *seen_dev) const {
-    a.few = counters;
+  int *few_counters(int batch, hipStream_t s) {
+    const size_t need = MVM_COUNT_WORDS + 7 * (size_t)batch;
+    if (s_count.n < need) { // a pass with settings of its own (io_other) that allow larger small calls than the tile's
+      s_count.ensure(need);
+      few_cleared = false;
+    }
+    if (!few_cleared) {
+      launch_fill(reinterpret_cast<float *>(s_count.p + MVM_COUNT_WORDS), 0.0f, s_count.n - MVM_COUNT_WORDS, s); // all-zero bits
+      hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+      RPU_HIP_CHECK(hipStreamIsCapturing(s, &capturing));
+      few_cleared = capturing == hipStreamCaptureStatusNone; // a captured launch clears when it is replayed
+    }
+    return s_count.p + MVM_COUNT_WORDS;
+  }
+  int few_args(MvmArgs &a, int call_number, const volatile int *seen_host, int *seen_dev, hipStream_t s) {
+    if (a.max_rounds < 2) return 1;
+    a.few = few_counters(a.m_batch, s);
+    a.st.count = s_count.p;
     a.few_seen = seen_dev;
     a.few_call = call_number;
     if (a.max_rounds < 3) return 1;
-    a.dual.buf[1] = rows;
-    a.dual.buf[2] = rows + (size_t)a.m_batch * a.O;
+    a.dual.buf[1] = a.xq[0];
+    a.dual.buf[2] = a.xq[1];
     if (fused_rounds >= 0) return fused_rounds & 1 ? 3 : 1;
     return seen_host[1] - seen_host[0] <= 8 ? 3 : 1;
   }
@@ -761,10 +777,12 @@ struct Tile {
     // large_tiles: whether rounds of this call run on the large-tile kernel (-1: what the shape alone decides)
     const bool tight = large_tiles < 0 ? mvm_uses_large_tiles(B, O) : large_tiles != 0;
     a.k_pad = mvm_k_pad(K, tight);
-    s_xq0.ensure((size_t)B * a.k_pad);
-    if (!io.perfect && io.p.bound_management != RPU_BM_NONE) s_xq1.ensure((size_t)B * a.k_pad);
-    a.xq[0] = s_xq0.p; a.xq[1] = s_xq1.p;
     a.max_rounds = io.perfect ? 0 : mvm_max_rounds(a.io);
+    size_t rows = (size_t)B * a.k_pad;
+    if (a.max_rounds > 2) rows = std::max(rows, (size_t)std::min(B, mvm_few_batch(a)) * O); // see few_args
+    s_xq0.ensure(rows);
+    if (!io.perfect && io.p.bound_management != RPU_BM_NONE) s_xq1.ensure(rows);
+    a.xq[0] = s_xq0.p; a.xq[1] = s_xq1.p;
     // rows for the next bound-management round are quantized ahead when the batch is small (shortest path between
     // rounds) or when at least four workgroups per sample tile share that work; a large batch on a narrow tile
     // quantizes only the rows of the samples that saturated
@@ -1009,16 +1027,10 @@ struct Tile {
 
     prof_begin(s);
     const bool running = io.p.noise_management == RPU_NM_AVERAGE_ABS_MAX || io.p.noise_management == RPU_NM_AVERAGE_ABS_MAX_SINGLE_VALUE;
-    const int few_batch = side || gather || running ? 0 : std::min(B, small_call_batch(a));
-    if (few_batch > 0 && a.max_rounds > 1) {
-      ensure_seen();
-      ensure_few(s_few, few_counters(a, few_batch), s_dual1, few_rows(a, few_batch), s);
-    }
-    if (few_batch == B && !writes_into_its_input(a)) {
-      int together = 1;
-      if (a.max_rounds > 1) {
-        together = few_args(a, s_few.p, s_dual1.p, few_calls++, seen_host + 4, seen_dev + 4);
-      }
+    const int few_batch = side || gather || running ? 0 : small_call_batch(a);
+    if (few_batch > 0 && a.max_rounds > 1) ensure_seen(); // by a larger call too: a small one after it may be captured
+    if (B <= few_batch && !writes_into_its_input(a)) {
+      const int together = a.max_rounds > 1 ? few_args(a, few_calls++, seen_host + 4, seen_dev + 4, s) : 1;
       const MvmArgs *call = &a;
       launch_mvm_few(a, mvm_few_variant(&call, 1), together, s);
       prof_mark(s, "mvm_few");
@@ -2611,9 +2623,7 @@ struct rpu_group {
   int device_id = -1;
   GroupArgs<MvmArgs> mvm_args;
   hipEvent_t copied = nullptr;
-  DevBuf<int> few_counters; // see Tile::few_args
-  DevBuf<float> few_rows;
-  int few_calls = 0;
+  int few_calls = 0; // see Tile::few_args
   Places inputs; // of the last call, kept for its memory
   // host-visible pairs (any tile listed a sample for round 1, batch), one per kernel variant of the group's last call:
   // the next call runs the rounds after round 0 in one launch where nothing was listed
@@ -2673,8 +2683,6 @@ struct rpu_group {
         if (seen_host) (void)hipHostFree(seen_host);
         update_args.release();
         mvm_args.release();
-        few_counters.release();
-        few_rows.release();
         for (auto &b : first_rows) b.release();
       } catch (...) {
       }
@@ -2918,7 +2926,7 @@ static int group_mvm(rpu_group_t *group, const float *const *x_dev, const long *
     bool all_big = use_big;
     // per tile: arguments of a plain forward call (row-major x [m_batch][x_size], y [m_batch][d_size])
     std::vector<MvmArgs> args(n);
-    std::vector<int> depth(n), mode(n), few(n), few_batch(n), few_rounds(n, 1);
+    std::vector<int> depth(n), mode(n), few(n), few_rounds(n, 1);
     if (!group->seen_host) {
       RPU_HIP_CHECK(hipHostMalloc((void **)&group->seen_host, (2 * kSeenPairs + 3) * sizeof(int), hipHostMallocMapped));
       for (int i = 0; i < 2 * kSeenPairs + 3; ++i) group->seen_host[i] = 0; // until the first calls say otherwise
@@ -2947,8 +2955,7 @@ static int group_mvm(rpu_group_t *group, const float *const *x_dev, const long *
       mvm_round_variant(a, depth[i], mode[i]);
       // (the test hook of the waits is about the other launches; the large-tile kernel takes all of its tiles through the
       // lists and marks that the init kernel sets up)
-      few_batch[i] = std::min(m_batch, t.small_call_batch(a));
-      few[i] = !big && !group->wait_spins_hook && !group->wait_extra_hook && few_batch[i] == m_batch ? 1 : 0;
+      few[i] = !big && !group->wait_spins_hook && !group->wait_extra_hook && m_batch <= t.small_call_batch(a) ? 1 : 0;
       rounds = std::max(rounds, a.max_rounds);
       args[i] = a;
       t.last_stream = s;
@@ -2963,22 +2970,11 @@ static int group_mvm(rpu_group_t *group, const float *const *x_dev, const long *
         break;
       }
     }
-    {
-      size_t counters = 0, rows = 0;
-      for (int i = 0; i < n; ++i) {
-        counters += Tile::few_counters(args[i], few_batch[i]);
-        rows += Tile::few_rows(args[i], few_batch[i]);
-      }
-      Tile::ensure_few(group->few_counters, counters, group->few_rows, rows, s);
-      ++group->few_calls;
-      counters = rows = 0;
-      for (int i = 0; i < n; ++i) {
-        if (!few[i]) continue;
-        few_rounds[i] = group->tiles[i]->t.few_args(args[i], group->few_counters.p + counters, group->few_rows.p + rows, group->few_calls,
-                                                    group->seen_host + 2 * kSeenPairs + 1, group->seen_dev + 2 * kSeenPairs + 1);
-        counters += Tile::few_counters(args[i], m_batch);
-        rows += Tile::few_rows(args[i], m_batch);
-      }
+    ++group->few_calls;
+    for (int i = 0; i < n; ++i) {
+      if (!few[i]) continue;
+      few_rounds[i] = group->tiles[i]->t.few_args(args[i], group->few_calls, group->seen_host + 2 * kSeenPairs + 1,
+                                                  group->seen_dev + 2 * kSeenPairs + 1, s);
     }
     // Tiles that quantize the same input the same way (the column blocks of a layer that was split over several
     // tiles) share the rows of rounds 0 and 1: one of them writes the rows, all of them read them.  Rows of later

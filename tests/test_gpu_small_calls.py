@@ -171,6 +171,53 @@ def test_small_calls_after_larger_ones_allocate_nothing(gpu_device, grouped):
     assert lib().rpu_device_allocation_count() == before
 
 
+def test_small_calls_captured_after_a_larger_one(gpu_device):
+    """The tile's first small call is captured, after a larger call only; replays on new inputs, with eager small calls and
+    synchronizations between them, find counters and marks as they have to be."""
+    rng = np.random.default_rng(8)
+    host, orc = exact_pair(rng, 300, 512, 0.5, 16)
+    gpu = tiles.CudaAnalogTile(host)
+    gpu.forward(torch.from_numpy(grid(rng, 64, (1024, 300), 64.0)).cuda(), False)
+    x_dev = torch.zeros(7, 300, device="cuda")
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y_dev = gpu.forward(x_dev, False, False, False, False, True)
+    most = 0
+    for replay in range(5):
+        x = grid(rng, 64, (7, 300), 64.0)
+        if replay % 2:                                           # before and after replays: a call that is not captured
+            assert np.array_equal(gpu.forward(torch.from_numpy(x).cuda(), False).cpu().numpy(), orc.forward(x))
+        x_dev.copy_(torch.from_numpy(x))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(y_dev.cpu().numpy(), orc.forward(x))
+        assert np.array_equal(gpu.get_bm_rounds(7).numpy(), orc.bm_rounds(7))
+        most = max(most, int(orc.bm_rounds(7).max()))
+    assert most >= 3
+
+
+def test_larger_calls_make_no_room_for_small_ones(gpu_device):
+    """The first call of a tile allocates the same number of buffers whether or not it could have small calls after it, and
+    more outputs than inputs (the results of rounds 1 and 2 are rows of outputs) still find their room."""
+    rng = np.random.default_rng(3)
+    allocations = []
+    for small in (True, False):
+        host, orc = exact_pair(rng, 40, 500, 0.5, 16)             # rounds 1 and 2 have samples
+        gpu = tiles.CudaAnalogTile(host)
+        gpu.set_small_calls(small)
+        x = grid(rng, 64, (700, 40), 64.0)
+        before = lib().rpu_device_allocation_count()
+        assert np.array_equal(gpu.forward(torch.from_numpy(x).cuda(), False).cpu().numpy(), orc.forward(x))
+        allocations.append(lib().rpu_device_allocation_count() - before)
+        before = lib().rpu_device_allocation_count()
+        for batch in (200, 3):
+            y = gpu.forward(torch.from_numpy(x[:batch]).cuda(), False).cpu().numpy()
+            assert np.array_equal(y, orc.forward(x[:batch])) and orc.bm_rounds(batch).max() >= 3
+        assert lib().rpu_device_allocation_count() == before or not small
+    assert allocations[0] == allocations[1]
+
+
 # outputs that lie over the inputs of the call (of another tile of the group): the inputs are read before anything is stored
 @pytest.mark.parametrize("size,batch", [(200, 7), (64, 3)])
 def test_small_calls_onto_their_own_input_equal_the_oracle(gpu_device, size, batch):
