@@ -2055,46 +2055,78 @@ __global__ __launch_bounds__(256, XP == 1 && BB == 64 ? 3 : 2) void k_mvm_big(Mv
 // lists nothing, eight launches of 2 to 5 us (large-tile and 32 x 32 kernel, four rounds) become one of 5 us.  A round that
 // does list samples runs on the kernel that its own launch would run it on (XP > 0: large tiles from a.big_from samples on;
 // the sum of an output does not depend on the tile's shape), so results are the same bits; on a few hundred workgroups it
-// takes longer, once: the next call is launched by what this one listed.
+// takes longer: once, as the next call is launched by what this one listed -- but in every replay of a captured call.
+// Nothing here can fail: a round's tiles are taken one by one from a counter, so none belongs to a workgroup that is not
+// running, and the one that finishes a round's last tile goes on at once.  The others wait for it within a limit and leave
+// when it runs out (CUs held by another stream): those that are left then have more tiles each.
+// First saturating call after quiet ones, us, separate launches / this one: 768 -> 2304, 1024 samples 119 / 174, 1024 x 1024,
+// 4096 178 / 282, 300 x 1000, 1300 67 / 63; quiet calls 63 / 48, 81 / 71, 48 / 28.
+
+// adds `mine` to a counter that all workgroups of k_mvm_rest_walk together bring to `total`, and waits until they have, for at
+// most `limit` polls: whether they have
+__device__ __forceinline__ bool walk_wait(int *counter, int mine, int total, int limit, int &sh) {
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int n = mine ? __hip_atomic_fetch_add(counter, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + mine : 0;
+    for (int spins = 0; n < total && spins < limit; ++spins) {
+      if (spins > 0) __builtin_amdgcn_s_sleep(8);
+      n = __hip_atomic_load(counter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    sh = n >= total ? 1 : 0;
+  }
+  __syncthreads();
+  return sh != 0;
+}
+
 template <int WMODE, int XP>
 __global__ __launch_bounds__(256, 2) void k_mvm_rest_walk(MvmArgs a) {
   constexpr int WT = WMODE == 1 ? 1 : 0;
   typedef BigLds<WT, 64, 2, XP ? XP : 1> Big;
   constexpr size_t RED = sizeof(float) * WAVES * 16 * 64, STAGE = sizeof(float) * WAVES * 2 * TILE * LDS_ROW;
   __shared__ __attribute__((aligned(16))) unsigned char lds[RED + STAGE > sizeof(Big) ? RED + STAGE : sizeof(Big)];
+  __shared__ int sh_next;
   float (*red)[16][64] = reinterpret_cast<float (*)[16][64]>(lds);
   float *stage = reinterpret_cast<float *>(lds + RED);
   if (a.dual.on == 2) {
     const int all = workgroups_for(a.O, a.m_batch);
     for (int n = blockIdx.x; n < all; n += gridDim.x) mvm_dual_select(a, n);
   }
-  const RoundWait wt = round_wait_of(a.st.count, a.dual.seen, a.wait_spins, a.wait_extra);
+  const int limit = a.wait_spins > 0 ? a.wait_spins : REST_SPIN_LIMIT;
   for (int r = a.round; r < a.max_rounds; ++r) {
+    // final since the launch before (first round) or since the last tile of the round before
     const int n_act = __hip_atomic_load(&a.st.count[r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     mvm_note_round(a, r, n_act, r == a.round && a.dual.on == 2);
     if (n_act == 0) return; // the same for every workgroup
-    if (r > a.round && !mvm_device_barrier(&a.st.count[MVM_ARRIVE_BASE + 4 * r + 2], (int)gridDim.x, wt, r)) return;
     const bool large = XP != 0 && runs_on_large_tiles(a, r, n_act);
-    if constexpr (XP != 0) {
-      if (large) {
-        const int total = 8 * ((((a.O + 63) / 64) * ((n_act + 63) / 64) + 7) / 8);
-        for (int n = blockIdx.x; n < total; n += gridDim.x) {
+    const int total = large ? 8 * ((((a.O + 63) / 64) * ((n_act + 63) / 64) + 7) / 8) : workgroups_for(a.O, n_act);
+    int *const taken = &a.st.count[MVM_ARRIVE_BASE + 4 * r], *const done = taken + 1, *const visible = taken + 2; // zero at first
+    int mine = 0;
+    for (;;) {
+      __syncthreads(); // LDS is reused by the next tile
+      if (threadIdx.x == 0) sh_next = __hip_atomic_fetch_add(taken, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __syncthreads();
+      const int n = sh_next;
+      if (n >= total) break;
+      ++mine;
+      if constexpr (XP != 0) {
+        if (large) {
           mvm_big_workgroup<WT, 64, 2, XP, false>(a, r, n, 0, *reinterpret_cast<Big *>(lds));
-          __syncthreads(); // LDS is reused by the next tile
+          continue;
         }
       }
-    }
-    const int total = large ? 0 : workgroups_for(a.O, n_act);
-    for (int n = blockIdx.x; n < total; n += gridDim.x) {
       if (a.in_index) {
         int tile_o, tile_b;
         if (tile_of(a, n, n_act, tile_o, tile_b)) mvm_gather_tile_rows(a, r, tile_b, n_act);
       }
       mvm_round_workgroup<1, WMODE>(a, r, n, n_act, red, stage);
-      __syncthreads(); // LDS is reused by the next tile
     }
     if (r + 1 == a.max_rounds) return;
-    if (!mvm_arrive(&a.st.count[MVM_ARRIVE_BASE + 4 * r], (int)gridDim.x, wt, r)) return;
+    // once all tiles are done the next list is final; only if it is not empty does the data have to reach every XCD as well
+    const bool all = walk_wait(done, mine, total, limit, sh_next);
+    if (all && __hip_atomic_load(&a.st.count[r + 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0) continue;
+    if (mine) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+    if (!walk_wait(visible, mine, total, all ? limit : 0, sh_next)) return;
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
   }
 }
 
@@ -3281,6 +3313,7 @@ int mvm_group_rest_resident_limit(int mode) {
 // the two-accumulator kernel).  Its workgroups wait for each other between rounds, so all of them must be resident at
 // once: resident_limit is what the GPU holds of that kernel when nothing else runs on it.  Another launch that holds
 // CUs at that moment (a second stream) can make a wait run out; that is reported (see RoundWait), never passed over.
+// (k_mvm_rest_walk goes on with the workgroups that are running.)
 bool mvm_can_merge_rest(const MvmArgs &a, int resident_limit) {
   if (a.io.perfect || a.io.bound_management == RPU_BM_NONE || a.max_rounds < 3 || a.transposed) return false;
   if (a.pre_add || a.skip_if_zero || a.nm_phase) return false;

@@ -686,9 +686,10 @@ int rpu_tile_set_extra(rpu_tile_t *tile, const int64_t *values_host, int count);
  * rounds after the last one that listed any sample in those calls
  * (the estimate rises at once and falls after eight calls below it), which are expected to be empty, share one
  * launch.  0: always the separate launches.  1 / 2 / 3 / 5 / 7: that shortcut whenever the shape allows it
- * (single tile, rounds on the 32 x 32 kernel, for 2 and 3 no more workgroups than the GPU holds of that kernel at once
- * -- what the occupancy query reports per CU times the CUs --, no per-line periphery terms).
- * The waits of shortcut 2 are bounded (some tens of milliseconds).  They assume that the launch has the GPU's CUs to
+ * (single tile, no per-line periphery terms; 1, 3, 5 and 7: rounds on the 32 x 32 kernel).
+ * A launch of shortcut 2 with a workgroup for every tile of a round, no more of them than the GPU has CUs, waits for all of
+ * its workgroups between rounds; one for larger or gathered calls hands the tiles out to whichever workgroups are running
+ * and cannot fail.  The waits of the former are bounded (some tens of milliseconds).  They assume that the launch has the GPU's CUs to
  * itself; work on another stream that holds CUs at that moment can make a wait run out.  That is never passed over: the
  * launch stops, and the next forward / backward / update call on the tile fails with "forward round barrier timed out
  * ...; results of call N are invalid", after which the tile runs one launch per round (setting a mode again re-arms

@@ -428,3 +428,56 @@ def test_large_calls_share_one_launch_for_the_later_rounds(gpu_device, shape):
         for (y0, r0), (y1, r1) in zip(results[0], other):
             assert np.array_equal(r0, r1)
             assert np.array_equal(y0, y1)
+
+
+def _quiet_and_loud(rng, x_size, d_size, batch):
+    io = noise_free_io(inp_res=1 / 64.0, out_res=1 / 256.0, out_bound=2.0, noise_management=NM.NONE, bound_management=BM.Iterative)
+    w = (rng.integers(-32, 33, (d_size, x_size)) / 64.0).astype(F)
+    host, _orc, _ = build_pair(make_meta(io, noise_free_io()), soft_bounds(construction_seed=3, w_max_dtod=0.0, w_min_dtod=0.0),
+                               x_size, d_size, gpu=False)
+    host.set_weights(torch.from_numpy(w))
+    loud = torch.from_numpy((rng.integers(-64, 65, (batch, x_size)) / 64.0).astype(F)).cuda()
+    quiet = torch.from_numpy((rng.integers(-1, 2, (batch, x_size)) / 64.0).astype(F)).cuda()
+    return host, quiet, loud
+
+
+@pytest.mark.parametrize("shape", [(160, 1100, 1030), (64, 80, 9000), (100, 700, 500)])
+def test_large_calls_go_on_without_the_workgroups_that_stop_waiting(gpu_device, shape):
+    """The launch that walks the rounds of a large call loses every workgroup that has waited for its limit, here one poll:
+    those that are left, at the end the one that finished a round, run the rounds to the same bits, and no call fails."""
+    host, quiet, loud = _quiet_and_loud(np.random.default_rng(shape[1]), *shape)
+    ref, tile = tiles.CudaAnalogTile(host), tiles.CudaAnalogTile(host)
+    ref.set_fused_rounds(0)
+    tile.set_fused_rounds(2)
+    tile.set_round_wait_test_hook(1, 0)
+    for x in (quiet, loud, loud, quiet, loud):
+        tile.set_profiling(True)
+        y = tile.forward(x)
+        assert sum(1 for name, _ms in tile.get_profile() if name == "mvm_round") == 2    # round 0, and all the others
+        tile.set_profiling(False)
+        assert torch.equal(y, ref.forward(x))
+        assert torch.equal(tile.get_bm_rounds(shape[2]), ref.get_bm_rounds(shape[2]))
+    assert ref.get_bm_rounds(shape[2]).max() >= 3
+
+
+@pytest.mark.parametrize("spins", [0, 1])
+def test_more_than_sixteen_rounds_walked_by_one_launch(gpu_device, spins):
+    """As test_more_than_sixteen_rounds_in_one_launch, with more 32 x 32 tiles than the GPU has CUs."""
+    rng = np.random.default_rng(17)
+    x_size, d_size, batch = 96, 64, 4200
+    io = io_params(inp_res=-1.0, out_res=-1.0, out_noise=0.0, out_bound=2e-5, max_bm_factor=1 << 22,
+                   noise_management=NM.AbsMax, bound_management=BM.Iterative)
+    host, _orc, _ = build_pair(make_meta(io, noise_free_io()), soft_bounds(construction_seed=9), x_size, d_size, gpu=False)
+    host.set_weights(torch.from_numpy(rng.uniform(-0.3, 0.3, (d_size, x_size)).astype(F)))
+    x = rng.uniform(-1, 1, (batch, x_size)).astype(F)
+    x[::3] *= F(1 / 64.0)
+    x[::3, 0] = 1.0
+    xin = torch.from_numpy(x).cuda()
+    ref, tile = tiles.CudaAnalogTile(host), tiles.CudaAnalogTile(host)
+    ref.set_fused_rounds(0)
+    tile.set_fused_rounds(2)
+    tile.set_round_wait_test_hook(spins, 0)
+    for _ in range(2):
+        assert torch.equal(tile.forward(xin), ref.forward(xin))
+        rounds = tile.get_bm_rounds(batch)
+        assert torch.equal(rounds, ref.get_bm_rounds(batch)) and rounds.max() >= 18
