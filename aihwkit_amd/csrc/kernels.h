@@ -361,7 +361,7 @@ bool update_reads_row_cost(const UpdateArgs &a); // by its shape: whether the pu
 int update_pulsed_workgroups(const UpdateArgs &a);
 bool update_takes_stream(const UpdateArgs &a); // by its shape: the call may set x_lane_masks (launch_update_lines, launch_update_pulsed)
 int update_mask_columns(const UpdateArgs &a);  // by its shape: the call may set x_lane_masks = 2 with these x_mask_columns; 0: not
-size_t update_mask_words(const UpdateArgs &a, int columns); // 64-bit words that such a call needs at x_planes
+size_t update_mask_room(const UpdateArgs &a, int rows); // 32-bit words at x_planes for calls of up to that many rows of words
 void launch_update_pulsed_group(const UpdateGroup &g, int variant, int total_workgroups, hipStream_t s);
 
 // tables of the update kernels on the current device (once per GPU; blocking copy, no allocation)

@@ -2535,22 +2535,31 @@ bool update_takes_stream(const UpdateArgs &a) {
   return update_pulsed_columns(a) == 1 && a.n_chunks >= 32 && a.m_batch < (1 << 23) &&
          (long)((a.x_size + 63) / 64) * a.d_size <= 4L * current_device_cus();
 }
+// rows of words whose masks have their offsets in 32 bits
+static long mask_rows(int x_size, int cols) { return (1L << 30) / (64L * cols * pulse_mask_spans(x_size, cols)); }
 // Columns per lane of the pulse loop on lane masks (k_update_pulsed_masks), 0: not for this call.  Its launches cost about
 // 4 us more than those on bit planes (a table of 64 KB, masks instead of planes), which a pass has to earn back, and a wave
 // on its own takes as long for a pass as before: it wants batch and units (256 columns per lane of a row) together.
-// Pulse trains and pulse loop of a call, planes / masks, us, soft bounds: 1024 x 1024 64 samples 30.2 / 29.0, 256 63 / 48,
-// 4096 648 / 396; 700 x 700 128 34 / 32, 1024 152 / 110; 512 x 512 128 24.9 / 25.1, 256 36.9 / 33.3; 512 x 256 256 33.4 /
-// 33.7; without noise 1024 x 1024 256 45 / 37, 700 x 700 128 27.0 / 26.6, 512 x 256 4096 228 / 240.
+// Pulse trains and pulse loop of a call, planes / masks, us, soft bounds, bit lines of up to 3 pulses: 1024 x 1024 64 samples
+// 30.2 / 29.0, 256 63 / 48, 4096 648 / 396; 700 x 700 128 34 / 32, 1024 152 / 110; 512 x 512 128 24.9 / 25.1, 256 36.9 / 33.3;
+// 512 x 256 256 33.4 / 33.7; without noise 1024 x 1024 256 45 / 37, 700 x 700 128 27.0 / 26.6, 512 x 256 4096 228 / 240.
+// Update calls with lines of 7 pulses: 1024 x 1024, 256 93 / 70; 700 x 700, 1024 263 / 195; 1024 x 256, 256 58 / 56, without
+// noise 47.8 / 46.9.  Longer ones, walked pulse by pulse by either kernel, of up to 13 and 31: 1024 x 1024, 256 661 / 660 and
+// 2227 / 2203; 700 x 700, 1024 1608 / 1429 and 5754 / 5198, without noise 1387 / 1388 and 4496 / 4499.
 int update_mask_columns(const UpdateArgs &a) {
   const int cols = update_pulsed_columns(a);
   const long spans = pulse_mask_spans(a.x_size, cols), units = spans / 4 * a.d_size, cus = current_device_cus();
   // (bit lines beyond seven pulses are walked as before, from planes and words: no use for lines that are all longer)
-  if (cols == 1 || a.x_index || a.d_group || !(a.up.update_bl_management || a.up.desired_bl <= UPDATE_PLANES_ONLY_KMAX) || 64L * cols * spans * a.m_batch > (1L << 30)) return 0; // offsets of masks in 32 bits
+  if (cols == 1 || a.x_index || a.d_group || !(a.up.update_bl_management || a.up.desired_bl <= UPDATE_PLANES_ONLY_KMAX) || a.m_batch > mask_rows(a.x_size, cols)) return 0;
   return a.m_batch >= 128 && units * a.m_batch >= 512 * cus && units > (a.dev.dw_min_std > 0.0f ? cus : 2 * cus - 1) ? cols : 0;
 }
-// 64-bit words of the masks of a call whose longest bit line has seven pulses
-size_t update_mask_words(const UpdateArgs &a, int columns) {
-  return (size_t)a.m_batch * (size_t)pulse_mask_spans(a.x_size, columns) * UPDATE_PLANES_ONLY_KMAX * 4u * (size_t)columns;
+// Masks of the largest call of at most `rows` rows of words, with a longest bit line of seven pulses.  By the shape of the tile
+// alone: a call on planes makes room for the masks of a smaller one after it.
+size_t update_mask_room(const UpdateArgs &a, int rows) {
+  const int cols = update_pulsed_columns(a);
+  if (cols == 1 || rows < 128) return 0;
+  return 2 * (size_t)std::min((long)rows, mask_rows(a.x_size, cols)) * (size_t)pulse_mask_spans(a.x_size, cols) *
+         UPDATE_PLANES_ONLY_KMAX * 4u * (size_t)cols;
 }
 template <bool NOISE, int C> static void launch_update_pulsed_masks(const UpdateArgs &a, hipStream_t s) {
   const long units = (long)((a.x_size + 256 * C - 1) / (256 * C)) * a.d_size;

@@ -1174,7 +1174,8 @@ struct Tile {
   void set_plane_args(UpdateArgs &a, int B) {
     const int slots = 32; // 31 pulse slots and the sign plane
     const int chunks = (B + 31) / 32;
-    u_xpl.ensure((size_t)chunks * slots * std::max(X, 16)); // 16: lane masks of a row of up to 64 elements
+    // 16: lane masks of a row of up to 64 elements; update_mask_room: those in the order of k_update_pulsed_masks
+    u_xpl.ensure(std::max((size_t)chunks * slots * std::max(X, 16), update_mask_room(a, B)));
     u_dpl.ensure((size_t)chunks * slots * D);
     if (!u_kmax.p) {
       u_kmax.ensure(4);
@@ -1731,8 +1732,6 @@ struct Tile {
         } else if (const int columns = update_mask_columns(a)) {
           a.x_lane_masks = 2;
           a.x_mask_columns = columns;
-          u_xpl.ensure(2 * update_mask_words(a, columns));
-          a.x_planes = u_xpl.p;
         }
       }
       launch_update_lines(a, s);

@@ -81,3 +81,19 @@ def test_pulse_loop_on_lane_masks_with_weights_outside_their_bounds(storage_mode
     assert torch.equal(results[0], results[1])
     assert bool((results[0][:, ::15] == 2.5).all())   # no x pulse: untouched
     assert float(results[0][:, 3].max()) < 2.5
+
+
+def test_masks_find_their_room_after_a_larger_call_on_planes(gpu_device):
+    """A row of 513 elements has masks for 1024: more words for 600 samples than bit planes for 1024 of them.  The larger call
+    (of a group: bit planes) makes room for both, so that the smaller one can be captured."""
+    from aihwkit_amd._cabi import lib
+    from aihwkit_amd.rpu_base.tiles import TileGroup
+    x, d = _data(513, 301, 1024, 0)
+    tile = _tile(513, 301, _device("soft_bounds"))
+    tile.set_learning_rate(0.01)
+    group = TileGroup([tile])
+    for _ in range(2):
+        group.update([x], [d])
+    before = lib().rpu_device_allocation_count()
+    tile.update(x[:600].contiguous(), d[:600].contiguous(), False)
+    assert lib().rpu_device_allocation_count() == before
