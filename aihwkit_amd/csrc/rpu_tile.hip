@@ -87,9 +87,10 @@ template <class A> struct GroupArgs {
     table_words = (n_table + 3) / 4 * 2;
     const size_t words = table_words + n_args * (sizeof(A) / 8);
     dev.ensure(words);
-    RPU_HIP_CHECK(hipHostMalloc((void **)&host, 8 * words, hipHostMallocMapped));
+    if (!host) RPU_HIP_CHECK(hipHostMalloc((void **)&host, 8 * words, hipHostMallocMapped));
     RPU_HIP_CHECK(hipHostGetDevicePointer((void **)&host_on_dev, host, 0));
   }
+  bool made() const { return host_on_dev != nullptr; } // the last step of make
   int *table() { return reinterpret_cast<int *>(host); }
   A *args() { return reinterpret_cast<A *>(host + 8 * table_words); }
   const int *dev_table() const { return reinterpret_cast<const int *>(dev.p); }
@@ -97,7 +98,7 @@ template <class A> struct GroupArgs {
   void upload(size_t n_args, hipStream_t s) { launch_upload(dev.p, host_on_dev, table_words + n_args * (sizeof(A) / 8), s); }
   void release() {
     if (host) (void)hipHostFree(host);
-    host = nullptr;
+    host = host_on_dev = nullptr;
     dev.release();
   }
 };
@@ -746,8 +747,8 @@ struct Tile {
   }
   // words 0 to 3: the launches of the rounds, 4 and 5: few_args
   void ensure_seen() {
-    if (seen_host) return;
-    RPU_HIP_CHECK(hipHostMalloc((void **)&seen_host, 6 * sizeof(int), hipHostMallocMapped));
+    if (seen_dev) return; // the last step
+    if (!seen_host) RPU_HIP_CHECK(hipHostMalloc((void **)&seen_host, 6 * sizeof(int), hipHostMallocMapped));
     for (int i = 0; i < 6; ++i) seen_host[i] = 0; // until the first calls say otherwise
     RPU_HIP_CHECK(hipHostGetDevicePointer((void **)&seen_dev, seen_host, 0));
   }
@@ -2726,7 +2727,7 @@ int rpu_group_update_strided(rpu_group_t *group, const float *const *x_dev, cons
     DeviceGuard dg(group->device_id);
     hipStream_t s = (hipStream_t)stream;
     const int n = (int)group->tiles.size();
-    if (!group->update_args.host) {
+    if (!group->update_args.made()) {
       // per tile the arguments of the kernels that make the lines and, after those of all tiles, the view that the
       // cross-point kernels take (the same, or with x and d exchanged for a tile that stores [x_size][d_size])
       group->update_args.make(2 * (size_t)n, 2 * (size_t)n + 16);
@@ -2926,13 +2927,13 @@ static int group_mvm(rpu_group_t *group, const float *const *x_dev, const long *
     // per tile: arguments of a plain forward call (row-major x [m_batch][x_size], y [m_batch][d_size])
     std::vector<MvmArgs> args(n);
     std::vector<int> depth(n), mode(n), few(n), few_rounds(n, 1);
-    if (!group->seen_host) {
-      RPU_HIP_CHECK(hipHostMalloc((void **)&group->seen_host, (2 * kSeenPairs + 3) * sizeof(int), hipHostMallocMapped));
-      for (int i = 0; i < 2 * kSeenPairs + 3; ++i) group->seen_host[i] = 0; // until the first calls say otherwise
-      RPU_HIP_CHECK(hipHostGetDevicePointer((void **)&group->seen_dev, group->seen_host, 0));
+    if (!group->seen_dev) { // made last
       hipDeviceProp_t prop;
       RPU_HIP_CHECK(hipGetDeviceProperties(&prop, group->device_id));
       group->cu_count = prop.multiProcessorCount;
+      if (!group->seen_host) RPU_HIP_CHECK(hipHostMalloc((void **)&group->seen_host, (2 * kSeenPairs + 3) * sizeof(int), hipHostMallocMapped));
+      for (int i = 0; i < 2 * kSeenPairs + 3; ++i) group->seen_host[i] = 0; // until the first calls say otherwise
+      RPU_HIP_CHECK(hipHostGetDevicePointer((void **)&group->seen_dev, group->seen_host, 0));
     }
     int rounds = 1;
     bool storage_xd = false;
