@@ -1743,7 +1743,7 @@ struct Tile {
         prof_mark(s, "update_aggregated");
       } else {
         launch_update_pulsed(a, s);
-        prof_mark(s, "update_pulsed");
+        prof_mark(s, a.x_lane_masks == 2 ? "update_pulsed_masks" : a.x_lane_masks ? "update_pulsed_stream" : "update_pulsed");
       }
     } else {
       launch_update_implicit_lines(a, s);

@@ -35,12 +35,12 @@ SPLIT_MFMA_PEAK_TFLOPS = 2500.0 / 3  # dense bf16 matrix, three products per ele
 # FETCH_SIZE / WRITE_SIZE are KiB per dispatch; a device copy of 64 MiB in the same runs reads FETCH_SIZE = 32782 and
 # WRITE_SIZE = 65536, so FETCH_SIZE is scaled by 2.0 and WRITE_SIZE by 1.0.
 PMC_TRAFFIC_BYTES = {
-    "k_update_pulsed": (16615 * 2.0 + 4096 * 1.0) * 1024,  # k_update_pulsed_masks
+    "k_update_pulsed_masks": (16615 * 2.0 + 4096 * 1.0) * 1024,
     "k_mvm_round": (6851 * 2.0 + 2115 * 1.0) * 1024,  # a round over all 256 samples
     # the launches of a forward call whose rounds 0 to 2 share one launch: k_mvm_dual<0, 3>, then k_mvm_rounds_rest
     "forward_fused_3": ((14557 + 586) * 2.0 + (3157 + 1024) * 1.0) * 1024,
 }
-PMC_SOURCE = {"k_update_pulsed": "profiles/k_update_pulsed_masks_config2.txt", "k_mvm_round": "profiles/k_mvm_round_config2.txt",
+PMC_SOURCE = {"k_update_pulsed_masks": "profiles/k_update_pulsed_masks_config2.txt", "k_mvm_round": "profiles/k_mvm_round_config2.txt",
               "forward_fused_3": "profiles/k_mvm_dual_config2.txt"}
 
 
@@ -244,6 +244,11 @@ def main() -> int:
         # (ms, launches) of a call's contraction: its round launches, or the one launch that runs a small batch
         return prof["mvm_few"] if "mvm_few" in prof else prof["mvm_round"]
 
+    def pulse_loop(prof):
+        # (kernel, ms) of the pulse loop of an update call: its plain form, the one on lane masks, the pipelined one
+        name = next(k for k in prof if k.startswith("update_pulsed"))
+        return "k_" + name, prof[name][0]
+
     def backward_kernel(prof):
         return "k_mvm_few (whole call)" if "mvm_few" in prof else "k_mvm_round"
 
@@ -332,9 +337,9 @@ def main() -> int:
                         "kernels_ms": {k: v[0] for k, v in px_f.items()}, "round_launches": contraction(px_f)[1]},
             "backward": {"ms_per_call": msx_b, "gflops": fl / (msx_b * 1e-3) / 1e9,
                          "kernels_ms": {k: v[0] for k, v in px_b.items()}},
-            "roofline": {"kernel": "k_update_pulsed", "bound": "hbm", "achieved": ubytes / (px_u["update_pulsed"][0] * 1e-3) / 1e9,
-                         "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": ubytes / (px_u["update_pulsed"][0] * 1e-3) / 1e9 / HBM_PEAK_GBS,
-                         "traffic": None, "algorithmic_bytes": ubytes, "kernel_ms": px_u["update_pulsed"][0]},
+            "roofline": {"kernel": pulse_loop(px_u)[0], "bound": "hbm", "achieved": ubytes / (pulse_loop(px_u)[1] * 1e-3) / 1e9,
+                         "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": ubytes / (pulse_loop(px_u)[1] * 1e-3) / 1e9 / HBM_PEAK_GBS,
+                         "traffic": None, "algorithmic_bytes": ubytes, "kernel_ms": pulse_loop(px_u)[1]},
             "roofline_forward": {"kernel": "all round launches of a call", "bound": "mfma",
                                  "achieved": fl / (contraction(px_f)[0] * 1e-3) / 1e12, "peak": FP32_MFMA_PEAK_TFLOPS,
                                  "unit": "TFLOP/s", "frac": fl / (contraction(px_f)[0] * 1e-3) / 1e12 / FP32_MFMA_PEAK_TFLOPS,
@@ -414,9 +419,9 @@ def main() -> int:
         prof_u8 = kernel_ms(lambda: tile.update(xg[:8].contiguous(), dg[:8].contiguous(), False, False, False, True), 10)
         tile.set_profiling(False)
         bytes8 = bytes_per_device * x_size * d_size + 4.0 * (x_size + d_size) * 8
-        other["update_batch_8"] = {"kernel": "k_update_pulsed", "kernel_ms": prof_u8["update_pulsed"][0],
-                                   "gbs": bytes8 / (prof_u8["update_pulsed"][0] * 1e-3) / 1e9,
-                                   "frac_of_hbm_peak": bytes8 / (prof_u8["update_pulsed"][0] * 1e-3) / 1e9 / HBM_PEAK_GBS,
+        other["update_batch_8"] = {"kernel": pulse_loop(prof_u8)[0], "kernel_ms": pulse_loop(prof_u8)[1],
+                                   "gbs": bytes8 / (pulse_loop(prof_u8)[1] * 1e-3) / 1e9,
+                                   "frac_of_hbm_peak": bytes8 / (pulse_loop(prof_u8)[1] * 1e-3) / 1e9 / HBM_PEAK_GBS,
                                    "note": "algorithmic bytes over kernel time; the calls repeat on the same 32 MB of "
                                            "arrays, part of which the memory-side cache still holds from the call "
                                            "before, so this can exceed what HBM alone delivers"}
@@ -424,7 +429,7 @@ def main() -> int:
     devices_per_call = float(x_size) * d_size * batch
     flops_per_call = 2.0 * x_size * d_size * batch
     update_bytes = bytes_per_device * x_size * d_size + 4.0 * (x_size + d_size) * batch
-    k_update_ms = prof_update["update_pulsed"][0]
+    k_update, k_update_ms = pulse_loop(prof_update)
     k_fwd_ms = contraction(prof_forward)[0]   # all round launches of one forward call
     fused_forward = contraction(prof_forward)[1] < 5 and args.config == 2  # rounds 0 and 1 ran as one launch
     fused_3 = fused_forward and contraction(prof_forward)[1] == 2           # rounds 0 to 2, then one launch for the rest
@@ -458,11 +463,11 @@ def main() -> int:
                             "launch (rpu_tile_set_fused_rounds, default: by what its last calls needed); same outputs"},
         "backward": {"ms_per_call": ms_backward, "gflops": flops_per_call / (ms_backward * 1e-3) / 1e9,
                      "kernels_ms": {k: v[0] for k, v in prof_backward.items()}},
-        "roofline": {"kernel": "k_update_pulsed", "bound": "hbm", "achieved": update_bytes / (k_update_ms * 1e-3) / 1e9,
+        "roofline": {"kernel": k_update, "bound": "hbm", "achieved": update_bytes / (k_update_ms * 1e-3) / 1e9,
                      "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": update_bytes / (k_update_ms * 1e-3) / 1e9 / HBM_PEAK_GBS,
-                     "traffic": PMC_TRAFFIC_BYTES["k_update_pulsed"] if args.config == 2 else None,
-                     "traffic_source": ("constant from " + PMC_SOURCE["k_update_pulsed"] + " (rocprofv3 --pmc FETCH_SIZE / "
+                     "traffic": PMC_TRAFFIC_BYTES["k_update_pulsed_masks"] if args.config == 2 else None,
+                     "traffic_source": ("constant from " + PMC_SOURCE["k_update_pulsed_masks"] + " (rocprofv3 --pmc FETCH_SIZE / "
                                         "WRITE_SIZE), not measured in this run") if args.config == 2 else None,
                      "algorithmic_bytes": update_bytes, "kernel_ms": k_update_ms},
         "roofline_forward": {"kernel": "k_mvm_dual + k_mvm_rounds_rest (all rounds of a call)" if fused_forward

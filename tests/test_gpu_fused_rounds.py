@@ -22,6 +22,7 @@ def both_ways(meta, dev, x_size, d_size, w, x, seed=5, bias=False, x_trans=False
     xin = torch.from_numpy(np.ascontiguousarray(x.T if x_trans else x)).cuda()
     for mode in (0, 1, 2, 3, 5, 7, -1):              # -1: the tile's own choice, which changes from call to call
         gpu = tiles.CudaAnalogTile(host)
+        gpu.set_small_calls(False)                   # those have no launches to share
         gpu.set_fused_rounds(mode)
         gpu.set_seed(seed)
         outs = []
@@ -135,6 +136,7 @@ def test_groups_share_one_launch_for_the_later_rounds_and_recover(gpu_device):
             host.set_weights(torch.from_numpy(w))
             orc.set_weights(w)
             grouped.append(tiles.CudaAnalogTile(host))
+            grouped[-1].set_small_calls(False)
             oracles.append(orc)
         group = tiles.TileGroup(grouped)
         sizes = [t.get_x_size() for t in grouped]
@@ -420,7 +422,11 @@ def test_large_calls_share_one_launch_for_the_later_rounds(gpu_device, shape):
         gpu.set_fused_rounds(mode)
         outs = []
         for x in [quiet] * 3 + [loud] * 2 + [quiet] * 2:
+            gpu.set_profiling(True)
             y = gpu.forward(torch.from_numpy(x).cuda()).cpu().numpy()
+            launches = sum(1 for name, _ms in gpu.get_profile() if name == "mvm_round")
+            assert mode < 0 or (launches == 2) == (mode == 2)     # round 0, and all the others
+            gpu.set_profiling(False)
             outs.append((y, gpu.get_bm_rounds(batch).numpy().copy()))
         results.append(outs)
     assert results[0][0][1].max() == 1 and results[0][3][1].max() >= 3

@@ -1,10 +1,11 @@
 """The pulse loop of tiles with several columns per lane runs on lane masks (k_update_pulsed_masks) where batch and rows are
 many enough (update_mask_columns).  A group call runs the plain pulse loop on the same pulse trains and noise streams, so
 both leave the same weights, bit for bit."""
+import numpy as np
 import pytest
 import torch
 
-from helpers import constant_step, soft_bounds
+from helpers import constant_step, make_meta, soft_bounds
 from test_gpu_pulse_stream import _additive, _tile
 
 pytestmark = pytest.mark.gpu
@@ -18,6 +19,14 @@ def _device(kind):
     if kind == "quiet":
         return soft_bounds(construction_seed=5, dw_min_std=0.0)
     return _additive(0.3 if kind == "additive" else 0.0)
+
+
+def _update(tile, kernel, *args):
+    """An update that has to run its pulse loop on that kernel."""
+    tile.set_profiling(True)
+    tile.update(*args)
+    assert [name for name, _ms in tile.get_profile()][-1] == kernel
+    tile.set_profiling(False)
 
 
 def _data(x_size, d_size, batch, sparse):
@@ -47,9 +56,9 @@ def test_pulse_loop_on_lane_masks_equals_the_plain_one(x_size, d_size, batch, lr
     group = TileGroup([other])
     for call in range(2):
         if call:  # lines along the batch
-            one.update(x.t().contiguous(), d.t().contiguous(), False, True, True)
+            _update(one, "update_pulsed_masks", x.t().contiguous(), d.t().contiguous(), False, True, True)
         else:
-            one.update(x, d, False)
+            _update(one, "update_pulsed_masks", x, d, False)
         group.update([x], [d])
     assert torch.equal(one.get_weights(), other.get_weights())
     assert not torch.equal(one.get_weights(), start)
@@ -76,7 +85,7 @@ def test_pulse_loop_on_lane_masks_with_weights_outside_their_bounds(storage_mode
         if grouped:
             TileGroup([tile]).update([x], [d])
         else:
-            tile.update(x, d, False)
+            _update(tile, "update_pulsed_masks", x, d, False)
         results.append(w.clone())
     assert torch.equal(results[0], results[1])
     assert bool((results[0][:, ::15] == 2.5).all())   # no x pulse: untouched
@@ -95,5 +104,31 @@ def test_masks_find_their_room_after_a_larger_call_on_planes(gpu_device):
     for _ in range(2):
         group.update([x], [d])
     before = lib().rpu_device_allocation_count()
-    tile.update(x[:600].contiguous(), d[:600].contiguous(), False)
+    _update(tile, "update_pulsed_masks", x[:600].contiguous(), d[:600].contiguous(), False)
     assert lib().rpu_device_allocation_count() == before
+
+
+@pytest.mark.parametrize("name,value", [("slope_up", float("nan")), ("dwmin_down", float("inf")), ("max_bound", float("inf"))])
+def test_pulse_loop_on_lane_masks_with_parameters_that_are_not_finite(name, value):
+    """They reach the cross-points that hold them, in the plain loop's way, and no other."""
+    from aihwkit_amd.rpu_base import tiles
+    from aihwkit_amd.rpu_base.tiles import TileGroup
+    x_size, d_size, batch = 600, 400, 300
+    host = make_meta(desired_bl=31).create_array(x_size, d_size, soft_bounds(construction_seed=5))
+    hidden = host.get_hidden_parameters()
+    hidden[host.get_hidden_parameter_names().index(name), :, ::3] = value
+    host.set_hidden_parameters(hidden)
+    host.set_weights(torch.from_numpy(np.random.default_rng(3).uniform(-0.4, 0.4, (d_size, x_size)).astype(np.float32)))
+    x, d = _data(x_size, d_size, batch, 0)
+    x[:, ::5] = 0.0
+    one, other = tiles.CudaAnalogTile(host), tiles.CudaAnalogTile(host)
+    before = one.get_weights().numpy()
+    for tile in (one, other):
+        tile.set_seed(17)
+        tile.set_learning_rate(0.01)
+    _update(one, "update_pulsed_masks", x, d, False)
+    TileGroup([other]).update([x], [d])
+    mine, theirs = one.get_weights().numpy(), other.get_weights().numpy()
+    assert np.array_equal(mine, theirs, equal_nan=True)
+    assert np.array_equal(mine[:, ::5], before[:, ::5], equal_nan=True)
+    assert np.isfinite(mine[:, 1::3]).all() and not np.array_equal(mine, before, equal_nan=True)
