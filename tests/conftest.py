@@ -28,7 +28,7 @@ def gpu_device():
 BOTH_STORAGES = ("test_gpu_parity", "test_gpu_statistics", "test_gpu_benchmark_configs", "test_gpu_fused_rounds",
                  "test_gpu_group_update", "test_gpu_inference", "test_gpu_indexed", "test_gpu_long_batches",
                  "test_gpu_state", "test_gpu_hwa", "test_zz_no_alloc", "test_gpu_pulse_stream",
-                 "test_gpu_large_tiles")
+                 "test_gpu_large_tiles", "test_gpu_pulse_masks", "test_gpu_small_calls")
 
 
 def pytest_generate_tests(metafunc):

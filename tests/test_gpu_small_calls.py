@@ -258,3 +258,41 @@ def test_small_calls_on_interleaved_columns(gpu_device, over, sets):
     assert group.get_shared_input_sets() == sets
     for y, w in zip(ys, want):
         assert np.array_equal(y.cpu().numpy(), w)
+
+
+# What is random in the converters, drawn for element, sample and round: a tile of the same seed in the launches of larger
+# batches draws the same.  Weights and inputs on a grid, so that sums in any order are the same bits; only noise on the inputs
+# takes them off it: sums of at most 300 terms below 1, each partial sum off by half an ulp of at most 2^-15 (300 < 2^9)
+@pytest.mark.parametrize("settings,off", [
+    (dict(out_noise=0.06), 0.0), (dict(inp_sto_round=True), 0.0), (dict(out_sto_round=True), 0.0),
+    (dict(out_noise=0.2, out_asymmetry=0.1, inp_asymmetry=0.5, out_res=-1.0), 0.0),
+    (dict(inp_noise=0.02, out_res=-1.0), 300 * 2.0 ** -16)])
+@pytest.mark.parametrize("x_size,d_size,batch,bias", [(130, 128, 1, False), (300, 512, 7, True), (64, 700, 3, False), (200, 65, 101, False)])
+def test_small_calls_draw_what_larger_ones_draw(gpu_device, settings, off, x_size, d_size, batch, bias):
+    rng = np.random.default_rng(x_size)
+    f_io = noise_free_io(**{**dict(inp_res=1 / 64.0, out_res=1 / 512.0, noise_management=NM.AbsMax,
+                                   bound_management=BM.Iterative, out_bound=1.0), **settings})
+    b_io = noise_free_io(**{**dict(inp_res=1 / 64.0, out_res=1 / 512.0, noise_management=NM.Max), **settings})
+    dev = constant_step(w_max_dtod=0.0, w_min_dtod=0.0, w_max=1.0, w_min=-1.0, construction_seed=1)
+    host, _orc, _ = build_pair(make_meta(f_io, b_io), dev, x_size, d_size, gpu=False)
+    host.set_weights(torch.from_numpy(grid(rng, 16, (d_size, x_size), 64.0)))
+    x = torch.from_numpy(grid(rng, 64, (batch, x_size - int(bias)), 64.0)).cuda()
+    d = torch.from_numpy(grid(rng, 64, (batch, d_size), 64.0)).cuda()
+    for mode in (0, 1):                              # round by round, rounds 0 to 2 together
+        tile = tiles.CudaAnalogTile(host)
+        tile.set_fused_rounds(mode)
+        got = []
+        for small in (False, True):
+            tile.set_small_calls(small)
+            tile.set_seed(11)
+            tile.set_profiling(True)
+            y = tile.forward(x, bias)
+            assert ([name for name, _ms in tile.get_profile()][1:] == ["mvm_few"]) == small
+            tile.set_profiling(False)
+            got.append((y, tile.get_bm_rounds(batch), tile.backward(d, bias)))
+        (y0, r0, g0), (y1, r1, g1) = got
+        assert torch.equal(r0, r1) and r0.max() >= 3
+        # (the output of a sample is scaled back by what its rounds scaled the input down)
+        scale = float(y0.abs().max()) if off else 1.0
+        assert float((y0 - y1).abs().max()) <= off * scale and float((g0 - g1).abs().max()) <= off
+        assert not off or float((y0 - y1).abs().max()) > 0.0      # noise did take them off the grid

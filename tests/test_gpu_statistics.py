@@ -7,7 +7,7 @@ import torch
 
 from aihwkit_amd.rpu_base import devices as dv
 from aihwkit_amd.rpu_base import tiles
-from helpers import build_pair, config2, config2_data, constant_step, io_params, make_meta, soft_bounds
+from helpers import build_pair, config2, config2_data, constant_step, io_params, make_meta, noise_free_io, soft_bounds
 
 pytestmark = pytest.mark.gpu
 
@@ -403,3 +403,43 @@ def test_discretized_pulse_probabilities_moments(gpu_device):
         orc.update(x, d)
         dwo.append(orc.get_weights() - w0)
     compare_moments(np.stack(dwg), np.stack(dwo), "discretized pulse probabilities")
+
+
+def _philox(c0, c1, c2, c3, k0, k1):
+    """Philox4x32-10 (Salmon et al., 2011) on arrays of counters."""
+    m = np.uint64(0xFFFFFFFF)
+    c = [np.broadcast_to(np.asarray(v, np.uint64), np.broadcast(c0, c1).shape) for v in (c0, c1, c2, c3)]
+    for r in range(10):
+        p0, p1 = c[0] * np.uint64(0xD2511F53), c[2] * np.uint64(0xCD9E8D57)
+        a, b = np.uint64((k0 + r * 0x9E3779B9) & 0xFFFFFFFF), np.uint64((k1 + r * 0xBB67AE85) & 0xFFFFFFFF)
+        c = [(p1 >> np.uint64(32)) ^ c[1] ^ a, p1 & m, (p0 >> np.uint64(32)) ^ c[3] ^ b, p0 & m]
+    return c
+
+
+@pytest.mark.parametrize("batch,d_size", [(1024, 1024), (5, 4096)])
+def test_output_noise_against_64_bits(gpu_device, batch, d_size):
+    """Normal numbers of the ADC stage: with no weights and a spread of one they are the outputs.  The hardware's logarithm,
+    square root, sine and cosine are off by about an ulp each, of a radius of at most sqrt(2 ln 2^24) = 5.8: 2e-6 is three of
+    its ulps and a half.  Root mean square 6.1e-8 over all pairs; a correctly rounded root of -2 ln u and an angle in radians
+    had 1.3e-7."""
+    seed = 0x1234567890ABCDEF
+    io = io_params(inp_res=-1.0, out_res=-1.0, out_noise=1.0, out_bound=1000.0)
+    dev = constant_step(construction_seed=1, w_max_dtod=0.0, w_min_dtod=0.0)     # (no bound below zero cuts a weight)
+    host, _orc, _ = build_pair(make_meta(io, noise_free_io()), dev, 8, d_size, gpu=False)
+    host.set_weights(torch.zeros(d_size, 8))
+    assert not host.get_weights().any()
+    tile = tiles.CudaAnalogTile(host)
+    tile.set_seed(seed)
+    y = tile.forward(torch.ones(batch, 8, device="cuda"), False).cpu().numpy().astype(np.float64)
+    b, o4 = np.meshgrid(np.arange(batch, dtype=np.uint64), np.arange(d_size // 4, dtype=np.uint64), indexing="ij")
+    r = _philox(o4, b, 0, 1, seed & 0xFFFFFFFF, seed >> 32)
+    want = np.empty((batch, d_size // 4, 4))
+    for pair in range(2):
+        u = ((r[2 * pair] >> np.uint64(8)).astype(np.float64) + 1.0) / 2.0 ** 24
+        turns = (r[2 * pair + 1] >> np.uint64(8)).astype(np.float64) / 2.0 ** 24
+        radius = np.sqrt(-2.0 * np.log(u))
+        want[..., 2 * pair] = radius * np.cos(2.0 * np.pi * turns)
+        want[..., 2 * pair + 1] = radius * np.sin(2.0 * np.pi * turns)
+    off = y - want.reshape(batch, d_size)
+    assert np.abs(off).max() <= 2e-6
+    assert np.sqrt((off ** 2).mean()) <= 1e-7
