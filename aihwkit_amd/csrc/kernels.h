@@ -197,6 +197,7 @@ int mvm_few_group_batch(long blocks);
 int mvm_few_variant(const MvmArgs *const *calls, int n); // blocks of a launch of n calls; the results do not depend on it
 int mvm_few_workgroups(const MvmArgs &a, int variant);
 void launch_mvm_few(const MvmArgs &a, int variant, int rounds, hipStream_t s);
+void launch_mvm_few_clear_group(const MvmGroup &g, hipStream_t s); // the counters of its calls
 void launch_mvm_few_group(const MvmGroup &g, int variant, int rounds, bool w_oc, int max_k, int total_workgroups, hipStream_t s);
 
 // Fused convolution forward (unfold + noisy MVM with its bound-management rounds) for tiles of at most 32 outputs:

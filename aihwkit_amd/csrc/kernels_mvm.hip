@@ -2580,6 +2580,13 @@ __global__ __launch_bounds__(256) void k_mvm_few(MvmArgs a) {
   if (f.block_of((int)blockIdx.x, block_b, block_o)) f.run(block_b, block_o);
 }
 
+// counters and marks of the tiles of a group, a workgroup for each tile
+__global__ __launch_bounds__(256) void k_mvm_few_clear_group(MvmGroup g) {
+  const MvmArgs &a = g.args[blockIdx.x];
+  if (a.max_rounds < 2) return;
+  for (int i = (int)threadIdx.x; i < 7 * a.m_batch; i += 256) a.few[i] = 0;
+}
+
 // several tiles in one launch: start[t] .. start[t + 1] are the workgroups of tile t
 template <bool WOC, int S, int OB, int R>
 __global__ __launch_bounds__(256) void k_mvm_few_group(MvmGroup g) {
@@ -3502,6 +3509,10 @@ void launch_mvm_few(const MvmArgs &a, int variant, int rounds, hipStream_t s) {
 #define RPU_LAUNCH_FEW(S, OB) RPU_LAUNCH_FEW_AS(k_mvm_few, a, a.K, a.w_oc, rounds, S, OB)
   RPU_FEW_VARIANT(variant, RPU_LAUNCH_FEW)
 #undef RPU_LAUNCH_FEW
+}
+
+void launch_mvm_few_clear_group(const MvmGroup &g, hipStream_t s) {
+  hipLaunchKernelGGL(k_mvm_few_clear_group, dim3((unsigned)g.n), dim3(256), 0, s, g);
 }
 
 void launch_mvm_few_group(const MvmGroup &g, int variant, int rounds, bool w_oc, int max_k, int total_workgroups, hipStream_t s) {

@@ -296,7 +296,7 @@ struct Tile {
   DevBuf<float> s_dual0, s_dual1, s_dual2, s_xq2;
   DevBuf<int> s_dsel, s_dhit1, s_dhit2;
   int few_calls = 0; // see few_args
-  bool few_cleared = false; // whether few_counters has cleared them
+  size_t few_zero = 0; // words for k_mvm_few that are zero between calls
   bool small_calls = true; // rpu_tile_set_small_calls
   // largest batch that the groups of this tile run as k_mvm_few, forward and backward: so does the tile in calls of its own,
   // whose sums are then those of a call of the group
@@ -531,7 +531,8 @@ struct Tile {
     last_bl = nullptr; last_a = last_b = nullptr; last_update = UpdateArgs{}; last_in_planes = false;
     t_unit.release(); t_read.release();
     i_ref.release(); i_prog.release(); i_nu_plus.release(); i_nu_minus.release(); i_scalar.release(); i_absmax.release();
-    has_reference = programmed = few_cleared = false;
+    has_reference = programmed = false;
+    few_zero = 0;
     x_idx.release(); x_idx_t.release(); x_fold_ptr.release(); x_fold_off.release(); fold_image_size = -1;
     x_mat.release(); d_mat.release();
     d_decay.release(); d_diff.release(); d_rbias.release(); s_clip.release();
@@ -694,10 +695,10 @@ struct Tile {
 
   // What a call of k_mvm_few needs beyond mvm_args.  Seven counters and saturation marks per sample, zero between calls: room
   // for the tile's largest small forward call stands behind the counts of the rounds from the start, so that neither a larger
-  // call nor a captured one has to make any.  The results of rounds 1 and 2 go where the other launches keep quantized rows,
-  // which mvm_args makes large enough.  `seen`: host-visible numbers of the last call (of this tile or group) in which a
-  // sample went on to a second round and of the last call that has ended.  Returns the rounds to work out together
-  // (launch_mvm_few).
+  // call nor a captured one has to make any; a call clears what none before it has.  The results of rounds 1 and 2 go where
+  // the other launches keep quantized rows, which mvm_args makes large enough.  `seen`: host-visible numbers of the last call
+  // (of this tile or group) in which a sample went on to a second round and of the last call that has ended.  Returns the
+  // rounds to work out together (launch_mvm_few).
   void make_counts() {
     MvmArgs a{};
     a.K = X;
@@ -706,24 +707,17 @@ struct Tile {
     a.max_rounds = fio.perfect ? 0 : mvm_max_rounds(a.io);
     s_count.ensure(MVM_COUNT_WORDS + (a.max_rounds > 1 ? 7 * (size_t)mvm_few_batch(a) : 0));
   }
-  int *few_counters(int batch, hipStream_t s) {
-    const size_t need = MVM_COUNT_WORDS + 7 * (size_t)batch;
-    if (s_count.n < need) { // a pass with settings of its own (io_other) that allow larger small calls than the tile's
-      s_count.ensure(need);
-      few_cleared = false;
-    }
-    if (!few_cleared) {
-      launch_fill(reinterpret_cast<float *>(s_count.p + MVM_COUNT_WORDS), 0.0f, s_count.n - MVM_COUNT_WORDS, s); // all-zero bits
-      hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-      RPU_HIP_CHECK(hipStreamIsCapturing(s, &capturing));
-      few_cleared = capturing == hipStreamCaptureStatusNone; // a captured launch clears when it is replayed
-    }
-    return s_count.p + MVM_COUNT_WORDS;
-  }
-  int few_args(MvmArgs &a, int call_number, const volatile int *seen_host, int *seen_dev, hipStream_t s) {
+  // `clear`: set where the counters of the call have to be cleared first (few_cleared)
+  int few_args(MvmArgs &a, int call_number, const volatile int *seen_host, int *seen_dev, bool &clear) {
     if (a.max_rounds < 2) return 1;
-    a.few = few_counters(a.m_batch, s);
+    const size_t words = 7 * (size_t)a.m_batch;
+    if (s_count.n < MVM_COUNT_WORDS + words) { // a pass with settings of its own (io_other) that allow larger small calls
+      s_count.ensure(MVM_COUNT_WORDS + words);
+      few_zero = 0;
+    }
+    if (few_zero < words) clear = true;
     a.st.count = s_count.p;
+    a.few = s_count.p + MVM_COUNT_WORDS;
     a.few_seen = seen_dev;
     a.few_call = call_number;
     if (a.max_rounds < 3) return 1;
@@ -731,6 +725,15 @@ struct Tile {
     a.dual.buf[2] = a.xq[1];
     if (fused_rounds >= 0) return fused_rounds & 1 ? 3 : 1;
     return seen_host[1] - seen_host[0] <= 8 ? 3 : 1;
+  }
+  // whether a launch on s runs now: a captured one clears when it is replayed
+  static bool runs_now(hipStream_t s) {
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    RPU_HIP_CHECK(hipStreamIsCapturing(s, &capturing));
+    return capturing == hipStreamCaptureStatusNone;
+  }
+  void few_cleared(const MvmArgs &a) {
+    if (a.max_rounds > 1) few_zero = std::max(few_zero, 7 * (size_t)a.m_batch);
   }
   // the largest batch whose calls take k_mvm_few, 0: none do
   int small_call_batch(const MvmArgs &a) const {
@@ -1031,7 +1034,12 @@ struct Tile {
     const int few_batch = side || gather || running ? 0 : small_call_batch(a);
     if (few_batch > 0 && a.max_rounds > 1) ensure_seen(); // by a larger call too: a small one after it may be captured
     if (B <= few_batch && !writes_into_its_input(a)) {
-      const int together = a.max_rounds > 1 ? few_args(a, few_calls++, seen_host + 4, seen_dev + 4, s) : 1;
+      bool clear = false;
+      const int together = a.max_rounds > 1 ? few_args(a, few_calls++, seen_host + 4, seen_dev + 4, clear) : 1;
+      if (clear) {
+        launch_fill(reinterpret_cast<float *>(a.few), 0.0f, 7 * (size_t)B, s); // all-zero bits
+        if (runs_now(s)) few_cleared(a);
+      }
       const MvmArgs *call = &a;
       launch_mvm_few(a, mvm_few_variant(&call, 1), together, s);
       prof_mark(s, "mvm_few");
@@ -2971,10 +2979,11 @@ static int group_mvm(rpu_group_t *group, const float *const *x_dev, const long *
       }
     }
     ++group->few_calls;
+    bool clear = false;
     for (int i = 0; i < n; ++i) {
       if (!few[i]) continue;
       few_rounds[i] = group->tiles[i]->t.few_args(args[i], group->few_calls, group->seen_host + 2 * kSeenPairs + 1,
-                                                  group->seen_dev + 2 * kSeenPairs + 1, s);
+                                                  group->seen_dev + 2 * kSeenPairs + 1, clear);
     }
     // Tiles that quantize the same input the same way (the column blocks of a layer that was split over several
     // tiles) share the rows of rounds 0 and 1: one of them writes the rows, all of them read them.  Rows of later
@@ -3085,6 +3094,12 @@ static int group_mvm(rpu_group_t *group, const float *const *x_dev, const long *
 
     if (n_few) {
       MvmGroup g{group->mvm_args.dev_args(), group->mvm_args.dev_table(), n_few, m_batch};
+      if (clear) {
+        launch_mvm_few_clear_group(g, s);
+        if (Tile::runs_now(s)) {
+          for (int i = 0; i < n_few; ++i) group->tiles[order[i]]->t.few_cleared(args[order[i]]);
+        }
+      }
       launch_mvm_few_group(g, few_variant, few_together, transposed != storage_xd, few_max_k, few_workgroups, s);
     }
     if (n_few == n) { // says nothing about the launches that the pairs choose
