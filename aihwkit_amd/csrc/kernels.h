@@ -19,7 +19,8 @@ struct IoDev {
 
 // Per-sample bookkeeping of the noisy MVM, all arrays of length >= m_batch.
 constexpr int MVM_COUNT_WORDS = 256; // MvmState::count: [0, 40) per round; [MVM_ARRIVE_BASE + 4 r, + 4): counter and flag of the
-                                     // arrivals after round r, counter and flag of the wait before round r
+                                     // arrivals after round r, counter and flag of the wait before round r (k_mvm_rest_walk:
+                                     // tiles taken, done and visible to all in round r); behind them MvmArgs::few
 constexpr int MVM_ARRIVE_BASE = 64;
 constexpr int MVM_ABORT_WORD = 255;  // MvmState::count[MVM_ABORT_WORD]: raised by a workgroup whose wait for the others ran out
 

@@ -299,7 +299,7 @@ struct Tile {
   size_t few_zero = 0; // words for k_mvm_few that are zero between calls
   bool small_calls = true; // rpu_tile_set_small_calls
   // largest batch that the groups of this tile run as k_mvm_few, forward and backward: so does the tile in calls of its own,
-  // whose sums are then those of a call of the group
+  // whose sums are then those of a call of the group (also when the group is gone)
   int group_batch[2] = {INT_MAX, INT_MAX};
   int cus = 0;       // MvmArgs::cus
   int *seen_host = nullptr, *seen_dev = nullptr;

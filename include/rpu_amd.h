@@ -698,7 +698,8 @@ int rpu_tile_set_fused_rounds(rpu_tile_t *tile, int mode);
 
 /* No counterpart in the reference.  A call of a small batch runs noise management, conversions, contraction and all
  * bound-management rounds in one launch, whose sums are added in another order than those of the launches for larger
- * batches.  enable = 0: the tile (alone and in a group) keeps to the latter for every batch. */
+ * batches.  Tiles of a group take it together or not at all, and from then on in calls of their own like in the group's.
+ * enable = 0: the tile (alone and in a group) keeps to the latter for every batch. */
 int rpu_tile_set_small_calls(rpu_tile_t *tile, int enable);
 
 /* No counterpart in the reference; for the test of the time-out path above only.  spin_limit > 0 shortens the bounded
