@@ -295,6 +295,7 @@ struct UpdateArgs {
   const float *wt_src;
   const float *x;
   long x_sb, x_sj; // x element (b, j) at x[b * x_sb + j * x_sj]
+  int x_one;       // 1: the last x line is the constant 1 and not stored (bias column)
   const float *d;
   long d_sb, d_si;
   // Lines read in place from the image tensors of the indexed interface (all zero / null otherwise; only the kernels

@@ -58,6 +58,7 @@ __device__ __forceinline__ float update_x_value(const UpdateArgs &a, int b, int 
     const int idx = a.x_index[(long)(b - n * a.x_group) * a.x_size + j];
     return idx <= 1 ? (float)idx : a.x[(long)n * a.x_gs + (idx - 2)];
   }
+  if (a.x_one && j == a.x_size - 1) return 1.0f;
   return a.x[(long)b * a.x_sb + (long)j * a.x_sj];
 }
 __device__ __forceinline__ const float *update_d_row(const UpdateArgs &a, int b) {
@@ -144,7 +145,8 @@ __device__ __forceinline__ void update_prepare_sample(const UpdateArgs &a, const
     if (a.x_index) {
       for (int j = t; j < a.x_size; j += SUB) xm = fmaxf(xm, fabsf(update_x_value(a, b, j)));
     } else {
-      xm = part_abs_max(a.x + (long)b * a.x_sb, a.x_size, a.x_sj, t, SUB);
+      xm = part_abs_max(a.x + (long)b * a.x_sb, a.x_size - a.x_one, a.x_sj, t, SUB);
+      if (a.x_one) xm = fmaxf(xm, 1.0f);
     }
     dm = part_abs_max(update_d_row(a, b), a.d_size, a.d_si, t, SUB);
 #pragma unroll
@@ -340,6 +342,7 @@ __device__ __forceinline__ void update_lines_block(const UpdateArgs &a, const in
   const int b0 = by * 64;
   const float *src = is_x ? a.x : a.d;
   const long s_b = is_x ? a.x_sb : a.d_sb, s_e = is_x ? a.x_sj : a.d_si;
+  const int stored = size - (is_x ? a.x_one : 0); // (a row of words behind the batch has no pulses, whatever its values)
   constexpr int ROWS_PER_PASS = 256 / LINES_E;
   const int col = threadIdx.x % LINES_E, row0 = threadIdx.x / LINES_E;
   const int wps = max(a.words_per_sample, 1);
@@ -381,7 +384,7 @@ __device__ __forceinline__ void update_lines_block(const UpdateArgs &a, const in
       const int rb = row0 + ROWS_PER_PASS * i;
       const int b = b0 + rb, e = e0 + col;
       const int sample = wps > 1 ? b / wps : b;
-      vals[rb][col] = (b < a.m_batch && e < size) ? src[(long)sample * s_b + (long)e * s_e] : 0.0f;
+      vals[rb][col] = (b < a.m_batch && e < stored) ? src[(long)sample * s_b + (long)e * s_e] : (e < size ? 1.0f : 0.0f);
     }
   }
   __syncthreads();
@@ -548,7 +551,7 @@ __global__ __launch_bounds__(256) void k_update_lines_stream(UpdateArgs a) {
     for (int i = 0; i < 16; ++i) {
       const int b = b0 + wave * 16 + i, e = e0 + lane;
       const int sample = wps > 1 ? b / wps : b;
-      vals[wave * 16 + i][lane] = (b < a.m_batch && e < a.x_size) ? a.x[(long)sample * a.x_sb + (long)e * a.x_sj] : 0.0f;
+      vals[wave * 16 + i][lane] = (b < a.m_batch && e < a.x_size - a.x_one) ? a.x[(long)sample * a.x_sb + (long)e * a.x_sj] : 1.0f;
     }
   }
   __syncthreads();
@@ -634,7 +637,7 @@ __global__ __launch_bounds__(256) void k_update_lines_masks(UpdateArgs a, int ro
 #pragma unroll
   for (int c = 0; c < C; ++c) {
     e[c] = pulse_mask_column<C>(span, c) + lane;
-    x[c] = a.x + (long)min(e[c], a.x_size - 1) * a.x_sj; // elements behind the end of the line never fire
+    x[c] = a.x + (long)max(min(e[c], a.x_size - 1 - a.x_one), 0) * a.x_sj; // elements behind the end of the line never fire
     v[c] = x[c][(long)(wps > 1 ? b0 / wps : b0) * a.x_sb];
     first[c] = philox_first((uint32_t)e[c], a.call, RNG_PULSE_X, a.key);
   }
@@ -645,7 +648,7 @@ __global__ __launch_bounds__(256) void k_update_lines_masks(UpdateArgs a, int ro
     const PhiloxSecond second = philox_second((uint32_t)sample, a.call, a.key);
     float now[C];
 #pragma unroll
-    for (int c = 0; c < C; ++c) now[c] = v[c];
+    for (int c = 0; c < C; ++c) now[c] = (a.x_one && e[c] == a.x_size - 1) ? 1.0f : v[c];
     if (b + 1 < b1) { // on their way while this row is worked out
       const int next = wps > 1 ? (b + 1) / wps : b + 1;
 #pragma unroll

@@ -1157,7 +1157,7 @@ struct Tile {
 
   // Carves the scratch of a stochastic pulsed update out of a caller-provided block (256-byte aligned parts) and
   // returns the bytes used; with base == nullptr only the size is computed.
-  static size_t carve_update_scratch(unsigned char *base, int X, int D, int B, bool bias, UpdateArgs *a, float **bias_rows) {
+  static size_t carve_update_scratch(unsigned char *base, int X, int D, int B, bool bias, UpdateArgs *a) {
     size_t off = 0;
     auto take = [&](size_t bytes) {
       unsigned char *p = base ? base + off : nullptr;
@@ -1171,12 +1171,11 @@ struct Tile {
     float *pa = (float *)take((size_t)B * 4), *pb = (float *)take((size_t)B * 4);
     uint32_t *xw = (uint32_t *)take((size_t)B * X * 4), *dw = (uint32_t *)take((size_t)B * D * 4);
     uint32_t *xpl = (uint32_t *)take(chunks * slots * X * 4), *dpl = (uint32_t *)take(chunks * slots * D * 4);
-    float *rows = bias ? (float *)take((size_t)B * X * 4) : nullptr;
+    if (bias) (void)take((size_t)B * X * 4); // (the limit on a call's size counts rows with the bias column)
     if (a) {
       a->kmax = kmax; a->row_cost = row_cost; a->bl = bl; a->prob_a = pa; a->prob_b = pb; a->x_words = xw; a->d_words = dw;
       a->x_planes = xpl; a->d_planes = dpl; a->n_chunks = (int)chunks;
     }
-    if (bias_rows) *bias_rows = rows;
     return off;
   }
 
@@ -1254,8 +1253,11 @@ struct Tile {
     }
     if (lr == 0.0f && !delta_w) return;
     const float *xin = x;
-    long x_sb = x_trans ? 1 : X, x_sj = x_trans ? B : 1;
-    if (bias) {
+    // (the kernels of a pulsed update know that the last line is 1, the others read whole rows)
+    const bool widened = bias && fp_update;
+    const int x_one = bias && !widened ? 1 : 0;
+    long x_sb = x_trans ? 1 : X - x_one, x_sj = x_trans ? B : 1;
+    if (widened) {
       s_bias.ensure((size_t)B * X);
       launch_make_bias(x, s_bias.p, B, X, x_trans ? 1 : 0, s);
       xin = s_bias.p; x_sb = X; x_sj = 1;
@@ -1307,12 +1309,12 @@ struct Tile {
     }
 
     if (is_transfer()) {
-      transfer_update(xin, x_sb, x_sj, d, d_sb, d_si, B, s);
+      transfer_update(xin, x_sb, x_sj, x_one, d, d_sb, d_si, B, s);
       return;
     }
     if (persistent() && delta_w) throw RpuError("Delta weights are not provided for a device with write noise.");
     DeviceView dv{wp_dev(), d_wmax.p, d_wmin.p, d_sup.p, d_sdown.p, d_slup.p, d_sldown.p, &dev, dev.p.dw_min};
-    pulsed_update_on(dv, up, lr, xin, x_sb, x_sj, d, d_sb, d_si, B, s);
+    pulsed_update_on(dv, up, lr, xin, x_sb, x_sj, d, d_sb, d_si, B, s, nullptr, x_one);
   }
 
   // ----- weight maintenance between steps (decay, diffusion, clipping, column reset) ------------------------------
@@ -1629,7 +1631,7 @@ struct Tile {
   // Arguments of the update kernels for one call (lr != 0): scratch sized for B samples (or carved out of ws), the
   // call's random-stream index taken; wps returns the rows of pulse words per sample.
   UpdateArgs pulsed_update_args(const DeviceView &dv, const UpdatePar &up, float lr, const float *xin, long x_sb, long x_sj,
-                                const float *d, long d_sb, long d_si, int B, hipStream_t s, unsigned char *ws, int &wps_out) {
+                                const float *d, long d_sb, long d_si, int B, hipStream_t s, unsigned char *ws, int &wps_out, int x_one = 0) {
     const DevicePar &dev = *dv.par;
     const int wps = words_per_sample_for(up, lr, dv.granularity);
     if (wps > 1 && ws) throw RpuError("update_noalloc holds bit lines of at most 31 pulses.");
@@ -1637,7 +1639,7 @@ struct Tile {
     const int rows = B * wps; // rows of pulse words
     UpdateArgs a{};
     a.w = dv.w; a.x_size = X; a.d_size = D; a.m_batch = B;
-    a.x = xin; a.x_sb = x_sb; a.x_sj = x_sj; a.d = d; a.d_sb = d_sb; a.d_si = d_si;
+    a.x = xin; a.x_sb = x_sb; a.x_sj = x_sj; a.x_one = x_one; a.d = d; a.d_sb = d_sb; a.d_si = d_si;
     if (lines_in_place) { // update_indexed: xin and d are the caller's image tensors
       a.x_index = lines_in_place->index_patch_major; a.x_index_lines = lines_in_place->index_line_major; a.x_group = lines_in_place->patches; a.x_gs = lines_in_place->image_size;
       a.x_sb = 0; a.x_sj = 0;
@@ -1655,7 +1657,7 @@ struct Tile {
     a.dev.slope_up = const_cast<float *>(dv.slope_up); a.dev.slope_down = const_cast<float *>(dv.slope_down);
     a.key = key(); a.call = call++;
     if (ws) {
-      carve_update_scratch(ws, X, D, B, false, &a, nullptr);
+      carve_update_scratch(ws, X, D, B, false, &a);
       // the array keeps the last call's contents: the largest-BL slots start from zero again
       hipLaunchKernelGGL(k_init_kmax, dim3(1), dim3(64), 0, s, a.kmax);
       a.kmax_slot = 0;
@@ -1712,16 +1714,16 @@ struct Tile {
   }
 
   void pulsed_update_on(const DeviceView &dv, const UpdatePar &up, float lr, const float *xin, long x_sb, long x_sj,
-                        const float *d, long d_sb, long d_si, int B, hipStream_t s, unsigned char *ws = nullptr) {
+                        const float *d, long d_sb, long d_si, int B, hipStream_t s, unsigned char *ws = nullptr, int x_one = 0) {
     if (lr == 0.0f) return;
     const DevicePar &dev = *dv.par;
     int wps = 1;
-    UpdateArgs a = pulsed_update_args(dv, up, lr, xin, x_sb, x_sj, d, d_sb, d_si, B, s, ws, wps);
+    UpdateArgs a = pulsed_update_args(dv, up, lr, xin, x_sb, x_sj, d, d_sb, d_si, B, s, ws, wps, x_one);
     const int rows = B * wps;
     prof_begin(s);
+    const bool counting = dev.p.count_pulses && !is_transfer();
     launch_update_prepare(a, s);
     prof_mark(s, "update_prepare");
-    const bool counting = dev.p.count_pulses && !is_transfer();
     if (up.p.pulse_type == RPU_PULSE_STOCHASTIC_COMPRESSED) {
       // from here on the kernels walk rows of words; a longer bit line is several rows of one sample in a row
       a.m_batch = rows;
@@ -1800,8 +1802,7 @@ struct Tile {
     if (is_transfer() || persistent() || delta_w || dev.p.count_pulses) {
       throw RpuError("update_noalloc is not provided for transfer compounds, write noise, delta weights or pulse counters.");
     }
-    float *rows = nullptr;
-    const size_t need = carve_update_scratch(nullptr, X, D, B, bias, nullptr, nullptr);
+    const size_t need = carve_update_scratch(nullptr, X, D, B, bias, nullptr);
     if (need > (size_t)RPU_NOALLOC_MAX_SCRATCH_BYTES) {
       throw RpuError("update_noalloc: this call needs " + std::to_string(need) + " bytes of scratch, the static array holds " +
                      std::to_string((size_t)RPU_NOALLOC_MAX_SCRATCH_BYTES) + ".");
@@ -1810,19 +1811,14 @@ struct Tile {
     // refused before anything is written to the shared array
     if (words_per_sample_for(up, lr, dev.p.dw_min) > 1) throw RpuError("update_noalloc holds bit lines of at most 31 pulses.");
     unsigned char *ws = noalloc_scratch(device_id);
-    carve_update_scratch(ws, X, D, B, bias, nullptr, &rows);
-    const float *xin = x;
-    long x_sb = x_trans ? 1 : X, x_sj = x_trans ? B : 1;
-    if (bias) {
-      launch_make_bias(x, rows, B, X, x_trans ? 1 : 0, s);
-      xin = rows; x_sb = X; x_sj = 1;
-    }
+    const int x_one = bias ? 1 : 0;
+    const long x_sb = x_trans ? 1 : X - x_one, x_sj = x_trans ? B : 1;
     const long d_sb = d_trans ? 1 : D, d_si = d_trans ? B : 1;
     DeviceView dv{wp_dev(), d_wmax.p, d_wmin.p, d_sup.p, d_sdown.p, d_slup.p, d_sldown.p, &dev, dev.p.dw_min};
     const bool was_profiling = profiling;
     profiling = false; // event creation allocates
     try {
-      pulsed_update_on(dv, up, lr, xin, x_sb, x_sj, d, d_sb, d_si, B, s, ws);
+      pulsed_update_on(dv, up, lr, x, x_sb, x_sj, d, d_sb, d_si, B, s, ws, x_one);
     } catch (...) {
       profiling = was_profiling;
       throw;
@@ -2125,7 +2121,7 @@ struct Tile {
   // TransferRPUDevice::doSparseUpdate / finishUpdateCycle per update vector (rpu_transfer_device.cpp:520-557):
   // the gradient goes onto device 0; after every vector the update counter advances and each device whose
   // period divides it transfers.  The batch is cut at those points (C/rpucuda_transfer_device.cu:393-510).
-  void transfer_update(const float *xin, long x_sb, long x_sj, const float *d, long d_sb, long d_si, int B, hipStream_t s) {
+  void transfer_update(const float *xin, long x_sb, long x_sj, int x_one, const float *d, long d_sb, long d_si, int B, hipStream_t s) {
     const TransferPar &tp = *tr;
     const float lr_fast = tp.fast_lr(lr);
     const int n_dev = tp.n();
@@ -2139,7 +2135,7 @@ struct Tile {
       for (int j = 0; j < n_dev; ++j) {
         if (every[j] > 0) chunk = std::min<uint64_t>(chunk, (uint64_t)every[j] - update_idx % (uint64_t)every[j]);
       }
-      pulsed_update_on(dv0, up, lr_fast, xin + (long)b0 * x_sb, x_sb, x_sj, d + (long)b0 * d_sb, d_sb, d_si, (int)chunk, s);
+      pulsed_update_on(dv0, up, lr_fast, xin + (long)b0 * x_sb, x_sb, x_sj, d + (long)b0 * d_sb, d_sb, d_si, (int)chunk, s, nullptr, x_one);
       update_idx += chunk;
       b0 += (int)chunk;
       for (int j = 0; j < n_dev; ++j) {

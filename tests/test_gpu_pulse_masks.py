@@ -132,3 +132,29 @@ def test_pulse_loop_on_lane_masks_with_parameters_that_are_not_finite(name, valu
     assert np.array_equal(mine, theirs, equal_nan=True)
     assert np.array_equal(mine[:, ::5], before[:, ::5], equal_nan=True)
     assert np.isfinite(mine[:, 1::3]).all() and not np.array_equal(mine, before, equal_nan=True)
+
+
+# every kernel that makes pulse trains reads a bias column that is not stored as the row that has it: a few samples, lane masks,
+# pipeline of waves, long lines, implicit pulses
+@pytest.mark.parametrize("x_size,d_size,batch,pulse_type,blm", [
+    (2, 3, 4, "StochasticCompressed", True), (129, 10, 64, "StochasticCompressed", True), (601, 400, 300, "StochasticCompressed", True),
+    (433, 48, 1030, "StochasticCompressed", True), (65, 20, 130, "StochasticCompressed", False), (70, 33, 20, "MeanCount", True)])
+@pytest.mark.parametrize("x_trans", [False, True])
+def test_bias_column_that_is_not_stored(x_size, d_size, batch, pulse_type, blm, x_trans, storage_mode):
+    from aihwkit_amd.rpu_base import devices as dv
+    from aihwkit_amd.rpu_base import tiles
+    x, d = _data(x_size - 1, d_size, batch, 0)
+    x *= 0.7  # the bias is the largest line
+    results = []
+    for bias in (True, False):
+        host = make_meta(desired_bl=31, pulse_type=getattr(dv.PulseType, pulse_type),
+                         update_bl_management=blm).create_array(x_size, d_size, _device("soft_bounds"))
+        host.set_weights(torch.zeros(d_size, x_size))
+        tile = tiles.CudaAnalogTile(host)
+        tile.set_seed(5)
+        tile.set_learning_rate(0.02)
+        line = x if bias else torch.cat([x, torch.ones(batch, 1, device="cuda")], 1)
+        tile.update(line.t().contiguous() if x_trans else line.contiguous(), d, bias, x_trans)
+        results.append(tile.get_weights())
+    assert torch.equal(results[0], results[1])
+    assert float(results[0][:, -1].abs().max()) > 0.0
