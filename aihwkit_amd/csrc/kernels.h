@@ -376,6 +376,10 @@ void launch_words_from_planes(const UpdateArgs &a, hipStream_t s);    // x_words
 void launch_update_planes(const UpdateArgs &a, hipStream_t s);        // bit planes of pulse words made elsewhere
 void launch_words_kmax(const UpdateArgs &a, hipStream_t s);           // a.kmax[a.kmax_slot] = longest bit line among such words
 void launch_update_pulsed(const UpdateArgs &a, hipStream_t s);        // coincidences + device steps
+// the same, where all bit lines are longer than seven pulses (update_takes_words).  On a tile that stores [x_size][d_size], wt_src
+// and w_out are that matrix, without a row-major copy (w is not used).
+bool update_takes_words(const UpdateArgs &a);
+void launch_update_pulsed_words(const UpdateArgs &a, hipStream_t s);
 // opt-in variant for LinearStep devices with multiplicative noise: per group of samples_per_step samples the
 // coincidences are counted and applied in closed form with one normal draw for their summed noise
 void launch_update_aggregated(const UpdateArgs &a, int samples_per_step, hipStream_t s);

@@ -87,12 +87,10 @@ __device__ __forceinline__ float part_abs_max(const float *v, int n, long stride
   return m;
 }
 
-// BL, A and B of sample b from the largest |x| and |d| of its lines (rpu_pulsed_meta_parameter.cpp:183-236), by one thread
-__device__ __forceinline__ void update_prepare_finish(const UpdateArgs &a, const int b, const float xm, const float dm) {
+// BL, A and B of a sample from the largest |x| and |d| of its lines (rpu_pulsed_meta_parameter.cpp:183-236)
+__device__ __forceinline__ void update_bl_ab(const UpdateArgs &a, const float xm, const float dm, int &BL, float &A, float &B) {
   const float lr = fabsf(a.lr);
   const float dw_min = a.dev.dw_min;
-  int BL;
-  float A, B;
   calc_bl_ab(a.up, BL, A, B, lr, dw_min);
   if ((a.up.update_management || a.up.update_bl_management) && lr > 0.0f) {
     if (dm == 0.0f || xm == 0.0f) {
@@ -116,6 +114,13 @@ __device__ __forceinline__ void update_prepare_finish(const UpdateArgs &a, const
       }
     }
   }
+}
+
+// ... of sample b, by one thread
+__device__ __forceinline__ void update_prepare_finish(const UpdateArgs &a, const int b, const float xm, const float dm) {
+  int BL;
+  float A, B;
+  update_bl_ab(a, xm, dm, BL, A, B);
   a.bl[b] = BL;
   // largest number of pulse slots in a row of words (a longer bit line takes several rows of 31): this call's slot
   // was zeroed by the previous call, which used the other one
@@ -1184,6 +1189,56 @@ template <int KIND, bool MULT, int NK, bool NOISE, int C> struct PulsedRows {
   }
 };
 
+// The pulses of a block of 128 samples for bit lines of any length: ev is the lane's set of samples with a coincidence,
+// `words` gives the two packed words of sample b, sample0 the number of the block's first sample.
+template <int KIND, bool MULT, typename Words>
+__device__ __forceinline__ float pulsed_events(const UpdateArgs &a, float w, const PulseCell<KIND> &cp, unsigned cell, uint32_t &refill,
+                                               const uint32_t (&ev)[4], unsigned sample0, const Words &words) {
+  const float std_ = a.dev.dw_min_std;
+  const uint32_t lr_neg = a.lr < 0.0f ? 1u : 0u;
+  unsigned long long cur = ((unsigned long long)ev[1] << 32) | ev[0]; // sample0: of bit 0 of cur
+  unsigned long long nxt = ((unsigned long long)ev[3] << 32) | ev[2];
+  uint32_t xw = 0u, dw = 0u; // of the lane's next event, fetched while the one before it is worked on
+  const auto fetch = [&] {
+    if (cur == 0ull) {
+      cur = nxt;
+      nxt = 0ull;
+      sample0 += 64u;
+    }
+    xw = 0u;
+    if (cur != 0ull) {
+      const int bit = __ffsll((long long)cur) - 1;
+      cur &= cur - 1ull;
+      words(sample0 + (unsigned)bit, xw, dw);
+    }
+  };
+  if (!__any((cur | nxt) != 0ull)) return w;
+  fetch();
+  int left = 0; // pulses left in the current event
+  float slope = 0.0f, scale = 0.0f;
+  for (;;) {
+    float f[8];
+    noise_factors(f, std_, cell, refill, a);
+    ++refill;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      if (left == 0) {
+        left = __popc(xw & dw & ~1u);
+        // step down when x and d have the same sign and lr > 0
+        const bool down = (((xw ^ dw) & 1u) ^ lr_neg) == 0u;
+        slope = down ? cp.slope_dn : cp.slope_up;
+        scale = down ? cp.scale_dn : cp.scale_up;
+        if (left != 0) fetch();
+      }
+      if (!__any(left > 0)) return w;
+      if (left > 0) {
+        w = pulse<KIND, MULT>(w, slope, scale, f[q], cp.lo, cp.hi);
+        --left;
+      }
+    }
+  }
+}
+
 // Pulse loop for any bit-line length.  The batch is walked in blocks of 128 samples.  For a block every lane
 // first builds the 128-bit set of samples in which its cross-point has a coincidence: OR over the pulse
 // slots of (x_plane & d_plane).  Then every lane walks its own set in batch order; the count and
@@ -1192,8 +1247,6 @@ template <int KIND, bool MULT, int NK, bool NOISE, int C> struct PulsedRows {
 template <int KIND, bool MULT>
 __device__ __forceinline__ float pulsed_gather(const UpdateArgs &a, float w, const PulseCell<KIND> &cp, unsigned cell,
                                                int i, int j, bool valid, int kmax) {
-  const float std_ = a.dev.dw_min_std;
-  const uint32_t lr_neg = a.lr < 0.0f ? 1u : 0u;
   const int n_chunks = a.n_chunks;
   const uint32_t *xpl = a.x_planes + j;
   const uint32_t *dpl = a.d_planes + i;
@@ -1219,47 +1272,10 @@ __device__ __forceinline__ float pulsed_gather(const UpdateArgs &a, float w, con
       }
       ev[cc] = valid ? e : 0u;
     }
-    unsigned long long cur = ((unsigned long long)ev[1] << 32) | ev[0];
-    unsigned long long nxt = ((unsigned long long)ev[3] << 32) | ev[2];
-    unsigned sample0 = (unsigned)c0 * 32u; // sample index of bit 0 of cur
-    int left = 0;                          // pulses left in the current event
-    float slope = 0.0f, scale = 0.0f;
-    bool block_done = !__any((cur | nxt) != 0ull);
-    while (!block_done) {
-      float f[8];
-      noise_factors(f, std_, cell, refill, a);
-      ++refill;
-#pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        if (left == 0) {
-          if (cur == 0ull) {
-            cur = nxt;
-            nxt = 0ull;
-            sample0 += 64u;
-          }
-          if (cur != 0ull) {
-            const int bit = __ffsll((long long)cur) - 1;
-            cur &= cur - 1ull;
-            const unsigned b = sample0 + (unsigned)bit;
-            const uint32_t xw = xwp[__umul24(b, xs)];
-            const uint32_t dw = dwp[__umul24(b, ds)];
-            left = __popc(xw & dw & ~1u);
-            // step down when x and d have the same sign and lr > 0
-            const bool down = (((xw ^ dw) & 1u) ^ lr_neg) == 0u;
-            slope = down ? cp.slope_dn : cp.slope_up;
-            scale = down ? cp.scale_dn : cp.scale_up;
-          }
-        }
-        if (!__any(left > 0)) {
-          block_done = true;
-          break;
-        }
-        if (left > 0) {
-          w = pulse<KIND, MULT>(w, slope, scale, f[q], cp.lo, cp.hi);
-          --left;
-        }
-      }
-    }
+    w = pulsed_events<KIND, MULT>(a, w, cp, cell, refill, ev, (unsigned)c0 * 32u, [&](unsigned b, uint32_t &xw, uint32_t &dw) {
+      xw = xwp[__umul24(b, xs)];
+      dw = dwp[__umul24(b, ds)];
+    });
   }
   return w;
 }
@@ -1981,6 +1997,63 @@ __global__ __launch_bounds__(1024) void k_update_pulsed_masks(UpdateArgs a, int 
   }
 }
 
+// ---- the pulse loop for long bit lines, its pulse words in LDS ------------------------------------------------------
+// Bit lines of more than seven pulses are walked event by event (pulsed_events): a lane needs the two packed words of the next
+// sample in which its cross-point has a coincidence, and from memory every one of them is a trip to the cache that the next
+// pulse waits for.  Here a workgroup of 16 waves brings the words of 16 rows and 64 columns into LDS, 128 samples at a time; a
+// wave takes a row.  Blocks of samples, the lanes of a wave and with them the noise are those of pulsed_gather: same weights.
+// 785 x 300, 37 samples of 31 pulses 40.7 -> 14.2 us; the training step 93 -> 68.
+constexpr int WORDS_ROWS = 16, WORDS_BATCH = 128, WORDS_LINES = 64 + WORDS_ROWS; // lines of a workgroup: columns, then rows
+
+template <int KIND, bool MULT>
+__global__ __launch_bounds__(1024) void k_update_pulsed_words(UpdateArgs a) {
+  __shared__ uint32_t words[WORDS_BATCH][WORDS_LINES];
+  const int lane = (int)threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int row0 = (int)blockIdx.y * WORDS_ROWS, i = row0 + wave, ic = min(i, a.d_size - 1), B = a.m_batch;
+  if (a.kmax[a.kmax_slot] <= UPDATE_PLANES_ONLY_KMAX) return; // no sample has pulses (update_takes_words)
+  const int jt = (int)blockIdx.x * 64 + lane, j = min(jt, a.x_size - 1);
+  const bool valid = jt < a.x_size && i < a.d_size;
+  const unsigned cell = (unsigned)ic * (unsigned)a.x_size + (unsigned)j;
+  PulseCell<KIND> cp;
+  cp.load(a.dev, cell);
+  float w = a.wt_src ? a.wt_src[(size_t)j * a.d_size + ic] : a.w[cell];
+  const int id = min(row0 + (lane & (WORDS_ROWS - 1)), a.d_size - 1);
+  uint32_t refill = 0u;
+  for (int b0 = 0; b0 < B; b0 += WORDS_BATCH) {
+    const int rows = min(WORDS_BATCH, B - b0);
+    const uint32_t *x = a.x_words + (size_t)b0 * a.x_size + j, *d = a.d_words + (size_t)b0 * a.d_size + id;
+    uint32_t vx[WORDS_BATCH / 16], vd[WORDS_BATCH / 16]; // all of them on their way at once
+#pragma unroll
+    for (int u = 0; u < WORDS_BATCH / 16; ++u) {
+      const size_t r = (size_t)min(wave + 16 * u, rows - 1);
+      vx[u] = x[r * a.x_size];
+      vd[u] = d[r * a.d_size];
+    }
+    __syncthreads(); // the block before has been walked
+#pragma unroll
+    for (int u = 0; u < WORDS_BATCH / 16; ++u) {
+      words[wave + 16 * u][lane] = vx[u];
+      if (lane < WORDS_ROWS) words[wave + 16 * u][64 + lane] = vd[u];
+    }
+    __syncthreads();
+    uint32_t ev[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      ev[q] = 0u;
+      const int last = valid ? min(32 * q + 32, rows) : 0;
+#pragma unroll 8
+      for (int b = 32 * q; b < last; ++b) ev[q] |= ((words[b][lane] & words[b][64 + wave]) > 1u ? 1u : 0u) << (b & 31);
+    }
+    w = pulsed_events<KIND, MULT>(a, w, cp, cell, refill, ev, 0u, [&](unsigned b, uint32_t &xw, uint32_t &dw) {
+      xw = words[b][lane];
+      dw = words[b][64 + wave];
+    });
+  }
+  if (!valid) return;
+  if (a.w_out) a.w_out[(long)i * a.wo_si + (long)j * a.wo_sj] = w; // see UpdateArgs::w_out
+  else a.w[cell] = w;
+}
+
 // Several tiles in one launch (same device kind, noise and columns per lane): start[t] .. start[t + 1] are the
 // workgroups of tile t, column blocks of a row next to each other.
 template <int KIND, bool MULT, bool NOISE, int C, bool DEEP = false>
@@ -2579,6 +2652,21 @@ template <bool NOISE, int C> static void launch_update_pulsed_masks(const Update
     hipLaunchKernelGGL((k_update_pulsed_masks<RPU_DEVICE_LINEAR_STEP, true, NOISE, C>), grid, block, 0, s, a, dealt);
   } else {
     hipLaunchKernelGGL((k_update_pulsed_masks<RPU_DEVICE_LINEAR_STEP, false, NOISE, C>), grid, block, 0, s, a, dealt);
+  }
+}
+// Whether all bit lines of this call are longer than seven pulses (k_update_pulsed_words): without BL management a sample has the
+// desired length or a longer one, or no pulses at all (calc_bl_ab).
+bool update_takes_words(const UpdateArgs &a) {
+  return !a.x_index && !a.d_group && !a.up.update_bl_management && a.up.desired_bl > UPDATE_PLANES_ONLY_KMAX;
+}
+void launch_update_pulsed_words(const UpdateArgs &a, hipStream_t s) {
+  const dim3 grid((unsigned)((a.x_size + 63) / 64), (unsigned)((a.d_size + WORDS_ROWS - 1) / WORDS_ROWS));
+  if (a.dev.kind == RPU_DEVICE_CONSTANT_STEP) {
+    hipLaunchKernelGGL((k_update_pulsed_words<RPU_DEVICE_CONSTANT_STEP, true>), grid, dim3(1024), 0, s, a);
+  } else if (a.dev.ls_mult_noise) {
+    hipLaunchKernelGGL((k_update_pulsed_words<RPU_DEVICE_LINEAR_STEP, true>), grid, dim3(1024), 0, s, a);
+  } else {
+    hipLaunchKernelGGL((k_update_pulsed_words<RPU_DEVICE_LINEAR_STEP, false>), grid, dim3(1024), 0, s, a);
   }
 }
 template <bool NOISE, int PARTS> static void launch_update_pulsed_stream(const UpdateArgs &a, hipStream_t s) {

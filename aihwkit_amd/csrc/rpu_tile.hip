@@ -1686,6 +1686,9 @@ struct Tile {
   void row_major_pulse_loop(UpdateArgs &a) {
     u_wrm.ensure(size());
     a.w = u_wrm.p;
+    row_major_parameters(a);
+  }
+  void row_major_parameters(UpdateArgs &a) {
     a.w_out = d_w.p; a.wo_si = 1; a.wo_sj = D;
     a.dev.w_max = r_wmax.p; a.dev.w_min = r_wmin.p; a.dev.scale_up = r_sup.p; a.dev.scale_down = r_sdown.p;
     a.dev.slope_up = r_slup.p; a.dev.slope_down = r_sldown.p;
@@ -1729,10 +1732,6 @@ struct Tile {
       a.m_batch = rows;
       a.words_per_sample = wps;
       const bool aggregated = update_variant == RPU_UPDATE_VARIANT_AGGREGATED && dev.linear() && dev.p.ls_mult_noise && !is_transfer();
-      if (xd && !aggregated && dv.w == d_w.p) {
-        row_major_pulse_loop(a);
-        a.wt_src = d_w.p; // the launch of the pulse trains makes the row-major copy
-      }
       // the static block belongs to all tiles of the GPU: its words are made now, a later inspection only reads them
       a.keep_words = ws ? 1 : 0;
       // (pulse counters and write noise read the bit planes; the static block is laid out for planes)
@@ -1745,10 +1744,23 @@ struct Tile {
           a.x_mask_columns = columns;
         }
       }
+      const bool words = !aggregated && !a.x_lane_masks && update_takes_words(a);
+      const bool transposed = xd && !aggregated && dv.w == d_w.p;
+      if (transposed && !words) {
+        row_major_pulse_loop(a);
+        a.wt_src = d_w.p; // the launch of the pulse trains makes the row-major copy
+      }
       launch_update_lines(a, s);
       prof_mark(s, "update_lines");
       if (counting) count_pulses(a, false, s);
-      if (aggregated) {
+      if (words) {
+        if (transposed) {
+          row_major_parameters(a);
+          a.wt_src = d_w.p;
+        }
+        launch_update_pulsed_words(a, s);
+        prof_mark(s, "update_pulsed_words");
+      } else if (aggregated) {
         launch_update_aggregated(cross_point_view(a), update_variant_samples, s);
         prof_mark(s, "update_aggregated");
       } else {

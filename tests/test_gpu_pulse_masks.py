@@ -134,6 +134,45 @@ def test_pulse_loop_on_lane_masks_with_parameters_that_are_not_finite(name, valu
     assert np.isfinite(mine[:, 1::3]).all() and not np.array_equal(mine, before, equal_nan=True)
 
 
+def _long_lines_tile(x_size, d_size, kind, desired_bl=31):
+    from aihwkit_amd.rpu_base import tiles
+    host = make_meta(desired_bl=desired_bl, update_bl_management=False).create_array(x_size, d_size, _device(kind))
+    host.set_weights(torch.from_numpy(np.random.default_rng(3).uniform(-0.4, 0.4, (d_size, x_size)).astype(np.float32)))
+    tile = tiles.CudaAnalogTile(host)
+    tile.set_seed(17)
+    return tile
+
+
+# without BL management all lines are long (k_update_pulsed_words): one lane, one wave and rows and columns just beyond them, a
+# block of 128 samples that is full, one short of it and one beyond it, two columns per lane in the kernel compared with, the
+# shortest such line (8), lines of two words (40 pulses), samples without a pulse, a step against the gradient
+@pytest.mark.parametrize("x_size,d_size,batch,desired_bl,lr,sparse", [
+    (1, 1, 3, 31, 0.02, 0), (64, 16, 128, 31, 0.02, 0), (65, 17, 129, 31, 0.02, 0), (63, 15, 127, 8, 0.004, 0),
+    (785, 300, 37, 31, 0.01, 0), (130, 70, 600, 31, 0.01, 0.9), (200, 33, 70, 31, 0.04, 0), (300, 500, 200, 12, -0.01, 0)])
+@pytest.mark.parametrize("kind", ["soft_bounds", "constant_step", "quiet", "additive"])
+def test_long_bit_lines_through_lds_equal_the_plain_loop(x_size, d_size, batch, desired_bl, lr, sparse, kind, storage_mode):
+    from aihwkit_amd.rpu_base.tiles import TileGroup
+    x, d = _data(x_size, d_size, batch, sparse)
+    one, other = (_long_lines_tile(x_size, d_size, kind, desired_bl) for _ in range(2))
+    start = one.get_weights()
+    for tile in (one, other):
+        tile.set_learning_rate(lr)
+    if lr > 31 * 0.001:  # lines of more than one word: not in groups; the longer call takes the pulse loop word by word
+        _update(one, "update_pulsed_words", x, d, False)
+        half = x.size(0) // 2
+        _update(other, "update_pulsed_words", x.clone(), d.clone(), False)
+        assert half and torch.equal(one.get_weights(), other.get_weights())
+        return
+    group = TileGroup([other])
+    for _ in range(2):
+        _update(one, "update_pulsed_words", x, d, False)
+        group.update([x], [d])
+    assert torch.equal(one.get_weights(), other.get_weights())
+    assert not torch.equal(one.get_weights(), start)
+    one.update(torch.zeros_like(x), d, False)  # no sample has pulses
+    assert torch.equal(one.get_weights(), other.get_weights())
+
+
 # every kernel that makes pulse trains reads a bias column that is not stored as the row that has it: a few samples, lane masks,
 # pipeline of waves, long lines, implicit pulses
 @pytest.mark.parametrize("x_size,d_size,batch,pulse_type,blm", [
