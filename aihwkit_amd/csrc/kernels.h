@@ -214,6 +214,21 @@ struct ConvArgs {
 bool conv_forward_supported(const MvmArgs &a);
 void launch_conv_forward(const MvmArgs &a, const ConvArgs &c, hipStream_t s);
 
+// ---- exact products of calls that fill the GPU (kernels_product.hip): MvmArgs with io.perfect, as launch_mvm_init and
+// launch_mvm_round take it, without the scratch of those
+constexpr int PRODUCT_TILE = 128; // outputs of a workgroup tile
+struct ProductArgs {
+  __bf16 *w_parts, *x_parts; // blocks of 128 rows x 32 terms, three planes each
+  int *w_flags, *x_flags;    // [64-row block][stage]: whether it holds a value out of the range of the parts
+  float *partial;            // [share][tile] sums, with more than one share
+  int tiles_o, tiles_b, stages, shares, stages_per_share;
+  int sample_tile;           // samples of a workgroup tile
+};
+bool product_plan(const MvmArgs &a, ProductArgs &p); // whether the call is one, and its sizes
+size_t product_scratch(const ProductArgs &p, unsigned char *base, ProductArgs *out); // bytes; places in `base` where it is not null
+void launch_product_parts(const MvmArgs &a, const ProductArgs &p, hipStream_t s);
+void launch_product(const MvmArgs &a, const ProductArgs &p, hipStream_t s);
+
 // ---- analog non-idealities before the ADC (kernels_nonideal.hip), rpu_forward_backward_pass.cpp:325-433, 535-560
 // transformed copy of the quantized input rows [rows][k_pad]: mode 0 x^2, 1 |x|, 2 x (1 - (1 - j / K)^2), 3 x
 // part -1 / +1: only the negative / positive inputs (the others read as zero), before the transformation

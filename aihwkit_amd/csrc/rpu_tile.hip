@@ -289,6 +289,7 @@ struct Tile {
   hipStream_t last_stream = nullptr;
   DevBuf<float> d_w, d_wmax, d_wmin, d_sup, d_sdown, d_slup, d_sldown;
   // MVM scratch
+  DevBuf<unsigned char> s_parts; // exact_product
   DevBuf<float> s_nsc0, s_nsc1, s_nm, s_nmnp, s_red, s_scale, s_fin, s_bias, s_xq0, s_xq1;
   // rounds 0 and 1 of a forward call in one launch: kept outputs of both, choice per sample, marks of round 1, rows of
   // round 2; the host-visible pair (samples of the last call that needed round 1, its batch) that the choice between
@@ -522,7 +523,7 @@ struct Tile {
       (void)hipHostFree(seen_host);
       seen_host = seen_dev = nullptr;
     }
-    s_nsc0.release(); s_nsc1.release(); s_nm.release(); s_nmnp.release(); s_red.release(); s_scale.release(); s_fin.release(); s_bias.release(); s_xq0.release(); s_xq1.release();
+    s_parts.release(); s_nsc0.release(); s_nsc1.release(); s_nm.release(); s_nmnp.release(); s_red.release(); s_scale.release(); s_fin.release(); s_bias.release(); s_xq0.release(); s_xq1.release();
     s_rounds.release(); s_hitup.release(); s_hitlo.release(); s_list0.release(); s_list1.release(); s_row0.release(); s_row1.release(); s_count.release(); s_tiledone.release();
     u_rowcost.release();
     u_bl.release(); u_a.release(); u_b.release(); u_xval.release(); u_dval.release(); u_xw.release(); u_dw.release();
@@ -973,6 +974,27 @@ struct Tile {
 
   const GatherSource *lines_in_place = nullptr; // set while update_indexed runs a pulsed update (pulsed_update_args)
 
+  // out = alpha * (weights * inputs) + beta * out
+  void exact_product(MvmArgs &a, hipStream_t s, const char *first, const char *second) {
+    ProductArgs p;
+    // (where values are out of the range of the parts, the product reads the inputs themselves)
+    const bool parts = product_plan(a, p) && !writes_into_its_input(a);
+    if (parts) {
+      s_parts.ensure(product_scratch(p, nullptr, nullptr));
+      (void)product_scratch(p, s_parts.p, &p);
+      launch_product_parts(a, p, s);
+    } else {
+      a.k_pad = a.k_pad ? a.k_pad : mvm_k_pad(a.K);
+      s_xq0.ensure((size_t)a.m_batch * a.k_pad);
+      a.xq[0] = s_xq0.p;
+      launch_mvm_init(a, s);
+    }
+    prof_mark(s, first);
+    if (parts) launch_product(a, p, s);
+    else launch_mvm_round(a, s);
+    prof_mark(s, second);
+  }
+
   // in_ld: row stride of a plain row-major input with padded rows (0: the rows are dense)
   void mvm(const float *in, float *out, int B, bool bias, bool in_trans, bool out_trans, bool transposed, hipStream_t s,
            const float *w_other = nullptr, const IOPar *io_other = nullptr, bool is_test = false, long in_ld = 0,
@@ -1045,10 +1067,7 @@ struct Tile {
       prof_mark(s, "mvm_few");
     } else if (io.perfect) {
       a.round = 0;
-      launch_mvm_init(a, s);
-      prof_mark(s, "mvm_init");
-      launch_mvm_round(a, s);
-      prof_mark(s, "mvm_round");
+      exact_product(a, s, "mvm_init", "mvm_round");
     } else {
       if (io.p.noise_management == RPU_NM_AVERAGE_ABS_MAX || io.p.noise_management == RPU_NM_AVERAGE_ABS_MAX_SINGLE_VALUE) {
         // per-sample maxima, the recurrence over the batch in its order, then the usual set-up with those scales
@@ -1293,14 +1312,8 @@ struct Tile {
       a.io = io_dev(fio); a.io.perfect = 1;
       a.alpha = delta_w ? 1.0f : -lr; a.beta = delta_w ? 0.0f : 1.0f; a.round = 0;
       a.key = key(); a.call = call++;
-      a.k_pad = mvm_k_pad(B);
-      s_xq0.ensure((size_t)X * a.k_pad);
-      a.xq[0] = s_xq0.p; a.xq[1] = nullptr;
       prof_begin(s);
-      launch_mvm_init(a, s);
-      prof_mark(s, "fp_update_gather");
-      launch_mvm_round(a, s);
-      prof_mark(s, "fp_update");
+      exact_product(a, s, "fp_update_gather", "fp_update");
       RPU_HIP_CHECK(hipGetLastError());
       last_stream = s;
       last_update_batch = B;

@@ -186,3 +186,51 @@ def test_grouped_products_in_three_parts_against_64_bit_sums(gpu_device, shapes,
         q = v.astype(np.float64) if perfect else np.rint(v / step) * step
         w64 = w.astype(np.float64)
         _close(got, q @ w64.T, np.abs(q) @ np.abs(w64).T, 4 * w.shape[1] + 16, w.shape[1])
+
+
+# exact calls that fill the GPU (k_product): a term, an output and a sample more than a tile holds, one less than that, the line
+# between eight and six products of the parts (512 terms), the terms in one and in several shares, a share of one stage
+@pytest.mark.parametrize("x_size,d_size,batch", [(1025, 900, 900), (2049, 129, 3100), (127, 2500, 2600), (511, 1200, 1400),
+                                                 (512, 1217, 1400), (100, 101, 16384), (1024, 1024, 769), (640, 257, 5000)])
+@pytest.mark.parametrize("trans", [False, True])
+def test_exact_products_of_calls_that_fill_the_gpu(gpu_device, x_size, d_size, batch, trans):
+    rng = np.random.default_rng(x_size)
+    io = noise_free_io()
+    io.is_perfect = True
+    w = (0.3 * rng.standard_normal((d_size, x_size))).astype(np.float32)
+    tile = _tile(x_size, d_size, io, w)
+    lay = (lambda v: torch.from_numpy(np.ascontiguousarray(v.T if trans else v)).cuda())
+    back = (lambda v: v.t() if trans else v)
+    x, d = rng.standard_normal((batch, x_size)).astype(np.float32), rng.standard_normal((batch, d_size)).astype(np.float32)
+    x[:, -1] = 1.0  # the bias column, which is not stored
+    x64, d64, w64 = x.astype(np.float64), d.astype(np.float64), w.astype(np.float64)
+    _close(back(tile.forward(lay(x[:, :-1]), True, trans, trans)), x64 @ w64.T, np.abs(x64) @ np.abs(w64).T, x_size)
+    _close(back(tile.backward(lay(d), True, trans, trans)), (d64 @ w64)[:, :-1], (np.abs(d64) @ np.abs(w64))[:, :-1], d_size)
+    lr = 0.125
+    tile.set_learning_rate(lr)
+    tile.update(lay(x[:, :-1]), lay(d), True, trans, trans)
+    want = w64 - lr * (d64.T @ x64)
+    _close(tile.get_weights(), want, np.abs(w64) + lr * (np.abs(d64).T @ np.abs(x64)), batch)
+
+
+@pytest.mark.parametrize("x_size,d_size,batch", [(1025, 900, 900), (300, 300, 12001)])
+def test_exact_products_with_values_out_of_the_range_of_the_parts(gpu_device, x_size, d_size, batch):
+    """In the last share of the terms, at the last rows, and none but there: the other tiles are as they are without them."""
+    rng = np.random.default_rng(2)
+    io = noise_free_io()
+    io.is_perfect = True
+    w = rng.uniform(-0.5, 0.5, (d_size, x_size)).astype(np.float32)
+    x = (rng.random((batch, x_size)) + 0.5).astype(np.float32)
+    plain = _tile(x_size, d_size, io, w).forward(torch.from_numpy(x).cuda()).cpu().numpy()
+    w[-1, -1], x[-1, -2], x[-2, -1], x[-3, 5] = np.inf, 3e38, np.nan, 1e30
+    got = _tile(x_size, d_size, io, w).forward(torch.from_numpy(x).cuda()).cpu().numpy()
+    with np.errstate(all="ignore"):
+        want = x.astype(np.float64) @ w.astype(np.float64).T
+        want32 = want.astype(np.float32)
+    assert np.array_equal(np.isnan(got), np.isnan(want32))
+    assert np.array_equal(got[np.isinf(want32)], want32[np.isinf(want32)])
+    fine = np.isfinite(want32)
+    with np.errstate(all="ignore"):
+        bound = (x_size + 2) * 2.0 ** -24 * (np.abs(x.astype(np.float64)) @ np.abs(w.astype(np.float64)).T)
+        assert np.all((np.abs(got.astype(np.float64) - want) <= bound + 1e-37)[fine])
+    assert np.array_equal(got[:-128 - batch % 128, :-128 - d_size % 128], plain[:-128 - batch % 128, :-128 - d_size % 128])
