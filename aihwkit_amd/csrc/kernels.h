@@ -386,6 +386,9 @@ void launch_update_pulsed_group(const UpdateGroup &g, int variant, int total_wor
 void ensure_update_tables();
 void launch_update_prepare(const UpdateArgs &a, hipStream_t s);       // BL, A, B per sample
 void launch_update_lines(const UpdateArgs &a, hipStream_t s);         // stochastic pulse words and their bit planes
+// both in one launch, for small calls with one row of words to a sample
+bool update_prepares_in_lines(const UpdateArgs &a);
+void launch_update_lines_small(const UpdateArgs &a, hipStream_t s);
 void launch_update_implicit_lines(const UpdateArgs &a, hipStream_t s); // deterministic line values
 void launch_words_from_planes(const UpdateArgs &a, hipStream_t s);    // x_words / d_words of an update that kept bit planes only
 void launch_update_planes(const UpdateArgs &a, hipStream_t s);        // bit planes of pulse words made elsewhere

@@ -337,7 +337,8 @@ constexpr int UPDATE_PLANES_ONLY_KMAX = 7;
 // there are four times as many workgroups.
 // bx: number of the workgroup's block of line elements (x blocks first, then d blocks), by: its block of 64 rows of words
 // IN_PLACE: the call may read its lines from the tensors of the indexed interface (UpdateArgs::x_index, d_group)
-template <int LINES_E, bool IN_PLACE = false>
+// THREADS: of the workgroup; more than 64 per element have nothing to do here (k_update_lines_small)
+template <int LINES_E, bool IN_PLACE = false, int THREADS = 256>
 __device__ __forceinline__ void update_lines_block(const UpdateArgs &a, const int bx, const int by,
                                                    float (*vals)[LINES_E + 1], uint32_t (*wt)[LINES_E + 1]) {
   const int tiles_x = (a.x_size + LINES_E - 1) / LINES_E;
@@ -348,7 +349,8 @@ __device__ __forceinline__ void update_lines_block(const UpdateArgs &a, const in
   const float *src = is_x ? a.x : a.d;
   const long s_b = is_x ? a.x_sb : a.d_sb, s_e = is_x ? a.x_sj : a.d_si;
   const int stored = size - (is_x ? a.x_one : 0); // (a row of words behind the batch has no pulses, whatever its values)
-  constexpr int ROWS_PER_PASS = 256 / LINES_E;
+  constexpr int ROWS_PER_PASS = THREADS / LINES_E, PASSES = ROWS_PER_PASS < 64 ? 64 / ROWS_PER_PASS : 1;
+  static_assert(!IN_PLACE || THREADS == 256, "lines in place");
   const int col = threadIdx.x % LINES_E, row0 = threadIdx.x / LINES_E;
   const int wps = max(a.words_per_sample, 1);
   if (IN_PLACE && is_x && a.x_index) {
@@ -385,8 +387,9 @@ __device__ __forceinline__ void update_lines_block(const UpdateArgs &a, const in
     }
   } else {
 #pragma unroll
-    for (int i = 0; i < 64 / ROWS_PER_PASS; ++i) {
+    for (int i = 0; i < PASSES; ++i) {
       const int rb = row0 + ROWS_PER_PASS * i;
+      if (ROWS_PER_PASS > 64 && rb >= 64) break;
       const int b = b0 + rb, e = e0 + col;
       const int sample = wps > 1 ? b / wps : b;
       vals[rb][col] = (b < a.m_batch && e < stored) ? src[(long)sample * s_b + (long)e * s_e] : (e < size ? 1.0f : 0.0f);
@@ -406,7 +409,7 @@ __device__ __forceinline__ void update_lines_block(const UpdateArgs &a, const in
   if (!keep_words && pulses_by_slot(a, kmax)) {
     // the element is the same for all lanes: its share of the generator is scalar work, the sample's is done once
     const PhiloxSecond second = philox_second((uint32_t)sample, a.call, a.key);
-    for (int el = wave; el < LINES_E; el += 4) {
+    for (int el = wave; el < LINES_E; el += THREADS / 64) {
       const int e = e0 + el;
       if (e >= size) break; // wave-uniform
       const float v = vals[lane][el], PP = fabsf(v) * P, most = PP * 16777216.0f;
@@ -433,7 +436,7 @@ __device__ __forceinline__ void update_lines_block(const UpdateArgs &a, const in
     }
     return;
   }
-  for (int el = wave; el < LINES_E; el += 4) {
+  for (int el = wave; el < LINES_E; el += THREADS / 64) {
     const int e = e0 + el;
     if (e >= size) break; // wave-uniform
     const uint32_t word = b_ok ? pulse_word(a, is_x, e, sample, vals[lane][el], P, K, wrow) : 0u;
@@ -461,8 +464,9 @@ __device__ __forceinline__ void update_lines_block(const UpdateArgs &a, const in
   __syncthreads();
   uint32_t *words = is_x ? a.x_words : a.d_words;
 #pragma unroll
-  for (int i = 0; i < 64 / ROWS_PER_PASS; ++i) {
+  for (int i = 0; i < PASSES; ++i) {
     const int rb = row0 + ROWS_PER_PASS * i;
+    if (ROWS_PER_PASS > 64 && rb >= 64) break;
     const int bb = b0 + rb, ee = e0 + col;
     if (bb < a.m_batch && ee < size) words[(long)bb * size + ee] = wt[rb][col];
   }
@@ -471,24 +475,104 @@ __device__ __forceinline__ void update_lines_block(const UpdateArgs &a, const in
 // Row-major copy a.w of the [x_size][d_size] matrix a.wt_src for the pulse loop, 32 x 32 tiles through LDS: made by
 // the `workers` workgroups that the launch of the pulse trains carries beyond its own, so that it costs no launch of its
 // own and runs beside that kernel's work (me: number of this one among them).
+template <int THREADS = 256>
 __device__ __forceinline__ void update_copy_weights(const UpdateArgs &a, int me, int workers, float (*tile)[33]) {
   const int tiles_j = (a.x_size + 31) / 32, tiles_i = (a.d_size + 31) / 32;
-  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5; // 8 rows of 32 per pass
+  constexpr int ROWS = THREADS / 32; // of 32 per pass
+  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
   for (int t = me; t < tiles_j * tiles_i; t += workers) {
     const int j0 = (t / tiles_i) * 32, i0 = (t % tiles_i) * 32;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int j = j0 + ty + 8 * r, i = i0 + tx;
-      tile[ty + 8 * r][tx] = (j < a.x_size && i < a.d_size) ? a.wt_src[(size_t)j * a.d_size + i] : 0.0f;
+    for (int r = 0; r < 32 / ROWS; ++r) {
+      const int j = j0 + ty + ROWS * r, i = i0 + tx;
+      tile[ty + ROWS * r][tx] = (j < a.x_size && i < a.d_size) ? a.wt_src[(size_t)j * a.d_size + i] : 0.0f;
     }
     __syncthreads();
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int i = i0 + ty + 8 * r, j = j0 + tx;
-      if (i < a.d_size && j < a.x_size) a.w[(size_t)i * a.x_size + j] = tile[tx][ty + 8 * r];
+    for (int r = 0; r < 32 / ROWS; ++r) {
+      const int i = i0 + ty + ROWS * r, j = j0 + tx;
+      if (i < a.d_size && j < a.x_size) a.w[(size_t)i * a.x_size + j] = tile[tx][ty + ROWS * r];
     }
     __syncthreads();
   }
+}
+
+// largest absolute value over the part of a line that thread `t` of `width` takes, four neighbours at a time from any address
+__device__ __forceinline__ float part_abs_max_wide(const float *v, int n, long stride, int t, int width) {
+  typedef float four __attribute__((ext_vector_type(4), aligned(4)));
+  float m = 0.0f;
+  const int whole = stride == 1 ? n & ~3 : 0;
+#pragma unroll 4
+  for (int j = 4 * t; j < whole; j += 4 * width) {
+    const four x = *reinterpret_cast<const four *>(v + j);
+    m = fmaxf(fmaxf(m, fmaxf(fabsf(x.x), fabsf(x.y))), fmaxf(fabsf(x.z), fabsf(x.w)));
+  }
+  for (int j = whole + t; j < n; j += width) m = fmaxf(m, fabsf(v[(long)j * stride]));
+  return m;
+}
+
+// k_update_prepare and k_update_lines in one launch, for a few samples of short lines: every workgroup finds the maxima of all
+// samples for itself, all sixteen waves, and the first four of them then make the pulse trains of four line elements.  Bound by
+// latencies, as the launch it saves: update of 129 x 10, 64 samples 14.7 -> 13.5 us, one sample 10.8 -> 7.7.
+constexpr int SMALL_LINES_SAMPLES = 64, SMALL_LINES_VALUES = 25600;
+__global__ __launch_bounds__(1024) void k_update_lines_small(UpdateArgs a) {
+  __shared__ float tile[32][33];
+  __shared__ uint32_t wt[64][5];
+  __shared__ int sh_max[2][SMALL_LINES_SAMPLES], sh_bl[SMALL_LINES_SAMPLES], sh_kmax;
+  __shared__ float sh_a[SMALL_LINES_SAMPLES], sh_b[SMALL_LINES_SAMPLES];
+  const int own = (a.x_size + 3) / 4 + (a.d_size + 3) / 4, t = (int)threadIdx.x;
+  if ((int)blockIdx.x >= own) { // only launched with a.wt_src set
+    update_copy_weights<1024>(a, (int)blockIdx.x - own, (int)gridDim.x - own, tile);
+    return;
+  }
+  if (t < 2 * SMALL_LINES_SAMPLES) sh_max[t / SMALL_LINES_SAMPLES][t % SMALL_LINES_SAMPLES] = 0;
+  if (t == 0) sh_kmax = 0;
+  __syncthreads();
+  if (a.up.update_management || a.up.update_bl_management) {
+    int shift = 4; // 16 to 1024 threads share a sample
+    while (shift < 10 && (a.m_batch << (shift + 1)) <= 1024) ++shift;
+    const int b = t >> shift, sub = t & ((1 << shift) - 1), lanes = min(1 << shift, 64);
+    if (b < a.m_batch) {
+      float xm = part_abs_max_wide(a.x + (long)b * a.x_sb, a.x_size - a.x_one, a.x_sj, sub, 1 << shift);
+      float dm = part_abs_max_wide(a.d + (long)b * a.d_sb, a.d_size, a.d_si, sub, 1 << shift);
+      if (a.x_one) xm = fmaxf(xm, 1.0f);
+      for (int off = lanes / 2; off > 0; off >>= 1) {
+        xm = fmaxf(xm, __shfl_xor(xm, off));
+        dm = fmaxf(dm, __shfl_xor(dm, off));
+      }
+      if ((sub & (lanes - 1)) == 0) { // (not negative, never NaN: in the order of their bits)
+        atomicMax(&sh_max[0][b], __float_as_int(xm));
+        atomicMax(&sh_max[1][b], __float_as_int(dm));
+      }
+    }
+    __syncthreads();
+  }
+  if (t < a.m_batch) {
+    int BL;
+    float A, B;
+    update_bl_ab(a, __int_as_float(sh_max[0][t]), __int_as_float(sh_max[1][t]), BL, A, B);
+    sh_bl[t] = BL;
+    sh_a[t] = A;
+    sh_b[t] = B;
+    if (BL > 0) atomicMax(&sh_kmax, min(BL, 31));
+    if (blockIdx.x == 0) {
+      a.bl[t] = BL;
+      a.prob_a[t] = A;
+      a.prob_b[t] = B;
+    }
+  }
+  __syncthreads();
+  if (blockIdx.x == 0 && t == 0) { // as update_prepare_finish leaves them
+    a.kmax[a.kmax_slot] = sh_kmax;
+    a.kmax[a.kmax_slot ^ 1] = 0;
+  }
+  UpdateArgs mine = a;
+  mine.bl = sh_bl;
+  mine.prob_a = sh_a;
+  mine.prob_b = sh_b;
+  mine.kmax = &sh_kmax;
+  mine.kmax_slot = 0;
+  update_lines_block<4, false, 1024>(mine, (int)blockIdx.x, 0, reinterpret_cast<float (*)[5]>(&tile[0][0]), wt);
 }
 
 template <int LINES_E, bool IN_PLACE = false>
@@ -2485,6 +2569,19 @@ void launch_update_prepare(const UpdateArgs &a, hipStream_t s) {
 // 1024 x 1024, 16 samples 27.2 / 23.3, 256 49.5 / 48.3, 1000 120 / 118.
 static unsigned update_copy_workgroups(const UpdateArgs &a) {
   return a.wt_src ? std::min(1024u, (unsigned)(((a.x_size + 31) / 32) * ((a.d_size + 31) / 32))) : 0u;
+}
+// Whether a call of one row of words to a sample takes k_update_lines_small: every workgroup reads all of its lines.  Updates, us,
+// two launches / one: 17 x 10, 5 samples 10.7 / 8.4; 129 x 10, 1 10.8 / 7.7, 64 14.7 / 13.5; 785 x 256, 1 11.3 / 9.5, 16 12.3 / 12.2;
+// 512 x 512, 16 12.4 / 10.9; 300 x 200, 50 14.5 / 14.3; 785 x 300, 20 13.1 / 12.7.  Beyond: 785 x 256, 32 14.0 / 15.0, 64 17.0 /
+// 20.1; 1024 x 1024, 1 14.6 / 15.0, 16 17.2 / 17.5.
+bool update_prepares_in_lines(const UpdateArgs &a) {
+  const long line = (long)a.x_size + a.d_size;
+  return !a.x_index && !a.d_group && !a.row_cost && a.kmax && a.m_batch <= SMALL_LINES_SAMPLES && (a.x_sj == 1 || a.m_batch == 1) &&
+         (a.d_si == 1 || a.m_batch == 1) && line <= 1536 && a.m_batch * line <= SMALL_LINES_VALUES && a.m_batch * line * line <= (1L << 24);
+}
+void launch_update_lines_small(const UpdateArgs &a, hipStream_t s) {
+  const unsigned own = (a.x_size + 3) / 4 + (a.d_size + 3) / 4;
+  hipLaunchKernelGGL(k_update_lines_small, dim3(own + update_copy_workgroups(a)), dim3(1024), 0, s, a);
 }
 void launch_update_lines(const UpdateArgs &a, hipStream_t s) {
   const unsigned sample_tiles = (a.m_batch + 63) / 64;

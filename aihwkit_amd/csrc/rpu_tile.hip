@@ -1738,8 +1738,12 @@ struct Tile {
     const int rows = B * wps;
     prof_begin(s);
     const bool counting = dev.p.count_pulses && !is_transfer();
-    launch_update_prepare(a, s);
-    prof_mark(s, "update_prepare");
+    // (batches as small as that take neither lane masks nor planes of long chains, so that all is decided here)
+    const bool prepares_in_lines = up.p.pulse_type == RPU_PULSE_STOCHASTIC_COMPRESSED && wps == 1 && !ws && update_prepares_in_lines(a);
+    if (!prepares_in_lines) {
+      launch_update_prepare(a, s);
+      prof_mark(s, "update_prepare");
+    }
     if (up.p.pulse_type == RPU_PULSE_STOCHASTIC_COMPRESSED) {
       // from here on the kernels walk rows of words; a longer bit line is several rows of one sample in a row
       a.m_batch = rows;
@@ -1763,7 +1767,8 @@ struct Tile {
         row_major_pulse_loop(a);
         a.wt_src = d_w.p; // the launch of the pulse trains makes the row-major copy
       }
-      launch_update_lines(a, s);
+      if (prepares_in_lines) launch_update_lines_small(a, s);
+      else launch_update_lines(a, s);
       prof_mark(s, "update_lines");
       if (counting) count_pulses(a, false, s);
       if (words) {

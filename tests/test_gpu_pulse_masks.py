@@ -197,3 +197,39 @@ def test_bias_column_that_is_not_stored(x_size, d_size, batch, pulse_type, blm, 
         results.append(tile.get_weights())
     assert torch.equal(results[0], results[1])
     assert float(results[0][:, -1].abs().max()) > 0.0
+
+
+# small calls find their maxima in the launch that makes the pulse trains (k_update_lines_small), the same tile in a group has a
+# launch for them: one sample (1024 threads to it, 16 at 64), samples and lines at and next to the ends of the range (25600 values,
+# lines of 1536), a last block of line elements that is not full, a gradient that is zero, values that are not finite
+@pytest.mark.parametrize("x_size,d_size,batch", [(1, 1, 1), (3, 2, 64), (129, 10, 63), (130, 11, 65), (785, 256, 1), (785, 751, 2), (785, 752, 2),
+                                                 (300, 100, 64), (301, 100, 64), (63, 5, 17), (1000, 17, 16)])
+@pytest.mark.parametrize("um,blm,desired_bl", [(True, True, 31), (True, False, 5), (False, False, 31)])
+def test_small_calls_prepare_in_the_launch_of_the_pulse_trains(x_size, d_size, batch, um, blm, desired_bl, storage_mode):
+    from aihwkit_amd.rpu_base import tiles
+    from aihwkit_amd.rpu_base.tiles import TileGroup
+    x, d = _data(x_size, d_size, batch, 0)
+    d[batch // 2] = 0.0
+    if batch > 2:
+        x[1, 0], d[2, -1] = float("inf"), float("nan")
+    pair = []
+    for _ in range(2):
+        host = make_meta(desired_bl=desired_bl, update_management=um, update_bl_management=blm).create_array(x_size, d_size, _device("soft_bounds"))
+        host.set_weights(torch.from_numpy(np.random.default_rng(3).uniform(-0.4, 0.4, (d_size, x_size)).astype(np.float32)))
+        tile = tiles.CudaAnalogTile(host)
+        tile.set_seed(17)
+        tile.set_learning_rate(0.004)
+        pair.append(tile)
+    one, other = pair
+    group = TileGroup([other])
+    for _ in range(2):
+        one.update(x, d, False)
+        group.update([x], [d])
+    assert torch.equal(one.get_weights(), other.get_weights())
+    for mine, theirs in zip(one.get_update_words(batch), other.get_update_words(batch)):
+        assert torch.equal(mine, theirs)
+    if batch > 1 and x_size > 1:  # lines that run the other way take the two launches
+        before = one.get_weights()
+        one.update(x.t().contiguous(), d.t().contiguous(), False, True, True)
+        group.update([x], [d])
+        assert torch.equal(one.get_weights(), other.get_weights()) and not torch.equal(one.get_weights(), before)
