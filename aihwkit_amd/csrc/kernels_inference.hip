@@ -250,10 +250,12 @@ void launch_gather_indexed(float *x_mat, const float *images, const int *indices
 // patch) in the order of the reference's loop (math_util / rpu.cpp:1130-1141 walks k, then p), added one after the
 // other from zero: the same bits on every run, and the reference's.  x_mat is line-major, [x_size][n_images * patches]:
 // neighbouring image elements meet the same lines at neighbouring patches, so a wave reads runs of a row.
+// A thread adds up one image element of NI images: the list entries, eight bytes for the four of a value, are read once for all of
+// them, U at a time with all values that they name on their way together.  Bound by memory: 48 -> 48
+// channels, 128 images of 34 x 34 (227 MB of patch entries): 121 us with four images and four entries, 70 with sixteen and nine.
+template <int NI, int U>
 __global__ __launch_bounds__(256) void k_fold_indexed(float *images, const float *x_mat, const int *ptr, const int2 *kp,
                                                       int patches, int n_images, long image_size) {
-  // a thread adds up one image element of four images: the list entries are read once for the four
-  constexpr int NI = 4;
   const int groups = (n_images + NI - 1) / NI;
   const size_t total = (size_t)groups * image_size;
   const long row = (long)n_images * patches;
@@ -266,20 +268,19 @@ __global__ __launch_bounds__(256) void k_fold_indexed(float *images, const float
 #pragma unroll
     for (int i = 0; i < NI; ++i) acc[i] = 0.0f;
     const int t_end = ptr[e + 1];
-    for (int t0 = ptr[e]; t0 < t_end; t0 += 4) { // sixteen loads in flight, added in list order
-      float v[4][NI];
+    for (int t0 = ptr[e]; t0 < t_end; t0 += U) { // added in list order
+      int2 q[U];
+      float v[U][NI];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        long at = 0;
-        if (t0 + u < t_end) {
-          const int2 q = kp[t0 + u];
-          at = (long)q.x * row + q.y;
-        }
+      for (int u = 0; u < U; ++u) q[u] = t0 + u < t_end ? kp[t0 + u] : make_int2(0, 0);
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const long at = (long)q[u].x * row + q[u].y;
 #pragma unroll
         for (int i = 0; i < NI; ++i) v[u][i] = (t0 + u < t_end && i < live) ? src[at + (long)i * patches] : 0.0f;
       }
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
+      for (int u = 0; u < U; ++u) {
         if (t0 + u < t_end) {
 #pragma unroll
           for (int i = 0; i < NI; ++i) acc[i] += v[u][i];
@@ -295,10 +296,19 @@ __global__ __launch_bounds__(256) void k_fold_indexed(float *images, const float
 
 void launch_fold_indexed(float *images, const float *x_mat, const int *ptr, const int *kp, int x_size, int patches,
                          int n_images, long image_size, hipStream_t s) {
-  (void)x_size;
-  const size_t total = (size_t)((n_images + 3) / 4) * image_size;
-  hipLaunchKernelGGL(k_fold_indexed, dim3(grid_of(total)), dim3(256), 0, s, images, x_mat, ptr,
-                     reinterpret_cast<const int2 *>(kp), patches, n_images, image_size);
+  const auto threads = [&](int images_per_thread) { return (size_t)((n_images + images_per_thread - 1) / images_per_thread) * image_size; };
+  const int2 *lists = reinterpret_cast<const int2 *>(kp);
+#define RPU_FOLD(NI, U) \
+  hipLaunchKernelGGL((k_fold_indexed<NI, U>), dim3(grid_of(threads(NI))), dim3(256), 0, s, images, x_mat, ptr, lists, patches, n_images, image_size)
+  // Lists of one to four entries on average (kernels no larger than their strides by more than that): four at a time, backward of 1 x
+  // 1, 64 -> 64 channels, 64 images of 16 x 16 28 us, with nine 29.  Nine are the lists of 3 x 3 kernels; of 5 x 5, 32 -> 32, 64
+  // images of 30 x 30 212 -> 165.  More images to a thread as long as two waves are left to a SIMD: 64 -> 64, 32 images of 36 x 36
+  // 109 -> 102, 48 150 -> 138; 16 of 16 x 16 (four to a thread) 26 -> 25.
+  if ((double)x_size * patches <= 4.0 * image_size) RPU_FOLD(4, 4);
+  else if (threads(16) >= (1u << 17)) RPU_FOLD(16, 9);
+  else if (threads(8) >= (1u << 17)) RPU_FOLD(8, 9);
+  else RPU_FOLD(4, 9);
+#undef RPU_FOLD
 }
 
 void launch_images_to_lines(float *lines_major, const float *images, int n_images, int lines, int patches, hipStream_t s) {

@@ -355,3 +355,26 @@ def test_pulsed_update_reads_patches_and_gradients_in_place(gpu_device, case):
         got.append(gpu.get_weights().clone())
     assert torch.equal(got[0], got[1])
     assert (got[0] - torch.from_numpy(np.clip(w.numpy(), -0.6, 0.6))).abs().max() > 1e-3
+
+
+# sixteen, eight and four images to a thread, with a last group of one image and one that is full; lists of one entry, of exactly
+# nine, of ten to twenty-five (three trips of nine) and of none (an edge that the stride passes over)
+@pytest.mark.parametrize("c_in,side,n,kernel,stride", [(16, 48, 49, 3, 1), (16, 48, 64, 5, 1), (16, 48, 33, 3, 1), (16, 48, 32, 4, 1), (5, 13, 7, 3, 1),
+                                                       (5, 13, 9, 5, 1), (16, 48, 49, 1, 1), (4, 17, 6, 2, 2), (3, 18, 21, 3, 2), (1, 6, 1, 6, 1)])
+def test_indexed_backward_of_whole_numbers_is_the_transposed_convolution(gpu_device, c_in, side, n, kernel, stride):
+    rng = np.random.default_rng(side)
+    c_out, out_side = 6, (side - kernel) // stride + 1
+    indices, patches = conv_indices((c_in, side, side), (kernel, kernel), (stride, stride), (0, 0), (1, 1), True)
+    x_size = c_in * kernel * kernel + 1
+    host = dv.FloatingPointTileParameter().create_array(x_size, c_out)
+    w = rng.integers(-3, 4, (c_out, x_size)).astype(np.float32)
+    host.set_weights(torch.from_numpy(w))
+    gpu = tiles.CudaFloatingPointTile(host)
+    gpu.set_matrix_indices(indices)
+    grad = rng.integers(-4, 5, (n, c_out, out_side, out_side)).astype(np.float32)
+    dx = gpu.backward_indexed(cuda(grad), torch.full((n, c_in, side, side), 7.0).cuda()).cpu()
+    weight = torch.from_numpy(w[:, :-1].reshape(c_out, c_in, kernel, kernel).astype(np.float64))
+    want = torch.zeros(n, c_in, side, side, dtype=torch.float64)
+    span = (out_side - 1) * stride + kernel
+    want[:, :, :span, :span] = F.conv_transpose2d(torch.from_numpy(grad.astype(np.float64)), weight, stride=stride)
+    assert torch.equal(dx.double(), want)
