@@ -322,7 +322,9 @@ bool product_plan(const MvmArgs &a, ProductArgs &p) {
   // 16384 268 / 47, but 64 x 3072 of 2048 26 / 29
   const long tiles_32 = (long)((a.O + 31) / 32) * ((a.m_batch + 31) / 32);
   const bool long_chain = (double)((tiles_32 + n_cus - 1) / n_cus) * a.K >= 4096.0 && work >= 0x1p27 && !mvm_uses_large_tiles(a.m_batch, a.O);
-  if (!(work >= 0x1.8p29 && a.K >= 128) && !long_chain) return false;
+  // products per split value: few outputs or few samples leave a launch that splits and little else
+  const double reuse = (double)a.m_batch * a.O / ((double)a.m_batch + a.O);
+  if (!(work >= 0x1.8p29 && a.K >= 128 && reuse >= 96.0) && !(long_chain && reuse >= 32.0)) return false;
   double best = 0.0;
   for (int bt = 64; bt <= 128; bt += 64) {
     const int tiles_b = (a.m_batch + bt - 1) / bt;
@@ -344,7 +346,7 @@ bool product_plan(const MvmArgs &a, ProductArgs &p) {
       }
     }
   }
-  return true;
+  return product_scratch(p, nullptr, nullptr) <= ((size_t)2 << 30); // rows padded to 128 are many times the operand of a long, narrow call
 }
 
 static int sample_blocks(const ProductArgs &p) { return p.sample_tile == PT ? p.tiles_b : (p.tiles_b + 1) / 2; } // of 128 rows
