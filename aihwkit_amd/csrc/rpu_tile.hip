@@ -785,7 +785,7 @@ struct Tile {
     a.max_rounds = io.perfect ? 0 : mvm_max_rounds(a.io);
     size_t rows = (size_t)B * a.k_pad;
     if (a.max_rounds > 2) rows = std::max(rows, (size_t)std::min(B, mvm_few_batch(a)) * O); // see few_args
-    s_xq0.ensure(rows);
+    if (!io.perfect) s_xq0.ensure(rows); // (exact calls may need none: exact_product, ensure_exact_rows)
     if (!io.perfect && io.p.bound_management != RPU_BM_NONE) s_xq1.ensure(rows);
     a.xq[0] = s_xq0.p; a.xq[1] = s_xq1.p;
     // rows for the next bound-management round are quantized ahead when the batch is small (shortest path between
@@ -974,19 +974,23 @@ struct Tile {
 
   const GatherSource *lines_in_place = nullptr; // set while update_indexed runs a pulsed update (pulsed_update_args)
 
+  void ensure_exact_rows(MvmArgs &a) {
+    s_xq0.ensure((size_t)a.m_batch * a.k_pad);
+    a.xq[0] = s_xq0.p;
+  }
   // out = alpha * (weights * inputs) + beta * out
   void exact_product(MvmArgs &a, hipStream_t s, const char *first, const char *second) {
     ProductArgs p;
     // (where values are out of the range of the parts, the product reads the inputs themselves)
     const bool parts = product_plan(a, p) && !writes_into_its_input(a);
     if (parts) {
-      s_parts.ensure(product_scratch(p, nullptr, nullptr));
+      const size_t bytes = product_scratch(p, nullptr, nullptr);
+      if (bytes > s_parts.n) s_parts.ensure(bytes + bytes / 4); // the other calls of a training step take about as much
       (void)product_scratch(p, s_parts.p, &p);
       launch_product_parts(a, p, s);
     } else {
       a.k_pad = a.k_pad ? a.k_pad : mvm_k_pad(a.K);
-      s_xq0.ensure((size_t)a.m_batch * a.k_pad);
-      a.xq[0] = s_xq0.p;
+      ensure_exact_rows(a);
       launch_mvm_init(a, s);
     }
     prof_mark(s, first);
@@ -2981,6 +2985,7 @@ static int group_mvm(rpu_group_t *group, const float *const *x_dev, const long *
       const int in_size = transposed ? t.D : t.X, out_size = transposed ? t.X : t.D;
       const bool big = use_big && out_size >= 128;
       MvmArgs a = t.mvm_args(m_batch, transposed, t.mvm_weights(is_test), transposed ? t.bio : t.fio, big ? 1 : 0);
+      if (a.io.perfect) t.ensure_exact_rows(a);
       a.in = x_dev[i]; a.in_sb = x_ld ? x_ld[i] : in_size; a.in_sk = 1;
       a.out = y_dev[i]; a.out_sb = y_ld ? y_ld[i] : out_size; a.out_so = 1;
       if (a.in_sb < in_size || a.out_sb < out_size) throw RpuError("A row stride is shorter than the row.");
