@@ -8,7 +8,7 @@
 //
 // In the kernels that split what they stage (k_mvm_big, three parts) a wave issues 220 vector instructions for the 16 MFMAs of a
 // stage and waits for a third of the rest: 27 % of the matrix pipe's time at 768 x 2304 outputs of 1024 terms.  Here a stage is
-// 24 or 32 MFMAs and 18 reads of LDS to a wave, a byte staged meets more multiply-adds, and splitting the terms fills the CUs that
+// 32 MFMAs and 18 reads of LDS to a wave, a byte staged meets more multiply-adds, and splitting the terms fills the CUs that
 // few large tiles leave idle.  768 -> 2304, 1024 samples, backward 79 -> 43 us (parts 8, product 30, sums 5).  What bounds it: the
 // matrix pipe (1024 x 1024, 16384 samples: 1.2 PFLOP/s of bf16 products, the rate of a large library product on this card).
 #include "bf16_parts.h"
@@ -144,15 +144,13 @@ __device__ __forceinline__ void product_place(int t, int i, int &o, int &b) {
   b = (wave >> 1) * 32 + (lane & 31);
 }
 
-// Of the nine products of the parts, that of the two low ones (2^-36 of the whole) is left out.  SIX: those of a low with a middle
-// one too (at most 2^-27 of the whole each), for sums of 512 terms and more, which round more than that: error against 64
-// bits, relative, nine parts but one / six products: 64 terms 4.91 / 4.95e-8, 256 8.93 / 8.95, 1024 1.30 / 1.29e-7, 2048 1.42 /
-// 1.42; the kernels that ran these sums before 4.92e-8, 8.93e-8, 1.9 to 2.9e-7 and 2.8 to 4.1e-7.  768 -> 2304, 1024 samples,
-// backward and update 47 -> 44 us.
+// Of the nine products of the parts, that of the two low ones (2^-36 of the whole) is left out.  Those of a low with a middle part
+// (up to 2^-26 of the whole together) are small beside the rounding of a long dense sum, but not where few terms count: one
+// term of 1024, largest error in units of the last place 0.51, without them 0.94.
 // BT samples of a workgroup tile: 128 (eight waves, 96 KB of LDS for two stages in turn, one workgroup to a CU) or 64 (four waves,
 // two workgroups to a CU).  Two waves to a SIMD either way: one reads fragments (18 for its 32 MFMAs) while the other multiplies.
 // The next stage is on its way to registers while one is worked on.
-template <int BT, bool SIX> __global__ __launch_bounds__(4 * BT, BT == 128 ? 1 : 2) void k_product(MvmArgs a, ProductArgs p) {
+template <int BT> __global__ __launch_bounds__(4 * BT, BT == 128 ? 1 : 2) void k_product(MvmArgs a, ProductArgs p) {
   constexpr int THREADS = 4 * BT, XPLANE = BT * PK;
   __shared__ __attribute__((aligned(16))) __bf16 lds_w[2][BLOCK], lds_x[2][3 * XPLANE];
   __shared__ int wide;
@@ -228,7 +226,7 @@ template <int BT, bool SIX> __global__ __launch_bounds__(4 * BT, BT == 128 ? 1 :
       }
       // part q of a weight with part m - q of an input, those that correct the product of the high parts to a sum of their own
 #pragma unroll
-      for (int m = SIX ? 2 : 3; m >= 0; --m) {
+      for (int m = 3; m >= 0; --m) {
 #pragma unroll
         for (int q = 0; q <= min(m, 2); ++q) {
           if (m - q > 2) continue;
@@ -376,14 +374,11 @@ void launch_product_parts(const MvmArgs &a, const ProductArgs &p, hipStream_t s)
 void launch_product(const MvmArgs &a, const ProductArgs &p, hipStream_t s) {
   const int tiles = p.tiles_o * p.tiles_b;
   const dim3 grid((unsigned)(8 * ((tiles * p.shares + 7) / 8))), sums((unsigned)(GROUPS * tiles)), block((unsigned)(4 * p.sample_tile));
-  const bool six = a.K >= 512;
   if (p.sample_tile == 128) {
-    if (six) hipLaunchKernelGGL((k_product<128, true>), grid, block, 0, s, a, p);
-    else hipLaunchKernelGGL((k_product<128, false>), grid, block, 0, s, a, p);
+    hipLaunchKernelGGL(k_product<128>, grid, block, 0, s, a, p);
     if (p.shares > 1) hipLaunchKernelGGL(k_product_sum<128>, sums, block, 0, s, a, p);
   } else {
-    if (six) hipLaunchKernelGGL((k_product<64, true>), grid, block, 0, s, a, p);
-    else hipLaunchKernelGGL((k_product<64, false>), grid, block, 0, s, a, p);
+    hipLaunchKernelGGL(k_product<64>, grid, block, 0, s, a, p);
     if (p.shares > 1) hipLaunchKernelGGL(k_product_sum<64>, sums, block, 0, s, a, p);
   }
 }

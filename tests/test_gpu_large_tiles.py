@@ -234,3 +234,35 @@ def test_exact_products_with_values_out_of_the_range_of_the_parts(gpu_device, x_
         bound = (x_size + 2) * 2.0 ** -24 * (np.abs(x.astype(np.float64)) @ np.abs(w.astype(np.float64)).T)
         assert np.all((np.abs(got.astype(np.float64) - want) <= bound + 1e-37)[fine])
     assert np.array_equal(got[:-128 - batch % 128, :-128 - d_size % 128], plain[:-128 - batch % 128, :-128 - d_size % 128])
+
+
+@pytest.mark.parametrize("x_size,d_size,batch", [(1024, 1100, 1024), (700, 3000, 1300), (2049, 2048, 600)])
+def test_one_term_that_is_not_zero(gpu_device, x_size, d_size, batch):
+    """One product, rounded once: half a unit in its last place.  The seven small products of its parts, together at most 2^-7
+    of it, round as often on the way to their sum: 7 * 2^-31 of the product, up to 2^24 units.  Two products left out, of a
+    low with a middle part, would be up to half a unit more."""
+    rng = np.random.default_rng(x_size)
+    io = noise_free_io()
+    io.is_perfect = True
+    w = rng.standard_normal((d_size, x_size)).astype(np.float32)
+    tile = _tile(x_size, d_size, io, w)
+    w64 = w.astype(np.float64)
+
+    def close(got, want):
+        unit = np.spacing(np.abs(want).astype(np.float32)).astype(np.float64)
+        assert np.max(np.abs(got.cpu().numpy().astype(np.float64) - want) / unit) <= 0.5 + 7.0 * 2.0 ** -7
+
+    def one_a_row(rows, width):
+        v = np.zeros((rows, width), np.float32)
+        v[np.arange(rows), rng.integers(0, width, rows)] = rng.standard_normal(rows)
+        return v
+
+    x, d = one_a_row(batch, x_size), one_a_row(batch, d_size)
+    close(tile.forward(torch.from_numpy(x).cuda()), x @ w64.T)
+    close(tile.backward(torch.from_numpy(d).cuda()), d @ w64)
+    x = np.ascontiguousarray(one_a_row(x_size, batch).T)  # every weight meets one sample
+    d = rng.standard_normal((batch, d_size)).astype(np.float32)
+    tile.set_weights(torch.zeros(d_size, x_size))
+    tile.set_learning_rate(0.5)
+    tile.update(torch.from_numpy(x).cuda(), torch.from_numpy(d).cuda(), False)
+    close(tile.get_weights(), -0.5 * (d.T.astype(np.float64) @ x))
