@@ -52,6 +52,12 @@ template <bool STAGED> __device__ __forceinline__ void split_bf16(const f32x4 v,
     lo[i] = pack_bf16<STAGED>(a1 - __uint_as_float(mid[i] << 16), b1 - __uint_as_float(mid[i] & 0xffff0000u));
   }
 }
+// Values of two operands, both split as 2^16 times themselves, below which the sum of `terms` of their products is finite before the
+// 2^32 is taken out of it: terms * safe^2 * 2^32 <= 2^127.  The largest power of two that is.
+__host__ __device__ inline float parts_safe(int terms) {
+  const int bits = terms > 1 ? 32 - __builtin_clz((unsigned)terms - 1u) : 0;
+  return __builtin_bit_cast(float, (uint32_t)(127 + (95 - bits) / 2) << 23);
+}
 __device__ __forceinline__ float max_abs4(float m, const f32x4 v) { // NaN do not count
   // two instructions; the compiler quiets every operand of fmaxf first, eight more
   asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(m) : "v"(v.x), "v"(v.y));

@@ -223,6 +223,7 @@ struct ProductArgs {
   float *partial;            // [share][tile] sums, with more than one share
   int tiles_o, tiles_b, stages, shares, stages_per_share;
   int sample_tile;           // samples of a workgroup tile
+  float safe;                // values from here on are out of the range of the parts (parts_safe)
 };
 bool product_plan(const MvmArgs &a, ProductArgs &p); // whether the call is one, and its sizes
 size_t product_scratch(const ProductArgs &p, unsigned char *base, ProductArgs *out); // bytes; places in `base` where it is not null

@@ -24,11 +24,10 @@ constexpr int PK = 32;                      // terms of a stage
 constexpr int PLANE = PT * PK;              // values of a plane of a block
 constexpr int BLOCK = 3 * PLANE;            // ... of a block: the parts of PT rows x PK terms
 constexpr float LIFT = 0x1p16f;             // the parts are those of this times the value (split_bf16)
-constexpr float SAFE = 0x1p44f;             // parts and products stay finite below it
 
 // 64 rows x 64 terms of an operand: element (row, k) at src[row * s_r + k * s_k]; term one_k is 1 and not stored (-1: none)
 __device__ __forceinline__ void product_parts_block(const float *src, long s_r, long s_k, int rows, int K, int one_k, int rb, int kb, __bf16 *parts,
-                                                    int *flags, int stages, float (*tile)[65]) {
+                                                    int *flags, int stages, float safe, float (*tile)[65]) {
   const int t = (int)threadIdx.x, r0 = rb * 64, k0 = kb * 64;
   const int stored = one_k >= 0 ? one_k : K;
   const bool along_k = s_k == 1;
@@ -86,7 +85,7 @@ __device__ __forceinline__ void product_parts_block(const float *src, long s_r, 
       part[1][2 * half] = mid.x; part[1][2 * half + 1] = mid.y;
       part[2][2 * half] = lo.x; part[2][2 * half + 1] = lo.y;
     }
-    wide[p] = !(m < SAFE);
+    wide[p] = !(m < safe);
     const int stage = 2 * kb + p;
     if (stage < stages) {
       __bf16 *dst = parts + ((long)(rb >> 1) * stages + stage) * BLOCK + big_x_offset((rb & 1) * 64 + row, chunk);
@@ -107,10 +106,10 @@ __global__ __launch_bounds__(256) void k_product_parts(MvmArgs a, ProductArgs p)
   const int kbs = (p.stages + 1) / 2, w_blocks = 2 * p.tiles_o * kbs;
   int n = (int)blockIdx.x;
   if (n < w_blocks) {
-    product_parts_block(a.w, a.w_oc ? 1 : a.w_ld, a.w_oc ? a.w_ld : 1, a.O, a.K, -1, n / kbs, n % kbs, p.w_parts, p.w_flags, p.stages, tile);
+    product_parts_block(a.w, a.w_oc ? 1 : a.w_ld, a.w_oc ? a.w_ld : 1, a.O, a.K, -1, n / kbs, n % kbs, p.w_parts, p.w_flags, p.stages, p.safe, tile);
   } else {
     n -= w_blocks;
-    product_parts_block(a.in, a.in_sb, a.in_sk, a.m_batch, a.K, a.in_one ? a.K - 1 : -1, n / kbs, n % kbs, p.x_parts, p.x_flags, p.stages, tile);
+    product_parts_block(a.in, a.in_sb, a.in_sk, a.m_batch, a.K, a.in_one ? a.K - 1 : -1, n / kbs, n % kbs, p.x_parts, p.x_flags, p.stages, p.safe, tile);
   }
 }
 
@@ -309,6 +308,7 @@ bool product_plan(const MvmArgs &a, ProductArgs &p) {
   if (!a.io.perfect || a.in_index || a.pre_add || a.skip_if_zero || a.nm_phase || a.small_tiles_only) return false;
   p.tiles_o = (a.O + PT - 1) / PT;
   p.stages = (a.K + PK - 1) / PK;
+  p.safe = parts_safe(a.K);
   const int n_cus = a.cus > 0 ? a.cus : current_device_cus();
   // us, the launches of k_mvm_init and k_mvm_round or k_mvm_big / these.  From 3/4 G multiply-adds: 784 -> 256, 4096 samples (0.8
   // G) forward 41 / 33, update 52 / 33; 2048 x 2048, 256 (1.1 G) 36 / 36, backward 40 / 35; 1024 x 1024, 1024 45 / 35, 16384 317 /

@@ -266,3 +266,20 @@ def test_one_term_that_is_not_zero(gpu_device, x_size, d_size, batch):
     tile.set_learning_rate(0.5)
     tile.update(torch.from_numpy(x).cuda(), torch.from_numpy(d).cuda(), False)
     close(tile.get_weights(), -0.5 * (d.T.astype(np.float64) @ x))
+
+
+# 2^86 a product: the parts of one are finite with 2^16 in either operand, the sum of 512 of them is not
+@pytest.mark.parametrize("x_size,d_size,batch", [(16384, 100, 100), (4097, 256, 256), (1024, 1024, 1024), (1024, 512, 16384)])
+def test_exact_products_of_large_values_have_the_sums_of_fp32(gpu_device, x_size, d_size, batch):
+    """No sum is near the end of the range of fp32; each has the error of one in fp32, half a unit a term."""
+    io = noise_free_io()
+    io.is_perfect = True
+    below = (95 - int(np.ceil(np.log2(x_size)))) // 2 - 1  # the largest values that are multiplied in parts
+    for e, few in ((43, False), (43, True), (below, False), (below, True)):
+        v = np.full((batch, x_size), 1.9 * 2.0 ** e, np.float32)
+        w = np.full((d_size, x_size), 1.9 * 2.0 ** e, np.float32)
+        if few:  # in the last of the tiles alone, of one sign
+            v[:-1], w[:-1] = 1.0, -0.5
+        got = _tile(x_size, d_size, io, w).forward(torch.from_numpy(v).cuda()).cpu().numpy().astype(np.float64)
+        want = np.outer(v[:, 0].astype(np.float64), w[:, 0].astype(np.float64)) * x_size
+        assert np.all(np.abs(got - want) <= (x_size + 2) * 2.0 ** -24 * np.abs(want))
