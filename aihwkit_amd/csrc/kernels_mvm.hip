@@ -1767,7 +1767,8 @@ __device__ __forceinline__ void mvm_big_workgroup(const MvmArgs &a, const int ro
   // k * step times 1 / step is k up to a few units in the 24th bit: rounding to bf16 returns k itself
   const float inv_step = XP == 1 ? 1.0f / a.x_step : 1.0f;
   constexpr float LIFT = 0x1p16f; // the operands in parts are this times their value (split_bf16)
-  constexpr float SAFE = XP == 1 ? 0x1p84f : 0x1p44f; // parts and products stay finite below it
+  // below it the sums of the products of the parts are finite; with inputs of at most 256 steps those of 2^19 terms
+  const float safe = XP == 1 ? 0x1p84f : parts_safe(K);
   auto lds_store = [&](int buf, const f32x4 (&gx)[XJ], const f32x4 (&gw)[WJ]) __attribute__((always_inline)) {
     float m = 0.0f;
 #pragma unroll
@@ -1797,7 +1798,7 @@ __device__ __forceinline__ void mvm_big_workgroup(const MvmArgs &a, const int ro
         *reinterpret_cast<f32x4 *>(&lds_w[buf][(wt_k + WROWS * j) * WPITCH + wt_col]) = w;
       }
     }
-    if (!(m < SAFE)) sh_slow = 1;
+    if (!(m < safe)) sh_slow = 1;
   };
 
   floatx16 acc[NB], low[XP == 3 ? NB : 1];

@@ -283,3 +283,17 @@ def test_exact_products_of_large_values_have_the_sums_of_fp32(gpu_device, x_size
         got = _tile(x_size, d_size, io, w).forward(torch.from_numpy(v).cuda()).cpu().numpy().astype(np.float64)
         want = np.outer(v[:, 0].astype(np.float64), w[:, 0].astype(np.float64)) * x_size
         assert np.all(np.abs(got - want) <= (x_size + 2) * 2.0 ** -24 * np.abs(want))
+
+
+def test_large_tiles_of_large_values_have_the_sums_of_fp32(gpu_device):
+    """As above, in the kernel that splits what it stages (exact calls of a group)."""
+    x_size, d_size, batch = 512, 512, 8192
+    io = noise_free_io()
+    io.is_perfect = True
+    for e in (43, 42):
+        w = np.full((d_size, x_size), 1.9 * 2.0 ** e, np.float32)
+        group = tiles.TileGroup([_tile(x_size, d_size, io, w) for _ in range(2)])
+        v = torch.full((batch, x_size), float(np.float32(1.9 * 2.0 ** e)), device="cuda")
+        want = float(w[0, 0]) ** 2 * x_size
+        for got in group.forward([v, v]):
+            assert float((got.double() - want).abs().max()) <= (x_size + 2) * 2.0 ** -24 * want
