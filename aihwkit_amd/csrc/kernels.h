@@ -227,6 +227,7 @@ struct ProductArgs {
 };
 bool product_plan(const MvmArgs &a, ProductArgs &p); // whether the call is one, and its sizes
 size_t product_scratch(const ProductArgs &p, unsigned char *base, ProductArgs *out); // bytes; places in `base` where it is not null
+size_t product_room(MvmArgs a, bool terms_are_samples); // scratch of the largest call of no more samples
 void launch_product_parts(const MvmArgs &a, const ProductArgs &p, hipStream_t s);
 void launch_product(const MvmArgs &a, const ProductArgs &p, hipStream_t s);
 

@@ -302,14 +302,9 @@ template <int BT> __global__ __launch_bounds__(4 * BT) void k_product_sum(MvmArg
 
 } // namespace
 
-// Whether an exact call runs as k_product, and how
-bool product_plan(const MvmArgs &a, ProductArgs &p) {
-  p = ProductArgs{};
-  if (!a.io.perfect || a.in_index || a.pre_add || a.skip_if_zero || a.nm_phase || a.small_tiles_only) return false;
-  p.tiles_o = (a.O + PT - 1) / PT;
-  p.stages = (a.K + PK - 1) / PK;
-  p.safe = parts_safe(a.K);
-  const int n_cus = a.cus > 0 ? a.cus : current_device_cus();
+// Whether a call of this size is worth the launch that splits its operands.  A tile makes room for the calls of fewer samples, too
+// (product_room): large_tiles_aside, whether one could be worth it.
+static bool product_pays(const MvmArgs &a, int n_cus, bool large_tiles_aside) {
   // us, the launches of k_mvm_init and k_mvm_round or k_mvm_big / these.  From 3/4 G multiply-adds: 784 -> 256, 4096 samples (0.8
   // G) forward 41 / 33, update 52 / 33; 2048 x 2048, 256 (1.1 G) 36 / 36, backward 40 / 35; 1024 x 1024, 1024 45 / 35, 16384 317 /
   // 252, update 623 / 259; 768 -> 2304, 1024 backward 79 / 43, update 60 / 44; 3072 x 3072, 512 146 / 105.  Below: 1024 x 1024, 512
@@ -319,10 +314,17 @@ bool product_plan(const MvmArgs &a, ProductArgs &p) {
   // Less than that where the 32 x 32 kernel would walk a long chain of terms: 256 x 256 outputs of 4096 terms 43 / 25, 100 x 100 of
   // 16384 268 / 47, but 64 x 3072 of 2048 26 / 29
   const long tiles_32 = (long)((a.O + 31) / 32) * ((a.m_batch + 31) / 32);
-  const bool long_chain = (double)((tiles_32 + n_cus - 1) / n_cus) * a.K >= 4096.0 && work >= 0x1p27 && !mvm_uses_large_tiles(a.m_batch, a.O);
+  const bool long_chain = (double)((tiles_32 + n_cus - 1) / n_cus) * a.K >= 4096.0 && work >= 0x1p27 && (large_tiles_aside || !mvm_uses_large_tiles(a.m_batch, a.O));
   // products per split value: few outputs or few samples leave a launch that splits and little else
   const double reuse = (double)a.m_batch * a.O / ((double)a.m_batch + a.O);
-  if (!(work >= 0x1.8p29 && a.K >= 128 && reuse >= 96.0) && !(long_chain && reuse >= 32.0)) return false;
+  return (work >= 0x1.8p29 && a.K >= 128 && reuse >= 96.0) || (long_chain && reuse >= 32.0);
+}
+// the work of the call dealt out: tiles, shares of the terms
+static void product_split(const MvmArgs &a, int n_cus, ProductArgs &p) {
+  p = ProductArgs{};
+  p.tiles_o = (a.O + PT - 1) / PT;
+  p.stages = (a.K + PK - 1) / PK;
+  p.safe = parts_safe(a.K);
   double best = 0.0;
   for (int bt = 64; bt <= 128; bt += 64) {
     const int tiles_b = (a.m_batch + bt - 1) / bt;
@@ -344,7 +346,33 @@ bool product_plan(const MvmArgs &a, ProductArgs &p) {
       }
     }
   }
-  return product_scratch(p, nullptr, nullptr) <= ((size_t)2 << 30); // rows padded to 128 are many times the operand of a long, narrow call
+}
+constexpr size_t MOST_SCRATCH = (size_t)2 << 30; // rows padded to 128 are many times the operand of a long, narrow call
+
+// Whether an exact call runs as k_product, and how
+bool product_plan(const MvmArgs &a, ProductArgs &p) {
+  if (!a.io.perfect || a.in_index || a.pre_add || a.skip_if_zero || a.nm_phase || a.small_tiles_only) return false;
+  const int n_cus = a.cus > 0 ? a.cus : current_device_cus();
+  if (!product_pays(a, n_cus, false)) return false;
+  product_split(a, n_cus, p);
+  return product_scratch(p, nullptr, nullptr) <= MOST_SCRATCH;
+}
+// Scratch of the largest such call with the sizes of `a` and no more samples (terms, where they are the samples): fewer samples can
+// take more shares of the terms, and with them more room for the sums.
+size_t product_room(MvmArgs a, bool terms_are_samples) {
+  const int n_cus = a.cus > 0 ? a.cus : current_device_cus();
+  int &samples = terms_are_samples ? a.K : a.m_batch;
+  const int most = samples, step = terms_are_samples ? PK : 64; // a stage, the smaller tile of samples
+  size_t room = 0;
+  for (samples = std::min(step, most);; samples = std::min(samples + step, most)) {
+    if (product_pays(a, n_cus, true)) {
+      ProductArgs p;
+      product_split(a, n_cus, p);
+      const size_t bytes = product_scratch(p, nullptr, nullptr);
+      if (bytes <= MOST_SCRATCH) room = std::max(room, bytes);
+    }
+    if (samples == most) return room;
+  }
 }
 
 static int sample_blocks(const ProductArgs &p) { return p.sample_tile == PT ? p.tiles_b : (p.tiles_b + 1) / 2; } // of 128 rows

@@ -289,7 +289,8 @@ struct Tile {
   hipStream_t last_stream = nullptr;
   DevBuf<float> d_w, d_wmax, d_wmin, d_sup, d_sdown, d_slup, d_sldown;
   // MVM scratch
-  DevBuf<unsigned char> s_parts; // exact_product
+  DevBuf<unsigned char> s_exact; // of exact calls of up to exact_batch samples (ensure_exact)
+  int exact_batch = 0;
   DevBuf<float> s_nsc0, s_nsc1, s_nm, s_nmnp, s_red, s_scale, s_fin, s_bias, s_xq0, s_xq1;
   // rounds 0 and 1 of a forward call in one launch: kept outputs of both, choice per sample, marks of round 1, rows of
   // round 2; the host-visible pair (samples of the last call that needed round 1, its batch) that the choice between
@@ -523,7 +524,7 @@ struct Tile {
       (void)hipHostFree(seen_host);
       seen_host = seen_dev = nullptr;
     }
-    s_parts.release(); s_nsc0.release(); s_nsc1.release(); s_nm.release(); s_nmnp.release(); s_red.release(); s_scale.release(); s_fin.release(); s_bias.release(); s_xq0.release(); s_xq1.release();
+    s_exact.release(); exact_batch = 0; s_nsc0.release(); s_nsc1.release(); s_nm.release(); s_nmnp.release(); s_red.release(); s_scale.release(); s_fin.release(); s_bias.release(); s_xq0.release(); s_xq1.release();
     s_rounds.release(); s_hitup.release(); s_hitlo.release(); s_list0.release(); s_list1.release(); s_row0.release(); s_row1.release(); s_count.release(); s_tiledone.release();
     u_rowcost.release();
     u_bl.release(); u_a.release(); u_b.release(); u_xval.release(); u_dval.release(); u_xw.release(); u_dw.release();
@@ -785,7 +786,7 @@ struct Tile {
     a.max_rounds = io.perfect ? 0 : mvm_max_rounds(a.io);
     size_t rows = (size_t)B * a.k_pad;
     if (a.max_rounds > 2) rows = std::max(rows, (size_t)std::min(B, mvm_few_batch(a)) * O); // see few_args
-    if (!io.perfect) s_xq0.ensure(rows); // (exact calls may need none: exact_product, ensure_exact_rows)
+    if (!io.perfect) s_xq0.ensure(rows); // (of exact calls: ensure_exact)
     if (!io.perfect && io.p.bound_management != RPU_BM_NONE) s_xq1.ensure(rows);
     a.xq[0] = s_xq0.p; a.xq[1] = s_xq1.p;
     // rows for the next bound-management round are quantized ahead when the batch is small (shortest path between
@@ -974,23 +975,43 @@ struct Tile {
 
   const GatherSource *lines_in_place = nullptr; // set while update_indexed runs a pulsed update (pulsed_update_args)
 
-  void ensure_exact_rows(MvmArgs &a) {
-    s_xq0.ensure((size_t)a.m_batch * a.k_pad);
-    a.xq[0] = s_xq0.p;
+  // Scratch of the exact calls of B samples, rows or parts: of all that this tile makes in a training step, so that it grows once,
+  // and of those of fewer samples, whichever launches they take, so that they can be captured after it.
+  size_t exact_room(const MvmArgs &call, bool terms_are_samples) const {
+    MvmArgs a{};
+    a.cus = call.cus;
+    size_t room = 0;
+    const auto add = [&](int samples, int outputs, int terms, bool over_terms) {
+      a.m_batch = samples; a.O = outputs; a.K = terms;
+      room = std::max({room, product_room(a, over_terms), (size_t)samples * mvm_k_pad(terms) * sizeof(float)});
+    };
+    add(call.m_batch, call.O, call.K, terms_are_samples);
+    const int B = terms_are_samples ? call.K : call.m_batch;
+    if (fio.perfect) add(B, D, X, false);
+    if (bio.perfect) add(B, X, D, false);
+    if (!dev.pulsed() || up.p.pulse_type == RPU_PULSE_NONE) add(X, D, B, true);
+    return room;
+  }
+  // room for the call, which needs `bytes` of it
+  void ensure_exact(MvmArgs &a, bool terms_are_samples, size_t bytes) {
+    const int B = terms_are_samples ? a.K : a.m_batch;
+    if (B > exact_batch || bytes > s_exact.n) {
+      s_exact.ensure(exact_room(a, terms_are_samples));
+      exact_batch = std::max(exact_batch, B);
+    }
+    a.xq[0] = reinterpret_cast<float *>(s_exact.p);
   }
   // out = alpha * (weights * inputs) + beta * out
-  void exact_product(MvmArgs &a, hipStream_t s, const char *first, const char *second) {
+  void exact_product(MvmArgs &a, bool terms_are_samples, hipStream_t s, const char *first, const char *second) {
     ProductArgs p;
     // (where values are out of the range of the parts, the product reads the inputs themselves)
     const bool parts = product_plan(a, p) && !writes_into_its_input(a);
+    a.k_pad = a.k_pad ? a.k_pad : mvm_k_pad(a.K);
+    ensure_exact(a, terms_are_samples, parts ? product_scratch(p, nullptr, nullptr) : (size_t)a.m_batch * a.k_pad * sizeof(float));
     if (parts) {
-      const size_t bytes = product_scratch(p, nullptr, nullptr);
-      if (bytes > s_parts.n) s_parts.ensure(bytes + bytes / 4); // the other calls of a training step take about as much
-      (void)product_scratch(p, s_parts.p, &p);
+      (void)product_scratch(p, s_exact.p, &p);
       launch_product_parts(a, p, s);
     } else {
-      a.k_pad = a.k_pad ? a.k_pad : mvm_k_pad(a.K);
-      ensure_exact_rows(a);
       launch_mvm_init(a, s);
     }
     prof_mark(s, first);
@@ -1071,7 +1092,7 @@ struct Tile {
       prof_mark(s, "mvm_few");
     } else if (io.perfect) {
       a.round = 0;
-      exact_product(a, s, "mvm_init", "mvm_round");
+      exact_product(a, false, s, "mvm_init", "mvm_round");
     } else {
       if (io.p.noise_management == RPU_NM_AVERAGE_ABS_MAX || io.p.noise_management == RPU_NM_AVERAGE_ABS_MAX_SINGLE_VALUE) {
         // per-sample maxima, the recurrence over the batch in its order, then the usual set-up with those scales
@@ -1317,7 +1338,7 @@ struct Tile {
       a.alpha = delta_w ? 1.0f : -lr; a.beta = delta_w ? 0.0f : 1.0f; a.round = 0;
       a.key = key(); a.call = call++;
       prof_begin(s);
-      exact_product(a, s, "fp_update_gather", "fp_update");
+      exact_product(a, true, s, "fp_update_gather", "fp_update");
       RPU_HIP_CHECK(hipGetLastError());
       last_stream = s;
       last_update_batch = B;
@@ -2985,7 +3006,7 @@ static int group_mvm(rpu_group_t *group, const float *const *x_dev, const long *
       const int in_size = transposed ? t.D : t.X, out_size = transposed ? t.X : t.D;
       const bool big = use_big && out_size >= 128;
       MvmArgs a = t.mvm_args(m_batch, transposed, t.mvm_weights(is_test), transposed ? t.bio : t.fio, big ? 1 : 0);
-      if (a.io.perfect) t.ensure_exact_rows(a);
+      if (a.io.perfect) t.ensure_exact(a, false, (size_t)m_batch * a.k_pad * sizeof(float));
       a.in = x_dev[i]; a.in_sb = x_ld ? x_ld[i] : in_size; a.in_sk = 1;
       a.out = y_dev[i]; a.out_sb = y_ld ? y_ld[i] : out_size; a.out_so = 1;
       if (a.in_sb < in_size || a.out_sb < out_size) throw RpuError("A row stride is shorter than the row.");

@@ -297,3 +297,31 @@ def test_large_tiles_of_large_values_have_the_sums_of_fp32(gpu_device):
         want = float(w[0, 0]) ** 2 * x_size
         for got in group.forward([v, v]):
             assert float((got.double() - want).abs().max()) <= (x_size + 2) * 2.0 ** -24 * want
+
+
+# fewer samples can take other launches (rows padded further, parts), and more shares of the terms
+@pytest.mark.parametrize("x_size,d_size,batch", [(768, 2304, 4096), (1024, 1024, 4096), (1000, 1500, 1203), (300, 300, 4096), (2048, 64, 16400)])
+def test_exact_calls_make_room_for_those_of_fewer_samples(gpu_device, x_size, d_size, batch):
+    """The first step makes room for every smaller one, so that those can be captured after it."""
+    from aihwkit_amd._cabi import lib
+    rng = np.random.default_rng(x_size)
+    io = noise_free_io()
+    io.is_perfect = True
+    w = rng.standard_normal((d_size, x_size)).astype(np.float32)
+    tile = _tile(x_size, d_size, io, w)
+    tile.set_learning_rate(2.0 ** -10)
+    x, d = torch.randn(batch, x_size, device="cuda"), torch.randn(batch, d_size, device="cuda")
+
+    def step(n):
+        tile.update(x[:n], d[:n], False)
+        return tile.forward(x[:n]), tile.backward(d[:n])
+
+    step(batch)
+    before = lib().rpu_device_allocation_count()
+    for n in range(batch - 31, 0, -(batch // 64 + 1)):
+        y, dx = step(n)
+        assert lib().rpu_device_allocation_count() == before, n
+    w64 = tile.get_weights().double()  # in the room of larger calls
+    for got, v, m in ((y, x[:n], w64.t()), (dx, d[:n], w64)):
+        want, terms = (v.double().cpu() @ m).numpy(), (v.double().cpu().abs() @ m.abs()).numpy()
+        _close(got, want, terms, m.shape[0])
