@@ -201,6 +201,7 @@ SYMBOLS = {
     "rpu_tile_set_fused_rounds": (C.c_int, [_P, C.c_int]),
     "rpu_tile_set_small_calls": (C.c_int, [_P, C.c_int]),
     "rpu_tile_set_round_wait_test_hook": (C.c_int, [_P, C.c_int, C.c_int]),
+    "rpu_tile_set_exact_scratch_test_hook": (C.c_int, [_P, C.c_size_t]),
     "rpu_group_set_round_wait_test_hook": (C.c_int, [_P, C.c_int, C.c_int]),
     "rpu_tile_get_update_ab": (C.c_int, [_P, _P, _P, C.c_int]),
     "rpu_tile_update_with_words": (C.c_int, [_P, _P, _P, C.c_int, _P]),

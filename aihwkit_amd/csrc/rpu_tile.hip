@@ -53,13 +53,32 @@ template <typename T> struct DevBuf {
   size_t n = 0;
   bool owned = true;
   void ensure(size_t count) {
-    if (count <= n) return;
+    const hipError_t e = grow(count);
+    RPU_HIP_CHECK(e);
+  }
+  // whether there is room for `count`; else, the GPU has no memory left for it, the buffer is empty
+  bool try_ensure(size_t count, size_t beyond = 0) {
+    const hipError_t e = grow(count, beyond);
+    if (e == hipErrorOutOfMemory) {
+      (void)hipGetLastError(); // not an error of the launches that follow
+      return false;
+    }
+    RPU_HIP_CHECK(e);
+    return true;
+  }
+  hipError_t grow(size_t count, size_t beyond = 0) {
+    if (count <= n) return hipSuccess;
     if (!owned) throw RpuError("A buffer that belongs to the caller cannot grow.");
     release();
-    RPU_HIP_CHECK(hipMalloc((void **)&p, count * sizeof(T)));
+    const hipError_t e = hipMalloc((void **)&p, count * sizeof(T) + beyond);
+    if (e != hipSuccess) {
+      p = nullptr;
+      return e;
+    }
     g_device_allocations.fetch_add(1, std::memory_order_relaxed);
     n = count;
     if (poison_new_buffers()) RPU_HIP_CHECK(hipMemset(p, 0xff, count * sizeof(T)));
+    return hipSuccess;
   }
   // use memory of the caller from now on (never freed here)
   void adopt(T *external, size_t count) {
@@ -291,6 +310,8 @@ struct Tile {
   // MVM scratch
   DevBuf<unsigned char> s_exact; // of exact calls of up to exact_batch samples (ensure_exact)
   int exact_batch = 0;
+  bool exact_parts = true;      // the GPU had room for parts
+  size_t exact_beyond_hook = 0; // rpu_tile_set_exact_scratch_test_hook
   DevBuf<float> s_nsc0, s_nsc1, s_nm, s_nmnp, s_red, s_scale, s_fin, s_bias, s_xq0, s_xq1;
   // rounds 0 and 1 of a forward call in one launch: kept outputs of both, choice per sample, marks of round 1, rows of
   // round 2; the host-visible pair (samples of the last call that needed round 1, its batch) that the choice between
@@ -524,7 +545,7 @@ struct Tile {
       (void)hipHostFree(seen_host);
       seen_host = seen_dev = nullptr;
     }
-    s_exact.release(); exact_batch = 0; s_nsc0.release(); s_nsc1.release(); s_nm.release(); s_nmnp.release(); s_red.release(); s_scale.release(); s_fin.release(); s_bias.release(); s_xq0.release(); s_xq1.release();
+    s_exact.release(); exact_batch = 0; exact_parts = true; s_nsc0.release(); s_nsc1.release(); s_nm.release(); s_nmnp.release(); s_red.release(); s_scale.release(); s_fin.release(); s_bias.release(); s_xq0.release(); s_xq1.release();
     s_rounds.release(); s_hitup.release(); s_hitlo.release(); s_list0.release(); s_list1.release(); s_row0.release(); s_row1.release(); s_count.release(); s_tiledone.release();
     u_rowcost.release();
     u_bl.release(); u_a.release(); u_b.release(); u_xval.release(); u_dval.release(); u_xw.release(); u_dw.release();
@@ -977,13 +998,13 @@ struct Tile {
 
   // Scratch of the exact calls of B samples, rows or parts: of all that this tile makes in a training step, so that it grows once,
   // and of those of fewer samples, whichever launches they take, so that they can be captured after it.
-  size_t exact_room(const MvmArgs &call, bool terms_are_samples) const {
+  size_t exact_room(const MvmArgs &call, bool terms_are_samples, bool parts) const {
     MvmArgs a{};
     a.cus = call.cus;
     size_t room = 0;
     const auto add = [&](int samples, int outputs, int terms, bool over_terms) {
       a.m_batch = samples; a.O = outputs; a.K = terms;
-      room = std::max({room, product_room(a, over_terms), (size_t)samples * mvm_k_pad(terms) * sizeof(float)});
+      room = std::max({room, parts ? product_room(a, over_terms) : 0, (size_t)samples * mvm_k_pad(terms) * sizeof(float)});
     };
     add(call.m_batch, call.O, call.K, terms_are_samples);
     const int B = terms_are_samples ? call.K : call.m_batch;
@@ -992,22 +1013,25 @@ struct Tile {
     if (!dev.pulsed() || up.p.pulse_type == RPU_PULSE_NONE) add(X, D, B, true);
     return room;
   }
-  // room for the call, which needs `bytes` of it
-  void ensure_exact(MvmArgs &a, bool terms_are_samples, size_t bytes) {
+  // Room for the call, which needs `bytes` of it; false: only for its rows, also of calls to come (parts take up to ten times as
+  // much, and a GPU that has no memory left for them still has the launches that do without).
+  bool ensure_exact(MvmArgs &a, bool terms_are_samples, size_t bytes) {
     const int B = terms_are_samples ? a.K : a.m_batch;
     if (B > exact_batch || bytes > s_exact.n) {
-      s_exact.ensure(exact_room(a, terms_are_samples));
+      if (exact_parts) exact_parts = s_exact.try_ensure(exact_room(a, terms_are_samples, true), exact_beyond_hook);
+      if (!exact_parts) s_exact.ensure(exact_room(a, terms_are_samples, false));
       exact_batch = std::max(exact_batch, B);
     }
     a.xq[0] = reinterpret_cast<float *>(s_exact.p);
+    return exact_parts;
   }
   // out = alpha * (weights * inputs) + beta * out
   void exact_product(MvmArgs &a, bool terms_are_samples, hipStream_t s, const char *first, const char *second) {
     ProductArgs p;
     // (where values are out of the range of the parts, the product reads the inputs themselves)
-    const bool parts = product_plan(a, p) && !writes_into_its_input(a);
-    a.k_pad = a.k_pad ? a.k_pad : mvm_k_pad(a.K);
-    ensure_exact(a, terms_are_samples, parts ? product_scratch(p, nullptr, nullptr) : (size_t)a.m_batch * a.k_pad * sizeof(float));
+    const size_t rows = (size_t)a.m_batch * (a.k_pad = a.k_pad ? a.k_pad : mvm_k_pad(a.K)) * sizeof(float);
+    bool parts = exact_parts && product_plan(a, p) && !writes_into_its_input(a);
+    parts = ensure_exact(a, terms_are_samples, parts ? product_scratch(p, nullptr, nullptr) : rows) && parts;
     if (parts) {
       (void)product_scratch(p, s_exact.p, &p);
       launch_product_parts(a, p, s);
@@ -3767,6 +3791,14 @@ int rpu_tile_set_round_wait_test_hook(rpu_tile_t *tile, int spin_limit, int extr
     std::lock_guard<std::mutex> lock(tile->t.mutex);
     tile->t.wait_spins_hook = spin_limit;
     tile->t.wait_extra_hook = extra_arrivals;
+  });
+}
+
+int rpu_tile_set_exact_scratch_test_hook(rpu_tile_t *tile, size_t beyond) {
+  return guarded([&] {
+    if (!tile) throw RpuError("null tile");
+    std::lock_guard<std::mutex> lock(tile->t.mutex);
+    tile->t.exact_beyond_hook = beyond;
   });
 }
 

@@ -538,6 +538,10 @@ class _CudaTileMixin:
         ``spin_limit`` polls and make them expect ``extra_arrivals`` workgroups more than the launch has."""
         check(lib().rpu_tile_set_round_wait_test_hook(self._h, int(spin_limit), int(extra_arrivals)))
 
+    def set_exact_scratch_test_hook(self, beyond: int = 0) -> None:
+        """For the test of exact calls without memory for their operands in parts only: ask for ``beyond`` bytes more."""
+        check(lib().rpu_tile_set_exact_scratch_test_hook(self._h, int(beyond)))
+
     def get_update_words_per_sample(self) -> int:
         """Rows of pulse words per sample of the last stochastic update: ceil(longest possible BL / 31)."""
         n = C.c_int32(0)

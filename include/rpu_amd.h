@@ -709,6 +709,10 @@ int rpu_tile_set_small_calls(rpu_tile_t *tile, int enable);
 int rpu_tile_set_round_wait_test_hook(rpu_tile_t *tile, int spin_limit, int extra_arrivals);
 int rpu_group_set_round_wait_test_hook(rpu_group_t *group, int spin_limit, int extra_arrivals);
 
+/* No counterpart in the reference; for the test of exact calls on a GPU without memory for their operands in parts only: the tile asks
+ * for `beyond` bytes more than it needs. */
+int rpu_tile_set_exact_scratch_test_hook(rpu_tile_t *tile, size_t beyond);
+
 /* ---- inspection hooks (mirror the reference's debug hooks) ------------------------------ */
 
 /* After rpu_tile_update with a stochastic pulse type: copies the packed pulse words of that call

@@ -325,3 +325,29 @@ def test_exact_calls_make_room_for_those_of_fewer_samples(gpu_device, x_size, d_
     for got, v, m in ((y, x[:n], w64.t()), (dx, d[:n], w64)):
         want, terms = (v.double().cpu() @ m).numpy(), (v.double().cpu().abs() @ m.abs()).numpy()
         _close(got, want, terms, m.shape[0])
+
+
+def test_exact_calls_without_memory_for_their_parts(gpu_device):
+    """The GPU refuses the scratch: the calls take the launches that need less, and find theirs from then on."""
+    from aihwkit_amd._cabi import lib
+    x_size, d_size, batch = 768, 1100, 1030
+    rng = np.random.default_rng(5)
+    io = noise_free_io()
+    io.is_perfect = True
+    w = (0.3 * rng.standard_normal((d_size, x_size))).astype(np.float32)
+    tile = _tile(x_size, d_size, io, w)
+    tile.set_exact_scratch_test_hook(1 << 50)  # more than any GPU has
+    lr = 0.125
+    tile.set_learning_rate(lr)
+    x, d = rng.standard_normal((batch, x_size)).astype(np.float32), rng.standard_normal((batch, d_size)).astype(np.float32)
+    x64, d64, w64 = x.astype(np.float64), d.astype(np.float64), w.astype(np.float64)
+    xg, dg = torch.from_numpy(x).cuda(), torch.from_numpy(d).cuda()
+    before = None
+    for _ in range(2):
+        tile.set_weights(torch.from_numpy(w))
+        _close(tile.forward(xg), x64 @ w64.T, np.abs(x64) @ np.abs(w64).T, x_size)
+        _close(tile.backward(dg), d64 @ w64, np.abs(d64) @ np.abs(w64), d_size)
+        tile.update(xg, dg, False)
+        _close(tile.get_weights(), w64 - lr * (d64.T @ x64), np.abs(w64) + lr * (np.abs(d64).T @ np.abs(x64)), batch)
+        assert before is None or lib().rpu_device_allocation_count() == before
+        before = lib().rpu_device_allocation_count()
