@@ -28,6 +28,7 @@
 #ifndef RPU_AMD_H
 #define RPU_AMD_H
 
+#include <stddef.h>
 #include <stdint.h>
 
 #ifdef __cplusplus
