@@ -1025,7 +1025,7 @@ struct Tile {
     a.xq[0] = reinterpret_cast<float *>(s_exact.p);
     return exact_parts;
   }
-  // out = alpha * (weights * inputs) + beta * out
+  // out = alpha * (weights * inputs) + beta * out; first, second: what the profile names the launches that do without parts
   void exact_product(MvmArgs &a, bool terms_are_samples, hipStream_t s, const char *first, const char *second) {
     ProductArgs p;
     // (where values are out of the range of the parts, the product reads the inputs themselves)
@@ -1038,10 +1038,10 @@ struct Tile {
     } else {
       launch_mvm_init(a, s);
     }
-    prof_mark(s, first);
+    prof_mark(s, parts ? "product_parts" : first);
     if (parts) launch_product(a, p, s);
     else launch_mvm_round(a, s);
-    prof_mark(s, second);
+    prof_mark(s, parts ? "product" : second);
   }
 
   // in_ld: row stride of a plain row-major input with padded rows (0: the rows are dense)

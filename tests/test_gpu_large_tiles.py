@@ -188,12 +188,23 @@ def test_grouped_products_in_three_parts_against_64_bit_sums(gpu_device, shapes,
         _close(got, q @ w64.T, np.abs(q) @ np.abs(w64).T, 4 * w.shape[1] + 16, w.shape[1])
 
 
-# exact calls that fill the GPU (k_product): a term, an output and a sample more than a tile holds, one less than that, the line
-# between eight and six products of the parts (512 terms), the terms in one and in several shares, a share of one stage
-@pytest.mark.parametrize("x_size,d_size,batch", [(1025, 900, 900), (2049, 129, 3100), (127, 2500, 2600), (511, 1200, 1400),
-                                                 (512, 1217, 1400), (100, 101, 16384), (1024, 1024, 769), (640, 257, 5000)])
+def _profiled(tile, parts, call, *args):
+    """The result of an exact call that has to run on the operands split into parts (k_product), or not to."""
+    tile.set_profiling(True)
+    out = call(*args)
+    assert ("product" in [name for name, _ms in tile.get_profile()]) == parts
+    tile.set_profiling(False)
+    return out
+
+
+# exact calls that fill the GPU (k_product): a term, an output and a sample more than a tile holds, one less than that, the terms
+# in one and in several shares, a share of one stage, the fewest terms, just above the least work; which of forward, backward and
+# update are such calls
+@pytest.mark.parametrize("x_size,d_size,batch,parts", [
+    (1025, 900, 900, "fbu"), (2049, 129, 3100, "fbu"), (127, 2500, 2600, "bu"), (128, 2500, 2600, "fbu"), (129, 2500, 2600, "fbu"),
+    (511, 1200, 1400, "fbu"), (512, 1217, 1400, "fbu"), (100, 101, 16384, "u"), (1024, 1024, 769, "fbu"), (640, 257, 5000, "fbu")])
 @pytest.mark.parametrize("trans", [False, True])
-def test_exact_products_of_calls_that_fill_the_gpu(gpu_device, x_size, d_size, batch, trans):
+def test_exact_products_of_calls_that_fill_the_gpu(gpu_device, x_size, d_size, batch, parts, trans):
     rng = np.random.default_rng(x_size)
     io = noise_free_io()
     io.is_perfect = True
@@ -204,13 +215,41 @@ def test_exact_products_of_calls_that_fill_the_gpu(gpu_device, x_size, d_size, b
     x, d = rng.standard_normal((batch, x_size)).astype(np.float32), rng.standard_normal((batch, d_size)).astype(np.float32)
     x[:, -1] = 1.0  # the bias column, which is not stored
     x64, d64, w64 = x.astype(np.float64), d.astype(np.float64), w.astype(np.float64)
-    _close(back(tile.forward(lay(x[:, :-1]), True, trans, trans)), x64 @ w64.T, np.abs(x64) @ np.abs(w64).T, x_size)
-    _close(back(tile.backward(lay(d), True, trans, trans)), (d64 @ w64)[:, :-1], (np.abs(d64) @ np.abs(w64))[:, :-1], d_size)
+    y = _profiled(tile, "f" in parts, tile.forward, lay(x[:, :-1]), True, trans, trans)
+    _close(back(y), x64 @ w64.T, np.abs(x64) @ np.abs(w64).T, x_size)
+    dx = _profiled(tile, "b" in parts, tile.backward, lay(d), True, trans, trans)
+    _close(back(dx), (d64 @ w64)[:, :-1], (np.abs(d64) @ np.abs(w64))[:, :-1], d_size)
     lr = 0.125
     tile.set_learning_rate(lr)
-    tile.update(lay(x[:, :-1]), lay(d), True, trans, trans)
-    want = w64 - lr * (d64.T @ x64)
-    _close(tile.get_weights(), want, np.abs(w64) + lr * (np.abs(d64).T @ np.abs(x64)), batch)
+    _profiled(tile, "u" in parts, tile.update, lay(x[:, :-1]), lay(d), True, trans, trans)
+    want, terms = d64.T @ x64, np.abs(d64).T @ np.abs(x64)
+    _close(tile.get_weights(), w64 - lr * want, np.abs(w64) + lr * terms, batch)
+    delta = torch.full((x_size, d_size), 7.0, device="cuda")  # overwritten, whatever it holds
+    tile.set_delta_weights(delta)
+    before = tile.get_weights()
+    _profiled(tile, "u" in parts, tile.update, lay(x[:, :-1]), lay(d), True, trans, trans)
+    assert torch.equal(tile.get_weights(), before)
+    _close(delta.t(), want, terms, batch)
+
+
+def test_exact_products_of_rows_that_are_slices_of_longer_ones(gpu_device):
+    """A group that holds a tile on running-average noise management runs its tiles one by one, on the slices that it is given:
+    unaligned ones here."""
+    rng = np.random.default_rng(7)
+    x_size, d_size, batch = 1025, 900, 901
+    io = noise_free_io()
+    io.is_perfect = True
+    average = noise_free_io(noise_management=dv.NoiseManagementType.AverageAbsMax)
+    w = rng.standard_normal((d_size, x_size)).astype(np.float32)
+    tile, other = _tile(x_size, d_size, io, w), _tile(20, 30, average, w[:30, :20])
+    group = tiles.TileGroup([tile, other])
+    for own, grouped, width, outputs, small in ((tile.forward, group.forward, x_size, d_size, 20), (tile.backward, group.backward, d_size, x_size, 30)):
+        v = torch.randn(batch, width + 6, device="cuda")[:, 3:3 + width]
+        out = torch.full((batch, outputs + 10), 7.0, device="cuda")
+        rows = [out[:, 5:5 + outputs], torch.empty(batch, 50 - small, device="cuda")]
+        _profiled(tile, True, lambda: grouped([v, torch.randn(batch, small, device="cuda")], outs=rows))
+        assert torch.equal(rows[0], own(v.contiguous()))
+        assert bool((out[:, :5] == 7.0).all()) and bool((out[:, 5 + outputs:] == 7.0).all())
 
 
 @pytest.mark.parametrize("x_size,d_size,batch", [(1025, 900, 900), (300, 300, 12001)])
