@@ -302,11 +302,13 @@ void launch_fold_indexed(float *images, const float *x_mat, const int *ptr, cons
   hipLaunchKernelGGL((k_fold_indexed<NI, U>), dim3(grid_of(threads(NI))), dim3(256), 0, s, images, x_mat, ptr, lists, patches, n_images, image_size)
   // Lists of one to four entries on average (kernels no larger than their strides by more than that): four at a time, backward of 1 x
   // 1, 64 -> 64 channels, 64 images of 16 x 16 28 us, with nine 29.  Nine are the lists of 3 x 3 kernels; of 5 x 5, 32 -> 32, 64
-  // images of 30 x 30 212 -> 165.  More images to a thread as long as two waves are left to a SIMD: 64 -> 64, 32 images of 36 x 36
-  // 109 -> 102, 48 150 -> 138; 16 of 16 x 16 (four to a thread) 26 -> 25.
+  // images of 30 x 30 212 -> 165.  More images to a thread as long as two waves of threads with all their images are left to a SIMD:
+  // 64 -> 64, 32 images of 36 x 36 109 -> 102, 48 150 -> 138; 16 of 16 x 16 (four to a thread) 26 -> 25.  Backward calls of 16 -> 16,
+  // images of 97 x 97, with four / sixteen to a thread: one image 27 / 31, three 39 / 45; two of 3 channels, 224 x 224, 5 x 5 81 / 96.
+  const auto fills = [&](int images_per_thread) { return n_images / images_per_thread * image_size >= 1L << 17; };
   if ((double)x_size * patches <= 4.0 * image_size) RPU_FOLD(4, 4);
-  else if (threads(16) >= (1u << 17)) RPU_FOLD(16, 9);
-  else if (threads(8) >= (1u << 17)) RPU_FOLD(8, 9);
+  else if (fills(16)) RPU_FOLD(16, 9);
+  else if (fills(8)) RPU_FOLD(8, 9);
   else RPU_FOLD(4, 9);
 #undef RPU_FOLD
 }

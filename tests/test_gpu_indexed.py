@@ -357,9 +357,9 @@ def test_pulsed_update_reads_patches_and_gradients_in_place(gpu_device, case):
     assert (got[0] - torch.from_numpy(np.clip(w.numpy(), -0.6, 0.6))).abs().max() > 1e-3
 
 
-# sixteen, eight and four images to a thread, with a last group of one image and one that is full; lists of one entry, of exactly
+# sixteen, eight and four images to a thread, with a last group of one image and one that is full, and one large image; lists of one entry, of exactly
 # nine, of ten to twenty-five (three trips of nine) and of none (an edge that the stride passes over)
-@pytest.mark.parametrize("c_in,side,n,kernel,stride", [(16, 48, 49, 3, 1), (16, 48, 64, 5, 1), (16, 48, 33, 3, 1), (16, 48, 32, 4, 1), (5, 13, 7, 3, 1),
+@pytest.mark.parametrize("c_in,side,n,kernel,stride", [(16, 48, 65, 3, 1), (16, 97, 1, 3, 1), (16, 48, 49, 3, 1), (16, 48, 64, 5, 1), (16, 48, 33, 3, 1), (16, 48, 32, 4, 1), (5, 13, 7, 3, 1),
                                                        (5, 13, 9, 5, 1), (16, 48, 49, 1, 1), (4, 17, 6, 2, 2), (3, 18, 21, 3, 2), (1, 6, 1, 6, 1)])
 def test_indexed_backward_of_whole_numbers_is_the_transposed_convolution(gpu_device, c_in, side, n, kernel, stride):
     rng = np.random.default_rng(side)
