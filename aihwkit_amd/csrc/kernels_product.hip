@@ -15,6 +15,7 @@
 #include "kernels.h"
 
 #include <algorithm>
+#include <cmath>
 
 namespace rpu_amd {
 namespace {
@@ -305,19 +306,35 @@ template <int BT> __global__ __launch_bounds__(4 * BT) void k_product_sum(MvmArg
 // Whether a call of this size is worth the launch that splits its operands.  A tile makes room for the calls of fewer samples, too
 // (product_room): large_tiles_aside, whether one could be worth it.
 static bool product_pays(const MvmArgs &a, int n_cus, bool large_tiles_aside) {
+  const auto padded = [](double n, int to) { return std::ceil(n / to) * to; };
   // us, the launches of k_mvm_init and k_mvm_round or k_mvm_big / these.  From 3/4 G multiply-adds: 784 -> 256, 4096 samples (0.8
-  // G) forward 41 / 33, update 52 / 33; 2048 x 2048, 256 (1.1 G) 36 / 36, backward 40 / 35; 1024 x 1024, 1024 45 / 35, 16384 317 /
-  // 252, update 623 / 259; 768 -> 2304, 1024 backward 79 / 43, update 60 / 44; 3072 x 3072, 512 146 / 105.  Below: 1024 x 1024, 512
-  // 23 / 28, 256 15 / 22; 512 x 512, 512 12 / 17; 3072 x 3072, 64 28 / 38, and few terms of a large product, which the split
-  // and the store are most of: 3072 x 3072 outputs of 64 terms 39 / 50, of 128 64 / 59.
+  // G) forward 43 / 35, update 53 / 34; 1024 x 1024, 1024 46 / 35, 16384 311 / 270, update 622 / 272; 768 -> 2304, 1024 58 / 52,
+  // backward 76 / 46, update 58 / 45; 3072 x 3072, 512 145 / 114.  Below: 1024 x 1024, 512 23 / 28, 256 15 / 22; 512 x 512, 512 12
+  // / 17; 3072 x 3072, 64 28 / 38, and few terms of a large product, which the split and the store are most of: 3072 x 3072 outputs
+  // of 64 terms 39 / 50, of 128 64 / 59.
   const double work = (double)a.m_batch * a.O * a.K;
-  // Less than that where the 32 x 32 kernel would walk a long chain of terms: 256 x 256 outputs of 4096 terms 43 / 25, 100 x 100 of
-  // 16384 268 / 47, but 64 x 3072 of 2048 26 / 29
+  // Less than that where the 32 x 32 kernel would walk a long chain of terms: 256 x 256 outputs of 4096 terms 35 / 27, 100 x 100 of
+  // 16384 103 / 49, but 64 x 3072 of 2048 26 / 29
   const long tiles_32 = (long)((a.O + 31) / 32) * ((a.m_batch + 31) / 32);
-  const bool long_chain = (double)((tiles_32 + n_cus - 1) / n_cus) * a.K >= 4096.0 && work >= 0x1p27 && (large_tiles_aside || !mvm_uses_large_tiles(a.m_batch, a.O));
+  const double chain = (double)((tiles_32 + n_cus - 1) / n_cus) * a.K;
+  const bool large = mvm_uses_large_tiles(a.m_batch, a.O);
+  const bool long_chain = chain >= 4096.0 && work >= 0x1p27 && (large_tiles_aside || !large);
   // products per split value: few outputs or few samples leave a launch that splits and little else
   const double reuse = (double)a.m_batch * a.O / ((double)a.m_batch + a.O);
-  return (work >= 0x1.8p29 && a.K >= 128 && reuse >= 96.0) || (long_chain && reuse >= 32.0);
+  if (!(work >= 0x1.8p29 && a.K >= 128 && reuse >= 96.0) && !(long_chain && reuse >= 32.0)) return false;
+  // Few samples of a large matrix, or the other way round: the split of the larger operand is most of the call.  Time of either, us,
+  // fitted to 570 calls of 36 to 49152 samples, 100 to 32768 outputs, 128 to 50000 terms (not the faster one of eight, by 9 % at
+  // most): 8192 x 8192, 40 samples 104 / 211, 4096 x 4096, 64 35 / 50, 128 54 / 62, 224 93 / 88, 2048 x 2048, 256 31.9 / 32.8, 288
+  // 41.9 / 36.4, 1024 -> 16384, 128 54 / 62.
+  const double samples = padded(a.m_batch, 64), outputs = padded(a.O, PT), terms = 1e-6 * a.K;
+  const double split = (padded(a.m_batch, PT) + outputs) * terms; // values
+  double rows = 11.0 + (a.w_oc ? 0.0068 : 0.005) * chain + (a.O % 32 && tiles_32 > n_cus ? 10.0 : 0.0);
+  if (large) { // two workgroups to a CU at a time
+    const double large_rows = 16.0 + 0.036 * a.K * std::max(1.0, (a.O + 63) / 64 * (samples / 64) / (2 * n_cus));
+    rows = large_tiles_aside ? std::max(rows, large_rows) : large_rows;
+  }
+  const double parts = 18.0 + 1.35 * split + 1.4 * std::max(split - 20.0, 0.0) + 10.5 * samples * outputs * a.K / 0x1p30; // 20 M: 120 MB
+  return rows + 1.7 * a.m_batch * terms > parts;
 }
 // the work of the call dealt out: tiles, shares of the terms
 static void product_split(const MvmArgs &a, int n_cus, ProductArgs &p) {
@@ -365,7 +382,9 @@ size_t product_room(MvmArgs a, bool terms_are_samples) {
   const int most = samples, step = terms_are_samples ? PK : 64; // a stage, the smaller tile of samples
   size_t room = 0;
   for (samples = std::min(step, most);; samples = std::min(samples + step, most)) {
-    if (product_pays(a, n_cus, true)) {
+    MvmArgs fewer = a;
+    if (terms_are_samples) fewer.K = std::max(a.K - (PK - 1), 1); // the fewest of this many stages
+    if (product_pays(a, n_cus, true) || (terms_are_samples && product_pays(fewer, n_cus, true))) {
       ProductArgs p;
       product_split(a, n_cus, p);
       const size_t bytes = product_scratch(p, nullptr, nullptr);

@@ -198,11 +198,12 @@ def _profiled(tile, parts, call, *args):
 
 
 # exact calls that fill the GPU (k_product): a term, an output and a sample more than a tile holds, one less than that, the terms
-# in one and in several shares, a share of one stage, the fewest terms, just above the least work; which of forward, backward and
-# update are such calls
+# in one and in several shares, a share of one stage, the fewest terms, just above the least work, few samples of large matrices (the
+# split of the weights would be most of the call); which of forward, backward and update are such calls
 @pytest.mark.parametrize("x_size,d_size,batch,parts", [
-    (1025, 900, 900, "fbu"), (2049, 129, 3100, "fbu"), (127, 2500, 2600, "bu"), (128, 2500, 2600, "fbu"), (129, 2500, 2600, "fbu"),
-    (511, 1200, 1400, "fbu"), (512, 1217, 1400, "fbu"), (100, 101, 16384, "u"), (1024, 1024, 769, "fbu"), (640, 257, 5000, "fbu")])
+    (1025, 900, 1000, "fbu"), (2049, 129, 3300, "fbu"), (127, 2500, 2600, "bu"), (128, 2500, 2600, "fbu"), (129, 2100, 4097, "fbu"),
+    (511, 1200, 1400, "fbu"), (512, 1217, 1400, "fbu"), (100, 101, 16384, "u"), (1024, 1024, 769, "fbu"), (640, 257, 5000, "fbu"),
+    (2048, 2048, 300, "fbu"), (4096, 4096, 64, ""), (1024, 16384, 128, "bu")])
 @pytest.mark.parametrize("trans", [False, True])
 def test_exact_products_of_calls_that_fill_the_gpu(gpu_device, x_size, d_size, batch, parts, trans):
     rng = np.random.default_rng(x_size)
