@@ -181,6 +181,33 @@ def test_long_bit_lines_through_lds_equal_the_plain_loop(x_size, d_size, batch, 
     assert torch.equal(one.get_weights(), other.get_weights())
 
 
+# k_update_lines_small at one and four lines of either operand, at its most samples, and at its most values and longest lines; the
+# last of each is a call beyond
+@pytest.mark.parametrize("x_size,d_size,batch,small", [
+    (1, 1, 1, True), (4, 5, 2, True), (129, 10, 64, True), (129, 10, 65, False), (200, 200, 64, True), (200, 201, 64, False),
+    (1100, 436, 7, True), (1100, 437, 7, False), (900, 636, 1, True), (512, 512, 16, True), (512, 513, 16, False)])
+@pytest.mark.parametrize("blm", [True, False])
+def test_small_updates_in_one_launch_of_pulse_trains_equal_those_of_a_group(x_size, d_size, batch, small, blm, storage_mode):
+    from aihwkit_amd.rpu_base.tiles import TileGroup
+    x, d = _data(x_size, d_size, batch, 0)
+    one, other = (_tile(x_size, d_size, _device("soft_bounds")) if blm else _long_lines_tile(x_size, d_size, "soft_bounds")
+                  for _ in range(2))
+    for tile in (one, other):
+        tile.set_learning_rate(0.02)
+    group = TileGroup([other])
+    for _ in range(2):
+        one.set_profiling(True)
+        one.update(x, d, False)
+        assert ("update_prepare" not in [name for name, _ms in one.get_profile()]) == small
+        one.set_profiling(False)
+        group.update([x], [d])
+        for mine, theirs in zip(one.get_update_words(batch), other.get_update_words(batch)):
+            assert torch.equal(mine, theirs)
+        for mine, theirs in zip(one.get_update_ab(batch), other.get_update_ab(batch)):
+            assert torch.equal(mine, theirs)
+    assert torch.equal(one.get_weights(), other.get_weights())
+
+
 # every kernel that makes pulse trains reads a bias column that is not stored as the row that has it: a few samples, lane masks,
 # pipeline of waves, long lines, implicit pulses
 @pytest.mark.parametrize("x_size,d_size,batch,pulse_type,blm", [
