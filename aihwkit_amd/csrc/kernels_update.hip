@@ -116,8 +116,15 @@ __device__ __forceinline__ void update_bl_ab(const UpdateArgs &a, const float xm
   }
 }
 
-// ... of sample b, by one thread
-__device__ __forceinline__ void update_prepare_finish(const UpdateArgs &a, const int b, const float xm, const float dm) {
+// a running maximum of at most 31: what is read first saves most of the atomics (with hundreds of thousands of samples those on the
+// one word were most of the kernel's time)
+__device__ __forceinline__ void update_kmax(const UpdateArgs &a, const int mine) {
+  if (mine > 0 && __hip_atomic_load(&a.kmax[a.kmax_slot], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < mine) {
+    atomicMax(&a.kmax[a.kmax_slot], mine);
+  }
+}
+// ... of sample b, by one thread.  most: where the largest number of slots goes that the workgroup sends once (null: the sample's at once)
+__device__ __forceinline__ void update_prepare_finish(const UpdateArgs &a, const int b, const float xm, const float dm, int *most = nullptr) {
   int BL;
   float A, B;
   update_bl_ab(a, xm, dm, BL, A, B);
@@ -125,12 +132,9 @@ __device__ __forceinline__ void update_prepare_finish(const UpdateArgs &a, const
   // largest number of pulse slots in a row of words (a longer bit line takes several rows of 31): this call's slot
   // was zeroed by the previous call, which used the other one
   if (a.kmax) {
-    // a running maximum of at most 31: a sample only sends its value when what it reads is still smaller (with
-    // hundreds of thousands of samples the atomics on the one word were most of this kernel's time)
     const int mine = min(BL, 31);
-    if (mine > 0 && __hip_atomic_load(&a.kmax[a.kmax_slot], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < mine) {
-      atomicMax(&a.kmax[a.kmax_slot], mine);
-    }
+    if (most) atomicMax(most, mine);
+    else update_kmax(a, mine);
     if (b == 0) a.kmax[a.kmax_slot ^ 1] = 0;
   }
   a.prob_a[b] = A;
@@ -142,7 +146,7 @@ __device__ __forceinline__ void update_prepare_finish(const UpdateArgs &a, const
 // SUB threads share a sample: the whole workgroup (long lines), a wave, or 16 lanes (the short patch rows of a
 // convolution come by the hundred thousand: a workgroup per sample would spend its time being launched)
 template <int SUB>
-__device__ __forceinline__ void update_prepare_sample(const UpdateArgs &a, const int b, float (*sh)[4]) {
+__device__ __forceinline__ void update_prepare_sample(const UpdateArgs &a, const int b, float (*sh)[4], int *most = nullptr) {
   const int t = threadIdx.x % SUB;
   const bool leader = t == 0;
   float xm = 0.0f, dm = 0.0f;
@@ -171,7 +175,7 @@ __device__ __forceinline__ void update_prepare_sample(const UpdateArgs &a, const
     }
   }
   if (!leader) return;
-  update_prepare_finish(a, b, xm, dm);
+  update_prepare_finish(a, b, xm, dm, most);
 }
 
 // The lines of the indexed interface read in place, for long batches.  A workgroup of 16 waves owns 64 patches, one per
@@ -257,12 +261,21 @@ __global__ __launch_bounds__(1024) void k_update_prepare_in_place(UpdateArgs a) 
 template <int SUB>
 __global__ __launch_bounds__(256) void k_update_prepare(UpdateArgs a) {
   __shared__ float sh[2][4];
+  __shared__ int most;
   if (a.row_cost) {
     for (int i = (int)(blockIdx.x * 256u + threadIdx.x); i < a.d_size; i += (int)(gridDim.x * 256u)) a.row_cost[i] = 0;
   }
   const int b = (int)blockIdx.x * (256 / SUB) + (int)threadIdx.x / SUB;
-  if (b >= a.m_batch) return; // all SUB threads of a sample leave together
-  update_prepare_sample<SUB>(a, b, sh);
+  if constexpr (SUB == 256) {
+    update_prepare_sample<SUB>(a, b, sh);
+  } else { // thousands of samples at a time find the word still smaller: 100 x 80, 4000 samples 22 to 47 us
+    // with an atomic to each, 11 to 13 with one to a workgroup
+    if (threadIdx.x == 0) most = 0;
+    __syncthreads();
+    if (b < a.m_batch) update_prepare_sample<SUB>(a, b, sh, &most); // all SUB threads of a sample together
+    __syncthreads();
+    if (threadIdx.x == 0 && a.kmax) update_kmax(a, most);
+  }
 }
 
 // The same for several tiles in one launch (all with the same batch): workgroup n works on sample n % m_batch of tile

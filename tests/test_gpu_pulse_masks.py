@@ -208,6 +208,28 @@ def test_small_updates_in_one_launch_of_pulse_trains_equal_those_of_a_group(x_si
     assert torch.equal(one.get_weights(), other.get_weights())
 
 
+# samples that share a workgroup of k_update_prepare, four or sixteen of them: one has bit lines several times longer than all others,
+# the first and the last of a workgroup, and the last of one that is not full
+@pytest.mark.parametrize("x_size,d_size,batch", [(70, 40, 1025), (70, 40, 2050), (60, 40, 1040), (60, 40, 1041)])
+@pytest.mark.parametrize("at", [0, 3, 15, -1])
+def test_the_longest_bit_line_of_many_short_samples(x_size, d_size, batch, at, storage_mode):
+    from aihwkit_amd.rpu_base.tiles import TileGroup
+    x, d = _data(x_size, d_size, batch, 0)
+    d[at] *= 6.0
+    one, other = (_tile(x_size, d_size, _device("soft_bounds")) for _ in range(2))
+    for tile in (one, other):
+        tile.set_learning_rate(0.02)
+    group = TileGroup([other])
+    for _ in range(2):
+        one.update(x, d, False)
+        group.update([x], [d])
+    for mine, theirs in zip(one.get_update_words(batch), other.get_update_words(batch)):
+        assert torch.equal(mine, theirs)
+    bl = one.get_update_words(batch)[2]
+    assert int(bl[at]) > 2 * int(torch.cat([bl[:at], bl[at + 1:] if at >= 0 else bl[:0]]).max())
+    assert torch.equal(one.get_weights(), other.get_weights())
+
+
 # every kernel that makes pulse trains reads a bias column that is not stored as the row that has it: a few samples, lane masks,
 # pipeline of waves, long lines, implicit pulses
 @pytest.mark.parametrize("x_size,d_size,batch,pulse_type,blm", [
