@@ -3,14 +3,16 @@
 //
 //   k_product_parts  an operand's rows as three bf16 planes, in blocks of 128 rows x 32 terms laid out as the contraction
 //                    stages them, whichever way the operand is stored (it takes the place of the copy into contiguous rows)
-//   k_product        a workgroup of four waves makes 128 outputs x 128 samples over a share of the terms
+//   k_product        a workgroup makes 128 outputs x 128 (or 64) samples over a share of the terms
 //   k_product_sum    adds the shares in their order, where there is more than one
 //
 // In the kernels that split what they stage (k_mvm_big, three parts) a wave issues 220 vector instructions for the 16 MFMAs of a
 // stage and waits for a third of the rest: 27 % of the matrix pipe's time at 768 x 2304 outputs of 1024 terms.  Here a stage is
 // 32 MFMAs and 18 reads of LDS to a wave, a byte staged meets more multiply-adds, and splitting the terms fills the CUs that
-// few large tiles leave idle.  768 -> 2304, 1024 samples, backward 79 -> 43 us (parts 8, product 30, sums 5).  What bounds it: the
-// matrix pipe (1024 x 1024, 16384 samples: 1.2 PFLOP/s of bf16 products, the rate of a large library product on this card).
+// few large tiles leave idle.  768 -> 2304, 1024 samples, row-major tile, backward call 76 -> 46 us (parts 9, product 32, sums 7);
+// 1024 x 1024, 16384 samples, forward 311 -> 272: 1.1 PFLOP/s of bf16 products, a large library product reaches 1.2 on this card.
+// There the matrix pipe is busy for 58 % of the cycles (at 1.9 GHz under that load), 49 % in the smaller call; what is left is the
+// waits of a stage, for LDS (27 % of the cycles, no bank conflicts) and at its barrier.
 #include "bf16_parts.h"
 #include "kernels.h"
 
@@ -24,6 +26,7 @@ constexpr int PT = PRODUCT_TILE;            // outputs of a workgroup tile, and 
 constexpr int PK = 32;                      // terms of a stage
 constexpr int PLANE = PT * PK;              // values of a plane of a block
 constexpr int BLOCK = 3 * PLANE;            // ... of a block: the parts of PT rows x PK terms
+constexpr int MOST_SHARES = 16;             // of the terms
 constexpr float LIFT = 0x1p16f;             // the parts are those of this times the value (split_bf16)
 
 // 64 rows x 64 terms of an operand: element (row, k) at src[row * s_r + k * s_k]; term one_k is 1 and not stored (-1: none)
@@ -346,7 +349,7 @@ static void product_split(const MvmArgs &a, int n_cus, ProductArgs &p) {
   for (int bt = 64; bt <= 128; bt += 64) {
     const int tiles_b = (a.m_batch + bt - 1) / bt;
     const long tiles = (long)p.tiles_o * tiles_b;
-    for (int shares = 1; shares <= 16 && shares <= p.stages; ++shares) {
+    for (int shares = 1; shares <= MOST_SHARES && shares <= p.stages; ++shares) {
       const int per = (p.stages + shares - 1) / shares;
       if (shares > 1 && (shares - 1) * per >= p.stages) continue; // the last share would be empty
       // in stages of a CU that is full: the rounds of workgroups, a half-full one faster, each with a start and an end, and the
@@ -379,19 +382,29 @@ bool product_plan(const MvmArgs &a, ProductArgs &p) {
 size_t product_room(MvmArgs a, bool terms_are_samples) {
   const int n_cus = a.cus > 0 ? a.cus : current_device_cus();
   int &samples = terms_are_samples ? a.K : a.m_batch;
-  const int most = samples, step = terms_are_samples ? PK : 64; // a stage, the smaller tile of samples
+  const int step = terms_are_samples ? PK : 64; // a stage, the smaller tile of samples
   size_t room = 0;
-  for (samples = std::min(step, most);; samples = std::min(samples + step, most)) {
+  for (; samples > 0; samples = (samples - 1) / step * step) {
+    ProductArgs p{};
+    p.tiles_o = (a.O + PT - 1) / PT;
+    p.tiles_b = (a.m_batch + PT - 1) / PT;
+    p.stages = (a.K + PK - 1) / PK;
+    p.sample_tile = PT;
+    p.shares = MOST_SHARES;
+    if (product_scratch(p, nullptr, nullptr) <= room) break; // nor can any smaller call need more
+    p.shares = 1;
+    // more shares save the last round of workgroups at most, and cost more than that for the sums of many tiles (product_split)
+    const double tiles = (double)p.tiles_o * (p.tiles_b - 0.5);
+    const bool one_share = 0.04 * tiles > p.stages + 1 + (double)p.tiles_o * (p.stages + 3 * MOST_SHARES) / (2 * n_cus);
+    if (one_share && product_scratch(p, nullptr, nullptr) <= room) continue;
     MvmArgs fewer = a;
     if (terms_are_samples) fewer.K = std::max(a.K - (PK - 1), 1); // the fewest of this many stages
-    if (product_pays(a, n_cus, true) || (terms_are_samples && product_pays(fewer, n_cus, true))) {
-      ProductArgs p;
-      product_split(a, n_cus, p);
-      const size_t bytes = product_scratch(p, nullptr, nullptr);
-      if (bytes <= MOST_SCRATCH) room = std::max(room, bytes);
-    }
-    if (samples == most) return room;
+    if (!product_pays(a, n_cus, true) && !(terms_are_samples && product_pays(fewer, n_cus, true))) continue;
+    if (!one_share) product_split(a, n_cus, p);
+    const size_t bytes = product_scratch(p, nullptr, nullptr);
+    if (bytes <= MOST_SCRATCH) room = std::max(room, bytes);
   }
+  return room;
 }
 
 static int sample_blocks(const ProductArgs &p) { return p.sample_tile == PT ? p.tiles_b : (p.tiles_b + 1) / 2; } // of 128 rows

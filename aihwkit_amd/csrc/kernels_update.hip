@@ -2099,7 +2099,8 @@ __global__ __launch_bounds__(1024) void k_update_pulsed_masks(UpdateArgs a, int 
 // sample in which its cross-point has a coincidence, and from memory every one of them is a trip to the cache that the next
 // pulse waits for.  Here a workgroup of 16 waves brings the words of 16 rows and 64 columns into LDS, 128 samples at a time; a
 // wave takes a row.  Blocks of samples, the lanes of a wave and with them the noise are those of pulsed_gather: same weights.
-// 785 x 300, 37 samples of 31 pulses 40.7 -> 14.2 us; the training step 93 -> 68.
+// 785 x 300, 37 samples of 31 pulses 40.7 -> 13.3 us; the training step 98 -> 68.  Bound by vector issue where the GPU is full (1024 x
+// 1024, 256 samples 165 us, all of its slots), by the chain of a wave's pulses where it is not.
 constexpr int WORDS_ROWS = 16, WORDS_BATCH = 128, WORDS_LINES = 64 + WORDS_ROWS; // lines of a workgroup: columns, then rows
 
 template <int KIND, bool MULT>
@@ -2584,9 +2585,9 @@ static unsigned update_copy_workgroups(const UpdateArgs &a) {
   return a.wt_src ? std::min(1024u, (unsigned)(((a.x_size + 31) / 32) * ((a.d_size + 31) / 32))) : 0u;
 }
 // Whether a call of one row of words to a sample takes k_update_lines_small: every workgroup reads all of its lines.  Updates, us,
-// two launches / one: 17 x 10, 5 samples 10.7 / 8.4; 129 x 10, 1 10.8 / 7.7, 64 14.7 / 13.5; 785 x 256, 1 11.3 / 9.5, 16 12.3 / 12.2;
-// 512 x 512, 16 12.4 / 10.9; 300 x 200, 50 14.5 / 14.3; 785 x 300, 20 13.1 / 12.7.  Beyond: 785 x 256, 32 14.0 / 15.0, 64 17.0 /
-// 20.1; 1024 x 1024, 1 14.6 / 15.0, 16 17.2 / 17.5.
+// two launches / one: 17 x 10, 5 samples 10.7 / 8.4; 129 x 10, 1 10.8 / 7.7, 64 14.7 / 13.5; 785 x 256, 1 11.3 / 9.5; 512 x 512, 16
+// 12.4 / 10.9; 300 x 200, 50 14.5 / 14.3.  Beyond, where every workgroup reads more than it saves: 785 x 256, 16 12.3 / 12.2, 32 14.0 /
+// 15.0, 64 17.0 / 20.1; 785 x 300, 20 13.1 / 12.7; 1024 x 1024, 1 14.6 / 15.0, 16 17.2 / 17.5.
 bool update_prepares_in_lines(const UpdateArgs &a) {
   const long line = (long)a.x_size + a.d_size;
   return !a.x_index && !a.d_group && !a.row_cost && a.kmax && a.m_batch <= SMALL_LINES_SAMPLES && (a.x_sj == 1 || a.m_batch == 1) &&
@@ -2764,7 +2765,11 @@ template <bool NOISE, int C> static void launch_update_pulsed_masks(const Update
   }
 }
 // Whether all bit lines of this call are longer than seven pulses (k_update_pulsed_words): without BL management a sample has the
-// desired length or a longer one, or no pulses at all (calc_bl_ab).
+// desired length or a longer one, or no pulses at all (calc_bl_ab).  Whatever the tile and the batch: update calls on row-major tiles,
+// us, the loop on bit planes and words in memory / this one, soft bounds, lines of 31 pulses 10 x 10, 5 samples 25 / 17; 1024 x 1, 256
+// 134 / 56 (fifteen of sixteen waves without a row); 64 x 64, 64 45 / 26; 26 x 16, 900 384 / 155; 512 x 512, 100 101 / 37; 1024 x 1024,
+// 1 39 / 29, 16 60 / 40, 256 406 / 192, 1000 1454 / 686; 2048 x 2048, 64 391 / 199; of 10 pulses 1024 x 1, 256 63 / 38; 1024 x 1024, 1
+// 25.5 / 25.5, 256 185 / 135.  (Longer batches on small tiles take the pipeline of waves, update_takes_stream.)
 bool update_takes_words(const UpdateArgs &a) {
   return !a.x_index && !a.d_group && !a.up.update_bl_management && a.up.desired_bl > UPDATE_PLANES_ONLY_KMAX;
 }
