@@ -325,19 +325,23 @@ static bool product_pays(const MvmArgs &a, int n_cus, bool large_tiles_aside) {
   // products per split value: few outputs or few samples leave a launch that splits and little else
   const double reuse = (double)a.m_batch * a.O / ((double)a.m_batch + a.O);
   if (!(work >= 0x1.8p29 && a.K >= 128 && reuse >= 96.0) && !(long_chain && reuse >= 32.0)) return false;
+  // an update of operands that both lie along the terms, which the launches before have little to copy for: 1024 x 4096, 192 terms 29.5
+  // / 32.9, 2048 x 2048, 192 31.0 / 32.6, 256 36.3 / 34.9
+  const bool update = a.beta != 0.0f;
+  if (update && a.in_sk == 1 && a.K < 256) return false;
   // Few samples of a large matrix, or the other way round: the split of the larger operand is most of the call.  Time of either, us,
-  // fitted to 570 calls of 36 to 49152 samples, 100 to 32768 outputs, 128 to 50000 terms (not the faster one of eight, by 9 % at
-  // most): 8192 x 8192, 40 samples 104 / 211, 4096 x 4096, 64 35 / 50, 128 54 / 62, 224 93 / 88, 2048 x 2048, 256 31.9 / 32.8, 288
-  // 41.9 / 36.4, 1024 -> 16384, 128 54 / 62.
+  // fitted to 629 calls of 36 to 49152 samples, 100 to 32768 outputs, 128 to 50000 terms (not the faster one of seven, by 11 % at
+  // most): 8192 x 8192, 40 samples 104 / 211, 4096 x 4096, 64 35 / 50, 128 54 / 64, 192 75 / 85, 224 93 / 88, 2048 x 2048, 256 31.9 /
+  // 33.2, 288 41.9 / 36.4, 1024 -> 16384, 128 54 / 62.
   const double samples = padded(a.m_batch, 64), outputs = padded(a.O, PT), terms = 1e-6 * a.K;
-  const double split = (padded(a.m_batch, PT) + outputs) * terms; // values
-  double rows = 11.0 + (a.w_oc ? 0.0068 : 0.005) * chain + (a.O % 32 && tiles_32 > n_cus ? 10.0 : 0.0);
+  double rows = 11.0 + (a.w_oc ? 0.0054 : 0.0042) * chain + (a.O % 32 && tiles_32 > n_cus ? 11.0 : 0.0);
   if (large) { // two workgroups to a CU at a time
-    const double large_rows = 16.0 + 0.036 * a.K * std::max(1.0, (a.O + 63) / 64 * (samples / 64) / (2 * n_cus));
+    const double large_rows = 20.5 + 0.022 * a.K * std::max(1.0, (a.O + 63) / 64 * (samples / 64) / (2 * n_cus));
     rows = large_tiles_aside ? std::max(rows, large_rows) : large_rows;
   }
-  const double parts = 18.0 + 1.35 * split + 1.4 * std::max(split - 20.0, 0.0) + 10.5 * samples * outputs * a.K / 0x1p30; // 20 M: 120 MB
-  return rows + 1.7 * a.m_batch * terms > parts;
+  rows += 1.5 * a.m_batch * terms + (update || large_tiles_aside ? 2e-6 * a.m_batch * a.O : 0.0);
+  const double parts = 15.0 + 1.35 * (padded(a.m_batch, PT) + outputs) * terms + 10.5 * samples * outputs * a.K / 0x1p30;
+  return rows > parts;
 }
 // the work of the call dealt out: tiles, shares of the terms
 static void product_split(const MvmArgs &a, int n_cus, ProductArgs &p) {
