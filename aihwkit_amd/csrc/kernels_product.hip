@@ -307,7 +307,7 @@ template <int BT> __global__ __launch_bounds__(4 * BT) void k_product_sum(MvmArg
 } // namespace
 
 // Whether a call of this size is worth the launch that splits its operands.  A tile makes room for the calls of fewer samples, too
-// (product_room): large_tiles_aside, whether one could be worth it.
+// (product_room): large_tiles_aside, whether this or one of up to 63 samples less, which might not take the large tiles, could be.
 static bool product_pays(const MvmArgs &a, int n_cus, bool large_tiles_aside) {
   const auto padded = [](double n, int to) { return std::ceil(n / to) * to; };
   // us, the launches of k_mvm_init and k_mvm_round or k_mvm_big / these.  From 3/4 G multiply-adds: 784 -> 256, 4096 samples (0.8
@@ -329,17 +329,18 @@ static bool product_pays(const MvmArgs &a, int n_cus, bool large_tiles_aside) {
   // / 32.9, 2048 x 2048, 192 31.0 / 32.6, 256 36.3 / 34.9
   const bool update = a.beta != 0.0f;
   if (update && a.in_sk == 1 && a.K < 256) return false;
-  // Few samples of a large matrix, or the other way round: the split of the larger operand is most of the call.  Time of either, us,
-  // fitted to 629 calls of 36 to 49152 samples, 100 to 32768 outputs, 128 to 50000 terms (not the faster one of seven, by 11 % at
-  // most): 8192 x 8192, 40 samples 104 / 211, 4096 x 4096, 64 35 / 50, 128 54 / 64, 192 75 / 85, 224 93 / 88, 2048 x 2048, 256 31.9 /
-  // 33.2, 288 41.9 / 36.4, 1024 -> 16384, 128 54 / 62.
+  if (large && a.m_batch > 256) return true;
+  // Few samples of a large matrix: the split of the weights is most of the call.  Time of either, us, fitted to 730 calls of 36 to 49152
+  // samples, 100 to 32768 outputs, 128 to 50000 terms (fourteen are left to the launches before that take up to 15 % longer, none
+  // is taken from them): 8192 x 8192, 40 samples 104 / 211, 4096 x 4096, 64 35 / 50, 128 54 / 64, 192 75 / 85, 224 93 / 88, 2048 x
+  // 2048, 256 31.9 / 33.2, 288 41.9 / 36.4, 1024 -> 16384, 128 62 / 74.
   const double samples = padded(a.m_batch, 64), outputs = padded(a.O, PT), terms = 1e-6 * a.K;
   double rows = 11.0 + (a.w_oc ? 0.0054 : 0.0042) * chain + (a.O % 32 && tiles_32 > n_cus ? 11.0 : 0.0);
   if (large) { // two workgroups to a CU at a time
     const double large_rows = 20.5 + 0.022 * a.K * std::max(1.0, (a.O + 63) / 64 * (samples / 64) / (2 * n_cus));
     rows = large_tiles_aside ? std::max(rows, large_rows) : large_rows;
   }
-  rows += 1.5 * a.m_batch * terms + (update || large_tiles_aside ? 2e-6 * a.m_batch * a.O : 0.0);
+  rows += 1.5 * a.m_batch * terms + (update ? 2e-6 * a.m_batch * a.O : 0.0);
   const double parts = 15.0 + 1.35 * (padded(a.m_batch, PT) + outputs) * terms + 10.5 * samples * outputs * a.K / 0x1p30;
   return rows > parts;
 }
@@ -387,6 +388,7 @@ size_t product_room(MvmArgs a, bool terms_are_samples) {
   const int n_cus = a.cus > 0 ? a.cus : current_device_cus();
   int &samples = terms_are_samples ? a.K : a.m_batch;
   const int step = terms_are_samples ? PK : 64; // a stage, the smaller tile of samples
+  a.beta = terms_are_samples ? 1.0f : 0.0f; // an update: those of delta weights pay for no smaller ones
   size_t room = 0;
   for (; samples > 0; samples = (samples - 1) / step * step) {
     ProductArgs p{};
@@ -403,7 +405,7 @@ size_t product_room(MvmArgs a, bool terms_are_samples) {
     if (one_share && product_scratch(p, nullptr, nullptr) <= room) continue;
     MvmArgs fewer = a;
     if (terms_are_samples) fewer.K = std::max(a.K - (PK - 1), 1); // the fewest of this many stages
-    if (!product_pays(a, n_cus, true) && !(terms_are_samples && product_pays(fewer, n_cus, true))) continue;
+    if (!product_pays(a, n_cus, !terms_are_samples) && !(terms_are_samples && product_pays(fewer, n_cus, false))) continue;
     if (!one_share) product_split(a, n_cus, p);
     const size_t bytes = product_scratch(p, nullptr, nullptr);
     if (bytes <= MOST_SCRATCH) room = std::max(room, bytes);
