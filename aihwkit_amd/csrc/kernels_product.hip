@@ -331,11 +331,11 @@ static bool product_pays(const MvmArgs &a, int n_cus, bool large_tiles_aside) {
   if (update && a.in_sk == 1 && a.K < 256) return false;
   if (large && a.m_batch > 256) return true;
   // Few samples of a large matrix: the split of the weights is most of the call.  Time of either, us, fitted to 730 calls of 36 to 49152
-  // samples, 100 to 32768 outputs, 128 to 50000 terms (fourteen are left to the launches before that take up to 15 % longer, none
-  // is taken from them): 8192 x 8192, 40 samples 104 / 211, 4096 x 4096, 64 35 / 50, 128 54 / 64, 192 75 / 85, 224 93 / 88, 2048 x
-  // 2048, 256 31.9 / 33.2, 288 41.9 / 36.4, 1024 -> 16384, 128 62 / 74.
+  // samples, 100 to 32768 outputs, 128 to 50000 terms (60 take up to 13 % longer than the faster one): 8192 x 8192, 40 samples 104 / 211,
+  // 4096 x 4096, 64 35 / 50, 128 54 / 64, 192 75 / 85, 224 93 / 88, 2048 x 2048, 256 31.9 / 33.2, 288 41.9 / 36.4, 1024 -> 16384, 128
+  // 62 / 74.  Not by the way the weights are stored (the 32 x 32 kernel takes 0.0042 or 0.0054 a term): either way the same bits.
   const double samples = padded(a.m_batch, 64), outputs = padded(a.O, PT), terms = 1e-6 * a.K;
-  double rows = 11.0 + (a.w_oc ? 0.0054 : 0.0042) * chain + (a.O % 32 && tiles_32 > n_cus ? 11.0 : 0.0);
+  double rows = 11.0 + 0.005 * chain + (a.O % 32 && tiles_32 > n_cus ? 11.0 : 0.0);
   if (large) { // two workgroups to a CU at a time
     const double large_rows = 20.5 + 0.022 * a.K * std::max(1.0, (a.O + 63) / 64 * (samples / 64) / (2 * n_cus));
     rows = large_tiles_aside ? std::max(rows, large_rows) : large_rows;

@@ -1002,15 +1002,15 @@ struct Tile {
     MvmArgs a{};
     a.cus = call.cus;
     size_t room = 0;
-    const auto add = [&](int samples, int outputs, int terms, bool over_terms, int w_oc) {
-      a.m_batch = samples; a.O = outputs; a.K = terms; a.w_oc = w_oc;
+    const auto add = [&](int samples, int outputs, int terms, bool over_terms) {
+      a.m_batch = samples; a.O = outputs; a.K = terms;
       room = std::max({room, parts ? product_room(a, over_terms) : 0, (size_t)samples * mvm_k_pad(terms) * sizeof(float)});
     };
-    add(call.m_batch, call.O, call.K, terms_are_samples, call.w_oc);
+    add(call.m_batch, call.O, call.K, terms_are_samples);
     const int B = terms_are_samples ? call.K : call.m_batch;
-    if (fio.perfect) add(B, D, X, false, xd ? 1 : 0);
-    if (bio.perfect) add(B, X, D, false, xd ? 0 : 1);
-    if (!dev.pulsed() || up.p.pulse_type == RPU_PULSE_NONE) add(X, D, B, true, 1);
+    if (fio.perfect) add(B, D, X, false);
+    if (bio.perfect) add(B, X, D, false);
+    if (!dev.pulsed() || up.p.pulse_type == RPU_PULSE_NONE) add(X, D, B, true);
     return room;
   }
   // Room for the call, which needs `bytes` of it; false: only for its rows, also of calls to come (parts take up to ten times as

@@ -633,7 +633,8 @@ class TileGroup:
 
     The reference runs the tiles of a tile array one after the other (TileModuleArray.forward,
     src/aihwkit/simulator/tiles/array.py:155-182); a group gives every tile the same result as its own
-    ``forward(x, False, False, False, is_test)`` would, with one launch per kernel variant and round for all of them.
+    ``forward(x, False, False, False, is_test)`` would, with one launch per kernel variant and round for all of them
+    (large batches and exact passes up to the order of the 32-bit sums, where another kernel adds them).
     """
 
     def __init__(self, tile_list):

@@ -432,7 +432,9 @@ int rpu_tile_update_indexed(rpu_tile_t *tile, const float *x_dev, const float *d
  * from Python (TileModuleArray.forward, src/aihwkit/simulator/tiles/array.py:155-182).  A group runs the forward
  * pass of all its tiles in a few launches (one per kernel variant and bound-management round) instead of
  * several per tile.  The tiles must be resident on the same GPU; each keeps its own state, seed and call
- * counter, and a grouped call gives every tile exactly what rpu_tile_forward with the same arguments would.
+ * counter, and a grouped call gives every tile what rpu_tile_forward with the same arguments would: the same bits, but
+ * where the sizes of the group or of the call give the contraction to another kernel than the tile's own call takes
+ * (large batches, exact passes) up to the order of its 32-bit sums.
  * x_dev[i] is [m_batch][x_size_i], y_dev[i] is [m_batch][d_size_i] (no bias column, no transposed layouts).
  * A group that holds a tile whose pass has periphery terms before the ADC (output-referred weight noise, IR drop,
  * per-line offsets and non-linearities, separate passes per input sign) or running-average noise management runs
@@ -449,7 +451,7 @@ int rpu_group_forward_strided(rpu_group_t *group, const float *const *x_dev, con
                               const long *y_ld, int m_batch, int is_test, void *stream);
 /* Backward pass of all tiles of the group: d_dev[i] is [m_batch][d_size_i] with row stride d_ld[i], x_dev[i] receives
  * [m_batch][x_size_i] with row stride x_ld[i] (null strides: dense rows); every tile gets what rpu_tile_backward
- * gives it. */
+ * gives it, as rpu_group_forward says. */
 int rpu_group_backward_strided(rpu_group_t *group, const float *const *d_dev, const long *d_ld, float *const *x_dev,
                                const long *x_ld, int m_batch, void *stream);
 /* Stochastic pulsed update of all tiles of the group (the reference updates the tiles of an array one after the other

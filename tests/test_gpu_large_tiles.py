@@ -233,6 +233,23 @@ def test_exact_products_of_calls_that_fill_the_gpu(gpu_device, x_size, d_size, b
     _close(delta.t(), want, terms, batch)
 
 
+# on either side of the line between the launches on parts and the 32 x 32 kernel, which takes longer for one of the storages
+@pytest.mark.parametrize("x_size,d_size,batch", [(1025, 900, 900), (2048, 2048, 130), (2048, 2048, 256), (1024, 4096, 192), (4096, 1024, 224),
+                                                 (3072, 3072, 96), (3072, 3072, 256), (4096, 4096, 192), (1024, 16384, 128)])
+def test_exact_calls_have_the_same_bits_on_either_storage(gpu_device, x_size, d_size, batch):
+    gen = torch.Generator("cuda").manual_seed(1)
+    io = noise_free_io()
+    io.is_perfect = True
+    w = np.random.default_rng(1).standard_normal((d_size, x_size)).astype(np.float32)
+    one, other = _tile(x_size, d_size, io, w), _tile(x_size, d_size, io, w)
+    if not tiles.CudaAnalogTile.bind_shared_weights:
+        bound = torch.empty(x_size, d_size, device="cuda")
+        other.set_shared_weights(bound)
+    x, d = torch.randn(batch, x_size, generator=gen, device="cuda"), torch.randn(batch, d_size, generator=gen, device="cuda")
+    assert torch.equal(one.forward(x), other.forward(x))
+    assert torch.equal(one.backward(d), other.backward(d))
+
+
 def test_exact_products_of_rows_that_are_slices_of_longer_ones(gpu_device):
     """A group that holds a tile on running-average noise management runs its tiles one by one, on the slices that it is given:
     unaligned ones here."""
