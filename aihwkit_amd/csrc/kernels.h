@@ -199,7 +199,8 @@ int mvm_few_variant(const MvmArgs *const *calls, int n); // blocks of a launch o
 int mvm_few_workgroups(const MvmArgs &a, int variant);
 void launch_mvm_few(const MvmArgs &a, int variant, int rounds, hipStream_t s);
 void launch_mvm_few_clear_group(const MvmGroup &g, hipStream_t s); // the counters of its calls
-void launch_mvm_few_group(const MvmGroup &g, int variant, int rounds, bool w_oc, int max_k, int total_workgroups, hipStream_t s);
+bool mvm_few_stoch(const MvmArgs &a); // whether the converters draw random numbers beyond the output noise
+void launch_mvm_few_group(const MvmGroup &g, int variant, int rounds, bool w_oc, bool stoch, int max_k, int total_workgroups, hipStream_t s);
 
 // Fused convolution forward (unfold + noisy MVM with its bound-management rounds) for tiles of at most 32 outputs:
 // images [n_images][image_size], idx_t the transposed index matrix [patches][x_size], out [n_images][d_size][patches].

@@ -30,7 +30,7 @@
 //                  management, DAC, contraction, ADC and the bound-management rounds in one kernel.
 //   *_group        the same kernels over the tiles of a group in one launch.
 #include "bf16_parts.h"
-#include "kernels.h"
+#include "mvm_device.h"
 
 #include <atomic>
 #include <cmath>
@@ -57,34 +57,6 @@ constexpr int TILE = 32;
 constexpr int WAVES = 4;
 constexpr int KSTEP = 32; // k-values per wave step: 128 bytes per operand row
 
-// STOCH = false: for callers that have checked that the DAC draws no random numbers (no stochastic rounding, no input
-// noise): the draws are then not even compiled in, which the fully unrolled callers pay for in registers
-template <bool STOCH = true>
-__device__ __forceinline__ float dac_value(float x, float scale, const IoDev &io, PhiloxKey key,
-                                           uint32_t call, int round, int b, int k) {
-  // value *= scale; discretize; clip; (+ noise); (asymmetry)      rpu_forward_backward_pass.cpp:583-602
-  float v = x * scale;
-  if (io.inp_res > 0.0f) {
-    float q = v / io.inp_res;
-    if (STOCH && io.inp_sto_round) {
-      const Philox4 r = philox4x32_10((uint32_t)k, (uint32_t)b, call, RNG_INP_SR | ((uint32_t)round << 8), key.k0, key.k1);
-      q = q + (u32_to_uniform(r.v[0]) - 0.5f);
-    }
-    v = rintf(q) * io.inp_res;
-  }
-  v = (v > io.inp_bound) ? io.inp_bound : v;
-  v = (v < -io.inp_bound) ? -io.inp_bound : v;
-  if (STOCH && io.inp_noise > 0.0f) {
-    float n[4];
-    philox_normal4((uint32_t)k, (uint32_t)b, call, RNG_INP_NOISE | ((uint32_t)round << 8), key, n);
-    v += io.inp_noise * n[0];
-  }
-  if (io.inp_asym != 0.0f) {
-    v = v < 0.0f ? v * (1.0f - io.inp_asym) : v;
-  }
-  return v;
-}
-
 // a sample's input row when the call gathers its input through an index (a.in_index)
 struct MvmGatherRow {
   const float *image; // element j - 2 at image[j]
@@ -98,12 +70,6 @@ __device__ __forceinline__ MvmGatherRow mvm_gather_row(const MvmArgs &a, int b) 
   const int n = b / a.in_group;
   return MvmGatherRow{a.in + (long)n * a.in_gs - 2, a.in_index + (long)(b - n * a.in_group) * a.K};
 }
-
-// Stored elements of a sample: all K, or without the 1 of the bias column.  Loops that put several loads in flight read the
-// elements below this number and set the 1 afterwards, in a branch that the whole wave takes or not: with a choice between
-// load and constant at every element the loads are issued one by one (k_mvm_init, 256 samples of 1024 elements: 8.1 us
-// instead of 6.9).
-__device__ __forceinline__ int mvm_stored(const MvmArgs &a) { return a.K - a.in_one; }
 
 // element k (< K) of a sample whose stored elements (one at least) start at `row`
 __device__ __forceinline__ float mvm_input(const MvmArgs &a, const float *__restrict__ row, int k) {
@@ -241,58 +207,12 @@ __device__ __forceinline__ void mvm_finish_outputs(const MvmArgs &a, int round, 
   }
 }
 
-// input scale of a round and the factor applied to its ADC output
-__device__ __forceinline__ float round_scales(const MvmArgs &a, float nm, float red, float &fin) {
-  const IoDev &io = a.io;
-  const bool use_nm = io.noise_management != RPU_NM_NONE;
-  const bool bm = io.bound_management != RPU_BM_NONE;
-  float scale;
-  if (a.transposed) {
-    // backward: scale = 1 / nm ; result *= out_scale * nm
-    if (use_nm && nm <= 0.0f) {
-      scale = 0.0f;
-      fin = 0.0f;
-    } else {
-      scale = use_nm ? 1.0f / nm : 1.0f;
-      fin = use_nm ? io.out_scale * nm : io.out_scale;
-    }
-  } else if (use_nm && nm <= 0.0f && io.inp_noise <= 0.0f) {
-    scale = 0.0f;
-    fin = 0.0f;
-  } else {
-    scale = 1.0f;
-    if (use_nm && nm > 0.0f) scale /= nm;
-    if (bm) scale /= red;
-    fin = io.out_scale / scale;
-  }
-  return scale;
-}
-
 __device__ __forceinline__ float set_round_scales(const MvmArgs &a, int b, float nm, float red) {
   float fin;
   const float scale = round_scales(a, nm, red, fin);
   a.st.scale[b] = scale;
   a.st.fin[b] = fin;
   return scale;
-}
-
-// Noise-management value and reduction that sample b, now at (nm, red) with output factor fin, would use in
-// the round after `round`; false when the reduction limit is reached or the sample is short-cut to zero
-// (rpu_forward_backward_pass.cpp:944-983).
-// np_known: the sample's AbsMaxNPSum scale where the caller has just computed it (the init kernel, whose other
-// threads must not read back what its first thread is storing); null: read from the per-sample state.
-__device__ __forceinline__ bool next_round_params(const MvmArgs &a, int round, int b, float fin, float &nm, float &red,
-                                                  const float *np_known = nullptr) {
-  const IoDev &io = a.io;
-  if (fin == 0.0f) return false;
-  const bool stop = ((int)red > io.max_bm_factor) || ((io.inp_res > 0.0f) && (red > io.max_bm_res / io.inp_res));
-  if (stop) return false;
-  red *= 2.0f;
-  if (round == 0 && io.bound_management == RPU_BM_ITERATIVE_WORST_CASE && io.noise_management != RPU_NM_ABS_MAX_NP_SUM) {
-    nm = np_known ? *np_known : a.st.nm_np[b];
-    red = 1.0f;
-  }
-  return true;
 }
 
 // input scale of the round after `round` for such a sample, 0 when there is none
@@ -2090,465 +2010,6 @@ __global__ __launch_bounds__(256, XP == 1 && BB == 64 ? 3 : 2) void k_mvm_big_gr
 }
 
 // ---------------------------------------------------------------------------------------------
-// Small batches in one launch: noise management, DAC, contraction, ADC and every bound-management round.
-//
-// A batch of a few dozen samples is latency from end to end: an init kernel, a round of 32 x 32 tiles on a handful of CUs
-// (each wave a chain of K / 4 matrix steps, mostly padding for one sample), and a launch for the rounds that are expected to
-// be empty -- 4, 12 and 4 us for one sample on a 512 x 512 tile.  Here a workgroup takes S samples and OB outputs.  It
-// reads and quantizes its samples' rows itself (every workgroup of a sample does: a few elements per thread), multiplies
-// with plain fp32 multiply-adds, 32 weights of a thread in flight, and adds its threads' partial sums (chains of K / 16 terms)
-// through LDS.  The workgroups of a sample count themselves off; the
-// last one knows whether the sample saturated.  Where the tile's recent calls did, R = 3: the workgroups multiply the same
-// weights with the inputs of rounds 0, 1 and 2 (V = R S rows) and keep all results, and the last one copies out what
-// stands (as k_mvm_dual); a round beyond those it runs alone, block by block.  No list, no later launch.
-// One sample on a 512 x 512 tile 21 -> 8 us, 27 -> 13 where it saturates; 64 samples on 785 -> 256 40 -> 22, on 129 -> 10 16 -> 7.
-// What bounds it: the chain from launch to loads, maximum, loads of weights, ADC, two atomics (about 1 us each).
-// The streams of random numbers are those of the other kernels (element k, sample, round; four outputs to a draw).
-template <bool WOC, int S, int OB, int R> struct MvmFew {
-  typedef MvmFew<WOC, S, 64, 1> Alone; // see alone()
-  static constexpr int V = R * S;
-  // A load of a wave, and the order of every sum, are the same in all variants, so that any of them can run a call: part p of
-  // an output's sixteen takes k = 4 p .. 4 p + 3 (mod 64) in ascending order, and the parts are added as a tree.
-  //   weights along k: sixteen lanes next to each other read 64 weights of a row, a wave OB / 4 rows
-  //   along the outputs: sixteen lanes read OB outputs of a row, each wave sixteen rows of 64
-  static constexpr int PARTS = 16, K_LOAD = 64;
-  static constexpr int WIDTH = WOC ? OB / 16 : 4;            // weights of a load
-  static constexpr int LOADS = WOC ? 4 : OB / 16;            // loads of a thread for 64 contraction indices
-  static constexpr int OUTPUTS = OB / 16;                    // sums of a thread, per row of inputs
-  static constexpr int AHEAD = 32 / (WIDTH * LOADS);         // of 64 contraction indices, in flight: 32 weights of a thread
-  static constexpr int PER_SUM = 256 / (S * OB);             // threads that add up an output
-  static constexpr int PITCH = PARTS + 1;                    // of an output's partial sums in LDS
-  typedef float Load __attribute__((ext_vector_type(WIDTH), aligned(4)));
-  typedef float Weights[AHEAD][LOADS][WIDTH];
-
-  const MvmArgs &a;
-  float *xs, *part; // LDS: [R][S][k_len] quantized inputs, zero padded; [S][OB][PITCH]
-  int *hits;        // LDS: [R][2][S] saturation marks: upper, lower
-  int k_len;
-  int lane, wave;
-
-  static __host__ __device__ int padded(int K) {
-    constexpr int STEP = K_LOAD * AHEAD;
-    return (K + STEP - 1) / STEP * STEP;
-  }
-  static __host__ __device__ size_t lds_bytes(int K) {
-    const size_t own = sizeof(float) * ((size_t)V * padded(K) + S * OB * PITCH);
-    if constexpr (OB == 64 && R == 1) return own;
-    else return own > Alone::lds_bytes(K) ? own : Alone::lds_bytes(K);
-  }
-
-  __device__ __forceinline__ MvmFew(const MvmArgs &a_, float *lds, int *hits_)
-      : a(a_), xs(lds), part(lds + V * padded(a_.K)), hits(hits_), k_len(padded(a_.K)), lane((int)threadIdx.x & 63), wave((int)threadIdx.x >> 6) {}
-
-  // weights of the outputs from o_first on for k0 .. k0 + 64 AHEAD - 1.  Nothing is read beyond a row's end, what stands for
-  // it is zero; beyond the last row the last one is read (k: the inputs are zero; outputs: never stored).
-  __device__ __forceinline__ void load(Weights &w, int o_first, int k0) const {
-    const bool whole = WOC ? o_first + OB <= a.O : k0 + K_LOAD * AHEAD <= a.K; // the same for the workgroup
-#pragma unroll
-    for (int u = 0; u < AHEAD; ++u) {
-#pragma unroll
-      for (int l = 0; l < LOADS; ++l) {
-        const float *row;
-        int at, end;
-        if (WOC) {
-          row = a.w + (long)min(k0 + u * K_LOAD + (wave * 4 + (lane >> 4)) * 4 + l, a.K - 1) * a.w_ld;
-          at = o_first + WIDTH * (lane & 15);
-          end = a.O;
-        } else {
-          row = a.w + (long)min(o_first + (wave * LOADS + l) * 4 + (lane >> 4), a.O - 1) * a.w_ld;
-          at = k0 + u * K_LOAD + 4 * (lane & 15);
-          end = a.K;
-        }
-        if (whole || at + WIDTH <= end) {
-          if constexpr (WIDTH == 1) {
-            w[u][l][0] = row[at];
-          } else {
-            const Load v = *reinterpret_cast<const Load *>(row + at);
-#pragma unroll
-            for (int q = 0; q < WIDTH; ++q) w[u][l][q] = v[q];
-          }
-        } else {
-#pragma unroll
-          for (int q = 0; q < WIDTH; ++q) w[u][l][q] = at + q < end ? row[at + q] : 0.0f;
-        }
-      }
-    }
-  }
-
-  // this thread's sums for the outputs from o_first on; w holds the weights from k = 0, and those of the outputs from `then`
-  // on afterwards
-  typedef float Sums[V][OUTPUTS];
-  __device__ __forceinline__ void contract(Weights &w, int o_first, Sums &sums, int then) const {
-#pragma unroll
-    for (int v = 0; v < V; ++v) {
-#pragma unroll
-      for (int o = 0; o < OUTPUTS; ++o) sums[v][o] = 0.0f;
-    }
-    for (int k0 = 0; k0 < k_len; k0 += K_LOAD * AHEAD) {
-      Weights now;
-#pragma unroll
-      for (int u = 0; u < AHEAD; ++u) {
-#pragma unroll
-        for (int l = 0; l < LOADS; ++l) {
-#pragma unroll
-          for (int q = 0; q < WIDTH; ++q) now[u][l][q] = w[u][l][q];
-        }
-      }
-      if (k0 + K_LOAD * AHEAD < k_len) load(w, o_first, k0 + K_LOAD * AHEAD);
-      else if (then < a.O) load(w, then, 0);
-#pragma unroll
-      for (int u = 0; u < AHEAD; ++u) {
-        const int k = k0 + u * K_LOAD + (WOC ? (wave * 4 + (lane >> 4)) * 4 : 4 * (lane & 15));
-#pragma unroll
-        for (int v = 0; v < V; ++v) {
-          const f32x4 x = *reinterpret_cast<const f32x4 *>(xs + v * k_len + k);
-#pragma unroll
-          for (int l = 0; l < LOADS; ++l) {
-#pragma unroll
-            for (int q = 0; q < WIDTH; ++q) {
-              if (WOC) sums[v][q] = __builtin_fmaf(now[u][l][q], x[l & 3], sums[v][q]);
-              else sums[v][l] = __builtin_fmaf(now[u][l][q], x[q & 3], sums[v][l]);
-            }
-          }
-        }
-      }
-    }
-  }
-  // the sums of round r (of R) to LDS
-  __device__ __forceinline__ void spread(const Sums &sums, int r) const {
-#pragma unroll
-    for (int s = 0; s < S; ++s) {
-#pragma unroll
-      for (int o = 0; o < OUTPUTS; ++o) {
-        float v = sums[s][o];
-#pragma unroll
-        for (int i = 1; i < R; ++i) v = r == i ? sums[i * S + s][o] : v;
-        if (WOC) part[(s * OB + OUTPUTS * (lane & 15) + o) * PITCH + wave * 4 + (lane >> 4)] = v;
-        else part[(s * OB + (wave * OUTPUTS + o) * 4 + (lane >> 4)) * PITCH + (lane & 15)] = v;
-      }
-    }
-  }
-
-  // adds up the partial sums and takes them through the ADC stage of `round` (mvm_adc_values, an output per thread), for the
-  // samples of the block with their bit set in `live`, marks to hits[at].  rows: where the results are kept, null: the call's
-  // output; shared: other workgroups read them, or have written the same outputs
-  __device__ __forceinline__ void finish(int b0, int o_first, int round, int at, unsigned live, const float (&fin)[S], float *rows,
-                                         bool shared) {
-    const int t = (int)threadIdx.x, sum = t / PER_SUM, s = sum / OB, o = o_first + sum % OB;
-    constexpr int MINE = PARTS / PER_SUM;
-    float p[MINE];
-#pragma unroll
-    for (int i = 0; i < MINE; ++i) p[i] = part[sum * PITCH + PER_SUM * i + t % PER_SUM];
-#pragma unroll
-    for (int half = MINE / 2; half > 0; half >>= 1) {
-#pragma unroll
-      for (int i = 0; i < half; ++i) p[i] += p[i + half];
-    }
-    float y = p[0];
-#pragma unroll
-    for (int off = PER_SUM / 2; off > 0; off >>= 1) y += __shfl_xor(y, off);
-    if (t % PER_SUM != 0 || o >= a.O || !((live >> s) & 1u)) return;
-    const IoDev &io = a.io;
-    const int b = b0 + s;
-    float f = fin[0];
-#pragma unroll
-    for (int i = 1; i < S; ++i) f = s == i ? fin[i] : f;
-    float *out = rows ? rows + (long)b * a.O + o : a.out + (long)b * a.out_sb + (long)o * a.out_so;
-    if (f == 0.0f) { // zero input: the reference short-cuts to a zero output
-      y = 0.0f;
-    } else {
-      if (io.out_asym > 0.0f) y = y < 0.0f ? y * (1.0f - io.out_asym) : y;
-      if (io.out_noise > 0.0f) {
-        const Philox4 r = philox4x32_10((uint32_t)(o >> 2), (uint32_t)b, a.call, RNG_OUT_NOISE | ((uint32_t)round << 8), a.key.k0, a.key.k1);
-        float n0, n1;
-        box_muller((o & 2) ? r.v[2] : r.v[0], (o & 2) ? r.v[3] : r.v[1], n0, n1);
-        y += io.out_noise * ((o & 1) ? n1 : n0);
-      }
-      if (io.out_res > 0.0f) {
-        float q = y / io.out_res;
-        if (io.out_sto_round) {
-          const Philox4 r = philox4x32_10((uint32_t)o, (uint32_t)b, a.call, RNG_OUT_SR | ((uint32_t)round << 8), a.key.k0, a.key.k1);
-          q = q + (u32_to_uniform(r.v[0]) - 0.5f);
-        }
-        y = rintf(q) * io.out_res;
-      }
-      const bool over = y > io.out_bound, under = y < -io.out_bound;
-      y = over ? io.out_bound : (under ? -io.out_bound : y);
-      if (over) atomicMax(&hits[2 * S * at + s], o + 1);
-      if (under) atomicMax(&hits[2 * S * at + S + s], o + 1);
-      y *= f;
-    }
-    if (o >= a.O - a.out_drop) return;
-    if (shared) __hip_atomic_store(out, y, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); // through the XCD's own L2
-    else *out = y;
-  }
-
-  __device__ __forceinline__ float stored_input(int b, int k) const {
-    const float v = a.in[(long)b * a.in_sb + (long)min(k, mvm_stored(a) - 1) * a.in_sk];
-    return k < mvm_stored(a) ? v : 1.0f;
-  }
-
-  // whether sample s, at (nm, red, fin) in `round` with the marks at hits[at], goes on to the next round; moves it there
-  __device__ __forceinline__ bool goes_on(int b, int s, int round, int at, float &nm, float &red, float &fin, float &scale) const {
-    const int up = hits[2 * S * at + s], lo = hits[2 * S * at + S + s];
-    const bool failed = a.io.bm_test_negative_bound ? (up > 0 || lo > 0) : (up > lo);
-    if (!failed || round + 1 >= a.max_rounds || !next_round_params(a, round, b, fin, nm, red)) return false;
-    scale = round_scales(a, nm, red, fin);
-    return true;
-  }
-
-  __device__ __forceinline__ void run(const int block_b, const int block_o) {
-    __shared__ float sh_max[2][4][S];
-    __shared__ int sh_last;
-    const IoDev &io = a.io;
-    const int t = (int)threadIdx.x, b0 = block_b * S, blocks_o = (a.O + OB - 1) / OB;
-    Weights w;
-    load(w, block_o * OB, 0); // on their way while the inputs are worked on
-    if (t < 2 * V) hits[t] = 0;
-    unsigned live = 0u;
-    float amax[S], vmax[S];
-#pragma unroll
-    for (int s = 0; s < S; ++s) {
-      amax[s] = 0.0f;
-      vmax[s] = -INFINITY;
-      live |= b0 + s < a.m_batch ? 1u << s : 0u;
-    }
-    for (int k = t; k < k_len; k += 256) {
-      float x[S];
-#pragma unroll
-      for (int s = 0; s < S; ++s) x[s] = stored_input(min(b0 + s, a.m_batch - 1), min(k, a.K - 1));
-#pragma unroll
-      for (int s = 0; s < S; ++s) {
-        xs[s * k_len + k] = k < a.K ? x[s] : 0.0f;
-        amax[s] = fmaxf(amax[s], k < a.K ? fabsf(x[s]) : 0.0f);
-        vmax[s] = fmaxf(vmax[s], k < a.K ? x[s] : -INFINITY);
-      }
-    }
-#pragma unroll
-    for (int s = 0; s < S; ++s) {
-#pragma unroll
-      for (int off = 32; off > 0; off >>= 1) {
-        amax[s] = fmaxf(amax[s], __shfl_xor(amax[s], off));
-        vmax[s] = fmaxf(vmax[s], __shfl_xor(vmax[s], off));
-      }
-      if (lane == 0) {
-        sh_max[0][wave][s] = amax[s];
-        sh_max[1][wave][s] = vmax[s];
-      }
-    }
-    __syncthreads();
-    // noise-management value, and reduction, input scale and output factor of the round a sample is in
-    float nm[S], red[S], scale[S], fin[S], fin_of[R][S];
-    int rounds[S];
-#pragma unroll
-    for (int s = 0; s < S; ++s) {
-      const int kind = io.noise_management == RPU_NM_MAX ? 1 : 0;
-      const float m = fmaxf(fmaxf(sh_max[kind][0][s], sh_max[kind][1][s]), fmaxf(sh_max[kind][2][s], sh_max[kind][3][s]));
-      nm[s] = 1.0f;
-      if (io.noise_management == RPU_NM_ABS_MAX || io.noise_management == RPU_NM_MAX) nm[s] = io.nm_thres > 0.0f ? fminf(m, io.nm_thres) : m;
-      else if (io.noise_management == RPU_NM_CONSTANT) nm[s] = io.nm_thres > 0.0f ? io.nm_thres : 1.0f;
-      red[s] = 1.0f;
-      scale[s] = round_scales(a, nm[s], 1.0f, fin[s]);
-      rounds[s] = fin[s] == 0.0f ? 0 : 1;
-    }
-    for (int k = t; k < k_len; k += 256) { // what this thread has written
-#pragma unroll
-      for (int s = 0; s < S; ++s) {
-        const float x = xs[s * k_len + k];
-        float rr = 1.0f;
-#pragma unroll
-        for (int r = 0; r < R; ++r, rr *= 2.0f) {
-          float f;
-          xs[(r * S + s) * k_len + k] = k < a.K ? dac_value(x, round_scales(a, nm[s], rr, f), io, a.key, a.call, r, b0 + s, k) : 0.0f;
-        }
-      }
-    }
-    {
-      float rr = 1.0f;
-#pragma unroll
-      for (int r = 0; r < R; ++r, rr *= 2.0f) {
-#pragma unroll
-        for (int s = 0; s < S; ++s) (void)round_scales(a, nm[s], rr, fin_of[r][s]);
-      }
-    }
-    __syncthreads();
-    Sums sums;
-    contract(w, block_o * OB, sums, a.O);
-    const bool managed = a.max_rounds > 1, shared = managed && blocks_o > 1;
-    int next = 0; // the first round that has not been run
-    if (!shared) {
-      // all outputs are here: the rounds one after the other, each for the samples that need it
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        if (r > 0) {
-          if (!managed) break;
-          live = advance(b0, live, r - 1, r - 1, nm, red, fin, scale, rounds);
-          if (!live) break;
-          __syncthreads();
-        }
-        spread(sums, r);
-        __syncthreads();
-        finish(b0, block_o * OB, r, r, live, fin, nullptr, false);
-        __syncthreads();
-        next = r + 1;
-      }
-      if (managed && live) live = advance(b0, live, next - 1, next - 1, nm, red, fin, scale, rounds);
-    } else {
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        if (r > 0) __syncthreads();
-        spread(sums, r);
-        __syncthreads();
-        finish(b0, block_o * OB, r, r, live, fin_of[r], r == 0 ? nullptr : (r == 1 ? a.dual.buf[1] : a.dual.buf[2]), true);
-      }
-      // what this workgroup stored has arrived before it counts itself off, and so have its marks
-      int *const marks = a.few + a.m_batch; // [R][2][m_batch]: upper, lower; the counters before them
-      __builtin_amdgcn_s_waitcnt(0);
-      __syncthreads();
-      const bool mine = t < 2 * V && b0 + t % S < a.m_batch;
-      if (mine && hits[t]) {
-        const int old = atomicMax(&marks[(t / S) * a.m_batch + b0 + t % S], hits[t]);
-        asm volatile("" ::"v"(old));
-      }
-      __syncthreads();
-      if (t == 0) sh_last = atomicAdd(&a.few[block_b], 1) == blocks_o - 1 ? 1 : 0;
-      __syncthreads();
-      if (!sh_last) return;
-      // the last one reads the marks of all, and leaves them and the counter as it found them at first: zero
-      if (t == 0) __hip_atomic_store(&a.few[block_b], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if (t < 2 * V) hits[t] = mine ? atomicExch(&marks[(t / S) * a.m_batch + b0 + t % S], 0) : 0;
-      __syncthreads();
-      unsigned chosen[R]; // samples whose result is that of round r
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        const unsigned before = live;
-        live = advance(b0, live, r, r, nm, red, fin, scale, rounds);
-        chosen[r] = before & ~live;
-      }
-      next = R;
-#pragma unroll
-      for (int r = 1; r < R; ++r) {
-        const float *rows = r == 1 ? a.dual.buf[1] : a.dual.buf[2];
-#pragma unroll
-        for (int s = 0; s < S; ++s) {
-          if (!((chosen[r] >> s) & 1u)) continue;
-          for (int o = t; o < a.O - a.out_drop; o += 256) {
-            const float v = __hip_atomic_load(rows + (long)(b0 + s) * a.O + o, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(a.out + (long)(b0 + s) * a.out_sb + (long)o * a.out_so, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          }
-        }
-      }
-    }
-    if (managed && live) { // the same for all threads
-      __syncthreads();
-      Alone(a, xs, hits).alone(b0, live, next, nm, red, fin, scale, rounds, shared);
-    }
-    if ((shared || block_o == 0) && t == 0) {
-      int most = 0;
-#pragma unroll
-      for (int s = 0; s < S; ++s) {
-        if (b0 + s >= a.m_batch) continue;
-        a.st.rounds[b0 + s] = rounds[s];
-        most = max(most, rounds[s]);
-      }
-      // the host picks R by what it knows of the last calls: the last one it hears of, the last one with samples that went on
-      if (managed && most > 1) __hip_atomic_store(a.few_seen, a.few_call, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-      if (managed && block_b == 0) __hip_atomic_store(a.few_seen + 1, a.few_call, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    }
-  }
-  // The rounds from `round` on for the samples of `live`, by this workgroup: block after block of 64 outputs, whatever the
-  // blocks of the launch are (a block is one trip through the ADC stage: with blocks
-  // of 16 a round of a 512 x 512 tile took 35 us)
-  __device__ __forceinline__ void alone(int b0, unsigned live, int round, float (&nm)[S], float (&red)[S], float (&fin)[S],
-                                        float (&scale)[S], int (&rounds)[S], bool shared) {
-    const int t = (int)threadIdx.x;
-    Sums sums;
-    Weights w;
-    for (; live; ++round) {
-      load(w, 0, 0);
-      if (t < 2 * S) hits[t] = 0;
-      for (int k = t; k < k_len; k += 256) {
-#pragma unroll
-        for (int s = 0; s < S; ++s) {
-          xs[s * k_len + k] = k < a.K ? dac_value(stored_input(min(b0 + s, a.m_batch - 1), k), scale[s], a.io, a.key, a.call, round, b0 + s, k) : 0.0f;
-        }
-      }
-      for (int o_first = 0; o_first < a.O; o_first += OB) {
-        __syncthreads(); // the inputs are there, the sums of the outputs before have been read
-        contract(w, o_first, sums, o_first + OB);
-        spread(sums, 0);
-        __syncthreads();
-        finish(b0, o_first, round, 0, live, fin, nullptr, shared);
-      }
-      __syncthreads();
-      live = advance(b0, live, round, 0, nm, red, fin, scale, rounds);
-      __syncthreads();
-    }
-  }
-  // the samples of `live` that go on after `round`
-  __device__ __forceinline__ unsigned advance(int b0, unsigned live, int round, int at, float (&nm)[S], float (&red)[S],
-                                              float (&fin)[S], float (&scale)[S], int (&rounds)[S]) const {
-    unsigned on = 0u;
-#pragma unroll
-    for (int s = 0; s < S; ++s) {
-      if (((live >> s) & 1u) && goes_on(b0 + s, s, round, at, nm[s], red[s], fin[s], scale[s])) {
-        rounds[s] += 1;
-        on |= 1u << s;
-      }
-    }
-    return on;
-  }
-
-  // workgroup number n of a tile -> block of samples, block of outputs.  From eight blocks of outputs on, those of an XCD
-  // (n % 8) are next to each other: each L2 holds its own part of the weights.
-  static __host__ __device__ int workgroups(int O, int m_batch) {
-    const int bo = (O + OB - 1) / OB, bb = (m_batch + S - 1) / S;
-    return bo < 8 ? bo * bb : 8 * ((bo + 7) / 8) * bb;
-  }
-  __device__ __forceinline__ bool block_of(int n, int &block_b, int &block_o) const {
-    const int bo = (a.O + OB - 1) / OB;
-    if (bo < 8) {
-      block_o = n % bo;
-      block_b = n / bo;
-    } else {
-      const int per = (bo + 7) / 8, m = n >> 3;
-      block_o = (n & 7) * per + m % per;
-      block_b = m / per;
-    }
-    return block_o < bo && block_b * S < a.m_batch;
-  }
-};
-
-template <bool WOC, int S, int OB, int R>
-__global__ __launch_bounds__(256) void k_mvm_few(MvmArgs a) {
-  extern __shared__ __attribute__((aligned(16))) float few_lds[];
-  __shared__ int hits[2 * R * S];
-  MvmFew<WOC, S, OB, R> f(a, few_lds, hits);
-  int block_b, block_o;
-  if (f.block_of((int)blockIdx.x, block_b, block_o)) f.run(block_b, block_o);
-}
-
-// counters and marks of the tiles of a group, a workgroup for each tile
-__global__ __launch_bounds__(256) void k_mvm_few_clear_group(MvmGroup g) {
-  const MvmArgs &a = g.args[blockIdx.x];
-  if (a.max_rounds < 2) return;
-  for (int i = (int)threadIdx.x; i < 7 * a.m_batch; i += 256) a.few[i] = 0;
-}
-
-// several tiles in one launch: start[t] .. start[t + 1] are the workgroups of tile t
-template <bool WOC, int S, int OB, int R>
-__global__ __launch_bounds__(256) void k_mvm_few_group(MvmGroup g) {
-  extern __shared__ __attribute__((aligned(16))) float few_lds[];
-  __shared__ int hits[2 * R * S];
-  int t = 0;
-  while (t + 1 < g.n && (int)blockIdx.x >= g.start[t + 1]) ++t;
-  const MvmArgs a = g.args[t]; // scalar loads: t is the same for the whole workgroup
-  MvmFew<WOC, S, OB, R> f(a, few_lds, hits);
-  int block_b, block_o;
-  if (f.block_of((int)blockIdx.x - g.start[t], block_b, block_o)) f.run(block_b, block_o);
-}
-
-// ---------------------------------------------------------------------------------------------
 // Convolution forward for a tile of at most 32 outputs, fused: unfold by the index matrix, noise management, DAC,
 // contraction, ADC and the bound-management rounds in one kernel, the result written in the image layout
 // [n][output][patch].  A wave owns 32 consecutive patches; it has all outputs of its patches, so whether a patch
@@ -3392,85 +2853,6 @@ void launch_mvm_round(const MvmArgs &a_in, hipStream_t s) {
   }
 #undef RPU_LAUNCH_ROUND
 }
-
-// Blocks of the largest kind (four samples by 64 outputs) that a call launches for four of its samples
-int mvm_few_blocks(int O) { return MvmFew<false, 4, 64, 1>::workgroups(O, 4); }
-
-// The largest batch whose calls run as k_mvm_few.  A second set of blocks on a CU that holds two doubles the launch: the GPU
-// has to hold all of them at once.  us, the other launches / one, at that line and beyond: 160 -> 100, backward, 600 samples
-// 11.4 / 9.9, 800 11.7 / 15.5; 64 -> 32, 1000 17.0 / 7.8, 3000 16.7 / 17.5, backward 6000 11.5 / 21.7; 64 -> 2048, 64 17.4 /
-// 16.6, 100 18.3 / 23.4; layers of tiles of at most 512 x 512, 768 -> 2304, 24 tokens 52 / 35, 32 28 / 32; 24 tiles of 300 x
-// 300, 16 tokens 33 / 26, 24 33 / 39; 24 of 130 x 125, 64 tokens 28.5 / 32.7 (mvm_few_group_batch).
-// Within it the multiply-adds, weights that saturate round 0 (the last workgroup of a sample runs the rounds from 3 on alone):
-//   forward: 512 x 512, 1 sample 27.5 / 13.3, 50 (13 M) 26.7 / 18.2, 100 26.9 / 26.0, 160 27.7 / 28.5; 1024 x 1024, 24 35.4 /
-//   26.4, 64 36.0 / 37.5; 1500 x 1500, 16 46 / 34, 32 (72 M) 47 / 69; the line is drawn well before the first loss
-//   backward: 512 x 512, 100 14.0 / 10.6, 256 (67 M) 14.3 / 12.2; 1024 x 1024, 64 (67 M) 17.4 / 14.9, 128 17.6 / 17.5; 1500 x
-//   1500, 64 (144 M) 30.0 / 34.6
-int mvm_few_batch(const MvmArgs &a) {
-  const IoDev &io = a.io;
-  const int nm = io.noise_management;
-  if (io.perfect || a.in_index || a.pre_add || a.skip_if_zero || a.nm_phase || a.small_tiles_only || a.K > 2048 || a.K <= a.in_one) return 0;
-  if (nm != RPU_NM_NONE && nm != RPU_NM_CONSTANT && nm != RPU_NM_ABS_MAX && nm != RPU_NM_MAX) return 0;
-  if (io.bound_management != RPU_BM_NONE && (io.bound_management != RPU_BM_ITERATIVE || a.transposed)) return 0;
-  const long per_cu = a.max_rounds > 1 ? 51200 : 262144; // multiply-adds
-  // (a sample takes a load of 64 inputs by 16 outputs at least: a long batch on a tiny tile is not a small call)
-  const long most = per_cu * cus_of(a) / ((long)((a.K + 63) & ~63) * ((a.O + 15) & ~15));
-  return (int)std::min(most, 4L * (2 * cus_of(a) / mvm_few_blocks(a.O)));
-}
-// The same for a group of tiles whose calls have `blocks` blocks for four samples, all tiles taken together.
-int mvm_few_group_batch(long blocks) { return (int)(4 * (2L * current_device_cus() / blocks)); }
-// the variant of a launch of such calls: the smallest blocks of samples and outputs with at most two workgroups to a CU
-int mvm_few_variant(const MvmArgs *const *calls, int n) {
-  for (int v = 0; v < 3; ++v) {
-    long workgroups = 0;
-    for (int i = 0; i < n; ++i) workgroups += mvm_few_workgroups(*calls[i], v);
-    if (workgroups <= 2L * current_device_cus()) return v;
-  }
-  return 3;
-}
-
-#define RPU_FEW_VARIANT(variant, CALL) \
-  switch (variant) { \
-  case 0: CALL(1, 16); break; \
-  case 1: CALL(2, 32); break; \
-  case 2: CALL(4, 32); break; \
-  default: CALL(4, 64); break; \
-  }
-
-int mvm_few_workgroups(const MvmArgs &a, int variant) {
-#define RPU_FEW_COUNT(S, OB) return MvmFew<false, S, OB, 1>::workgroups(a.O, a.m_batch)
-  RPU_FEW_VARIANT(variant, RPU_FEW_COUNT)
-#undef RPU_FEW_COUNT
-}
-
-#define RPU_LAUNCH_FEW_AS(KERNEL, ARGS, K, W_OC, ROUNDS, S, OB) \
-  if (W_OC) { \
-    if (ROUNDS == 3) hipLaunchKernelGGL((KERNEL<true, S, OB, 3>), grid, dim3(256), (MvmFew<true, S, OB, 3>::lds_bytes(K)), s, ARGS); \
-    else hipLaunchKernelGGL((KERNEL<true, S, OB, 1>), grid, dim3(256), (MvmFew<true, S, OB, 1>::lds_bytes(K)), s, ARGS); \
-  } else { \
-    if (ROUNDS == 3) hipLaunchKernelGGL((KERNEL<false, S, OB, 3>), grid, dim3(256), (MvmFew<false, S, OB, 3>::lds_bytes(K)), s, ARGS); \
-    else hipLaunchKernelGGL((KERNEL<false, S, OB, 1>), grid, dim3(256), (MvmFew<false, S, OB, 1>::lds_bytes(K)), s, ARGS); \
-  }
-
-void launch_mvm_few(const MvmArgs &a, int variant, int rounds, hipStream_t s) {
-  const dim3 grid((unsigned)mvm_few_workgroups(a, variant));
-#define RPU_LAUNCH_FEW(S, OB) RPU_LAUNCH_FEW_AS(k_mvm_few, a, a.K, a.w_oc, rounds, S, OB)
-  RPU_FEW_VARIANT(variant, RPU_LAUNCH_FEW)
-#undef RPU_LAUNCH_FEW
-}
-
-void launch_mvm_few_clear_group(const MvmGroup &g, hipStream_t s) {
-  hipLaunchKernelGGL(k_mvm_few_clear_group, dim3((unsigned)g.n), dim3(256), 0, s, g);
-}
-
-void launch_mvm_few_group(const MvmGroup &g, int variant, int rounds, bool w_oc, int max_k, int total_workgroups, hipStream_t s) {
-  const dim3 grid((unsigned)total_workgroups);
-#define RPU_LAUNCH_FEW(S, OB) RPU_LAUNCH_FEW_AS(k_mvm_few_group, g, max_k, w_oc, rounds, S, OB)
-  RPU_FEW_VARIANT(variant, RPU_LAUNCH_FEW)
-#undef RPU_LAUNCH_FEW
-}
-#undef RPU_LAUNCH_FEW_AS
-#undef RPU_FEW_VARIANT
 
 bool conv_forward_supported(const MvmArgs &a) {
   if (a.O > 32 || a.transposed) return false;

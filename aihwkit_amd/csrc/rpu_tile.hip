@@ -743,7 +743,8 @@ struct Tile {
     a.few = s_count.p + MVM_COUNT_WORDS;
     a.few_seen = seen_dev;
     a.few_call = call_number;
-    if (a.max_rounds < 3) return 1;
+    // (the launch takes the inputs of rounds 1 and 2 as halves of those of round 0 before the clipping)
+    if (a.max_rounds < 3 || !(a.io.inp_bound < 0x1p96f)) return 1;
     a.dual.buf[1] = a.xq[0];
     a.dual.buf[2] = a.xq[1];
     if (fused_rounds >= 0) return fused_rounds & 1 ? 3 : 1;
@@ -3133,11 +3134,13 @@ static int group_mvm(rpu_group_t *group, const float *const *x_dev, const long *
     std::vector<const MvmArgs *> few_calls;
     while ((int)few_calls.size() < n && few[order[few_calls.size()]]) few_calls.push_back(&args[order[few_calls.size()]]);
     const int n_few = (int)few_calls.size(), few_variant = mvm_few_variant(few_calls.data(), n_few);
+    bool few_stoch = false;
     int few_workgroups = 0, few_max_k = 0, few_together = 3; // a launch has one form; the buffers of three rounds serve one
     for (int i = 0; i < n_few; ++i) {
       table[cursor++] = few_workgroups;
       few_workgroups += mvm_few_workgroups(*few_calls[i], few_variant);
       few_max_k = std::max(few_max_k, few_calls[i]->K);
+      few_stoch = few_stoch || mvm_few_stoch(*few_calls[i]);
       few_together = std::min(few_together, few_rounds[order[i]]);
     }
     if (n_few) table[cursor++] = few_workgroups;
@@ -3176,7 +3179,7 @@ static int group_mvm(rpu_group_t *group, const float *const *x_dev, const long *
           for (int i = 0; i < n_few; ++i) group->tiles[order[i]]->t.few_cleared(args[order[i]]);
         }
       }
-      launch_mvm_few_group(g, few_variant, few_together, transposed != storage_xd, few_max_k, few_workgroups, s);
+      launch_mvm_few_group(g, few_variant, few_together, transposed != storage_xd, few_stoch, few_max_k, few_workgroups, s);
     }
     if (n_few == n) { // says nothing about the launches that the pairs choose
       RPU_HIP_CHECK(hipGetLastError());
