@@ -201,6 +201,11 @@ void launch_mvm_few(const MvmArgs &a, int variant, int rounds, hipStream_t s);
 void launch_mvm_few_clear_group(const MvmGroup &g, hipStream_t s); // the counters of its calls
 bool mvm_few_stoch(const MvmArgs &a); // whether the converters draw random numbers beyond the output noise
 void launch_mvm_few_group(const MvmGroup &g, int variant, int rounds, bool w_oc, bool stoch, int max_k, int total_workgroups, hipStream_t s);
+// Calls between those and the large tiles, also in one launch (k_mvm_whole), with the bits of the launches one by one.
+// outputs: of a workgroup, mvm_whole_outputs(), 0 where a call does not take that launch; the rest as for k_mvm_few.
+int mvm_whole_outputs(const MvmArgs &a);
+int mvm_whole_batch(const MvmArgs &a); // at least the largest batch whose calls take it
+void launch_mvm_whole(const MvmArgs &a, int outputs, int rounds, hipStream_t s);
 
 // Fused convolution forward (unfold + noisy MVM with its bound-management rounds) for tiles of at most 32 outputs:
 // images [n_images][image_size], idx_t the transposed index matrix [patches][x_size], out [n_images][d_size][patches].

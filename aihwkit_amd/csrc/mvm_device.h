@@ -5,6 +5,16 @@
 namespace rpu_amd {
 namespace {
 
+// lane i: the value of lane i ^ off, within rows of 16 lanes, where the values of lanes i and i ^ (2 off) (and above, in the
+// row) are the same already: a butterfly that starts with the largest offset
+template <int OFF> __device__ __forceinline__ float row_xor(float v) {
+  static_assert(OFF == 8 || OFF == 4 || OFF == 2 || OFF == 1);
+  constexpr int CTRL = OFF == 8 ? 0x128 : (OFF == 4 ? 0x124 : (OFF == 2 ? 0x4e : 0xb1)); // row_ror:8, row_ror:4, quad_perm
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, false));
+}
+
+__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+
 // STOCH = false: for callers that have checked that the DAC draws no random numbers (no stochastic rounding, no input
 // noise): the draws are then not even compiled in, which the fully unrolled callers pay for in registers
 template <bool STOCH = true>

@@ -728,8 +728,10 @@ struct Tile {
     a.O = D;
     a.io = io_dev(fio);
     a.max_rounds = fio.perfect ? 0 : mvm_max_rounds(a.io);
-    s_count.ensure(MVM_COUNT_WORDS + (a.max_rounds > 1 ? 7 * (size_t)mvm_few_batch(a) : 0));
+    s_count.ensure(MVM_COUNT_WORDS + (a.max_rounds > 1 ? 7 * (size_t)one_launch_batch(a) : 0));
   }
+  // the largest batch that may need what few_args sets up
+  static int one_launch_batch(const MvmArgs &a) { return std::max(mvm_few_batch(a), mvm_whole_batch(a)); }
   // `clear`: set where the counters of the call have to be cleared first (few_cleared)
   int few_args(MvmArgs &a, int call_number, const volatile int *seen_host, int *seen_dev, bool &clear) {
     if (a.max_rounds < 2) return 1;
@@ -807,7 +809,7 @@ struct Tile {
     a.k_pad = mvm_k_pad(K, tight);
     a.max_rounds = io.perfect ? 0 : mvm_max_rounds(a.io);
     size_t rows = (size_t)B * a.k_pad;
-    if (a.max_rounds > 2) rows = std::max(rows, (size_t)std::min(B, mvm_few_batch(a)) * O); // see few_args
+    if (a.max_rounds > 2) rows = std::max(rows, (size_t)std::min(B, one_launch_batch(a)) * O); // see few_args
     if (!io.perfect) s_xq0.ensure(rows); // (of exact calls: ensure_exact)
     if (!io.perfect && io.p.bound_management != RPU_BM_NONE) s_xq1.ensure(rows);
     a.xq[0] = s_xq0.p; a.xq[1] = s_xq1.p;
@@ -1105,7 +1107,12 @@ struct Tile {
     const bool running = io.p.noise_management == RPU_NM_AVERAGE_ABS_MAX || io.p.noise_management == RPU_NM_AVERAGE_ABS_MAX_SINGLE_VALUE;
     const int few_batch = side || gather || running ? 0 : small_call_batch(a);
     if (few_batch > 0 && a.max_rounds > 1) ensure_seen(); // by a larger call too: a small one after it may be captured
-    if (B <= few_batch && !writes_into_its_input(a)) {
+    const bool few = B <= few_batch;
+    // (the hooks of tests are about the other launches)
+    const bool other_launches = !small_calls || fused_rounds >= 0 || wait_spins_hook || wait_extra_hook;
+    const int whole = few || side || gather || running || other_launches ? 0 : mvm_whole_outputs(a);
+    if (whole && a.max_rounds > 1) ensure_seen();
+    if ((few || whole) && !writes_into_its_input(a)) {
       bool clear = false;
       const int together = a.max_rounds > 1 ? few_args(a, few_calls++, seen_host + 4, seen_dev + 4, clear) : 1;
       if (clear) {
@@ -1113,8 +1120,9 @@ struct Tile {
         if (runs_now(s)) few_cleared(a);
       }
       const MvmArgs *call = &a;
-      launch_mvm_few(a, mvm_few_variant(&call, 1), together, s);
-      prof_mark(s, "mvm_few");
+      if (few) launch_mvm_few(a, mvm_few_variant(&call, 1), together, s);
+      else launch_mvm_whole(a, whole, together, s);
+      prof_mark(s, few ? "mvm_few" : "mvm_whole");
     } else if (io.perfect) {
       a.round = 0;
       exact_product(a, false, s, "mvm_init", "mvm_round");
