@@ -809,7 +809,7 @@ struct Tile {
     a.k_pad = mvm_k_pad(K, tight);
     a.max_rounds = io.perfect ? 0 : mvm_max_rounds(a.io);
     size_t rows = (size_t)B * a.k_pad;
-    if (a.max_rounds > 2) rows = std::max(rows, (size_t)std::min(B, one_launch_batch(a)) * O); // see few_args
+    if (a.max_rounds > 2) rows = std::max(rows, (size_t)std::min(B, mvm_few_batch(a)) * O); // see few_args
     if (!io.perfect) s_xq0.ensure(rows); // (of exact calls: ensure_exact)
     if (!io.perfect && io.p.bound_management != RPU_BM_NONE) s_xq1.ensure(rows);
     a.xq[0] = s_xq0.p; a.xq[1] = s_xq1.p;
@@ -1114,7 +1114,17 @@ struct Tile {
     if (whole && a.max_rounds > 1) ensure_seen();
     if ((few || whole) && !writes_into_its_input(a)) {
       bool clear = false;
-      const int together = a.max_rounds > 1 ? few_args(a, few_calls++, seen_host + 4, seen_dev + 4, clear) : 1;
+      int together = a.max_rounds > 1 ? few_args(a, few_calls++, seen_host + 4, seen_dev + 4, clear) : 1;
+      const size_t results = (size_t)B * a.O;
+      if (whole && together > 1 && (s_xq0.n < results || s_xq1.n < results)) {
+        // where the fused launches keep theirs; the tile's first call and captured ones make no room and work out one round
+        if ((s_dual1.n < results || s_dual2.n < results) && (few_calls == 1 || !runs_now(s))) {
+          together = 1;
+        } else {
+          s_dual1.ensure(results); s_dual2.ensure(results);
+          a.dual.buf[1] = s_dual1.p; a.dual.buf[2] = s_dual2.p;
+        }
+      }
       if (clear) {
         launch_fill(reinterpret_cast<float *>(a.few), 0.0f, 7 * (size_t)B, s); // all-zero bits
         if (runs_now(s)) few_cleared(a);

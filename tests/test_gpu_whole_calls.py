@@ -140,14 +140,18 @@ def test_rows_that_are_not_finite_stay_to_themselves(gpu_device):
     assert bool(torch.isfinite(y[:, keep]).all()) and torch.equal(y[:, keep], y_other[:, keep])
 
 
-def test_captured_after_a_larger_call(gpu_device):
-    """Scratch is there after a larger call; replays, with eager calls between them, find counters and marks as they have to be."""
+@pytest.mark.parametrize("warm", [False, True])
+def test_captured_after_a_larger_call(gpu_device, warm):
+    """The captured call makes no room, whether or not a call before it has (round by round, or three together); replays, with eager
+    calls between them, find counters and marks as they have to be."""
     rng = np.random.default_rng(8)
     host = host_tile(rng, 300, 512, 2.0)
     gpu, other = pair_of(host)
     for tile in (gpu, other):
         tile.forward(torch.zeros(4096, 300, device="cuda"), False)
     x_dev = torch.zeros(140, 300, device="cuda")
+    if warm:
+        gpu.forward(x_dev, False)
     torch.cuda.synchronize()
     before = lib().rpu_device_allocation_count()
     state = gpu.dump_extra()
@@ -156,7 +160,7 @@ def test_captured_after_a_larger_call(gpu_device):
         y_dev = gpu.forward(x_dev, False, False, False, False, True)
     for replay in range(4):
         x = torch.from_numpy(rng.uniform(-1, 1, (140, 300)).astype(np.float32)).cuda()
-        if replay % 2:
+        if replay % 2 and warm:
             gpu.forward(x[:100], False)
         x_dev.copy_(x)
         graph.replay()
