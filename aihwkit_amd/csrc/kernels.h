@@ -200,7 +200,17 @@ int mvm_few_workgroups(const MvmArgs &a, int variant);
 void launch_mvm_few(const MvmArgs &a, int variant, int rounds, hipStream_t s);
 void launch_mvm_few_clear_group(const MvmGroup &g, hipStream_t s); // the counters of its calls
 bool mvm_few_stoch(const MvmArgs &a); // whether the converters draw random numbers beyond the output noise
-void launch_mvm_few_group(const MvmGroup &g, int variant, int rounds, bool w_oc, bool stoch, int max_k, int total_workgroups, hipStream_t s);
+// What differs from one call of a group to the next, in the launch's own arguments: the argument blocks in HBM can then stay as
+// they are (count: tiles; 0: the blocks hold these values too)
+struct MvmFewCalls {
+  static constexpr int MOST = 64;
+  int count, few_call;
+  const float *in[MOST];
+  float *out[MOST];
+  uint32_t call[MOST];
+};
+void launch_mvm_few_group(const MvmGroup &g, const MvmFewCalls &calls, int variant, int rounds, bool w_oc, bool stoch, int max_k,
+                          int total_workgroups, hipStream_t s);
 // Calls between those and the large tiles, also in one launch (k_mvm_whole), with the bits of the launches one by one.
 // outputs: of a workgroup, mvm_whole_outputs(), 0 where a call does not take that launch; the rest as for k_mvm_few.
 int mvm_whole_outputs(const MvmArgs &a);

@@ -534,9 +534,15 @@ __global__ __launch_bounds__(256) void k_mvm_few_clear_group(MvmGroup g) {
   for (int i = (int)threadIdx.x; i < 7 * a.m_batch; i += 256) a.few[i] = 0;
 }
 
+struct MvmFewGroup {
+  MvmGroup group;
+  MvmFewCalls calls;
+};
+
 // several tiles in one launch: start[t] .. start[t + 1] are the workgroups of tile t
 template <bool WOC, int S, int OB, int R, bool STOCH>
-__global__ __launch_bounds__(256, 2) void k_mvm_few_group(MvmGroup g) {
+__global__ __launch_bounds__(256, 2) void k_mvm_few_group(MvmFewGroup launch) {
+  const MvmGroup &g = launch.group;
   extern __shared__ __attribute__((aligned(16))) float few_lds[];
   __shared__ FewShared sh;
   typedef MvmFew<WOC, S, OB, R, STOCH> Few;
@@ -549,7 +555,13 @@ __global__ __launch_bounds__(256, 2) void k_mvm_few_group(MvmGroup g) {
     if (before != ~0ull) break;
   }
   t = uniform(t);
-  const MvmArgs a = g.args[t]; // scalar loads: t is the same for the whole workgroup
+  MvmArgs a = g.args[t]; // scalar loads: t is the same for the whole workgroup
+  if (launch.calls.count > 0) {
+    a.in = launch.calls.in[t];
+    a.out = launch.calls.out[t];
+    a.call = launch.calls.call[t];
+    a.few_call = launch.calls.few_call;
+  }
   int block_b, block_o;
   if (Few::block_of(a, (int)blockIdx.x - g.start[t], block_b, block_o)) Few(a, few_lds, sh).run(block_b, block_o);
 }
@@ -639,10 +651,12 @@ void launch_mvm_few_clear_group(const MvmGroup &g, hipStream_t s) {
   hipLaunchKernelGGL(k_mvm_few_clear_group, dim3((unsigned)g.n), dim3(256), 0, s, g);
 }
 
-void launch_mvm_few_group(const MvmGroup &g, int variant, int rounds, bool w_oc, bool stoch, int max_k, int total_workgroups, hipStream_t s) {
+void launch_mvm_few_group(const MvmGroup &g, const MvmFewCalls &calls, int variant, int rounds, bool w_oc, bool stoch, int max_k,
+                          int total_workgroups, hipStream_t s) {
+  const MvmFewGroup launch{g, calls};
   const dim3 grid((unsigned)total_workgroups);
-#define RPU_LAUNCH_FEW(S, OB) RPU_LAUNCH_FEW_AS(k_mvm_few_group, g, max_k, w_oc, rounds, false, S, OB)
-#define RPU_LAUNCH_FEW_STOCH(S, OB) RPU_LAUNCH_FEW_AS(k_mvm_few_group, g, max_k, w_oc, rounds, true, S, OB)
+#define RPU_LAUNCH_FEW(S, OB) RPU_LAUNCH_FEW_AS(k_mvm_few_group, launch, max_k, w_oc, rounds, false, S, OB)
+#define RPU_LAUNCH_FEW_STOCH(S, OB) RPU_LAUNCH_FEW_AS(k_mvm_few_group, launch, max_k, w_oc, rounds, true, S, OB)
   if (stoch) {
     RPU_FEW_VARIANT(variant, RPU_LAUNCH_FEW_STOCH)
   } else {

@@ -114,7 +114,8 @@ template <class A> struct GroupArgs {
   A *args() { return reinterpret_cast<A *>(host + 8 * table_words); }
   const int *dev_table() const { return reinterpret_cast<const int *>(dev.p); }
   const A *dev_args() const { return reinterpret_cast<const A *>(dev.p + table_words); }
-  void upload(size_t n_args, hipStream_t s) { launch_upload(dev.p, host_on_dev, table_words + n_args * (sizeof(A) / 8), s); }
+  size_t words(size_t n_args) const { return table_words + n_args * (sizeof(A) / 8); }
+  void upload(size_t n_args, hipStream_t s) { launch_upload(dev.p, host_on_dev, words(n_args), s); }
   void release() {
     if (host) (void)hipHostFree(host);
     host = host_on_dev = nullptr;
@@ -2724,6 +2725,10 @@ struct rpu_group {
   std::vector<rpu_tile *> tiles;
   int device_id = -1;
   GroupArgs<MvmArgs> mvm_args;
+  // Table and argument blocks of the call that is being put together, and those that lie in HBM (empty: others).  Calls that take
+  // the one launch of small batches hand it what differs from call to call (MvmFewCalls; zeros here) and upload the rest only
+  // when it has changed: the upload reads host memory, 3 us and a gap before each launch of 8 to 15.
+  std::vector<unsigned long long> next_args, uploaded_args;
   hipEvent_t copied = nullptr;
   int few_calls = 0; // see Tile::few_args
   Places inputs; // of the last call, kept for its memory
@@ -3147,7 +3152,8 @@ static int group_mvm(rpu_group_t *group, const float *const *x_dev, const long *
     });
     struct Segment { int first, count, depth, mode, start_offset, workgroups; };
     std::vector<Segment> segments;
-    int *const table = group->mvm_args.table();
+    group->next_args.assign(group->mvm_args.words((size_t)n), 0);
+    int *const table = reinterpret_cast<int *>(group->next_args.data());
     int cursor = 0; // position in the table
     std::vector<const MvmArgs *> few_calls;
     while ((int)few_calls.size() < n && few[order[few_calls.size()]]) few_calls.push_back(&args[order[few_calls.size()]]);
@@ -3185,9 +3191,28 @@ static int group_mvm(rpu_group_t *group, const float *const *x_dev, const long *
       }
       table[cursor++] = wg;
     }
-    for (int i = 0; i < n; ++i) group->mvm_args.args()[i] = args[order[i]];
-    group->mvm_args.upload((size_t)n, s);
-    RPU_HIP_CHECK(hipEventRecord(group->copied, s));
+    MvmFewCalls calls{};
+    const bool now = Tile::runs_now(s); // (a replay uploads what the pinned memory holds then, and reads no other values)
+    if (n_few == n && n <= MvmFewCalls::MOST && now) {
+      calls.count = n;
+      calls.few_call = group->few_calls;
+    }
+    MvmArgs *const blocks = reinterpret_cast<MvmArgs *>(group->next_args.data() + group->mvm_args.table_words);
+    for (int i = 0; i < n; ++i) {
+      std::memcpy((void *)&blocks[i], (const void *)&args[order[i]], sizeof(MvmArgs));
+      if (calls.count == 0) continue;
+      MvmArgs &a = blocks[i];
+      calls.in[i] = a.in; calls.out[i] = a.out; calls.call[i] = a.call;
+      a.in = nullptr; a.out = nullptr; a.call = 0; a.few_call = 0;
+    }
+    if (calls.count == 0 || group->next_args != group->uploaded_args) {
+      group->uploaded_args.clear();
+      std::memcpy(group->mvm_args.table(), group->next_args.data(), 8 * group->mvm_args.table_words);
+      for (int i = 0; i < n; ++i) group->mvm_args.args()[i] = args[order[i]];
+      group->mvm_args.upload((size_t)n, s);
+      RPU_HIP_CHECK(hipEventRecord(group->copied, s));
+      if (calls.count > 0) group->uploaded_args.swap(group->next_args);
+    }
 
     if (n_few) {
       MvmGroup g{group->mvm_args.dev_args(), group->mvm_args.dev_table(), n_few, m_batch};
@@ -3197,7 +3222,7 @@ static int group_mvm(rpu_group_t *group, const float *const *x_dev, const long *
           for (int i = 0; i < n_few; ++i) group->tiles[order[i]]->t.few_cleared(args[order[i]]);
         }
       }
-      launch_mvm_few_group(g, few_variant, few_together, transposed != storage_xd, few_stoch, few_max_k, few_workgroups, s);
+      launch_mvm_few_group(g, calls, few_variant, few_together, transposed != storage_xd, few_stoch, few_max_k, few_workgroups, s);
     }
     if (n_few == n) { // says nothing about the launches that the pairs choose
       RPU_HIP_CHECK(hipGetLastError());
