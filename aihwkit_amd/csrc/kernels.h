@@ -127,7 +127,9 @@ struct MvmArgs {
   int in_group;
   long in_gs;
   int *few;      // calls of k_mvm_few: [7][m_batch] counters and saturation marks, zero between calls
-  int *few_seen; // host-visible: few_call of the last call in which a sample needed a second round, and of the last call
+  // host-visible: few_call of the last call in which a sample needed a second round, and of the last call; k_mvm_whole: behind them
+  // 1 + few_call of the last one in which a sample went beyond MVM_WHOLE_ROUNDS
+  int *few_seen;
   int few_call;
   int cus; // compute units of the tile's GPU: the rules of a launch ask for them several times (a query of the runtime each)
 };
@@ -213,6 +215,7 @@ void launch_mvm_few_group(const MvmGroup &g, const MvmFewCalls &calls, int varia
                           int total_workgroups, hipStream_t s);
 // Calls between those and the large tiles, also in one launch (k_mvm_whole), with the bits of the launches one by one.
 // outputs: of a workgroup, mvm_whole_outputs(), 0 where a call does not take that launch; the rest as for k_mvm_few.
+constexpr int MVM_WHOLE_ROUNDS = 3; // that such a call works out together
 int mvm_whole_outputs(const MvmArgs &a);
 int mvm_whole_batch(const MvmArgs &a); // at least the largest batch whose calls take it
 void launch_mvm_whole(const MvmArgs &a, int outputs, int rounds, hipStream_t s);

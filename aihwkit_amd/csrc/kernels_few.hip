@@ -15,6 +15,8 @@
 // the clock between them, on the version before).  So the random draws of the converters are compiled in only where
 // the settings have them (STOCH), a thread works on one sample's row and not on all, loads have no branches (buffer
 // loads: what lies beyond the matrix reads as zero) and what few calls need stands at the end.
+// One sample on 512 x 512 8.8 -> 7.8 us a launch, 12 tiles of 512 x 512 with 8 samples 17.2 -> 10.1, 785 x 300 with 37 samples and
+// three rounds 23.2 -> 16.8, backward 16.6 -> 7.0, 129 x 10 with 64 samples 9.3 -> 5.6.
 // The streams of random numbers are those of the other kernels (element k, sample, round; four outputs to a draw).
 #include "bf16_parts.h"
 #include "mvm_device.h"
@@ -581,11 +583,15 @@ int mvm_few_blocks(int O) { return MvmFew<false, 4, 64, 1, false>::workgroups(O,
 // 11.4 / 9.9, 800 11.7 / 15.5; 64 -> 32, 1000 17.0 / 7.8, 3000 16.7 / 17.5, backward 6000 11.5 / 21.7; 64 -> 2048, 64 17.4 /
 // 16.6, 100 18.3 / 23.4; layers of tiles of at most 512 x 512, 768 -> 2304, 24 tokens 52 / 35, 32 28 / 32; 24 tiles of 300 x
 // 300, 16 tokens 33 / 26, 24 33 / 39; 24 of 130 x 125, 64 tokens 28.5 / 32.7 (mvm_few_group_batch).
-// Within it the multiply-adds, weights that saturate round 0 (the last workgroup of a sample runs the rounds from 3 on alone):
-//   forward: 512 x 512, 1 sample 27.5 / 13.3, 50 (13 M) 26.7 / 18.2, 100 26.9 / 26.0, 160 27.7 / 28.5; 1024 x 1024, 24 35.4 /
-//   26.4, 64 36.0 / 37.5; 1500 x 1500, 16 46 / 34, 32 (72 M) 47 / 69; the line is drawn well before the first loss
-//   backward: 512 x 512, 100 14.0 / 10.6, 256 (67 M) 14.3 / 12.2; 1024 x 1024, 64 (67 M) 17.4 / 14.9, 128 17.6 / 17.5; 1500 x
-//   1500, 64 (144 M) 30.0 / 34.6
+// (Measured on the kernel as it was with branches and all draws; this one is faster, the line is where it was: a call on this
+// side of it adds in another order than one beyond.)
+// Within it the multiply-adds: on either side of the line the launches cost the same.  The last samples here, the launches one
+// by one / this one, and one sample more on k_mvm_whole:
+//   forward, no saturation: 512 x 512, 50 (13 M) 18.1 / 9.6, 9.8; 1024 x 1024, 12 20.8 / 10.3, 11.9; 1500 x 1500, 5 28.1 / 12.9,
+//   14.2; 785 x 300, 51 26.9 / 10.0, 11.2; 160 -> 100, 609 16.9 / 7.5, 9.0; 64 -> 32, 2048 15.3 / 5.7, 7.9
+//   every sample in round 3 or later, which the last workgroup of a sample runs alone: 512 x 512, 50 70 / 54; 785 x 300, 51 108 /
+//   45; 160 -> 100, 609 65 / 26; but 1024 x 1024, 12 64 / 87; 1500 x 1500, 5 82 / 205
+//   backward: 512 x 512, 256 (67 M) 14.6 / 8.4, 9.3; 1024 x 1024, 64 17.6 / 11.0, 12.2; 1500 x 1500, 29 29.4 / 15.1, 12.3
 int mvm_few_batch(const MvmArgs &a) {
   const IoDev &io = a.io;
   const int nm = io.noise_management;

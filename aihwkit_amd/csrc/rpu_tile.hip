@@ -320,6 +320,7 @@ struct Tile {
   DevBuf<float> s_dual0, s_dual1, s_dual2, s_xq2;
   DevBuf<int> s_dsel, s_dhit1, s_dhit2;
   int few_calls = 0; // see few_args
+  int beyond_call = 0, beyond_calls = 0; // see rounds_beyond
   size_t few_zero = 0; // words for k_mvm_few that are zero between calls
   bool small_calls = true; // rpu_tile_set_small_calls
   // largest batch that the groups of this tile run as k_mvm_few, forward and backward: so does the tile in calls of its own,
@@ -775,11 +776,28 @@ struct Tile {
     p.add(in);
     return p.meets(out);
   }
-  // words 0 to 3: the launches of the rounds, 4 and 5: few_args
+  // Whether forward calls that could take k_mvm_whole keep to the other launches, with the same bits: a sample of one of the recent
+  // calls went beyond the rounds that are worked out together.  A workgroup runs those alone, all outputs of its samples one after
+  // the other.  us, the other launches / the one, every sample in round 3 or later: 512 x 512, 100 samples 71 / 138; 1024 x 1024, 24
+  // 85 / 361; 1500 x 1500, 10 86 / 544; 64 -> 1024, 129 59 / 139; but 160 -> 100, 1218 67 / 42, 64 -> 32, 4096 91 / 25: matrices of up
+  // to 2^14 weights stay.  Such a call sends the next 64 to the other launches, which say
+  // for themselves when a sample needs those rounds again (a call without any is 10 to 30 us slower on them).
+  bool rounds_beyond(bool reports) {
+    const volatile int *const seen = seen_host;
+    if (seen[6] != beyond_call) {
+      beyond_call = seen[6];
+      beyond_calls = 64;
+    } else if (beyond_calls > 0) {
+      if (beyond_calls < 64 && reports && seen[1] > 0 && seen[2] >= 3) beyond_calls = 64;
+      --beyond_calls;
+    }
+    return beyond_calls > 0;
+  }
+  // words 0 to 3: the launches of the rounds, 4 and 5: few_args, 6: the last call on k_mvm_whole with a sample in round 3 or later
   void ensure_seen() {
     if (seen_dev) return; // the last step
-    if (!seen_host) RPU_HIP_CHECK(hipHostMalloc((void **)&seen_host, 6 * sizeof(int), hipHostMallocMapped));
-    for (int i = 0; i < 6; ++i) seen_host[i] = 0; // until the first calls say otherwise
+    if (!seen_host) RPU_HIP_CHECK(hipHostMalloc((void **)&seen_host, 7 * sizeof(int), hipHostMallocMapped));
+    for (int i = 0; i < 7; ++i) seen_host[i] = 0; // until the first calls say otherwise
     RPU_HIP_CHECK(hipHostGetDevicePointer((void **)&seen_dev, seen_host, 0));
   }
 
@@ -1111,21 +1129,26 @@ struct Tile {
     const bool few = B <= few_batch;
     // (the hooks of tests are about the other launches)
     const bool other_launches = !small_calls || fused_rounds >= 0 || wait_spins_hook || wait_extra_hook;
-    const int whole = few || side || gather || running || other_launches ? 0 : mvm_whole_outputs(a);
+    int whole = few || side || gather || running || other_launches ? 0 : mvm_whole_outputs(a);
     if (whole && a.max_rounds > 1) ensure_seen();
-    if ((few || whole) && !writes_into_its_input(a)) {
-      bool clear = false;
-      int together = a.max_rounds > 1 ? few_args(a, few_calls++, seen_host + 4, seen_dev + 4, clear) : 1;
-      const size_t results = (size_t)B * a.O;
-      if (whole && together > 1 && (s_xq0.n < results || s_xq1.n < results)) {
-        // where the fused launches keep theirs; the tile's first call and captured ones make no room and work out one round
-        if ((s_dual1.n < results || s_dual2.n < results) && (few_calls == 1 || !runs_now(s))) {
-          together = 1;
-        } else {
-          s_dual1.ensure(results); s_dual2.ensure(results);
-          a.dual.buf[1] = s_dual1.p; a.dual.buf[2] = s_dual2.p;
-        }
+    if (whole && a.max_rounds > MVM_WHOLE_ROUNDS && (long)a.K * a.O > 1L << 14 && rounds_beyond(!w_other)) whole = 0;
+    bool clear = false;
+    int together = 1;
+    const bool one_launch = (few || whole) && !writes_into_its_input(a);
+    if (one_launch && a.max_rounds > 1) together = few_args(a, few_calls++, seen_host + 4, seen_dev + 4, clear);
+    const size_t results = (size_t)B * a.O;
+    if (one_launch && whole && together > 1 && (s_xq0.n < results || s_xq1.n < results)) {
+      // where the fused launches keep theirs; the tile's first call and captured ones make no room, and one round in the launch
+      // would leave the others to workgroups alone (rounds_beyond)
+      if ((s_dual1.n < results || s_dual2.n < results) && (few_calls == 1 || !runs_now(s))) {
+        whole = 0;
+        a.dual.buf[1] = a.dual.buf[2] = nullptr;
+      } else {
+        s_dual1.ensure(results); s_dual2.ensure(results);
+        a.dual.buf[1] = s_dual1.p; a.dual.buf[2] = s_dual2.p;
       }
+    }
+    if (one_launch && (few || whole)) {
       if (clear) {
         launch_fill(reinterpret_cast<float *>(a.few), 0.0f, 7 * (size_t)B, s); // all-zero bits
         if (runs_now(s)) few_cleared(a);
@@ -1159,7 +1182,11 @@ struct Tile {
         a.dual.seen = seen_dev;
         const int needed = *(volatile int *)&seen_host[0], of = *(volatile int *)&seen_host[1];
         const int last_listed = *(volatile int *)&seen_host[2];
-        fuse = mvm_can_fuse_rounds(a) &&
+        // (a captured call makes no room; after calls in one launch it may be the first of its size here)
+        const bool room = s_dual0.n >= results && s_dual1.n >= results && s_xq2.n >= (size_t)B * a.k_pad && s_dsel.n >= (size_t)B &&
+                          s_dhit1.n >= 2 * (size_t)B;
+        const bool room_for_3 = s_dual2.n >= results && s_dhit2.n >= 2 * (size_t)B;
+        fuse = mvm_can_fuse_rounds(a) && (room || few_calls == 0 || runs_now(s)) &&
                ((fused_rounds > 0 && (fused_rounds & 1)) || (fused_rounds < 0 && of > 0 && 2 * (long)needed > of));
         // The last round that listed samples in the recent calls is expected to be the last one of this call too: the
         // rounds after it share a launch, whose workgroups find the first of their lists empty and leave.  The
@@ -1177,6 +1204,7 @@ struct Tile {
         }
         // a third round in the fused launch costs half of what its own launch does, even for a few samples
         if (fuse) fused = (a.max_rounds >= 4 && ((fused_rounds > 0 && (fused_rounds & 4)) || (fused_rounds < 0 && rest_from >= 2))) ? 3 : 2;
+        if (fused == 3 && !room_for_3 && few_calls > 0 && !runs_now(s)) fused = 2;
         const int first_mergeable = fuse ? fused : 1;
         if (!merged_off && mvm_can_merge_rest(a, mvm_rest_resident_limit(a))) {
           if (fused_rounds > 0 && (fused_rounds & 2)) merge_from = first_mergeable;
