@@ -241,8 +241,11 @@ def main() -> int:
         return out
 
     def contraction(prof):
-        # (ms, launches) of a call's contraction: its round launches, or the one launch that runs a small batch
-        return prof["mvm_few"] if "mvm_few" in prof else prof["mvm_round"]
+        # (ms, launches) of a call's contraction: its round launches, or the one launch that runs a small or medium batch
+        return prof[next(k for k in ("mvm_few", "mvm_whole", "mvm_round") if k in prof)]
+
+    def one_launch(prof):
+        return next(("k_%s (whole call)" % k for k in ("mvm_few", "mvm_whole") if k in prof), None)
 
     def pulse_loop(prof):
         # (kernel, ms) of the pulse loop of an update call: its plain form, the one on lane masks, the pipelined one
@@ -250,7 +253,7 @@ def main() -> int:
         return "k_" + name, prof[name][0]
 
     def backward_kernel(prof):
-        return "k_mvm_few (whole call)" if "mvm_few" in prof else "k_mvm_round"
+        return one_launch(prof) or "k_mvm_round"
 
     n = max(args.steps, 10)
     # forward / backward alone, on the initial weights (they do not change the tile)
@@ -471,8 +474,7 @@ def main() -> int:
                                         "WRITE_SIZE), not measured in this run") if args.config == 2 else None,
                      "algorithmic_bytes": update_bytes, "kernel_ms": k_update_ms},
         "roofline_forward": {"kernel": "k_mvm_dual + k_mvm_rounds_rest (all rounds of a call)" if fused_forward
-                             else "k_mvm_few (whole call)" if "mvm_few" in prof_forward
-                             else "k_mvm_round (all rounds of a call)", "bound": "mfma",
+                             else one_launch(prof_forward) or "k_mvm_round (all rounds of a call)", "bound": "mfma",
                              "achieved": flops_per_call / (k_fwd_ms * 1e-3) / 1e12, "peak": FP32_MFMA_PEAK_TFLOPS,
                              "unit": "TFLOP/s", "frac": flops_per_call / (k_fwd_ms * 1e-3) / 1e12 / FP32_MFMA_PEAK_TFLOPS,
                              "traffic": PMC_TRAFFIC_BYTES[fwd_traffic] if fwd_traffic else None,
