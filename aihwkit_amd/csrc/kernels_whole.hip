@@ -519,7 +519,9 @@ template <bool WOC, int NB, int R> struct MvmWhole {
       for (int u = 0; u < 8; ++u) {
         const int end = o0 + 64 * u + 4;
         if (a.out_so == 1 && end <= stored) {
-          const __amdgpu_buffer_rsrc_t out = __builtin_amdgcn_make_buffer_rsrc(a.out + (long)b0 * a.out_sb, 0, (int)(4u * (unsigned)(S * a.out_sb)), 0x00020000);
+          // up to the last output of the block's last sample (for one sample the distance to the next may be anything)
+          const unsigned end_of_block = (unsigned)((long)(min(S, a.m_batch - b0) - 1) * a.out_sb + stored);
+          const __amdgpu_buffer_rsrc_t out = __builtin_amdgcn_make_buffer_rsrc(a.out + (long)b0 * a.out_sb, 0, (int)(4u * end_of_block), 0x00020000);
           __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_bits, v[u]), out, 4u * (unsigned)(s * a.out_sb + end - 4), 0, THROUGH);
           continue;
         }

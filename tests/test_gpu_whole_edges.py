@@ -1,0 +1,42 @@
+"""Edges of the one launch of medium batches (k_mvm_whole): few samples and strides that coincide.  Compared bit for bit with the
+launches that such calls take otherwise."""
+import numpy as np
+import pytest
+import torch
+
+from aihwkit_amd.rpu_base import tiles
+from test_gpu_whole_calls import host_tile, names_of, pair_of
+
+pytestmark = pytest.mark.gpu
+
+
+def without_small_calls(tile, rng):
+    """Puts the tile into a group with one whose rows are too long for the launch of small batches: its own calls of few samples
+    then take the launch of medium ones."""
+    return tiles.TileGroup([tile, tiles.CudaAnalogTile(host_tile(rng, 2100, 16, 12.0))])
+
+
+# one sample with transposed output has strides of one element both ways; 13.3 million weights are too many
+# for the launch of small batches
+@pytest.mark.parametrize("x_size,d_size,batch,grouped", [
+    (300, 270, 1, True), (300, 270, 5, True), (300, 270, 15, True), (512, 512, 16, True), (100, 70, 17, True), (300, 20, 1, True),
+    (300, 17, 1, True), (96, 30000, 1, True), (512, 26000, 1, False)])
+@pytest.mark.parametrize("trans", [False, True])
+def test_few_samples(gpu_device, x_size, d_size, batch, grouped, trans):
+    rng = np.random.default_rng(x_size + d_size + batch)
+    spread = 0.2 * np.sqrt(x_size)
+    stood = set()
+    for out_bound in (0.45 * spread, 0.9 * spread, 1.5 * spread, 2.4 * spread, 100.0 * spread):
+        pair = pair_of(host_tile(rng, x_size, d_size, out_bound))
+        group = without_small_calls(pair[0], rng) if grouped else None
+        for call in range(3):
+            x = torch.from_numpy(rng.uniform(-1, 1, (x_size, batch) if trans else (batch, x_size)).astype(np.float32)).cuda()
+            (y, names), (y_other, names_other) = (names_of(t, lambda t: t.forward(x, False, trans, trans)) for t in pair)
+            rounds = pair[0].get_bm_rounds(batch)
+            if names == ["mvm_whole"]:
+                stood.update(rounds.tolist())
+            assert "mvm_whole" not in names_other
+            assert torch.equal(y, y_other), (out_bound, call)
+            assert torch.equal(rounds, pair[1].get_bm_rounds(batch))
+        del group
+    assert {1, 2, 3} <= stood
