@@ -191,8 +191,8 @@ template <bool WOC, int NB, int R> struct MvmWhole {
     *reinterpret_cast<f32x2 *>(to + 16) = f32x2{v[1], v[3]};
   }
   // v / divisor, rounded as the division rounds it: with the divisor's reciprocal rounded to nearest, a product and one
-  // correction are exact (Markstein 1990), except where the remainder leaves the range of numbers (larger quotients are clipped,
-  // smaller ones round to zero).
+  // correction are exact (Markstein 1990; compared with the division for 2400 divisors, with every mantissa), except where the
+  // remainder leaves the range of numbers: smaller quotients round to zero, and larger ones are clipped (steps_are_exact).
   __device__ __forceinline__ static float quotient(float v, float divisor, float reciprocal) {
     const float first = v * reciprocal, second = __builtin_fmaf(__builtin_fmaf(-first, divisor, v), reciprocal, first);
     return fabsf(first) < 0x1p60f ? second : first;
@@ -603,6 +603,11 @@ template <int NB, int R> int held(int K, int cus) {
 
 } // namespace
 
+// Whether quotient() is the division for every value that a converter does not clip
+static bool steps_are_exact(float resolution, float bound) {
+  return !(resolution > 0.0f) || (resolution > 0x1p-60f && resolution < 0x1p60f && bound < 0x1p59f * resolution);
+}
+
 // The outputs of a workgroup: 16 where the GPU holds all of the call's workgroups at once, else 64, up to one set of those with
 // bound management and two without.  us, the launches one by one / this one (forward: weights that saturate round 0 / that do
 // not):
@@ -624,6 +629,7 @@ int mvm_whole_outputs(const MvmArgs &a) {
   const int nm = io.noise_management, cus = a.cus > 0 ? a.cus : current_device_cus();
   if (io.perfect || a.in_index || a.pre_add || a.skip_if_zero || a.nm_phase || a.small_tiles_only || a.K > 2048 || a.K <= a.in_one) return 0;
   if (io.inp_sto_round || io.out_sto_round || io.inp_noise > 0.0f || !(io.inp_bound < 0x1p96f)) return 0;
+  if (!steps_are_exact(io.inp_res, io.inp_bound) || !steps_are_exact(io.out_res, io.out_bound)) return 0;
   if (nm != RPU_NM_NONE && nm != RPU_NM_CONSTANT && nm != RPU_NM_ABS_MAX && nm != RPU_NM_MAX) return 0;
   if (io.bound_management != RPU_BM_NONE && (io.bound_management != RPU_BM_ITERATIVE || a.transposed)) return 0;
   if (mvm_uses_large_tiles(a.m_batch, a.O)) return 0;

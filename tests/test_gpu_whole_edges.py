@@ -1,5 +1,5 @@
-"""Edges of the one launch of medium batches (k_mvm_whole): few samples and strides that coincide.  Compared bit for bit with the
-launches that such calls take otherwise."""
+"""Edges of the one launch of medium batches (k_mvm_whole): few samples, strides that coincide, converters of more steps than its
+division is exact for.  Compared bit for bit with the launches that such calls take otherwise."""
 import numpy as np
 import pytest
 import torch
@@ -40,3 +40,19 @@ def test_few_samples(gpu_device, x_size, d_size, batch, grouped, trans):
             assert torch.equal(rounds, pair[1].get_bm_rounds(batch))
         del group
     assert {1, 2, 3} <= stood
+
+
+# steps of a converter: more than 2^60, and as many as its rule still lets through
+@pytest.mark.parametrize("settings", [dict(inp_res=3e-19), dict(out_res=3e-19, out_noise=0.0), dict(inp_res=1 / 1.1e18),
+                                      dict(out_res=1 / 1.1e18, out_noise=0.0)])
+def test_converters_of_many_steps(gpu_device, settings):
+    rng = np.random.default_rng(7)
+    x_size, d_size, batch = 300, 600, 203
+    pair = pair_of(host_tile(rng, x_size, d_size, 30.0, **settings))
+    for call in range(2):
+        x = torch.from_numpy(rng.uniform(-1, 1, (batch, x_size)).astype(np.float32)).cuda()
+        d = torch.from_numpy(rng.normal(0, 0.05, (400, d_size)).astype(np.float32)).cuda()
+        y, y_other = (t.forward(x, False) for t in pair)
+        assert torch.equal(y, y_other)
+        g, g_other = (t.backward(d, False) for t in pair)
+        assert torch.equal(g, g_other)
