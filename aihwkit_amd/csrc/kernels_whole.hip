@@ -247,16 +247,21 @@ template <bool WOC, int NB, int R> struct MvmWhole {
     const f32x4 x[2] = {*reinterpret_cast<const f32x4 *>(from), *reinterpret_cast<const f32x4 *>(from + 4)};
     float v[NB][8], in[R][8];
     operands(w, v);
-    if (!WOC && step * KSTEP + KSTEP > a.K) { // beyond the row: the next one's
-      const int left = a.K - step * KSTEP - 16 * ((lane >> 4) & 1) - (lane >> 5);
-#pragma unroll
-      for (int n = 0; n < NB; ++n) {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) v[n][j] = 2 * j < left ? v[n][j] : 0.0f;
-      }
-    }
 #pragma unroll
     for (int j = 0; j < 8; ++j) in[0][j] = x[j / 4][j & 3] * by.scale;
+    if (step * KSTEP + KSTEP > a.K) {
+      // beyond the row: the next one's weights, and zeros times a scale that is infinite where the row's largest input is below
+      // 2^-128
+      const int left = a.K - step * KSTEP - 16 * ((lane >> 4) & 1) - (lane >> 5);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        in[0][j] = 2 * j < left ? in[0][j] : 0.0f;
+        if constexpr (!WOC) {
+#pragma unroll
+          for (int n = 0; n < NB; ++n) v[n][j] = 2 * j < left ? v[n][j] : 0.0f;
+        }
+      }
+    }
     if (by.resolution > 0.0f) {
 #pragma unroll
       for (int j = 0; j < 8; ++j) {

@@ -1,5 +1,5 @@
 """Edges of the one launch of medium batches (k_mvm_whole): few samples, strides that coincide, converters of more steps than its
-division is exact for.  Compared bit for bit with the launches that such calls take otherwise."""
+division is exact for, inputs at the ends of their range.  Compared bit for bit with the launches that such calls take otherwise."""
 import numpy as np
 import pytest
 import torch
@@ -56,3 +56,27 @@ def test_converters_of_many_steps(gpu_device, settings):
         assert torch.equal(y, y_other)
         g, g_other = (t.backward(d, False) for t in pair)
         assert torch.equal(g, g_other)
+
+
+# gradients so small that the factor of their noise management is infinite, on rows that end within a step of the contraction and on
+# whole ones; and values that are not numbers: the rest of the batch is as ever, and so are the rows themselves
+@pytest.mark.parametrize("x_size,d_size,batch", [(300, 270, 800), (300, 300, 700), (200, 512, 600)])
+@pytest.mark.parametrize("value", [1e-40, 1e-38, 3e38, float("inf"), float("nan")])
+def test_inputs_at_the_ends_of_their_range(gpu_device, x_size, d_size, batch, value):
+    rng = np.random.default_rng(d_size)
+    pair = pair_of(host_tile(rng, x_size, d_size, 12.0))
+    d = rng.normal(0, 0.05, (batch, d_size)).astype(np.float32)
+    d[17] = value
+    d[18] = value * np.sign(d[18])
+    d[19, 5] = value
+    x = rng.normal(0, 0.05, (203, x_size)).astype(np.float32)
+    x[17] = value
+    x[18] = value * np.sign(x[18])
+    x[19, 5] = value
+    d, x = torch.from_numpy(d).cuda(), torch.from_numpy(x).cuda()
+    (g, names), (g_other, _) = (names_of(t, lambda t: t.backward(d, False)) for t in pair)
+    assert names == ["mvm_whole"]
+    assert torch.equal(torch.nan_to_num(g, 1e30), torch.nan_to_num(g_other, 1e30))
+    (y, names), (y_other, _) = (names_of(t, lambda t: t.forward(x, False)) for t in pair)
+    assert names == ["mvm_whole"] or d_size > x_size
+    assert torch.equal(torch.nan_to_num(y, 1e30), torch.nan_to_num(y_other, 1e30))
