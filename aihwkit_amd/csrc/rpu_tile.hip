@@ -320,7 +320,24 @@ struct Tile {
   DevBuf<float> s_dual0, s_dual1, s_dual2, s_xq2;
   DevBuf<int> s_dsel, s_dhit1, s_dhit2;
   int few_calls = 0; // see few_args
-  int beyond_call = 0, beyond_calls = 0; // see rounds_beyond
+  // Calls for which a tile keeps away from a launch that cost it time, after a call of which the GPU reports so: 64, and twice as many
+  // (4096 at most) each time that it happens again after them, so that what it costs to try stays small beside them
+  struct KeepAway {
+    int reported = 0, length = 32, left = 0;
+    bool on(int report) {
+      if (report != reported) {
+        reported = report;
+        if (left == 0) length = std::min(2 * length, 4096);
+        left = length;
+      } else if (left > 0) {
+        --left;
+      }
+      return left > 0;
+    }
+  };
+  KeepAway beyond, one_round; // see rounds_beyond, whole_rounds
+  int one_from = 0, one_to = 0; // numbers of the last calls in a row that worked out one round
+  bool last_was_whole = false;  // of the tile's forward calls
   size_t few_zero = 0; // words for k_mvm_few that are zero between calls
   bool small_calls = true; // rpu_tile_set_small_calls
   // largest batch that the groups of this tile run as k_mvm_few, forward and backward: so does the tile in calls of its own,
@@ -747,13 +764,14 @@ struct Tile {
     a.few = s_count.p + MVM_COUNT_WORDS;
     a.few_seen = seen_dev;
     a.few_call = call_number;
-    // (the launch takes the inputs of rounds 1 and 2 as halves of those of round 0 before the clipping)
-    if (a.max_rounds < 3 || !(a.io.inp_bound < 0x1p96f)) return 1;
     a.dual.buf[1] = a.xq[0];
     a.dual.buf[2] = a.xq[1];
+    // (the launch takes the inputs of rounds 1 and 2 as halves of those of round 0 before the clipping)
+    if (a.max_rounds < 3 || !(a.io.inp_bound < 0x1p96f)) return 1;
     if (fused_rounds >= 0) return fused_rounds & 1 ? 3 : 1;
-    return seen_host[1] - seen_host[0] <= 8 ? 3 : 1;
+    return saturated_lately(seen_host) ? 3 : 1;
   }
+  static bool saturated_lately(const volatile int *seen_host) { return seen_host[1] - seen_host[0] <= 8; }
   // whether a launch on s runs now: a captured one clears when it is replayed
   static bool runs_now(hipStream_t s) {
     hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
@@ -776,28 +794,63 @@ struct Tile {
     p.add(in);
     return p.meets(out);
   }
+  // Rounds that k_mvm_whole does not work out together it leaves to one workgroup per 16 samples, which runs all of their outputs
+  // one after the other.  us, the other launches / this one, every sample in round 3 or later: 512 x 512, 100 samples 62 / 138; 1024
+  // x 1024, 24 77 / 361; 1500 x 1500, 10 81 / 544; 64 -> 1024, 129 52 / 139; 16 -> 1024, 300 57 / 108; but 40 -> 400, 600 60 / 61; 160 ->
+  // 100, 1218 60 / 31; 64 -> 32, 4096 86 / 63.  Small matrices with few outputs can leave them there; other calls go as follows.
+  static bool leaves_rounds_alone(const MvmArgs &a) {
+    return a.max_rounds > 1 && ((long)a.K * a.O > 1L << 14 || a.O > 256);
+  }
   // Whether forward calls that could take k_mvm_whole keep to the other launches, with the same bits: a sample of one of the recent
-  // calls went beyond the rounds that are worked out together.  A workgroup runs those alone, all outputs of its samples one after
-  // the other.  us, the other launches / the one, every sample in round 3 or later: 512 x 512, 100 samples 71 / 138; 1024 x 1024, 24
-  // 85 / 361; 1500 x 1500, 10 86 / 544; 64 -> 1024, 129 59 / 139; but 160 -> 100, 1218 67 / 42, 64 -> 32, 4096 91 / 25: matrices of up
-  // to 2^14 weights stay.  Such a call sends the next 64 to the other launches, which say
-  // for themselves when a sample needs those rounds again (a call without any is 10 to 30 us slower on them).
+  // calls went beyond the rounds that are worked out together.  The other launches say for themselves when a sample needs those
+  // rounds again (a call without any is 6 to 16 us slower on them).
   bool rounds_beyond(bool reports) {
     const volatile int *const seen = seen_host;
-    if (seen[6] != beyond_call) {
-      beyond_call = seen[6];
-      beyond_calls = 64;
-    } else if (beyond_calls > 0) {
-      if (beyond_calls < 64 && reports && seen[1] > 0 && seen[2] >= 3) beyond_calls = 64;
-      --beyond_calls;
-    }
-    return beyond_calls > 0;
+    const bool on = beyond.on(seen[6]);
+    if (on && reports && seen[1] > 0 && seen[2] >= MVM_WHOLE_ROUNDS) beyond.left = beyond.length;
+    return on;
+  }
+  // Rounds that call number few_calls works out together on k_mvm_whole: one where no recent call needed more, unless that has cost time
+  // lately -- a call whose samples went on took 73 us instead of 26 (512 x 512, 100 samples; 1024 x 1024, 24: 221 and 31), three rounds
+  // together take 16 and 20 where one takes 11 and 12.
+  int whole_rounds(const MvmArgs &a) {
+    if (a.max_rounds < 2) return 1;
+    const int saturated = *(volatile int *)&seen_host[4];
+    const bool was_one = saturated >= one_from && saturated < one_to;
+    const bool keep = one_round.on(was_one ? saturated + 1 : one_round.reported);
+    if (keep || saturated_lately(seen_host + 4)) return MVM_WHOLE_ROUNDS;
+    if (one_to != few_calls) one_from = few_calls;
+    one_to = few_calls + 1;
+    return 1;
+  }
+  // what the launch of several rounds (k_mvm_dual) needs for a call
+  bool has_fused_room(const MvmArgs &a, int rounds) const {
+    const size_t results = (size_t)a.m_batch * a.O, marks = 2 * (size_t)a.m_batch;
+    return s_dual0.n >= results && s_dual1.n >= results && s_xq2.n >= (size_t)a.m_batch * a.k_pad && s_dsel.n >= (size_t)a.m_batch &&
+           s_dhit1.n >= marks && (rounds < 3 || (s_dual2.n >= results && s_dhit2.n >= marks));
+  }
+  void make_fused_room(const MvmArgs &a, int rounds) {
+    const size_t results = (size_t)a.m_batch * a.O, marks = 2 * (size_t)a.m_batch;
+    auto make_marks = [&](DevBuf<int> &buf) {
+      if (buf.n >= marks) return;
+      buf.ensure(marks);
+      RPU_HIP_CHECK(hipMemset(buf.p, 0, buf.n * sizeof(int))); // cleared by every call after use
+    };
+    s_dual0.ensure(results); s_dual1.ensure(results); s_xq2.ensure((size_t)a.m_batch * a.k_pad);
+    s_dsel.ensure((size_t)a.m_batch);
+    make_marks(s_dhit1);
+    if (rounds < 3) return;
+    s_dual2.ensure(results);
+    make_marks(s_dhit2);
   }
   // words 0 to 3: the launches of the rounds, 4 and 5: few_args, 6: the last call on k_mvm_whole with a sample in round 3 or later
+  static constexpr int SEEN_WORDS = 7;
   void ensure_seen() {
     if (seen_dev) return; // the last step
-    if (!seen_host) RPU_HIP_CHECK(hipHostMalloc((void **)&seen_host, 7 * sizeof(int), hipHostMallocMapped));
-    for (int i = 0; i < 7; ++i) seen_host[i] = 0; // until the first calls say otherwise
+    if (!seen_host) RPU_HIP_CHECK(hipHostMalloc((void **)&seen_host, SEEN_WORDS * sizeof(int), hipHostMallocMapped));
+    for (int i = 0; i < SEEN_WORDS; ++i) seen_host[i] = 0; // until the first calls say otherwise
+    beyond = one_round = KeepAway{};
+    one_from = one_to = 0;
     RPU_HIP_CHECK(hipHostGetDevicePointer((void **)&seen_dev, seen_host, 0));
   }
 
@@ -1131,11 +1184,17 @@ struct Tile {
     const bool other_launches = !small_calls || fused_rounds >= 0 || wait_spins_hook || wait_extra_hook;
     int whole = few || side || gather || running || other_launches ? 0 : mvm_whole_outputs(a);
     if (whole && a.max_rounds > 1) ensure_seen();
-    if (whole && a.max_rounds > MVM_WHOLE_ROUNDS && (long)a.K * a.O > 1L << 14 && rounds_beyond(!w_other)) whole = 0;
+    // a captured call takes the launch only if every round is worked out together: what its replays need is not known here
+    const bool captured = whole && leaves_rounds_alone(a) && !runs_now(s);
+    if (whole && leaves_rounds_alone(a) && a.max_rounds > MVM_WHOLE_ROUNDS && (captured || rounds_beyond(!w_other))) whole = 0;
     bool clear = false;
     int together = 1;
     const bool one_launch = (few || whole) && !writes_into_its_input(a);
-    if (one_launch && a.max_rounds > 1) together = few_args(a, few_calls++, seen_host + 4, seen_dev + 4, clear);
+    if (one_launch && whole) together = captured ? MVM_WHOLE_ROUNDS : whole_rounds(a);
+    if (one_launch && a.max_rounds > 1) {
+      const int few_together = few_args(a, few_calls++, seen_host + 4, seen_dev + 4, clear);
+      if (few) together = few_together;
+    }
     const size_t results = (size_t)B * a.O;
     if (one_launch && whole && together > 1 && (s_xq0.n < results || s_xq1.n < results)) {
       // where the fused launches keep theirs; the tile's first call and captured ones make no room, and one round in the launch
@@ -1156,6 +1215,13 @@ struct Tile {
       const MvmArgs *call = &a;
       if (few) launch_mvm_few(a, mvm_few_variant(&call, 1), together, s);
       else launch_mvm_whole(a, whole, together, s);
+      if (!transposed && !w_other) last_was_whole = whole != 0;
+      // where samples go on to further rounds call after call, a captured one, which takes the other launches, finds the room to share
+      // them (512 x 512, 100 samples in round 1: 30 us instead of 37)
+      if (whole && together > 1 && !captured && leaves_rounds_alone(a) && !w_other && *(volatile int *)&seen_host[4] >= 2 &&
+          saturated_lately(seen_host + 4) && !has_fused_room(a, 3) && mvm_can_fuse_rounds(a)) {
+        make_fused_room(a, 3);
+      }
       prof_mark(s, few ? "mvm_few" : "mvm_whole");
     } else if (io.perfect) {
       a.round = 0;
@@ -1180,12 +1246,16 @@ struct Tile {
       if (!transposed && !w_other && !side && io.p.bound_management != RPU_BM_NONE && fused_rounds != 0) {
         ensure_seen();
         a.dual.seen = seen_dev;
-        const int needed = *(volatile int *)&seen_host[0], of = *(volatile int *)&seen_host[1];
-        const int last_listed = *(volatile int *)&seen_host[2];
+        int needed = *(volatile int *)&seen_host[0], of = *(volatile int *)&seen_host[1];
+        int last_listed = *(volatile int *)&seen_host[2];
+        if (captured && last_was_whole) { // those calls know better
+          const bool saturated = saturated_lately(seen_host + 4);
+          of = B;
+          needed = saturated ? B : 0;
+          last_listed = rest_from = saturated ? 2 : 0;
+        }
         // (a captured call makes no room; after calls in one launch it may be the first of its size here)
-        const bool room = s_dual0.n >= results && s_dual1.n >= results && s_xq2.n >= (size_t)B * a.k_pad && s_dsel.n >= (size_t)B &&
-                          s_dhit1.n >= 2 * (size_t)B;
-        const bool room_for_3 = s_dual2.n >= results && s_dhit2.n >= 2 * (size_t)B;
+        const bool room = has_fused_room(a, 2), room_for_3 = has_fused_room(a, 3);
         fuse = mvm_can_fuse_rounds(a) && (room || few_calls == 0 || runs_now(s)) &&
                ((fused_rounds > 0 && (fused_rounds & 1)) || (fused_rounds < 0 && of > 0 && 2 * (long)needed > of));
         // The last round that listed samples in the recent calls is expected to be the last one of this call too: the
@@ -1218,24 +1288,15 @@ struct Tile {
         }
       }
       if (fuse) {
-        s_dual0.ensure((size_t)B * a.O); s_dual1.ensure((size_t)B * a.O); s_xq2.ensure((size_t)B * a.k_pad);
-        s_dsel.ensure((size_t)B);
-        if (s_dhit1.n < 2 * (size_t)B) {
-          s_dhit1.ensure(2 * (size_t)B);
-          RPU_HIP_CHECK(hipMemset(s_dhit1.p, 0, s_dhit1.n * sizeof(int))); // cleared by every call after use
-        }
+        make_fused_room(a, fused);
         a.dual.buf[0] = s_dual0.p; a.dual.buf[1] = s_dual1.p; a.dual.sel = s_dsel.p; a.dual.hit1 = s_dhit1.p;
         a.dual.xq2 = s_xq2.p;
         a.dual.rounds = fused;
         if (fused == 3) {
-          s_dual2.ensure((size_t)B * a.O);
-          if (s_dhit2.n < 2 * (size_t)B) {
-            s_dhit2.ensure(2 * (size_t)B);
-            RPU_HIP_CHECK(hipMemset(s_dhit2.p, 0, s_dhit2.n * sizeof(int)));
-          }
           a.dual.buf[2] = s_dual2.p; a.dual.hit2 = s_dhit2.p;
         }
       }
+      if (!transposed && !w_other) last_was_whole = false;
       launch_mvm_init(a, s);
       prof_mark(s, "mvm_init");
       // every round after the first works on the samples whose ADC saturated in the one before; the

@@ -1,11 +1,12 @@
 """Edges of the one launch of medium batches (k_mvm_whole): few samples, strides that coincide, converters of more steps than its
-division is exact for, inputs at the ends of their range.  Compared bit for bit with the launches that such calls take otherwise."""
+division is exact for, inputs at the ends of their range, rounds that it leaves to one workgroup.  Compared bit for bit with the
+launches that such calls take otherwise."""
 import numpy as np
 import pytest
 import torch
 
 from aihwkit_amd.rpu_base import tiles
-from test_gpu_whole_calls import host_tile, names_of, pair_of
+from test_gpu_whole_calls import binds, host_tile, names_of, pair_of
 
 pytestmark = pytest.mark.gpu
 
@@ -80,3 +81,70 @@ def test_inputs_at_the_ends_of_their_range(gpu_device, x_size, d_size, batch, va
     (y, names), (y_other, _) = (names_of(t, lambda t: t.forward(x, False)) for t in pair)
     assert names == ["mvm_whole"] or d_size > x_size
     assert torch.equal(torch.nan_to_num(y, 1e30), torch.nan_to_num(y_other, 1e30))
+
+
+def microseconds(call, calls=40):
+    start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+    call()
+    torch.cuda.synchronize()
+    start.record()
+    for _ in range(calls):
+        call()
+    end.record()
+    torch.cuda.synchronize()
+    return start.elapsed_time(end) * 1000 / calls
+
+
+# 1500 x 1500, 10 samples: a round that one workgroup runs alone takes 400 us, the launches of the others 25 to 45.  two: there are no more
+# than two rounds; captured: without saturation, replayed with it; alternating: calls without saturation, now and then one with it
+@binds
+@pytest.mark.parametrize("program", ["two", "captured", "alternating"])
+def test_no_rounds_are_left_alone_time_and_again(gpu_device, program):
+    rng = np.random.default_rng(1)
+    x_size, d_size, batch = 1500, 1500, 10
+    pair = pair_of(host_tile(rng, x_size, d_size, 4.0, **(dict(max_bm_factor=1) if program == "two" else {})))
+    x = torch.from_numpy(rng.uniform(-1, 1, (batch, x_size)).astype(np.float32)).cuda()
+    weights = torch.from_numpy(rng.uniform(-1, 1, (d_size, x_size)).astype(np.float32)).cuda()
+    weights /= float((x / x.abs().amax(dim=1, keepdim=True) @ weights.t()).abs().amax())   # largest output of a sample: up to 1
+    calm, saturating = weights, weights * (6.0 if program != "alternating" else 12.0)       # beyond 4, beyond 8
+    took, results, graphs = [], [], []
+    for tile in pair:
+        tile.live = torch.empty(d_size, x_size, device="cuda")
+        tile.set_shared_weights_row_major(tile.live)
+        tile.live.copy_(calm)
+        torch.cuda.synchronize()
+
+        def forward():
+            return tile.forward(x, False, False, False, False, True)
+
+        if program == "two":
+            tile.live.copy_(saturating)
+            call = forward
+        elif program == "captured":
+            for _ in range(12):
+                forward()
+            torch.cuda.synchronize()
+            graphs.append(torch.cuda.CUDAGraph())
+            with torch.cuda.graph(graphs[-1]):
+                y = forward()
+            tile.live.copy_(saturating)
+            graph = graphs[-1]
+
+            def call():
+                graph.replay()
+                return y
+        else:
+            def call():
+                tile.live.copy_(saturating)
+                y = forward()
+                tile.live.copy_(calm)
+                for _ in range(10):
+                    forward()
+                return y
+        torch.cuda.synchronize()
+        took.append(min(microseconds(call) for _ in range(3)))
+        results.append(call().clone())
+        if program != "alternating":
+            assert int(tile.get_bm_rounds(batch).max()) == 2
+    assert torch.equal(*results)
+    assert took[0] < 1.5 * took[1], took
