@@ -101,21 +101,24 @@ template <class A> struct GroupArgs {
   DevBuf<unsigned long long> dev;
   char *host = nullptr, *host_on_dev = nullptr;
   size_t table_words = 0; // of eight bytes, before the argument blocks
+  size_t set_words = 0;   // of a set: table and argument blocks of one kind of call
+  size_t set_at = 0;      // of the set that the members below are about, see use
   static_assert(sizeof(A) % 8 == 0 && alignof(A) <= 16, "argument blocks are uploaded in words of eight bytes");
-  void make(size_t n_args, size_t n_table) {
+  void make(size_t n_args, size_t n_table, size_t sets = 1) {
     table_words = (n_table + 3) / 4 * 2;
-    const size_t words = table_words + n_args * (sizeof(A) / 8);
-    dev.ensure(words);
-    if (!host) RPU_HIP_CHECK(hipHostMalloc((void **)&host, 8 * words, hipHostMallocMapped));
+    set_words = (words(n_args) + 1) / 2 * 2;
+    dev.ensure(sets * set_words);
+    if (!host) RPU_HIP_CHECK(hipHostMalloc((void **)&host, 8 * sets * set_words, hipHostMallocMapped));
     RPU_HIP_CHECK(hipHostGetDevicePointer((void **)&host_on_dev, host, 0));
   }
   bool made() const { return host_on_dev != nullptr; } // the last step of make
-  int *table() { return reinterpret_cast<int *>(host); }
-  A *args() { return reinterpret_cast<A *>(host + 8 * table_words); }
-  const int *dev_table() const { return reinterpret_cast<const int *>(dev.p); }
-  const A *dev_args() const { return reinterpret_cast<const A *>(dev.p + table_words); }
+  void use(size_t set) { set_at = set * set_words; }
+  int *table() { return reinterpret_cast<int *>(host + 8 * set_at); }
+  A *args() { return reinterpret_cast<A *>(host + 8 * (set_at + table_words)); }
+  const int *dev_table() const { return reinterpret_cast<const int *>(dev.p + set_at); }
+  const A *dev_args() const { return reinterpret_cast<const A *>(dev.p + set_at + table_words); }
   size_t words(size_t n_args) const { return table_words + n_args * (sizeof(A) / 8); }
-  void upload(size_t n_args, hipStream_t s) { launch_upload(dev.p, host_on_dev, words(n_args), s); }
+  void upload(size_t n_args, hipStream_t s) { launch_upload(dev.p + set_at, host_on_dev + 8 * set_at, words(n_args), s); }
   void release() {
     if (host) (void)hipHostFree(host);
     host = host_on_dev = nullptr;
@@ -2813,11 +2816,12 @@ int rpu_tile_set_extra(rpu_tile_t *tile, const int64_t *values_host, int count) 
 struct rpu_group {
   std::vector<rpu_tile *> tiles;
   int device_id = -1;
-  GroupArgs<MvmArgs> mvm_args;
-  // Table and argument blocks of the call that is being put together, and those that lie in HBM (empty: others).  Calls that take
-  // the one launch of small batches hand it what differs from call to call (MvmFewCalls; zeros here) and upload the rest only
-  // when it has changed: the upload reads host memory, 3 us and a gap before each launch of 8 to 15.
-  std::vector<unsigned long long> next_args, uploaded_args;
+  GroupArgs<MvmArgs> mvm_args; // two sets: of forward and of backward calls, which a training step runs in turn
+  // Table and argument blocks of the call that is being put together, and those of either set that lie in HBM (empty: others).  Calls
+  // that take the one launch of small batches hand it what differs from call to call (MvmFewCalls; zeros here) and upload the rest only
+  // when it has changed: the upload reads host memory, 3 us and a gap before each launch of 8 to 15.  (Forward and backward in turn, 38
+  // tiles of 128 x 128, 4 samples: with one set for both 1 % slower than with an upload in every call, with two 69 -> 56 us.)
+  std::vector<unsigned long long> next_args, uploaded_args[2];
   hipEvent_t copied = nullptr;
   int few_calls = 0; // see Tile::few_args
   Places inputs; // of the last call, kept for its memory
@@ -2905,7 +2909,7 @@ int rpu_group_create(rpu_group_t **out, rpu_tile_t *const *tiles, int n_tiles) {
     DeviceGuard dg(g->device_id);
     g->limit_small_calls();
     const size_t n = (size_t)n_tiles;
-    g->mvm_args.make(n, 3 * n + 4);
+    g->mvm_args.make(n, 3 * n + 4, 2);
     RPU_HIP_CHECK(hipEventCreateWithFlags(&g->copied, hipEventDisableTiming));
     *out = g.release();
   });
@@ -3241,12 +3245,17 @@ static int group_mvm(rpu_group_t *group, const float *const *x_dev, const long *
     });
     struct Segment { int first, count, depth, mode, start_offset, workgroups; };
     std::vector<Segment> segments;
-    group->next_args.assign(group->mvm_args.words((size_t)n), 0);
-    int *const table = reinterpret_cast<int *>(group->next_args.data());
-    int cursor = 0; // position in the table
     std::vector<const MvmArgs *> few_calls;
     while ((int)few_calls.size() < n && few[order[few_calls.size()]]) few_calls.push_back(&args[order[few_calls.size()]]);
     const int n_few = (int)few_calls.size(), few_variant = mvm_few_variant(few_calls.data(), n_few);
+    // (a replay uploads what the pinned memory holds then, and reads no other values)
+    const bool keeps_args = n_few == n && n <= MvmFewCalls::MOST && Tile::runs_now(s);
+    group->mvm_args.use(transposed ? 1 : 0);
+    std::vector<unsigned long long> &uploaded_args = group->uploaded_args[transposed ? 1 : 0];
+    if (keeps_args) group->next_args.assign(group->mvm_args.words((size_t)n), 0);
+    else uploaded_args.clear();
+    int *const table = keeps_args ? reinterpret_cast<int *>(group->next_args.data()) : group->mvm_args.table();
+    int cursor = 0; // position in the table
     bool few_stoch = false;
     int few_workgroups = 0, few_max_k = 0, few_together = 3; // a launch has one form; the buffers of three rounds serve one
     for (int i = 0; i < n_few; ++i) {
@@ -3281,26 +3290,24 @@ static int group_mvm(rpu_group_t *group, const float *const *x_dev, const long *
       table[cursor++] = wg;
     }
     MvmFewCalls calls{};
-    const bool now = Tile::runs_now(s); // (a replay uploads what the pinned memory holds then, and reads no other values)
-    if (n_few == n && n <= MvmFewCalls::MOST && now) {
+    if (keeps_args) {
       calls.count = n;
       calls.few_call = group->few_calls;
+      MvmArgs *const blocks = reinterpret_cast<MvmArgs *>(group->next_args.data() + group->mvm_args.table_words);
+      for (int i = 0; i < n; ++i) {
+        std::memcpy((void *)&blocks[i], (const void *)&args[order[i]], sizeof(MvmArgs));
+        MvmArgs &a = blocks[i];
+        calls.in[i] = a.in; calls.out[i] = a.out; calls.call[i] = a.call;
+        a.in = nullptr; a.out = nullptr; a.call = 0; a.few_call = 0;
+      }
     }
-    MvmArgs *const blocks = reinterpret_cast<MvmArgs *>(group->next_args.data() + group->mvm_args.table_words);
-    for (int i = 0; i < n; ++i) {
-      std::memcpy((void *)&blocks[i], (const void *)&args[order[i]], sizeof(MvmArgs));
-      if (calls.count == 0) continue;
-      MvmArgs &a = blocks[i];
-      calls.in[i] = a.in; calls.out[i] = a.out; calls.call[i] = a.call;
-      a.in = nullptr; a.out = nullptr; a.call = 0; a.few_call = 0;
-    }
-    if (calls.count == 0 || group->next_args != group->uploaded_args) {
-      group->uploaded_args.clear();
-      std::memcpy(group->mvm_args.table(), group->next_args.data(), 8 * group->mvm_args.table_words);
+    if (!keeps_args || group->next_args != uploaded_args) {
+      uploaded_args.clear();
+      if (keeps_args) std::memcpy(group->mvm_args.table(), group->next_args.data(), 8 * group->mvm_args.table_words);
       for (int i = 0; i < n; ++i) group->mvm_args.args()[i] = args[order[i]];
       group->mvm_args.upload((size_t)n, s);
       RPU_HIP_CHECK(hipEventRecord(group->copied, s));
-      if (calls.count > 0) group->uploaded_args.swap(group->next_args);
+      if (keeps_args) uploaded_args.swap(group->next_args);
     }
 
     if (n_few) {
