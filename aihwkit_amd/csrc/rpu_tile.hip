@@ -798,11 +798,11 @@ struct Tile {
     return p.meets(out);
   }
   // Rounds that k_mvm_whole does not work out together it leaves to one workgroup per 16 samples, which runs all of their outputs
-  // one after the other.  us, the other launches / this one, every sample in round 3 or later: 512 x 512, 100 samples 62 / 138; 1024
-  // x 1024, 24 77 / 361; 1500 x 1500, 10 81 / 544; 64 -> 1024, 129 52 / 139; 16 -> 1024, 300 57 / 108; but 40 -> 400, 600 60 / 61; 160 ->
-  // 100, 1218 60 / 31; 64 -> 32, 4096 86 / 63.  Small matrices with few outputs can leave them there; other calls go as follows.
+  // one after the other.  us for a round of all samples, in launches of its own / alone: 512 x 512, 100 samples 19 / 61; 1024 x 1024, 24
+  // 19 / 206; 1500 x 1500, 10 24 / 415; 785 -> 256, 64 26 / 48; 64 -> 1024, 129 22 / 61; 32 -> 512, 500 30 / 31; but 40 -> 400, 600 38 /
+  // 30; 160 -> 100, 1218 25 / 16; 64 -> 32, 4096 36 / 17.  Small matrices with few outputs can leave them there; other calls go as follows.
   static bool leaves_rounds_alone(const MvmArgs &a) {
-    return a.max_rounds > 1 && ((long)a.K * a.O > 1L << 14 || a.O > 256);
+    return a.max_rounds > 1 && ((long)a.K * a.O > 1L << 14 || a.O > 400);
   }
   // Whether forward calls that could take k_mvm_whole keep to the other launches, with the same bits: a sample of one of the recent
   // calls went beyond the rounds that are worked out together.  The other launches say for themselves when a sample needs those
