@@ -11,8 +11,8 @@
 // weights with the inputs of rounds 0, 1 and 2 (V = R S rows) and keep all results, and the last one copies out what
 // stands (as k_mvm_dual); a round beyond those it runs alone, block by block.  No list, no later launch.
 // What bounds it: the chain from launch to loads, maximum, ADC and two atomics (about 1 us each), and how fast its code comes:
-// it runs once through, and a jump over code that the call does not need waits for instructions (1.1 us for two of them, by
-// the clock between them, on the version before).  So the random draws of the converters are compiled in only where
+// it runs once through, and a jump over code that the call does not need waits for instructions.  So the random draws of the
+// converters are compiled in only where
 // the settings have them (STOCH), a thread works on one sample's row and not on all, loads have no branches (buffer
 // loads: what lies beyond the matrix reads as zero) and what few calls need stands at the end.
 // One sample on 512 x 512 8.8 -> 7.8 us a launch, 12 tiles of 512 x 512 with 8 samples 17.2 -> 10.1, 785 x 300 with 37 samples and

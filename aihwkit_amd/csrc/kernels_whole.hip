@@ -9,7 +9,9 @@
 // underneath the matrix instructions) and decides about further rounds as k_mvm_few does: the workgroups of a sample count
 // themselves off, the last one copies out the round that stands (R = 3), or runs the rounds from R on alone.
 //
-// What bounds it: the rows' way through LDS and the conversions in front of the matrix instructions, then the chain of counters.
+// What bounds it: the chain from the inputs' loads over their maximum, the contraction, the barriers and the counters to the output.
+// 512 x 512, 100 samples, three rounds: of the waves' cycles 58 % wait for such results, 19 % issue vector instructions, the matrix
+// pipe is busy 11 %, LDS is waited for 0.3 % (one round: 63, 18, 5, 0.1).
 // Launches one by one -> this one: 512 x 512, 100 samples 27.1 -> 15.8 us, 785 -> 256, 64 samples 39.3 -> 17.2.
 //
 // Sums are those of mvm_round_tile, bit for bit: four chains over the quarters of the padded contraction, wave w the w-th,
@@ -600,7 +602,7 @@ template <bool WOC, int NB, int R> __global__ __launch_bounds__(256, 2) void k_m
   if (Whole::block_of(a, (int)blockIdx.x, block_b, block_o)) Whole(a, whole_lds, sh).run(block_b, block_o);
 }
 
-// workgroups that the GPU holds at once: two to a CU by their registers, one where rows of more than 1000 inputs take half of
+// workgroups that the GPU holds at once: two to a CU by their registers, one where rows of more than 1088 inputs take half of
 // its 160 KB of LDS
 template <int NB, int R> int held(int K, int cus) {
   return std::min<int>(2, (int)(160 * 1024 / (MvmWhole<false, NB, R>::lds_bytes(K) + sizeof(WholeShared)))) * cus;
@@ -627,8 +629,11 @@ static bool steps_are_exact(float resolution, float bound) {
 // (1500 x 1500, one workgroup to a CU, 200 81 / 81, 37 / 43).
 // Long aligned rows along the inputs, a single round: not with 64 outputs, whose 64 rows a wave reads 16 bytes at a time from 16
 // of them (1024 x 1024 stored the other way round, backward, 256 16.6 / 16.6, 300 22.1 / 23.6, 1000 38 / 46).
-// Large matrices whose 32 x 32 tiles are one to a CU stay with the rounds in one launch (k_mvm_dual), which read the weights once
-// for 32 samples: 1024 x 1024, 256 samples 41.5 / 39.5, 24.9 / 21.7.
+// Large matrices whose 32 x 32 tiles are one to a CU stay with the others: these share the launch of rounds 0 and 1 there (k_mvm_dual)
+// and read the weights once for 32 samples, where all samples end in round 1.  Without saturation / in round 1 / in round 2, the others
+// and this one: 1024 x 1024, 256 samples 25.2 21.5 / 36.4 38.6 / 42.0 38.9, 160 23.1 19.8 / 34.1 35.0 / 38.7 35.4; 1024 -> 768, 320 25.1 25.8
+// / 37.6 50.5 / 42.6 50.8; 544 -> 2048, 128 24.2 20.5 / 34.8 40.2 / 39.3 40.3; 1504 x 1504, 96 25.7 24.0 / 39.1 44.7 / 44.9 45.0 (so a call
+// that does not saturate would gain up to 16 %).
 int mvm_whole_outputs(const MvmArgs &a) {
   const IoDev &io = a.io;
   const int nm = io.noise_management, cus = a.cus > 0 ? a.cus : current_device_cus();

@@ -529,8 +529,8 @@ class _CudaTileMixin:
         check(lib().rpu_tile_set_fused_rounds(self._h, int(mode)))
 
     def set_small_calls(self, enable: bool = True) -> None:
-        """Whether small batches may run as one launch (default).  ``False``: the launches of larger batches, whose sums are
-        added in another order, serve every batch."""
+        """Whether small and medium batches may run as one launch (default).  ``False``: the launches of larger batches serve
+        every batch; those of small ones add in another order, those of medium ones give the same results."""
         check(lib().rpu_tile_set_small_calls(self._h, int(enable)))
 
     def set_round_wait_test_hook(self, spin_limit: int = 0, extra_arrivals: int = 0) -> None:

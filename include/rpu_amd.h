@@ -702,7 +702,10 @@ int rpu_tile_set_fused_rounds(rpu_tile_t *tile, int mode);
 /* No counterpart in the reference.  A call of a small batch runs noise management, conversions, contraction and all
  * bound-management rounds in one launch, whose sums are added in another order than those of the launches for larger
  * batches.  Tiles of a group take it together or not at all, and from then on in calls of their own like in the group's.
- * enable = 0: the tile (alone and in a group) keeps to the latter for every batch. */
+ * A tile's own calls of larger batches, below those of thousands of samples, may run as one launch too, with the same results as
+ * the launches that they take otherwise; forward calls with bound management keep away from it where recent ones went through more
+ * rounds than it works out together, and so do captured ones, whose replays may.
+ * enable = 0: the tile (alone and in a group) keeps to the launches for larger batches for every batch. */
 int rpu_tile_set_small_calls(rpu_tile_t *tile, int enable);
 
 /* No counterpart in the reference; for the test of the time-out path above only.  spin_limit > 0 shortens the bounded

@@ -6,7 +6,7 @@ import pytest
 import torch
 
 from aihwkit_amd.rpu_base import tiles
-from test_gpu_whole_calls import binds, host_tile, names_of, pair_of
+from test_gpu_whole_calls import NM, binds, host_tile, names_of, pair_of
 
 pytestmark = pytest.mark.gpu
 
@@ -148,3 +148,27 @@ def test_no_rounds_are_left_alone_time_and_again(gpu_device, program):
             assert int(tile.get_bm_rounds(batch).max()) == 2
     assert torch.equal(*results)
     assert took[0] < 1.5 * took[1], took
+
+
+def test_padded_rows(gpu_device):
+    """Rows of inputs and outputs that are slices of wider ones: a group whose tiles run one by one (running averages) takes the launch
+    for the others, and what lies between the rows stays as it was."""
+    rng = np.random.default_rng(12)
+    x_size, d_size, batch = 300, 270, 203
+    host = host_tile(rng, x_size, d_size, 1.7 * 0.2 * np.sqrt(x_size))
+    x = torch.from_numpy(rng.uniform(-1, 1, (batch, x_size + 7)).astype(np.float32)).cuda()
+    results = []
+    for tile in pair_of(host):
+        average = tiles.CudaAnalogTile(host_tile(rng, 64, 32, 12.0, nm=NM.AverageAbsMax))
+        group = tiles.TileGroup([tile, average])
+        wide = torch.full((batch, d_size + 13), 5.0, device="cuda")
+        other = torch.empty(batch, 32, device="cuda")
+        took = []
+        for _ in range(2):
+            _, names = names_of(tile, lambda t: group.forward([x[:, 3:3 + x_size], x[:, :64]], outs=[wide[:, :d_size], other]))
+            took.append(names == ["mvm_whole"])
+        assert bool((wide[:, d_size:] == 5.0).all())
+        results.append((wide, tile.get_bm_rounds(batch), took))
+    assert any(results[0][2]) and not any(results[1][2])
+    assert torch.equal(results[0][0], results[1][0]) and torch.equal(results[0][1], results[1][1])
+    assert int(results[0][1].max()) > 1
